@@ -76,10 +76,13 @@ __global__ __launch_bounds__(SK_WAVES * 64, DUMP ? 2 : 4) void gemm_skinny_kerne
 		a_q_off[i]		= real ? 16 * lane : 16 * (STRIP_ROWS - 1);
 		a_d_off[i]		= real ? 8 * r : 8 * (STRIP_ROWS - 1);
 	}
+	// With an odd number of activation strips the last group of two has only one: its second strip's loads go to the last strip that
+	// exists (its results belong to no row and are dropped at the store).
+	const int last_m_strip = (M + STRIP_ROWS - 1) / STRIP_ROWS - 1;
 	auto issue_a = [&](int g, a_regs& b) {
 #pragma unroll
 		for (int i = 0; i < MS; ++i) {
-			const uint8_t* am = A + macro_offset(mg * MS + i, g, groups);
+			const uint8_t* am = A + macro_offset(min(mg * MS + i, last_m_strip), g, groups);
 #pragma unroll
 			for (int j = 0; j < GROUP_BLOCKS; ++j) {
 				b.q[i][j] = *reinterpret_cast<const v4i*>(am + j * TILE_BYTES + a_q_off[i]);

@@ -55,6 +55,37 @@ def test_gemm_residual(q8, oracle, m, n, k):
     assert np.array_equal(to_host(acc), got)
 
 
+@pytest.mark.parametrize("m,n,k", [(77, 4096, 512), (65, 8192, 256), (225, 4096, 256), (461, 1024, 384)])
+def test_odd_number_of_activation_strips(q8, oracle, m, n, k):
+    # more than 64 rows on a small grid, in an odd number of 32-row strips: the last pair of strips has only one.  The operand ends
+    # where its allocation ends, so that nothing behind it belongs to the process.
+    import ctypes
+
+    import torch
+
+    from nihilus_amd import _lib
+
+    w, x, aq = _inputs(oracle, m, n, k, seed=m + n)
+    wt, at = q8.tile(to_dev(w), n, k), q8.tile(to_dev(aq.reshape(-1)), m, k)
+    lib, stream = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    buf = ctypes.c_void_p()
+    size = (at.numel() + 4095) // 4096 * 4096
+    _lib.check("nh_malloc", lib.nh_malloc(ctypes.byref(buf), size))
+    try:
+        operand = buf.value + (size - at.numel()) // 16 * 16
+        raw = to_host(at)
+        _lib.check("nh_memcpy_h2d", lib.nh_memcpy_h2d(operand, raw.ctypes.data, at.numel(), stream))
+        c = torch.empty((m, n), dtype=torch.float32, device="cuda")
+        _lib.check("nh_q8_0_gemm_tiled", lib.nh_q8_0_gemm_tiled(wt.data_ptr(), operand, c.data_ptr(), m, n, k, stream))
+        _lib.check("nh_stream_sync", lib.nh_stream_sync(stream))
+    finally:
+        lib.nh_free(buf)
+    want = oracle.gemm(w, aq, m, n, k, threads=8) if (k // 32) % 16 == 0 else oracle.gemm(w, aq, m, n, k)
+    got = to_host(c)
+    for i in range(m):
+        assert rel_l2(got[i], want[i]) <= REL_L2_TOL, i
+
+
 def test_mul_mat_residual_every_row_count(q8, oracle):
     # y = mul_mat(W, x) + residual through one entry point whatever M picks underneath: mat-vec, 2- and 3-row form, streaming and
     # tile mat-mat; one fp32 add per element after its sum
