@@ -259,11 +259,11 @@ int nh_q8_0_gemm_tiled_residual(const void* W_tiled, const void* Aq_tiled, const
 /* The prefill FFN's first half as one call: act = quantize_row_q8_0(silu(W_gate . Aq) * (W_up . Aq)), written in the tiled layout as the
  * activation operand of the down projection (rows padded with zero blocks to a multiple of 32).  Stands for the ffn_gate and ffn_up
  * mul_mat -> ffn_silu -> ffn_gate_par (mul) chain of the reference's mega_ffn core in the prompt phase (infra/core_traits.hpp:976-989).
- * Where each matrix alone would take the prefill MFMA kernel it is ONE launch: every workgroup computes the same tiles of both
+ * Where each matrix alone would take the prefill MFMA kernel, and up to 32 rows against matrices of enough rows, it is ONE launch: every workgroup computes the same tiles of both
  * mat-mats against one activation image and applies SiLU * up and the quantizer to them in registers, so the two fp32 [M x N_ff]
  * intermediates are never written and no separate quantize launch runs (nh_q8_0_gate_up_silu_workspace_bytes == 0 for such a
  * shape).  Other shapes run nh_q8_0_gemm_tiled twice into `workspace` and nh_q8_0_silu_mul_quantize_tiled.  Either way the bytes are
- * those of that three-call sequence.  W_gate, W_up: [N_ff x K] tiled; Aq: [M x K] tiled; act: [M x N_ff] tiled; N_ff, K % 128 == 0. */
+ * those of that three-call sequence (where that sums K in the same order; else the fp32 sums differ in their last bits, and single quants with them).  W_gate, W_up: [N_ff x K] tiled; Aq: [M x K] tiled; act: [M x N_ff] tiled; N_ff, K % 128 == 0. */
 int64_t nh_q8_0_gate_up_silu_workspace_bytes(int64_t M, int64_t N_ff, int64_t K);
 int nh_q8_0_gemm_tiled_gate_up_silu(const void* W_gate_tiled, const void* W_up_tiled, const void* Aq_tiled, void* act_tiled_out, void* workspace, int64_t workspace_bytes, int64_t M, int64_t N_ff,
 	int64_t K, void* stream);
@@ -355,7 +355,8 @@ int nh_q8_0_debug_ffn_gate_up(float* gate_out, float* up_out, int64_t N_ff, void
  *       inside (small matrices);
  *   [1] 1 when the activations are quantized by a launch of their own into the workspace (kernels 3, 4, 5);
  *   kernel 1, 6: [2] workgroups per 32-row strip along K, [3] 128-quant groups per wave, [4] row parts per strip;
- *   kernel 3:    [2] 32-row activation strips per workgroup, [3] workgroups per weight strip along K;
+ *   kernel 3:    [2] 32-row activation strips per workgroup, [3] workgroups per weight strip along K (up to 32 rows: the form of
+ *                q8_0_gemm_rows.hip, one strip);
  *   kernel 4, 5: [2] activation strips per wave, [3] K sets of four waves per workgroup, [4] workgroups per tile along K,
  *                [5], [6] the grid (column blocks of 128 weight rows, groups of activation strips);
  *   the rest 0.  The same shape under HIP graph capture may take a form without state between launches (no K split). */

@@ -605,7 +605,7 @@ int64_t nh_q8_0_gate_up_silu_workspace_bytes(int64_t M, int64_t N_ff, int64_t K)
 	if (M < 0 || N_ff < 0 || K < 0 || K % nh::GROUP_K != 0 || N_ff % nh::GROUP_K != 0) {
 		return NH_ERR_SHAPE;
 	}
-	if (M == 0 || N_ff == 0 || nh::plan_gate_up_fused(M, N_ff, K)) {
+	if (M == 0 || N_ff == 0 || nh::gate_up_rows_suits(M, N_ff, K) || nh::plan_gate_up_fused(M, N_ff, K)) {
 		return 0;
 	}
 	return 2 * M * N_ff * 4;
@@ -701,8 +701,8 @@ int nh_q8_0_debug_plan_mul_mat(int64_t M, int64_t N, int64_t K, int32_t* host_pl
 			host_plan[4] = p.gemv_row_parts;
 			break;
 		case nh::MM_GEMM_SKINNY:
-			host_plan[2] = p.gemm.skinny.ms;
-			host_plan[3] = p.gemm.skinny.splits;
+			host_plan[2] = p.gemm.rows_splits > 0 ? 1 : p.gemm.skinny.ms;
+			host_plan[3] = p.gemm.rows_splits > 0 ? p.gemm.rows_splits : p.gemm.skinny.splits;
 			break;
 		case nh::MM_GEMM_TILE_STREAM:
 		case nh::MM_GEMM_TILE:

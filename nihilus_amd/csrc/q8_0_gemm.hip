@@ -657,6 +657,9 @@ hipError_t launch_gemm_gate_up_silu(const void* w_gate, const void* w_up, const 
 	if (M == 0 || n_ff == 0) {
 		return hipSuccess;
 	}
+	if (gate_up_rows_suits(M, n_ff, K)) {
+		return launch_gemm_rows_gate_up(w_gate, w_up, aq, act_out, gate_dbg, up_dbg, M, n_ff, K, s);
+	}
 	gemm_tile_cut cut{};
 	if (plan_gate_up_fused(M, n_ff, K, &cut)) {
 		const uint8_t* wg = static_cast<const uint8_t*>(w_gate);
@@ -710,6 +713,10 @@ hipError_t launch_gemm(const void* W, const void* Aq, float* C, int32_t* sums, i
 		}
 		const gemm_plan plan = plan_gemm(M, N, K); // which kernel and how it cuts the work: q8_0_plan.h
 		if (plan.kernel == MM_GEMM_SKINNY) {
+			// (a launch that hands K parts' sums over by epoch cannot be replayed from a graph: the streaming kernel's counters can)
+			if (plan.rows_splits == 1 || (plan.rows_splits > 1 && !stream_is_capturing(s))) {
+				return launch_gemm_rows(W, Aq, C, residual, M, N, K, plan.rows_splits, s);
+			}
 			return launch_gemm_skinny(W, Aq, C, sums, M, N, K, s, residual);
 		}
 		return launch_gemm_tiled(plan.tile, w, a, C, residual, sums, m, n, k, s, plan.kernel == MM_GEMM_TILE_STREAM);

@@ -1,0 +1,329 @@
+// Batched decode with 2 ... 32 already quantized activation rows: C[m][n] = dot(W row n, Aq row m), and the FFN's gate / up pair with
+// SiLU * up and the quantizer behind it in the same launch, gfx950.
+//
+// What bounds it is HBM and, at these sizes, latency: the weights are read once, so the kernel is the streaming mat-vec again -- a
+// workgroup per (32-row weight strip, K part), its waves splitting the K range, every weight load of a wave's share in flight
+// before anything is waited for, one reduction at the end -- with the int8 MFMA as the inner product.  The weight tile as loaded is
+// the B operand; the activation rows are the A operand.  Eight waves per workgroup and at most 128 registers: two workgroups per
+// CU, so that one streams while the other reduces and leaves.
+//
+// The activations come memory -> LDS without registers, and only the rows that exist: a 128-quant group of R rows (R = 8, 16 or 32) is
+// R / 8 transfers of 1 KiB (lane l fetches the 16 bytes of one (block, k half, row)), so that eight rows cost a quarter of the weight
+// tile's requests; operand rows past R repeat them and their sums are never looked at.
+#include "q8_0_plan.h"
+
+namespace nh {
+
+namespace {
+
+// memory -> LDS, 16 bytes per lane: base (wave-uniform) + lane_off to LDS byte address lds_addr + 16 * lane
+__device__ __forceinline__ void dma_b128(const uint8_t* base, uint32_t lane_off, uint32_t lds_addr) {
+	uint32_t saved_m0;
+	asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0" : "=&s"(saved_m0) : "v"(lane_off), "s"(base), "s"(lds_addr) : "memory");
+}
+
+typedef _Float16 rq_v4h __attribute__((ext_vector_type(4)));
+typedef float rq_v16f __attribute__((ext_vector_type(16)));
+
+// With 8 or 16 rows a lane multiplies the two scales of its 4 or 8 sums itself; with 32 (16 sums per lane) the products come from an
+// f16 MFMA (measured at 32 rows, [14336 x 4096] 14.9 -> 14.4 us, [8192 x 8192] 15.6 -> 14.9; at 16 rows 12.2 -> 12.8).
+template<int R> constexpr bool rows_scale_mfma = R == 32;
+template<int R> constexpr int rows_group_bytes = R / 8 * 1024; // a group's operand rows in LDS: [block][k half][row][16 bytes]
+
+// Groups [gc, gc + CNT) of a wave's K range, against MATS weight strips that share the activations.  CNT is a template parameter so
+// that every wait is a count of younger loads.
+template<int R, int T, int MATS, int CNT>
+__device__ __forceinline__ void rows_chunk_n(const uint8_t* __restrict__ w_strip, const uint8_t* __restrict__ w_strip2, const uint8_t* __restrict__ a_strip, uint8_t* a_tiles, uint8_t* a_scales, int gc,
+	int lane, float (&acc)[MATS][R / 2]) {
+	static_assert(R * T <= 64, "one scale load per lane covers the chunk");
+	const int r	   = lane & 31;
+	const int half = lane >> 5;
+	// ---- 1. the activation rows, requested first: memory -> LDS, then the scales of (group lane / R, row lane % R) through a
+	// register; loads return in issue order, so whoever has the scales has the rows too ----
+	const uint32_t lds_addr = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)a_tiles));
+#pragma unroll
+	for (int c = 0; c < CNT; ++c) {
+		const uint8_t* macro = a_strip + static_cast<int64_t>(gc + c) * MACRO_BYTES;
+#pragma unroll
+		for (int d = 0; d < R / 8; ++d) {
+			// lane l of transfer d: byte 1024 d + 16 l of the group's LDS image = block (64 d + l) / (2 R), half (l / R) % 2, row l % R
+			const int unit = lane; // + 64 d: whole blocks further on
+			const int off  = unit / (2 * R) * TILE_BYTES + (unit / R) % 2 * (TILE_BYTES / 2) + unit % R * 16;
+			dma_b128(macro + d * (64 / (2 * R)) * TILE_BYTES, off, lds_addr + c * rows_group_bytes<R> + d * 1024);
+		}
+	}
+	const int sg = min(lane / R, CNT - 1), sr = lane % R;
+	uint32_t sc_off = sg * MACRO_BYTES + MACRO_D_OFFSET + 8 * sr;
+	asm volatile("" : "+v"(sc_off)::"memory"); // the load below takes its address from behind the transfers: it cannot be issued ahead of them
+	const v2u sc = *reinterpret_cast<const v2u*>(a_strip + static_cast<int64_t>(gc) * MACRO_BYTES + sc_off);
+	asm volatile("" ::: "memory");
+	// ---- 2. every weight byte of the chunk ----
+	v4i q[MATS][T][GROUP_BLOCKS];
+	v2u dd[MATS][T];
+#pragma unroll
+	for (int c = 0; c < CNT; ++c) {
+#pragma unroll
+		for (int k = 0; k < MATS; ++k) {
+			const uint8_t* macro = (k == 0 ? w_strip : w_strip2) + static_cast<int64_t>(gc + c) * MACRO_BYTES;
+#pragma unroll
+			for (int j = 0; j < GROUP_BLOCKS; ++j) {
+				q[k][c][j] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(macro + j * TILE_BYTES + 16 * lane));
+			}
+			dd[k][c] = __builtin_nontemporal_load(reinterpret_cast<const v2u*>(macro + MACRO_D_OFFSET + 8 * r));
+		}
+	}
+	__builtin_amdgcn_sched_barrier(0);
+	// ---- 3. the scales, [block][row]: as fp32, or (32 rows) as the scale MFMA's operand {d in half-word t, zeros} ----
+	if (lane / R < CNT) {
+		if constexpr (rows_scale_mfma<R>) {
+			v2u* out   = reinterpret_cast<v2u*>(a_scales) + (lane / R) * GROUP_BLOCKS * R + sr;
+			out[0]	   = v2u{ sc.x & 0xFFFFu, 0u };
+			out[R]	   = v2u{ sc.x & 0xFFFF0000u, 0u };
+			out[2 * R] = v2u{ 0u, sc.y & 0xFFFFu };
+			out[3 * R] = v2u{ 0u, sc.y & 0xFFFF0000u };
+		} else {
+			float* out = reinterpret_cast<float*>(a_scales) + (lane / R) * GROUP_BLOCKS * R + sr;
+			out[0]	   = half_bits_to_float(static_cast<uint16_t>(sc.x & 0xFFFFu));
+			out[R]	   = half_bits_to_float(static_cast<uint16_t>(sc.x >> 16));
+			out[2 * R] = half_bits_to_float(static_cast<uint16_t>(sc.y & 0xFFFFu));
+			out[3 * R] = half_bits_to_float(static_cast<uint16_t>(sc.y >> 16));
+		}
+	}
+	asm volatile("" ::"v"(sc) : "memory"); // the rows have landed (issue order): no LDS read of them above this point
+	__builtin_amdgcn_wave_barrier();
+	// ---- 4. one MFMA per block and matrix; lane (r, half) gets column r's sums for rows 8 i + 4 half + (0..3) in s[4 i .. 4 i + 3] ----
+#pragma unroll
+	for (int c = 0; c < CNT; ++c) {
+#pragma unroll
+		for (int j = 0; j < GROUP_BLOCKS; ++j) {
+			const v4i a = *reinterpret_cast<const v4i*>(a_tiles + c * rows_group_bytes<R> + j * (32 * R) + half * (16 * R) + (r & (R - 1)) * 16);
+			if constexpr (rows_scale_mfma<R>) {
+				// the products d_x * d_w on the matrix pipe: the weights' four scales as loaded are the operand, the activation's picks
+				// block j's; the k = 4..7 slots (lanes 32..63) hold zeros
+				const v2u dx = reinterpret_cast<const v2u*>(a_scales)[(c * GROUP_BLOCKS + j) * R + (r & (R - 1))];
+#pragma unroll
+				for (int k = 0; k < MATS; ++k) {
+					const v16i zi	 = { 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0 };
+					const rq_v16f zf = { 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0 };
+					const v2u dw	 = half ? v2u{ 0u, 0u } : dd[k][c];
+					const v16i s	 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, q[k][c][j], zi, 0, 0, 0);
+					const rq_v16f p	 = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(rq_v4h, dx), __builtin_bit_cast(rq_v4h, dw), zf, 0, 0, 0);
+#pragma unroll
+					for (int e = 0; e < R / 2; ++e) {
+						acc[k][e] = fmaf(static_cast<float>(s[e]), p[e], acc[k][e]);
+					}
+				}
+				__builtin_amdgcn_sched_barrier(0); // left alone the compiler forms every block's operands at once and spills
+				continue;
+			}
+#pragma unroll
+			for (int k = 0; k < MATS; ++k) {
+				const uint32_t dp = (j & 2) ? dd[k][c].y : dd[k][c].x;
+				const float dw	  = half_bits_to_float(static_cast<uint16_t>((j & 1) ? (dp >> 16) : (dp & 0xFFFFu)));
+				const v16i zi	  = { 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0 };
+				const v16i s	  = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, q[k][c][j], zi, 0, 0, 0);
+#pragma unroll
+				for (int e4 = 0; e4 < R / 8; ++e4) {
+					const float4 dx	   = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(a_scales) + (c * GROUP_BLOCKS + j) * R + 8 * e4 + 4 * half);
+					acc[k][4 * e4 + 0] = fmaf(static_cast<float>(s[4 * e4 + 0]), dw * dx.x, acc[k][4 * e4 + 0]);
+					acc[k][4 * e4 + 1] = fmaf(static_cast<float>(s[4 * e4 + 1]), dw * dx.y, acc[k][4 * e4 + 1]);
+					acc[k][4 * e4 + 2] = fmaf(static_cast<float>(s[4 * e4 + 2]), dw * dx.z, acc[k][4 * e4 + 2]);
+					acc[k][4 * e4 + 3] = fmaf(static_cast<float>(s[4 * e4 + 3]), dw * dx.w, acc[k][4 * e4 + 3]);
+				}
+			}
+		}
+	}
+}
+
+template<int R, int T, int MATS>
+__device__ __forceinline__ void rows_chunk(const uint8_t* __restrict__ w_strip, const uint8_t* __restrict__ w_strip2, const uint8_t* __restrict__ a_strip, uint8_t* a_tiles, uint8_t* a_scales, int gc,
+	int cnt, int lane, float (&acc)[MATS][R / 2]) {
+	switch (cnt) { // wave-uniform; 0: an idle wave (still takes part in the reduction)
+		case 1:
+			rows_chunk_n<R, T, MATS, 1>(w_strip, w_strip2, a_strip, a_tiles, a_scales, gc, lane, acc);
+			break;
+		case 2:
+			if constexpr (T >= 2) {
+				rows_chunk_n<R, T, MATS, 2>(w_strip, w_strip2, a_strip, a_tiles, a_scales, gc, lane, acc);
+			}
+			break;
+		case 3:
+			if constexpr (T >= 3) {
+				rows_chunk_n<R, T, MATS, 3>(w_strip, w_strip2, a_strip, a_tiles, a_scales, gc, lane, acc);
+			}
+			break;
+		case 4:
+			if constexpr (T >= 4) {
+				rows_chunk_n<R, T, MATS, 4>(w_strip, w_strip2, a_strip, a_tiles, a_scales, gc, lane, acc);
+			}
+			break;
+		default:
+			break;
+	}
+}
+
+// The workgroup's LDS: the waves' activation tiles and scales, then (behind a barrier) the partial sums in the same place.
+template<int R, int T, int MATS> struct rows_lds {
+	static constexpr int TILES	= T * rows_group_bytes<R>; // per wave
+	static constexpr int SCALES = T * GROUP_BLOCKS * R * (rows_scale_mfma<R> ? 8 : 4); // per wave
+	static constexpr int STAGE	= ROWS_WAVES * (TILES + SCALES);
+	static constexpr int RED	= MATS * (R / 2) * ROWS_WAVES * 64 * 4;
+	static constexpr int BYTES	= STAGE > RED ? STAGE : RED;
+};
+
+// A workgroup's K part of a strip, all waves' partial sums left in LDS: red[matrix][value][wave][lane]
+template<int R, int T, int MATS>
+__device__ __forceinline__ void rows_strip(const uint8_t* __restrict__ w_strip, const uint8_t* __restrict__ w_strip2, const uint8_t* __restrict__ A, uint8_t* lds, int groups, int split_shift, int split,
+	int lane, int wave) {
+	using L = rows_lds<R, T, MATS>;
+	int g0, g1;
+	wave_k_range(groups, split_shift, split, ROWS_WAVES, wave, g0, g1);
+	uint8_t* a_tiles = lds + wave * L::TILES;
+	uint8_t* a_scales = lds + ROWS_WAVES * L::TILES + wave * L::SCALES;
+	float acc[MATS][R / 2];
+#pragma unroll
+	for (int k = 0; k < MATS; ++k) {
+#pragma unroll
+		for (int e = 0; e < R / 2; ++e) {
+			acc[k][e] = 0.0f;
+		}
+	}
+	for (int gc = g0; gc < g1; gc += T) {
+		rows_chunk<R, T, MATS>(w_strip, w_strip2, A, a_tiles, a_scales, gc, min(T, g1 - gc), lane, acc);
+		__builtin_amdgcn_wave_barrier(); // the next chunk overwrites this wave's tiles
+	}
+	__syncthreads(); // everybody is through with the tiles
+	float* red = reinterpret_cast<float*>(lds);
+#pragma unroll
+	for (int k = 0; k < MATS; ++k) {
+#pragma unroll
+		for (int e = 0; e < R / 2; ++e) {
+			red[((k * (R / 2) + e) * ROWS_WAVES + wave) * 64 + lane] = acc[k][e];
+		}
+	}
+	__syncthreads();
+}
+// output (row m, strip column l) of matrix k: the waves' partial sums in wave order
+template<int R> __device__ __forceinline__ float rows_total(const uint8_t* lds, int k, int m, int l) {
+	const float* red = reinterpret_cast<const float*>(lds);
+	const int e = 4 * (m >> 3) + (m & 3), at = 32 * ((m >> 2) & 1) + l;
+	float total = 0.0f;
+#pragma unroll
+	for (int w = 0; w < ROWS_WAVES; ++w) {
+		total += red[((k * (R / 2) + e) * ROWS_WAVES + w) * 64 + at];
+	}
+	return total;
+}
+
+} // namespace
+
+template<int R, int T>
+__global__ __launch_bounds__(ROWS_WAVES * 64, 4) void gemm_rows_kernel(const uint8_t* __restrict__ W, const uint8_t* __restrict__ A, float* C, const float* residual, uint64_t* __restrict__ tagged,
+	unsigned epoch, int M, int N, int groups, int split_shift) {
+	__shared__ __align__(16) uint8_t lds[rows_lds<R, T, 1>::BYTES];
+	const int tid	= threadIdx.x;
+	const int lane	= tid & 63;
+	const int wave	= __builtin_amdgcn_readfirstlane(tid >> 6);
+	const int strip = static_cast<int>(blockIdx.x >> split_shift);
+	const int split = static_cast<int>(blockIdx.x) & ((1 << split_shift) - 1);
+	rows_strip<R, T, 1>(W + macro_offset(strip, 0, groups), nullptr, A, lds, groups, split_shift, split, lane, wave);
+#pragma unroll
+	for (int o = 0; o < R * STRIP_ROWS; o += ROWS_WAVES * 64) {
+		const int m = (o + tid) >> 5, l = tid & 31;
+		if (m >= M || m >= R) {
+			continue;
+		}
+		const float total = rows_total<R>(lds, 0, m, l);
+		const int n		  = strip * STRIP_ROWS + l;
+		float* cm		  = C + static_cast<int64_t>(m) * N;
+		const float* rm	  = residual ? residual + static_cast<int64_t>(m) * N : nullptr; // may be cm: read before the write, by the same thread
+		if (split_shift == 0) {
+			if (n < N) {
+				cm[n] = rm ? total + rm[n] : total;
+			}
+		} else {
+			split_k_finish(tagged, epoch, strip * R + m, 1 << split_shift, split, l, total, cm, n, N, rm);
+		}
+	}
+}
+
+// The gate and up strips of the same 32 rows against one activation, then silu(g) * u and quantize_row_q8_0: the 32 values of an
+// activation row are one block of the down projection's operand and sit in one half-wave.
+template<int R, int T>
+__global__ __launch_bounds__(ROWS_WAVES * 64, 4) void gemm_rows_gate_up_kernel(const uint8_t* __restrict__ W_gate, const uint8_t* __restrict__ W_up, const uint8_t* __restrict__ A,
+	uint8_t* __restrict__ act_out, float* __restrict__ gate_out, float* __restrict__ up_out, int M, int N, int groups) {
+	__shared__ __align__(16) uint8_t lds[rows_lds<R, T, 2>::BYTES];
+	const int tid	= threadIdx.x;
+	const int lane	= tid & 63;
+	const int wave	= __builtin_amdgcn_readfirstlane(tid >> 6);
+	const int strip = static_cast<int>(blockIdx.x);
+	rows_strip<R, T, 2>(W_gate + macro_offset(strip, 0, groups), W_up + macro_offset(strip, 0, groups), A, lds, groups, 0, 0, lane, wave);
+	uint8_t* macro = act_out + macro_offset(0, strip / GROUP_BLOCKS, N / GROUP_K);
+	const int t	   = strip % GROUP_BLOCKS;
+#pragma unroll
+	for (int o = 0; o < STRIP_ROWS * STRIP_ROWS; o += ROWS_WAVES * 64) {
+		const int m = (o + tid) >> 5, l = tid & 31;
+		float v = 0.0f; // rows past M are the operand's padding: zero blocks
+		if (m < M && m < R) {
+			const float g = rows_total<R>(lds, 0, m, l), u = rows_total<R>(lds, 1, m, l);
+			v = silu_mul(g, u);
+			if (gate_out) {
+				gate_out[static_cast<int64_t>(m) * N + strip * STRIP_ROWS + l] = g;
+				up_out[static_cast<int64_t>(m) * N + strip * STRIP_ROWS + l]   = u;
+			}
+		}
+		float amax = fabsf(v);
+#pragma unroll
+		for (int off = 16; off >= 1; off >>= 1) {
+			amax = fmaxf(amax, __shfl_xor(amax, off));
+		}
+		const float d  = __fdiv_rn(amax, 127.0f);
+		const float id = (amax != 0.0f) ? __fdiv_rn(127.0f, amax) : 0.0f;
+		macro[t * TILE_BYTES + 16 * (m + 32 * (l >> 4)) + (l & 15)] = static_cast<uint8_t>(quantize_value(v, id));
+		if (l == 0) {
+			*reinterpret_cast<uint16_t*>(macro + MACRO_D_OFFSET + 8 * m + 2 * t) = float_to_half_bits(d);
+		}
+	}
+}
+
+// 1 <= M <= 32, K > 0; splits: plan_gemm_rows_splits
+hipError_t launch_gemm_rows(const void* W, const void* Aq, float* C, const float* residual, int64_t M, int64_t N, int64_t K, int splits, hipStream_t s) {
+	const int64_t strips = (N + STRIP_ROWS - 1) / STRIP_ROWS;
+	gemv_scratch sc;
+	if (splits > 1) {
+		const hipError_t e = get_gemv_scratch(&sc, true, s);
+		if (e != hipSuccess) {
+			return e;
+		}
+	}
+	int shift = 0;
+	while ((1 << shift) < splits) {
+		++shift;
+	}
+	const dim3 grid(static_cast<unsigned>(strips * splits)), block(ROWS_WAVES * 64);
+	const uint8_t *w = static_cast<const uint8_t*>(W), *a = static_cast<const uint8_t*>(Aq);
+	const int m = static_cast<int>(M), n = static_cast<int>(N), groups = static_cast<int>(K / GROUP_K);
+	if (M <= 8) {
+		return launch_kernel(KIND_GEMM, gemm_rows_kernel<8, 2>, grid, block, 0, s, w, a, C, residual, sc.tagged, sc.epoch, m, n, groups, shift);
+	}
+	if (M <= 16) {
+		return launch_kernel(KIND_GEMM, gemm_rows_kernel<16, 2>, grid, block, 0, s, w, a, C, residual, sc.tagged, sc.epoch, m, n, groups, shift);
+	}
+	return launch_kernel(KIND_GEMM, gemm_rows_kernel<32, 2>, grid, block, 0, s, w, a, C, residual, sc.tagged, sc.epoch, m, n, groups, shift);
+}
+
+hipError_t launch_gemm_rows_gate_up(const void* w_gate, const void* w_up, const void* aq, void* act_out, float* gate_dbg, float* up_dbg, int64_t M, int64_t n_ff, int64_t K, hipStream_t s) {
+	const dim3 grid(static_cast<unsigned>(n_ff / STRIP_ROWS)), block(ROWS_WAVES * 64);
+	const uint8_t *wg = static_cast<const uint8_t*>(w_gate), *wu = static_cast<const uint8_t*>(w_up), *a = static_cast<const uint8_t*>(aq);
+	uint8_t* out = static_cast<uint8_t*>(act_out);
+	const int m = static_cast<int>(M), n = static_cast<int>(n_ff), groups = static_cast<int>(K / GROUP_K);
+	if (M <= 8) {
+		return launch_kernel(KIND_GEMM, gemm_rows_gate_up_kernel<8, 1>, grid, block, 0, s, wg, wu, a, out, gate_dbg, up_dbg, m, n, groups);
+	}
+	if (M <= 16) {
+		return launch_kernel(KIND_GEMM, gemm_rows_gate_up_kernel<16, 1>, grid, block, 0, s, wg, wu, a, out, gate_dbg, up_dbg, m, n, groups);
+	}
+	return launch_kernel(KIND_GEMM, gemm_rows_gate_up_kernel<32, 1>, grid, block, 0, s, wg, wu, a, out, gate_dbg, up_dbg, m, n, groups);
+}
+
+} // namespace nh

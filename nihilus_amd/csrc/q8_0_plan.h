@@ -84,11 +84,47 @@ inline gemm_skinny_cut plan_gemm_skinny(int64_t M, int64_t N, int64_t K) {
 	return c;
 }
 
+// The same for up to 32 rows (q8_0_gemm_rows.hip): workgroups of ROWS_WAVES waves, a strip's K over `splits` of them.
+constexpr int ROWS_WAVES		= 8;
+constexpr int64_t GEMM_ROWS_MAX = 32;
+inline int gemm_rows_operand(int64_t M) { // operand rows the kernel is instantiated for
+	return M <= 8 ? 8 : M <= 16 ? 16 : 32;
+}
+// Until the launch has a workgroup per CU, while every wave keeps a group.  ([4096 x 4096] at 4 rows 5.7 us with 256 workgroups, 6.0 with
+// 512; [4096 x 14336] 12.6 and 13.3; [1024 x 4096] 4.6 us with 128, 8.0 with 32 (the kernel it replaced there).)
+inline int plan_gemm_rows_splits(int64_t M, int64_t N, int64_t K) {
+	const int64_t strips = (N + STRIP_ROWS - 1) / STRIP_ROWS, groups = K / GROUP_K;
+	int splits			 = 1;
+	while (strips * splits * 2 <= 256 && groups >= 2 * ROWS_WAVES * splits && strips * gemm_rows_operand(M) * splits * 2 <= GEMV_MAX_SPLIT_UNITS) {
+		splits *= 2;
+	}
+	return splits;
+}
+// Measured against the kernels that had these shapes (weights rotated, kernel times, us):
+//   rows                4            16            32
+//   [4096 x 4096]    5.7 /  9.8    6.3 /  9.1    8.7 /  9.4   (streaming kernel with eight waves' operand tiles from L2)
+//   [1024 x 4096]    4.6 /  8.0    5.0 /  8.2    6.9 /  8.8
+//   [4096 x 14336]  12.3 / 18.1   13.2 / 17.9   15.8 / 18.4
+//   [14336 x 4096]  11.0 / 13.9   12.1 / 14.7   14.4 / 15.8
+//   [8192 x 8192]                               14.9 / 17.8   (tile kernel, K over workgroups)
+//   [128256 x 4096] 80.7 / 83.9   86.1 / 88.1  106   / 91     (tile kernel)
+//   [28672 x 8192]  39.1 / 39.4   41.5 / 39.6   47   / 40
+// Every wave takes its own copy of the activations out of L2, M / 32 times the weight bytes, which the tile kernel shares over four
+// strips: that decides large matrices from 17 rows on, and long K from 9.
+inline bool gemm_rows_suits(int64_t M, int64_t N, int64_t K) {
+	const int64_t column_blocks = (N + 127) / 128;
+	if (M > GEMM_ROWS_MAX) {
+		return false;
+	}
+	return column_blocks < GEMM_STREAM_TILE_MIN_COLUMN_BLOCKS || (M <= 16 && K <= 4096);
+}
+
 // A mat-mat on tiled, already quantized operands (nh_q8_0_gemm_tiled, and the second half of nh_q8_0_mul_mat wherever the activations are quantized by a launch of their own).
 struct gemm_plan {
 	int kernel; // MM_GEMM_SKINNY, MM_GEMM_TILE_STREAM or MM_GEMM_TILE (MM_NOTHING for an empty problem)
 	gemm_tile_cut tile; // when a tile kernel runs
 	gemm_skinny_cut skinny; // when the streaming kernel runs
+	int rows_splits; // > 0: it runs as the form for up to 32 rows, with a strip's K over this many workgroups
 };
 inline gemm_plan plan_gemm(int64_t M, int64_t N, int64_t K) {
 	gemm_plan p{};
@@ -112,7 +148,7 @@ inline gemm_plan plan_gemm(int64_t M, int64_t N, int64_t K) {
 		// against 182 / - / 221 us).  Below that the tile kernel's grid leaves CUs idle ([14336 x 4096] at M = 64: 30 us
 		// against 23 us) and the streaming kernel, which can split K over workgroups, stays.
 		if (column_blocks >= GEMM_STREAM_TILE_MIN_COLUMN_BLOCKS) {
-			stream_tile = true;
+			stream_tile = !gemm_rows_suits(M, N, K);
 		} else if (M > 32 ? (column_blocks >= 32 && weights >= (48ll << 20)) : (M >= 16 && column_blocks >= 64 && weights >= (64ll << 20))) {
 			// Between the two, with K long enough to cut: the tile kernel with K over several workgroups per tile as well, so
 			// that 32 to 191 column blocks still put a workgroup on every CU.  Measured against the streaming kernel:
@@ -132,6 +168,9 @@ inline gemm_plan plan_gemm(int64_t M, int64_t N, int64_t K) {
 	} else if (M <= GEMM_SKINNY_MAX_M || tile_workgroups <= 256) {
 		p.kernel = MM_GEMM_SKINNY;
 		p.skinny = plan_gemm_skinny(M, N, K);
+		if (gemm_rows_suits(M, N, K)) {
+			p.rows_splits = plan_gemm_rows_splits(M, N, K);
+		}
 	} else {
 		p.kernel = MM_GEMM_TILE;
 		p.tile	 = plan_gemm_tile(M, N, K, false);
@@ -142,6 +181,16 @@ inline gemm_plan plan_gemm(int64_t M, int64_t N, int64_t K) {
 // The prefill FFN's gate and up mat-mats with SiLU * up and the quantizer behind them: one launch of the tile kernel's fused form
 // where each matrix alone would take the prefill tile kernel and the doubled grid runs one K set per workgroup; otherwise the two
 // mat-mats and the quantizer as launches of their own (through an fp32 workspace).
+//
+// Up to 32 rows the pair runs as the rows kernel's fused form (gate_up_rows_suits), which cuts no strip's K over workgroups: matrices
+// of enough strips only.  Measured against the three launches (us): [2 x 14336 x 4096] at 4 / 16 / 32 rows 20.9 / 22.5 / 26.3 against
+// 31.8 / 33.0 / 36.0; [2 x 28672 x 8192] at 16 rows 79.8 against 84.9.
+inline bool gate_up_rows_suits(int64_t M, int64_t n_ff, int64_t K) {
+	if (M <= 0 || M > GEMM_ROWS_MAX || n_ff <= 0 || K <= 0 || n_ff % GROUP_K != 0 || K % GROUP_K != 0) {
+		return false;
+	}
+	return plan_gemm_rows_splits(M, n_ff, K) == 1 && (M <= 16 || gemm_rows_suits(M, n_ff, K));
+}
 inline bool plan_gate_up_fused(int64_t M, int64_t n_ff, int64_t K, gemm_tile_cut* cut = nullptr) {
 	if (M <= 0 || n_ff <= 0 || K <= 0 || n_ff % GROUP_K != 0 || K % GROUP_K != 0) {
 		return false;

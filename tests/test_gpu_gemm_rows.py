@@ -1,0 +1,77 @@
+"""GPU parity: the streaming MFMA kernel for up to 32 quantized rows, and its fused gate / up form, at the edges of its tiles."""
+import numpy as np
+import pytest
+
+from helpers import REL_L2_TOL, rel_l2, to_dev, to_host
+
+pytestmark = pytest.mark.gpu
+
+
+def _gemm(oracle, w, aq, m, n, k):  # the threaded checker takes block counts that are multiples of 16
+    return oracle.gemm(w, aq, m, n, k, threads=8) if (k // 32) % 16 == 0 else oracle.gemm(w, aq, m, n, k)
+
+
+# rows at either side of the 8-, 16- and 32-row operands; N with a ragged last strip; K of one group, fewer groups than waves, a last chunk
+# of one group, and long enough for two and four workgroups per strip
+@pytest.mark.parametrize("m", [1, 2, 8, 9, 16, 17, 31, 32])
+@pytest.mark.parametrize("n,k", [(33, 128), (100, 128 * 7), (8200, 128 * 17), (257, 128 * 35), (1024, 4096), (4096, 128 * 21)])
+def test_gemm_rows(q8, oracle, m, n, k):
+    w = oracle.fill_weights(m + n, n, k)
+    x = oracle.fill_activations(m + k, m * k).reshape(m, k)
+    aq = oracle.quantize_rows(x)
+    want = _gemm(oracle, w, aq, m, n, k)
+    wt, at = q8.tile(to_dev(w), n, k), q8.quantize_row_q8_0(to_dev(x), tiled=True)
+    got = to_host(q8.gemm(wt, at, m, n, k, tiled=True))
+    for i in range(m):
+        assert rel_l2(got[i], want[i]) <= REL_L2_TOL, i
+    res = oracle.fill_activations(5, m * n).reshape(m, n)
+    acc = to_dev(res.copy())
+    q8.gemm_residual(wt, at, acc, m, n, k, out=acc)
+    assert np.array_equal(to_host(acc), got + res)  # one fp32 add after the sum, in place; the sum itself is bit-stable
+
+
+# [2 x n_ff x k] with a strip's K uncut (>= 129 strips, or a short K), several chunks per wave and ragged rows
+@pytest.mark.parametrize("m", [1, 8, 11, 16, 23, 32])
+@pytest.mark.parametrize("n_ff,k", [(128, 128), (4224, 128 * 9), (8192, 2048)])
+def test_gate_up_rows(q8, oracle, m, n_ff, k):
+    lib = q8._lib.lib()
+    assert lib.nh_q8_0_gate_up_silu_workspace_bytes(m, n_ff, k) == 0
+    wg, wu = oracle.fill_weights(1 + m, n_ff, k), oracle.fill_weights(2 + m, n_ff, k)
+    x = oracle.fill_activations(m + k, m * k).reshape(m, k)
+    aq = oracle.quantize_rows(x)
+    tg, tu = q8.tile(to_dev(wg), n_ff, k), q8.tile(to_dev(wu), n_ff, k)
+    at = q8.quantize_row_q8_0(to_dev(x), tiled=True)
+    act, gate, up = q8.gate_up_silu(tg, tu, at, m, n_ff, k, debug=True)
+    gate, up = to_host(gate), to_host(up)
+    assert rel_l2(gate, _gemm(oracle, wg, aq, m, n_ff, k)) <= REL_L2_TOL
+    assert rel_l2(up, _gemm(oracle, wu, aq, m, n_ff, k)) <= REL_L2_TOL
+    # the quantizer on the launch's own sums, byte for byte, and zero blocks in the rows past M
+    whole = to_host(q8.untile(act, 32, n_ff)).reshape(32, -1)
+    assert np.array_equal(whole[:m], oracle.silu_mul_quantize_rows(gate, up))
+    assert not whole[m:].any()
+    assert np.array_equal(to_host(q8.gate_up_silu(tg, tu, at, m, n_ff, k)), to_host(act))
+
+
+def test_gemm_rows_in_a_graph(q8, oracle):
+    # a captured launch takes no form whose hand-off is tagged by a number that a replay could not renew
+    import torch
+
+    m, n, k = 12, 1024, 4096
+    w = oracle.fill_weights(3, n, k)
+    wt = q8.tile(to_dev(w), n, k)
+    xs = [oracle.fill_activations(20 + i, m * k).reshape(m, k) for i in range(3)]
+    at = q8.quantize_row_q8_0(to_dev(xs[0]), tiled=True)
+    lib, c = q8._lib.lib(), torch.empty((m, n), dtype=torch.float32, device="cuda")
+    q8._lib.check("nh_q8_0_prepare", lib.nh_q8_0_prepare())
+    q8.gemm(wt, at, m, n, k, tiled=True)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        q8._lib.check("gemm", lib.nh_q8_0_gemm_tiled(wt.data_ptr(), at.data_ptr(), c.data_ptr(), m, n, k, torch.cuda.current_stream().cuda_stream))
+    for x in xs:
+        at.copy_(q8.quantize_row_q8_0(to_dev(x), tiled=True))
+        graph.replay()
+        torch.cuda.synchronize()
+        eager = to_host(q8.gemm(wt, at, m, n, k, tiled=True))
+        assert rel_l2(to_host(c), eager) < 2e-6
+        assert rel_l2(eager, oracle.gemm(w, oracle.quantize_rows(x), m, n, k, threads=8)) <= REL_L2_TOL
