@@ -40,6 +40,29 @@ __device__ __forceinline__ int dot16(v4i a, v4i b) {
 	s	  = dot4(a.z, b.z, s);
 	return dot4(a.w, b.w, s);
 }
+typedef float v16f __attribute__((ext_vector_type(16)));
+// One result tile (rows m0 + 8 (e / 4) + 4 half + e % 4, column n0 + r) to C, + R if given.  R may be C: an element is read and written by
+// the same thread.  The sixteen reads are issued together: written one by one behind stores that they may alias, they were a chain of
+// sixteen memory latencies.
+__device__ __forceinline__ void store_tile(const v16f& v, int m0, int n0, int half, int r, float* C, const float* R, int M, int N) {
+	const int n = n0 + r;
+	if (n >= N) {
+		return;
+	}
+	float add[16];
+#pragma unroll
+	for (int e = 0; e < 16; ++e) {
+		const int m = m0 + 8 * (e >> 2) + 4 * half + (e & 3);
+		add[e]		= (R && m < M) ? R[static_cast<int64_t>(m) * N + n] : 0.0f;
+	}
+#pragma unroll
+	for (int e = 0; e < 16; ++e) {
+		const int m = m0 + 8 * (e >> 2) + 4 * half + (e & 3);
+		if (m < M) {
+			C[static_cast<int64_t>(m) * N + n] = R ? v[e] + add[e] : v[e];
+		}
+	}
+}
 // 16 bytes from an address that is only 2-byte aligned (the qs field of a packed 34-byte block).
 __device__ __forceinline__ v4i load16_unaligned(const uint8_t* p) {
 	v4i v;

@@ -220,7 +220,6 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 	constexpr int LDS_BYTES	   = LDS_BASE > FUSE_BYTES ? LDS_BASE : FUSE_BYTES;
 	__shared__ __align__(16) uint8_t lds_raw[LDS_BYTES];
 	typedef _Float16 v4h __attribute__((ext_vector_type(4)));
-	typedef float v16f __attribute__((ext_vector_type(16)));
 
 	const int tid	   = threadIdx.x;
 	const int lane	   = tid & 63;
@@ -428,8 +427,17 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 				}
 			}
 		}
-		__syncthreads();
 		const int n = ns * 32 + (lane & 31);
+		// the residual of this wave's rows, requested together and before the sums are: R may be C, every element is read here and written
+		// below by the same thread
+		float add[TM * PER];
+#pragma unroll
+		for (int j = 0; j < TM * PER; ++j) {
+			const int ee = kr * PER + j % PER;
+			const int m	 = (ms0 + j / PER) * 32 + 8 * (ee >> 2) + 4 * half + (ee & 3);
+			add[j]		 = (R && m < M && n < N) ? R[static_cast<int64_t>(m) * N + n] : 0.0f;
+		}
+		__syncthreads();
 		float mine[TM * PER]; // this wave's rows of the workgroup's tile (SPLIT: of its share of K)
 #pragma unroll
 		for (int q = 0; q < KS; ++q) {
@@ -493,16 +501,11 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 			}
 		}
 #pragma unroll
-		for (int i = 0; i < TM; ++i) {
-#pragma unroll
-			for (int e = 0; e < PER; ++e) {
-				const int ee = kr * PER + e;
-				const int m	 = (ms0 + i) * 32 + 8 * (ee >> 2) + 4 * half + (ee & 3);
-				if (m < M && n < N) {
-					const int64_t at = static_cast<int64_t>(m) * N + n;
-					const float v	 = mine[i * PER + e];
-					C[at]			 = R ? v + R[at] : v; // R may be C: read before the write, by the same thread
-				}
+		for (int j = 0; j < TM * PER; ++j) {
+			const int ee = kr * PER + j % PER;
+			const int m	 = (ms0 + j / PER) * 32 + 8 * (ee >> 2) + 4 * half + (ee & 3);
+			if (m < M && n < N) {
+				C[static_cast<int64_t>(m) * N + n] = R ? mine[j] + add[j] : mine[j];
 			}
 		}
 		return;
@@ -583,17 +586,9 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 		return;
 	}
 	if constexpr (!DUMP) {
-		const int n = ns * 32 + (lane & 31);
 #pragma unroll
 		for (int i = 0; i < TM; ++i) {
-#pragma unroll
-			for (int e = 0; e < 16; ++e) {
-				const int m = (ms0 + i) * 32 + 8 * (e >> 2) + 4 * half + (e & 3);
-				if (m < M && n < N) {
-					const int64_t at = static_cast<int64_t>(m) * N + n;
-					C[at]			 = R ? acc[i][e] + R[at] : acc[i][e]; // R may be C: read before the write, by the same thread
-				}
-			}
+			store_tile(acc[i], (ms0 + i) * 32, ns * 32, half, lane & 31, C, R, M, N);
 		}
 	}
 }
