@@ -3,7 +3,7 @@
 // The reference keeps weights as rows of packed block_q8_0 (common/data_types.hpp:38-44) and copies them
 // into its device arena at load time (infra/model_parser.hpp:151-154).  tile_kernel is that copy with a byte
 // permutation: after it, one 64-lane wavefront reads a 32-row x 32-quant tile as one contiguous KiB.
-// Both directions are lossless; one thread moves four quants.
+// Both directions are lossless.
 #include "q8_0_device.h"
 
 namespace nh {
@@ -19,29 +19,49 @@ __device__ __forceinline__ int64_t tiled_d_offset(int64_t row, int64_t b, int64_
 	return macro_offset(row / STRIP_ROWS, b / GROUP_BLOCKS, groups) + MACRO_D_OFFSET + 8 * (row % STRIP_ROWS) + 2 * (b % GROUP_BLOCKS);
 }
 
-__global__ __launch_bounds__(256) void tile_kernel(const uint8_t* __restrict__ blocks, uint8_t* __restrict__ tiled, int64_t rows, int64_t rows_padded, int64_t K) {
-	const int64_t nb  = K / QK;
-	const int64_t t	  = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-	const int64_t blk = t >> 3;
-	const int j		  = static_cast<int>(t & 7);
-	if (blk >= rows_padded * nb) {
+// One wave per macro-tile (32 rows x 4 blocks), a workgroup's four waves on consecutive groups of a strip.  Lane (row r, half h) takes 68
+// contiguous bytes of its row, blocks 2h and 2h + 1 of the group, and owns what they become: 16 bytes of either half of tiles 2h and
+// 2h + 1 and a dword of the scale table; per store instruction 32 lanes fill 512 contiguous bytes.  It is a copy and bounded by memory:
+// [14336 x 4096] 25 us = 4.9 TB/s read and written, a plain copy on this card 5.1.  A thread per four quants (half-word loads, dword
+// stores, divisions of a 64-bit index) was bounded by its instructions: 57 us, 2.2 TB/s; [1024 x 4096] 8.3 us against 5.7.
+constexpr int TILE_WAVES = 4;
+__global__ __launch_bounds__(TILE_WAVES * 64) void tile_kernel(const uint8_t* __restrict__ blocks, uint8_t* __restrict__ tiled, int64_t rows, int groups, int wg_per_strip) {
+	const int lane	 = threadIdx.x & 63;
+	const int r		 = lane & 31;
+	const int h		 = lane >> 5;
+	const int64_t strip = blockIdx.x / static_cast<unsigned>(wg_per_strip);
+	const int g		 = static_cast<int>(blockIdx.x % static_cast<unsigned>(wg_per_strip)) * TILE_WAVES + static_cast<int>(threadIdx.x >> 6);
+	if (g >= groups) {
 		return;
 	}
-	const int64_t row = blk / nb;
-	const int64_t b	  = blk - row * nb;
-	uint32_t q		  = 0;
-	uint16_t d		  = 0;
+	const int64_t row = strip * STRIP_ROWS + r;
+	uint32_t v[17]; // d0 q0[0..31] d1 q1[0..31], little-endian
+#pragma unroll
+	for (int i = 0; i < 17; ++i) {
+		v[i] = 0u;
+	}
 	if (row < rows) {
-		const uint8_t* src = blocks + blk * BLOCK_BYTES;
-		q				   = static_cast<uint32_t>(load_u16(src + 2 + 4 * j)) | (static_cast<uint32_t>(load_u16(src + 4 + 4 * j)) << 16);
-		d				   = load_u16(src);
+		const uint32_t* src = reinterpret_cast<const uint32_t*>(blocks + (row * groups + g) * (GROUP_BLOCKS * BLOCK_BYTES) + h * (2 * BLOCK_BYTES)); // 4-byte aligned: 136 and 68 are multiples of 4
+		__builtin_memcpy(v, src, sizeof(v));
 	}
-	*reinterpret_cast<uint32_t*>(tiled + tiled_q_offset(row, b, j, K / GROUP_K)) = q;
-	if (j == 0) {
-		*reinterpret_cast<uint16_t*>(tiled + tiled_d_offset(row, b, K / GROUP_K)) = d;
+	uint8_t* macro = tiled + macro_offset(strip, g, groups);
+	// quants of block 2h start at byte 2 (every dword straddles two of v), of block 2h + 1 at byte 36 = v[9]
+#pragma unroll
+	for (int part = 0; part < 2; ++part) {
+		v4i a, b;
+#pragma unroll
+		for (int i = 0; i < 4; ++i) {
+			a[i] = static_cast<int>(__builtin_amdgcn_alignbyte(v[4 * part + i + 1], v[4 * part + i], 2));
+			b[i] = static_cast<int>(v[9 + 4 * part + i]);
+		}
+		*reinterpret_cast<v4i*>(macro + (2 * h) * TILE_BYTES + 16 * (r + 32 * part))	 = a;
+		*reinterpret_cast<v4i*>(macro + (2 * h + 1) * TILE_BYTES + 16 * (r + 32 * part)) = b;
 	}
+	// the two scales: the low half of v[0], the high half of v[8]
+	*reinterpret_cast<uint32_t*>(macro + MACRO_D_OFFSET + 8 * r + 4 * h) = (v[0] & 0xFFFFu) | (v[8] & 0xFFFF0000u);
 }
 
+// one thread moves four quants
 __global__ __launch_bounds__(256) void untile_kernel(const uint8_t* __restrict__ tiled, uint8_t* __restrict__ blocks, int64_t rows, int64_t K) {
 	const int64_t nb  = K / QK;
 	const int64_t t	  = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -62,12 +82,13 @@ __global__ __launch_bounds__(256) void untile_kernel(const uint8_t* __restrict__
 }
 
 hipError_t launch_tile(const void* blocks, void* tiled, int64_t rows, int64_t K, hipStream_t s) {
-	const int64_t rows_padded = (rows + STRIP_ROWS - 1) / STRIP_ROWS * STRIP_ROWS;
-	const int64_t threads	  = rows_padded * (K / QK) * 8;
-	if (threads == 0) {
+	const int64_t strips = (rows + STRIP_ROWS - 1) / STRIP_ROWS;
+	const int groups	 = static_cast<int>(K / GROUP_K);
+	if (strips == 0 || groups == 0) {
 		return hipSuccess;
 	}
-	tile_kernel<<<dim3(static_cast<unsigned>((threads + 255) / 256)), dim3(256), 0, s>>>(static_cast<const uint8_t*>(blocks), static_cast<uint8_t*>(tiled), rows, rows_padded, K);
+	const int wg_per_strip = (groups + TILE_WAVES - 1) / TILE_WAVES;
+	tile_kernel<<<dim3(static_cast<unsigned>(strips * wg_per_strip)), dim3(TILE_WAVES * 64), 0, s>>>(static_cast<const uint8_t*>(blocks), static_cast<uint8_t*>(tiled), rows, groups, wg_per_strip);
 	return hipGetLastError();
 }
 

@@ -37,3 +37,18 @@ def test_device_generator_matches_cpu(q8, oracle):
         assert np.array_equal(got, oracle.fill_weights(seed, n, k, first_block=first))
         x = to_host(q8.fill_activations(seed, 4097))
         assert np.array_equal(x, oracle.fill_activations(seed, 4097))
+
+
+@pytest.mark.parametrize("rows", [1, 31, 32, 65])
+@pytest.mark.parametrize("groups", [1, 3, 4, 5, 9])  # a wave takes a group, a workgroup four: full, short and single
+def test_tile_is_the_documented_permutation(q8, rows, groups):
+    rng = np.random.default_rng(rows * 16 + groups)
+    w = random_blocks(rng, rows, groups * 128)
+    strips = (rows + 31) // 32
+    padded = np.zeros((strips * 32, groups, 4, 34), dtype=np.uint8)  # rows past the last are zero blocks
+    padded[:rows] = w.reshape(rows, groups, 4, 34)
+    by_strip = padded.reshape(strips, 32, groups, 4, 34).transpose(0, 2, 3, 1, 4)  # strip, group, tile, row, bytes
+    quants = by_strip[..., 2:].reshape(strips, groups, 4, 32, 2, 16).transpose(0, 1, 2, 4, 3, 5).reshape(strips, groups, 4096)
+    scales = by_strip[..., :2].transpose(0, 1, 3, 2, 4).reshape(strips, groups, 256)
+    want = np.concatenate([quants, scales], axis=2).reshape(-1)
+    assert np.array_equal(to_host(q8.tile(to_dev(w), rows, groups * 128)), want)
