@@ -293,6 +293,21 @@ inline hipError_t query_stream_any_capture_mode(hipStream_t s) {
 	return q;
 }
 
+// hipErrorNotReady when `prev` still has work in flight; anything else (a destroyed stream, a capturing one) counts as drained
+inline hipError_t stream_drained(hipStream_t prev) {
+	if (stream_is_capturing(prev)) {
+		return hipSuccess; // must not be queried; its launches take forms that keep no state in the scratch
+	}
+	const hipError_t q = query_stream_any_capture_mode(prev);
+	if (q == hipErrorNotReady) {
+		return q;
+	}
+	if (q != hipSuccess) {
+		(void)hipGetLastError();
+	}
+	return hipSuccess;
+}
+
 // When timing is on for `kind` and the event pool has room, hands out an event pair for the next launch.
 bool profile_next(int kind, hipEvent_t* start, hipEvent_t* stop);
 
@@ -379,6 +394,8 @@ hipError_t launch_gemm_gate_up_silu(const void* w_gate, const void* w_up, const 
 constexpr int64_t GEMM_SKINNY_MAX_M = 64;
 // Tiled operands, 1 <= M <= 32: the streaming mat-vec's shape with the int8 MFMA as inner product (q8_0_gemm_rows.hip), K of a strip over
 // `splits` workgroups, and the same for a gate / up pair with SiLU * up and the quantizer behind it (n_ff % 128 == 0).
+// hipErrorNotReady: another stream's launch may still be handing sums over (the streaming kernel of q8_0_gemm_skinny.hip takes the shape too).
+hipError_t prepare_gemm_rows_scratch();
 hipError_t launch_gemm_rows(const void* W, const void* Aq, float* C, const float* residual, int64_t M, int64_t N, int64_t K, int splits, hipStream_t s);
 hipError_t launch_gemm_rows_gate_up(const void* w_gate, const void* w_up, const void* aq, void* act_out, float* gate_dbg, float* up_dbg, int64_t M, int64_t n_ff, int64_t K, hipStream_t s);
 // Make this device's K-split scratch buffers now (otherwise: on the first launch that needs one).

@@ -708,9 +708,13 @@ hipError_t launch_gemm(const void* W, const void* Aq, float* C, int32_t* sums, i
 		}
 		const gemm_plan plan = plan_gemm(M, N, K); // which kernel and how it cuts the work: q8_0_plan.h
 		if (plan.kernel == MM_GEMM_SKINNY) {
-			// (a launch that hands K parts' sums over by epoch cannot be replayed from a graph: the streaming kernel's counters can)
+			// (a launch that hands K parts' sums over by epoch cannot be replayed from a graph, and is refused while another stream's is
+			// under way: the streaming kernel, with counters or without a K split, takes those calls)
 			if (plan.rows_splits == 1 || (plan.rows_splits > 1 && !stream_is_capturing(s))) {
-				return launch_gemm_rows(W, Aq, C, residual, M, N, K, plan.rows_splits, s);
+				const hipError_t e = launch_gemm_rows(W, Aq, C, residual, M, N, K, plan.rows_splits, s);
+				if (e != hipErrorNotReady || plan.rows_splits == 1) {
+					return e;
+				}
 			}
 			return launch_gemm_skinny(W, Aq, C, sums, M, N, K, s, residual);
 		}

@@ -12,6 +12,8 @@
 // tile's requests; operand rows past R repeat them and their sums are never looked at.
 #include "q8_0_plan.h"
 
+#include <mutex>
+
 namespace nh {
 
 namespace {
@@ -286,12 +288,71 @@ __global__ __launch_bounds__(ROWS_WAVES * 64, 4) void gemm_rows_gate_up_kernel(c
 	}
 }
 
+// The tagged partial sums of a K split: this kernel's own (shared with the mat-vecs' scratch, a mat-mat on one stream and a mat-vec on
+// another refused each other), one allocation per device on first use, in two parts: the null stream's, which may not be queried while
+// some other stream is being captured and so never shares, and one that serves the other streams one at a time.
+namespace {
+	struct rows_scratch {
+		uint64_t* tagged = nullptr; // [GEMV_MAX_SPLIT_UNITS][32] {epoch, partial sum}
+		unsigned epoch	 = 0;
+		hipStream_t user = nullptr; // stream of the last launch that used this part
+	};
+	constexpr size_t ROWS_SCRATCH_WORDS = static_cast<size_t>(GEMV_MAX_SPLIT_UNITS) * STRIP_ROWS;
+	hipError_t get_rows_scratch(rows_scratch* out, bool launching, hipStream_t s) {
+		static std::mutex lock;
+		static rows_scratch per_device[64][2];
+		int dev		 = 0;
+		hipError_t e = hipGetDevice(&dev);
+		if (e != hipSuccess) {
+			return e;
+		}
+		if (dev < 0 || dev >= 64) {
+			return hipErrorInvalidDevice;
+		}
+		std::lock_guard<std::mutex> g(lock);
+		if (!per_device[dev][0].tagged) {
+			void* p = nullptr;
+			e		= hipMalloc(&p, 2 * ROWS_SCRATCH_WORDS * 8);
+			if (e != hipSuccess) {
+				return e;
+			}
+			e = hipMemset(p, 0, 2 * ROWS_SCRATCH_WORDS * 8); // synchronous, once: every tag starts at epoch 0, which no launch uses
+			if (e != hipSuccess) {
+				(void)hipFree(p);
+				return e;
+			}
+			per_device[dev][0].tagged = static_cast<uint64_t*>(p);
+			per_device[dev][1].tagged = static_cast<uint64_t*>(p) + ROWS_SCRATCH_WORDS;
+		}
+		rows_scratch& sc = per_device[dev][s != nullptr];
+		if (launching) {
+			if (sc.user != s && sc.user != nullptr) {
+				e = stream_drained(sc.user);
+				if (e != hipSuccess) {
+					return e;
+				}
+			}
+			sc.user = s;
+			if (++sc.epoch == 0) {
+				++sc.epoch;
+			}
+		}
+		*out = sc;
+		return hipSuccess;
+	}
+} // namespace
+
+hipError_t prepare_gemm_rows_scratch() {
+	rows_scratch sc;
+	return get_rows_scratch(&sc, false, nullptr);
+}
+
 // 1 <= M <= 32, K > 0; splits: plan_gemm_rows_splits
 hipError_t launch_gemm_rows(const void* W, const void* Aq, float* C, const float* residual, int64_t M, int64_t N, int64_t K, int splits, hipStream_t s) {
 	const int64_t strips = (N + STRIP_ROWS - 1) / STRIP_ROWS;
-	gemv_scratch sc;
+	rows_scratch sc;
 	if (splits > 1) {
-		const hipError_t e = get_gemv_scratch(&sc, true, s);
+		const hipError_t e = get_rows_scratch(&sc, true, s);
 		if (e != hipSuccess) {
 			return e;
 		}

@@ -311,7 +311,8 @@ hipError_t acquire_gemm_split_scratch(float** partials, unsigned** counters, hip
 
 hipError_t prepare_gemm_scratch() {
 	skinny_scratch sc;
-	return get_skinny_scratch(&sc);
+	const hipError_t e = get_skinny_scratch(&sc);
+	return e != hipSuccess ? e : prepare_gemm_rows_scratch();
 }
 
 template<int MS> static hipError_t launch_skinny_t(int splits, const uint8_t* w, const uint8_t* a, float* C, const float* R, int32_t* sums, int m, int n, int groups, hipStream_t s) {

@@ -225,21 +225,6 @@ namespace {
 	std::mutex scratch_lock;
 	scratch_state scratch_per_device[64];
 	int published_spin_limit = PUBLISHED_SPIN_LIMIT;
-
-	// hipErrorNotReady when `prev` still has work in flight; anything else (a destroyed stream, a capturing one) counts as drained
-	hipError_t stream_drained(hipStream_t prev) {
-		if (stream_is_capturing(prev)) {
-			return hipSuccess; // must not be queried; its launches take forms that keep no state in the scratch
-		}
-		const hipError_t q = query_stream_any_capture_mode(prev);
-		if (q == hipErrorNotReady) {
-			return q;
-		}
-		if (q != hipSuccess) {
-			(void)hipGetLastError();
-		}
-		return hipSuccess;
-	}
 } // namespace
 
 hipError_t get_gemv_scratch(gemv_scratch* out, bool next_epoch, hipStream_t s) {
