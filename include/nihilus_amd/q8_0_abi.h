@@ -259,7 +259,7 @@ int nh_q8_0_gemm_tiled_residual(const void* W_tiled, const void* Aq_tiled, const
 /* The prefill FFN's first half as one call: act = quantize_row_q8_0(silu(W_gate . Aq) * (W_up . Aq)), written in the tiled layout as the
  * activation operand of the down projection (rows padded with zero blocks to a multiple of 32).  Stands for the ffn_gate and ffn_up
  * mul_mat -> ffn_silu -> ffn_gate_par (mul) chain of the reference's mega_ffn core in the prompt phase (infra/core_traits.hpp:976-989).
- * Where each matrix alone would take the prefill MFMA kernel, and up to 32 rows against matrices of enough rows, it is ONE launch: every workgroup computes the same tiles of both
+ * Where the two matrices have rows enough to occupy the GPU it is ONE launch: every workgroup computes the same tiles of both
  * mat-mats against one activation image and applies SiLU * up and the quantizer to them in registers, so the two fp32 [M x N_ff]
  * intermediates are never written and no separate quantize launch runs (nh_q8_0_gate_up_silu_workspace_bytes == 0 for such a
  * shape).  Other shapes run nh_q8_0_gemm_tiled twice into `workspace` and nh_q8_0_silu_mul_quantize_tiled.  Either way the bytes are

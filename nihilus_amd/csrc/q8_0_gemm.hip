@@ -200,7 +200,8 @@ template<typename T, bool NT> __device__ __forceinline__ T load_sv(gptr_u8 p, ui
 // kernel's.  Behind it the up waves hand their tiles to the gate waves through LDS, and those apply silu(g) * u and quantize: a
 // 32-value block of the down projection's activation is one activation row against one 32-row weight strip, i.e. one (register,
 // half-wave) of an MFMA result tile -- 32 lanes hold it, its maximum is five cross-lane steps, and the quants go out in the tiled
-// operand layout (through an LDS image of the tile, one 16-byte store per lane).  The two fp32 [M x N] intermediates are never
+// operand layout (through an LDS image of the tile, one 16-byte store per lane).  With several K sets the sets' tiles are summed first, as
+// in the plain kernel, and each set finishes the rows it has summed.  The two fp32 [M x N] intermediates are never
 // written, the activation is read once for both matrices, and two launches (the second mat-mat and the SiLU * up quantizer) are gone.
 // The arithmetic per value is that of the stand-alone kernels (same fp32 sums, silu_mul, quantize_row_q8_0), so the bytes are theirs.
 // C / C2 (optional, inspection): the fp32 gate / up tiles as the launch computed them.
@@ -208,7 +209,7 @@ template<int TM, bool DUMP, int KS, bool STREAM, bool SPLIT, bool GATE_UP>
 __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, const uint8_t* __restrict__ A, float* C, const float* R, int32_t* __restrict__ sums, int M, int N, int groups,
 	float* __restrict__ partials, unsigned* __restrict__ counters, const uint8_t* __restrict__ W2, uint8_t* __restrict__ act_out, float* __restrict__ C2) {
 	static_assert(!SPLIT || (KS > 1 && !DUMP), "K over several workgroups continues the K sets' sum");
-	static_assert(!GATE_UP || (KS == 1 && !DUMP && !SPLIT && !STREAM), "the fused gate/up form runs one K set per workgroup");
+	static_assert(!GATE_UP || (!DUMP && !SPLIT), "the fused gate/up form leaves a workgroup's tile quantized");
 	constexpr int DATA_BYTES  = TM * MACRO_BYTES;
 	constexpr int STAGE_BYTES = DATA_BYTES + 16;
 	constexpr int SET_BYTES	   = 2 * STAGE_BYTES + 256; // + 256: where waves that copy no scale table put theirs
@@ -403,12 +404,13 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 			trip(g + 1, wb, wa);
 		}
 	}
+	constexpr int PER = 16 / KS; // values of a lane's 16 per strip that a K set finishes: registers PER * kr .. PER * kr + PER - 1
+	float mine[TM * PER]; // this wave's share of the workgroup's tile (SPLIT: of its part of K)
 	if constexpr (KS > 1 && !DUMP) {
 		// The K sets' tiles are summed by all of them at once: set q keeps PER = 16 / KS of a lane's 16 values per strip (with
 		// four sets: rows 8q .. 8q+7 of every 32-row strip), parks the other sets' shares in LDS, and after one barrier adds what
 		// the others parked for it, in set order (s0 + s1 + s2 + s3 whatever q is, so the result does not depend on who adds),
 		// and stores its own rows.  One set adding the others' whole tiles in turn took 12 % of the launch at M=512, N=K=4096.
-		constexpr int PER = 16 / KS;
 		__syncthreads(); // every set is through with its stages
 		float* park = reinterpret_cast<float*>(lds_raw);
 		auto slot	= [&](int q, int src) { // where set src parks its share of part q (src != q), this wave's strip
@@ -435,10 +437,9 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 		for (int j = 0; j < TM * PER; ++j) {
 			const int ee = kr * PER + j % PER;
 			const int m	 = (ms0 + j / PER) * 32 + 8 * (ee >> 2) + 4 * half + (ee & 3);
-			add[j]		 = (R && m < M && n < N) ? R[static_cast<int64_t>(m) * N + n] : 0.0f;
+			add[j]		 = (!GATE_UP && R && m < M && n < N) ? R[static_cast<int64_t>(m) * N + n] : 0.0f;
 		}
 		__syncthreads();
-		float mine[TM * PER]; // this wave's rows of the workgroup's tile (SPLIT: of its share of K)
 #pragma unroll
 		for (int q = 0; q < KS; ++q) {
 			if (q == kr) {
@@ -500,43 +501,49 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 				}
 			}
 		}
+		if constexpr (!GATE_UP) {
+#pragma unroll
+			for (int j = 0; j < TM * PER; ++j) {
+				const int ee = kr * PER + j % PER;
+				const int m	 = (ms0 + j / PER) * 32 + 8 * (ee >> 2) + 4 * half + (ee & 3);
+				if (m < M && n < N) {
+					C[static_cast<int64_t>(m) * N + n] = R ? mine[j] + add[j] : mine[j];
+				}
+			}
+			return;
+		}
+		__syncthreads(); // the sets have read each other's sums: the exchange below goes to the same place
+	} else {
 #pragma unroll
 		for (int j = 0; j < TM * PER; ++j) {
-			const int ee = kr * PER + j % PER;
-			const int m	 = (ms0 + j / PER) * 32 + 8 * (ee >> 2) + 4 * half + (ee & 3);
-			if (m < M && n < N) {
-				C[static_cast<int64_t>(m) * N + n] = R ? mine[j] + add[j] : mine[j];
-			}
+			mine[j] = acc[j / PER][j % PER];
 		}
-		return;
 	}
 	if constexpr (GATE_UP) {
-		// Every wave is through with the stages (the last trip ended in a barrier).  The gate wave and the up wave of a strip share
-		// the work behind the loop: registers 0..7 of every tile are finished by the gate wave, 8..15 by the up wave, each handing
-		// the other the half it does not finish (the exp and the divides of SiLU and of the quantizer are a quarter of the loop's
-		// VALU work; on two of the four waves alone they cost the launch 6 %).
+		// Every wave is through with the stages (the last trip ended in a barrier).  The gate wave and the up wave of a strip (and K set)
+		// share the work behind the loop: the first half of their PER registers of every tile is finished by the gate wave, the second by
+		// the up wave, each handing the other the half it does not finish (the exp and the divides of SiLU and of the quantizer are a
+		// quarter of the loop's VALU work; on the gate waves alone they cost the launch 6 %).
 		const int pair	 = wave & 1;
 		const bool is_up = wave >= 2;
 		float* xch		 = reinterpret_cast<float*>(lds_raw); // [pair][TM][16][64]: slot (i, e) holds the value of the wave that does not finish it
 #pragma unroll
 		for (int i = 0; i < TM; ++i) {
 #pragma unroll
-			for (int e = 0; e < 8; ++e) {
-				const int give						  = is_up ? e : e + 8;
-				xch[((pair * TM + i) * 16 + give) * 64 + lane] = acc[i][give];
+			for (int x = 0; x < PER / 2; ++x) {
+				const int give															   = kr * PER + (is_up ? x : x + PER / 2);
+				xch[((pair * TM + i) * 16 + give) * 64 + lane] = is_up ? mine[i * PER + x] : mine[i * PER + x + PER / 2];
 			}
 		}
 		float* dbg = is_up ? C2 : C; // inspection copies of the fp32 tiles
 		if (dbg) {
 			const int n = ns * 32 + (lane & 31);
 #pragma unroll
-			for (int i = 0; i < TM; ++i) {
-#pragma unroll
-				for (int e = 0; e < 16; ++e) {
-					const int m = (ms0 + i) * 32 + 8 * (e >> 2) + 4 * half + (e & 3);
-					if (m < M && n < N) {
-						dbg[static_cast<int64_t>(m) * N + n] = acc[i][e];
-					}
+			for (int j = 0; j < TM * PER; ++j) {
+				const int e = kr * PER + j % PER;
+				const int m = (ms0 + j / PER) * 32 + 8 * (e >> 2) + 4 * half + (e & 3);
+				if (m < M && n < N) {
+					dbg[static_cast<int64_t>(m) * N + n] = mine[j];
 				}
 			}
 		}
@@ -548,10 +555,11 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 			uint8_t* tile	 = image + i * (TILE_BYTES + 64);
 			uint16_t* scales = reinterpret_cast<uint16_t*>(tile + TILE_BYTES);
 #pragma unroll
-			for (int e8 = 0; e8 < 8; ++e8) {
-				const int e		  = is_up ? e8 + 8 : e8;
+			for (int x = 0; x < PER / 2; ++x) {
+				const int e		  = kr * PER + (is_up ? x + PER / 2 : x);
+				const float own	  = is_up ? mine[i * PER + x + PER / 2] : mine[i * PER + x];
 				const float other = xch[((pair * TM + i) * 16 + e) * 64 + lane];
-				const float v	  = is_up ? silu_mul(other, acc[i][e]) : silu_mul(acc[i][e], other);
+				const float v	  = is_up ? silu_mul(other, own) : silu_mul(own, other);
 				// the block = this register over the 32 lanes of the half-wave: quantize_row_q8_0 on it
 				float amax = fabsf(v);
 #pragma unroll
@@ -567,10 +575,10 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 				}
 			}
 		}
-		__syncthreads(); // both waves of a pair have filled its images
-		// tile i of the pair goes out through the gate wave (even i) or the up wave (odd i): one 16-byte store per lane
+		__syncthreads(); // the waves of a pair have filled its images
+		// tile i of the pair goes out through the first K set's gate wave (even i) or up wave (odd i): one 16-byte store per lane
 		const int out_groups = N / GROUP_K; // the activation is [M x N]: N / 128 groups per strip, this strip's block is ns
-		if (ns < n_strips) {
+		if (ns < n_strips && kr == 0) {
 #pragma unroll
 			for (int i = 0; i < TM; ++i) {
 				if ((i & 1) == (is_up ? 1 : 0) && ms0 + i < m_strips) {
@@ -600,10 +608,10 @@ __global__ __launch_bounds__(256 * KS, 4) void gemm_tiled_kernel(const uint8_t* 
 }
 
 // the fused gate / up form (GATE_UP above): N = rows of each of the two matrices; gate_out / up_out optional
-template<int TM>
-__global__ __launch_bounds__(256, 4) void gemm_gate_up_kernel(const uint8_t* __restrict__ W_gate, const uint8_t* __restrict__ W_up, const uint8_t* __restrict__ A, uint8_t* __restrict__ act_out,
+template<int TM, int KS, bool STREAM>
+__global__ __launch_bounds__(256 * KS, 4) void gemm_gate_up_kernel(const uint8_t* __restrict__ W_gate, const uint8_t* __restrict__ W_up, const uint8_t* __restrict__ A, uint8_t* __restrict__ act_out,
 	float* __restrict__ gate_out, float* __restrict__ up_out, int M, int N, int groups) {
-	gemm_tiled_body<TM, false, 1, false, false, true>(W_gate, A, gate_out, nullptr, nullptr, M, N, groups, nullptr, nullptr, W_up, act_out, up_out);
+	gemm_tiled_body<TM, false, KS, STREAM, false, true>(W_gate, A, gate_out, nullptr, nullptr, M, N, groups, nullptr, nullptr, W_up, act_out, up_out);
 }
 
 // Executes a cut made by plan_gemm_tile (q8_0_plan.h): TM activation strips per wave, KS sets of four waves per workgroup,
@@ -663,10 +671,14 @@ hipError_t launch_gemm_gate_up_silu(const void* w_gate, const void* w_up, const 
 		uint8_t* out	  = static_cast<uint8_t*>(act_out);
 		const int m = static_cast<int>(M), n = static_cast<int>(n_ff), groups = static_cast<int>(K / GROUP_K);
 		const dim3 grid(cut.grid_x, cut.grid_y);
-		if (cut.tm == 2) {
-			return launch_kernel(KIND_GEMM, gemm_gate_up_kernel<2>, grid, dim3(256), 0, s, wg, wu, a, out, gate_dbg, up_dbg, m, n, groups);
+		auto launch = [&](auto kernel, int ks) { return launch_kernel(KIND_GEMM, kernel, grid, dim3(256 * ks), 0, s, wg, wu, a, out, gate_dbg, up_dbg, m, n, groups); };
+		if (cut.tm == 1) { // 17 to 32 rows on matrices of 192 column blocks and more (the rows kernel has the others): four K sets are never cut
+			return cut.ks == 2 ? launch(gemm_gate_up_kernel<1, 2, true>, 2) : launch(gemm_gate_up_kernel<1, 1, true>, 1);
 		}
-		return launch_kernel(KIND_GEMM, gemm_gate_up_kernel<1>, grid, dim3(256), 0, s, wg, wu, a, out, gate_dbg, up_dbg, m, n, groups);
+		if (cut.grid_y == 1) { // up to 64 rows: the weights are read once
+			return cut.ks == 4 ? launch(gemm_gate_up_kernel<2, 4, true>, 4) : cut.ks == 2 ? launch(gemm_gate_up_kernel<2, 2, true>, 2) : launch(gemm_gate_up_kernel<2, 1, true>, 1);
+		}
+		return cut.ks == 4 ? launch(gemm_gate_up_kernel<2, 4, false>, 4) : cut.ks == 2 ? launch(gemm_gate_up_kernel<2, 2, false>, 2) : launch(gemm_gate_up_kernel<2, 1, false>, 1);
 	}
 	float* gate = gate_dbg ? gate_dbg : workspace;
 	float* up	= up_dbg ? up_dbg : workspace + M * n_ff;

@@ -178,9 +178,8 @@ inline gemm_plan plan_gemm(int64_t M, int64_t N, int64_t K) {
 	return p;
 }
 
-// The prefill FFN's gate and up mat-mats with SiLU * up and the quantizer behind them: one launch of the tile kernel's fused form
-// where each matrix alone would take the prefill tile kernel and the doubled grid runs one K set per workgroup; otherwise the two
-// mat-mats and the quantizer as launches of their own (through an fp32 workspace).
+// The prefill FFN's gate and up mat-mats with SiLU * up and the quantizer behind them: one launch of the tile kernel's fused form, or the
+// two mat-mats and the quantizer as launches of their own (through an fp32 workspace).
 //
 // Up to 32 rows the pair runs as the rows kernel's fused form (gate_up_rows_suits), which cuts no strip's K over workgroups: matrices
 // of enough strips only.  Measured against the three launches (us): [2 x 14336 x 4096] at 4 / 16 / 32 rows 20.9 / 22.5 / 26.3 against
@@ -191,15 +190,22 @@ inline bool gate_up_rows_suits(int64_t M, int64_t n_ff, int64_t K) {
 	}
 	return plan_gemm_rows_splits(M, n_ff, K) == 1 && (M <= 16 || gemm_rows_suits(M, n_ff, K));
 }
+// The tile kernel's fused form, K sets included, wherever its grid has the chip's SIMDs two waves each, or about one where the matrices are
+// small enough that the launches saved count for more than idle CUs.  Whole calls, us, fused / three launches:
+//   rows      [2 x 14336 x 4096]   [2 x 28672 x 8192]   [2 x 11008 x 4096]   [2 x 8192 x 8192]   [2 x 5632 x 2048]   [2 x 4096 x 1024]
+//   64        30.8 / 43.1          105 / 114            26.6 / 43.2                              16.2 / 19.5
+//   117, 128  51.7 / 57.0                                                    54.5 / 82.5
+//   256                                                                                                              11.6 / 20.8
+// and below two waves per SIMD: [2 x 5632 x 4096] at 40 rows (1408 waves, 46 Mi weights) 24.7 / 29.0, but [2 x 6144 x 8192] at 64 rows
+// (1536 waves, 101 Mi) 42.0 / 39.4.
+constexpr int64_t GATE_UP_MIN_WAVES = 2048, GATE_UP_MIN_WAVES_SMALL = 1100, GATE_UP_SMALL_WEIGHTS = 48ll << 20;
 inline bool plan_gate_up_fused(int64_t M, int64_t n_ff, int64_t K, gemm_tile_cut* cut = nullptr) {
 	if (M <= 0 || n_ff <= 0 || K <= 0 || n_ff % GROUP_K != 0 || K % GROUP_K != 0) {
 		return false;
 	}
-	if (plan_gemm(M, n_ff, K).kernel != MM_GEMM_TILE) {
-		return false;
-	}
 	const gemm_tile_cut c = plan_gemm_tile(M, 2 * n_ff, K, false); // grid_x = n_ff / 64 workgroups of two gate and two up strips
-	if (c.ks != 1) {
+	const int64_t waves	  = int64_t{ 4 } * c.ks * c.grid_x * c.grid_y;
+	if (waves < (2 * n_ff * K <= GATE_UP_SMALL_WEIGHTS ? GATE_UP_MIN_WAVES_SMALL : GATE_UP_MIN_WAVES) && !(c.ks == 1 && plan_gemm(M, n_ff, K).kernel == MM_GEMM_TILE)) {
 		return false;
 	}
 	if (cut) {

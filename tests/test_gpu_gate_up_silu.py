@@ -83,3 +83,26 @@ def test_gate_up_silu_arguments(q8):
     assert lib.nh_q8_0_gemm_tiled_gate_up_silu(None, None, None, out.data_ptr(), ws.data_ptr(), ws.numel(), 37, 3584, 0, None) == 0
     torch.cuda.synchronize()
     assert not out.cpu().numpy().any()
+
+
+# the fused kernel with K sets: two and four of them, one row of workgroups (non-temporal weights) and several, ragged and odd strips, the
+# one-strip form, and a single set read once
+@pytest.mark.parametrize("m,n_ff,k", [(64, 4608, 2048), (33, 4608, 2048), (97, 2304, 2048), (129, 1536, 2048), (64, 8960, 1024), (70, 4480, 1024), (33, 17664, 384), (20, 24576, 512), (31, 24576, 1024)])
+def test_gate_up_silu_k_sets(q8, oracle, m, n_ff, k):
+    assert q8._lib.lib().nh_q8_0_gate_up_silu_workspace_bytes(m, n_ff, k) == 0
+    wg, wu = oracle.fill_weights(21 + m, n_ff, k), oracle.fill_weights(22 + m, n_ff, k)
+    x = oracle.fill_activations(m + k, m * k).reshape(m, k)
+    aq_cpu = oracle.quantize_rows(x)
+    tg, tu = q8.tile(to_dev(wg), n_ff, k), q8.tile(to_dev(wu), n_ff, k)
+    aq = q8.quantize_row_q8_0(to_dev(x), tiled=True)
+    act, gate, up = q8.gate_up_silu(tg, tu, aq, m, n_ff, k, debug=True)
+    gate, up = to_host(gate), to_host(up)
+    for got, w in ((gate, wg), (up, wu)):
+        want = oracle.gemm(w, aq_cpu, m, n_ff, k, threads=8) if (k // 32) % 16 == 0 else oracle.gemm(w, aq_cpu, m, n_ff, k)
+        assert rel_l2(got, want) <= REL_L2_TOL
+        for i in (0, m // 2, m - 1):
+            assert rel_l2(got[i], want[i]) <= REL_L2_TOL, i
+    padded = (m + 31) // 32 * 32
+    whole = to_host(q8.untile(act, padded, n_ff)).reshape(padded, -1)
+    assert np.array_equal(whole[:m], oracle.silu_mul_quantize_rows(gate, up)) and not whole[m:].any()
+    assert np.array_equal(to_host(q8.gate_up_silu(tg, tu, aq, m, n_ff, k)), to_host(act))
