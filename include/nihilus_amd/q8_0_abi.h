@@ -18,7 +18,7 @@
  * Streams
  *   Launches that hand data between workgroups do so through scratch memory that the library keeps per GPU (made on first
  *   use or by nh_q8_0_prepare): nh_q8_0_gemv_tiled*, nh_q8_0_gemv_tiled_group_f32, nh_q8_0_mul_mat*, nh_q8_0_mul_mat_batch,
- *   nh_q8_0_mul_mat_f32_activations (each when the shape makes them split K over workgroups), nh_q8_0_gemm_tiled* for M <= 64,
+ *   nh_q8_0_mul_mat_f32_activations (each when the shape makes them split K over workgroups), nh_q8_0_gemm_tiled*,
  *   and nh_q8_0_ffn_f32 and nh_q8_0_decode_layer_f32 always.  That scratch serves ONE stream at a time per GPU: enqueue such calls on one stream, or let
  *   the other stream drain first.  A call that would use the scratch while a launch from a different stream may still be
  *   running returns NH_ERR_BUSY and launches nothing (not detected: work on a capturing stream, work that followed a
@@ -107,7 +107,7 @@ int nh_q8_0_clear_error(void);
  * previous setting (1 or 0); 1 by default.  Takes effect for calls made afterwards; needs no GPU. */
 int nh_q8_0_set_in_kernel_waits(int enabled);
 /* Allocates, for the current device, the three internal scratch buffers that K-split launches hand partial sums through
- * (about 2.6, 16 and 4 MiB; otherwise made by the first launch that needs one).  After it no launch entry point of this library
+ * (about 2.6, 32 and 4 MiB; otherwise made by the first launch that needs one).  After it no launch entry point of this library
  * allocates device memory: call it once per device before capturing launches into a HIP graph or entering a serving loop.
  * No counterpart in the reference, whose kernels never allocate (infra/model.hpp:241 owns the arena). */
 int nh_q8_0_prepare(void);

@@ -615,7 +615,7 @@ __global__ __launch_bounds__(256 * KS, 4) void gemm_gate_up_kernel(const uint8_t
 }
 
 // Executes a cut made by plan_gemm_tile (q8_0_plan.h): TM activation strips per wave, KS sets of four waves per workgroup,
-// and, with non-temporal weights, K over kz workgroups per tile whose tiles are added through the scratch.
+// and K over kz workgroups per tile whose tiles are added through the scratch.
 template<int TM, bool STREAM> static hipError_t launch_gemm_tiled_t(const gemm_tile_cut& cut, const uint8_t* w, const uint8_t* a, float* C, const float* R, int32_t* sums, int m, int n, int k, hipStream_t s) {
 	const int groups = k / GROUP_K;
 	const dim3 grid(cut.grid_x, cut.grid_y);
@@ -624,7 +624,7 @@ template<int TM, bool STREAM> static hipError_t launch_gemm_tiled_t(const gemm_t
 		return hipGetLastError();
 	}
 	const int ks = cut.ks;
-	if constexpr (STREAM) {
+	if constexpr (STREAM || TM == 2) {
 		if (cut.kz > 1) {
 			float* partials	   = nullptr;
 			unsigned* counters = nullptr;
@@ -632,7 +632,7 @@ template<int TM, bool STREAM> static hipError_t launch_gemm_tiled_t(const gemm_t
 			if (e != hipSuccess) {
 				return e;
 			}
-			return launch_kernel(KIND_GEMM, gemm_tiled_kernel<TM, false, 4, true, true>, dim3(grid.x, grid.y, static_cast<unsigned>(cut.kz)), dim3(1024), 0, s, w, a, C, R, sums, m, n, groups, partials,
+			return launch_kernel(KIND_GEMM, gemm_tiled_kernel<TM, false, 4, STREAM, true>, dim3(grid.x, grid.y, static_cast<unsigned>(cut.kz)), dim3(1024), 0, s, w, a, C, R, sums, m, n, groups, partials,
 				counters);
 		}
 	}
@@ -730,7 +730,16 @@ hipError_t launch_gemm(const void* W, const void* Aq, float* C, int32_t* sums, i
 			}
 			return launch_gemm_skinny(W, Aq, C, sums, M, N, K, s, residual);
 		}
-		return launch_gemm_tiled(plan.tile, w, a, C, residual, sums, m, n, k, s, plan.kernel == MM_GEMM_TILE_STREAM);
+		// K over workgroups with more than 64 rows: where the scratch is another stream's for now, or the launch goes into a graph that may be
+		// replayed beside another (the scratch would be both's), the streaming kernel, which seldom needs any
+		const bool split_rows = plan.kernel == MM_GEMM_TILE && plan.tile.kz > 1;
+		if (!split_rows || !stream_is_capturing(s)) {
+			const hipError_t e = launch_gemm_tiled(plan.tile, w, a, C, residual, sums, m, n, k, s, plan.kernel == MM_GEMM_TILE_STREAM);
+			if (!split_rows || e != hipErrorNotReady) {
+				return e;
+			}
+		}
+		return launch_gemm_skinny(W, Aq, C, sums, M, N, K, s, residual);
 	} else {
 		if (sums) {
 			gemm_kernel<false, true><<<grid, dim3(GEMM_THREADS), 0, s>>>(w, a, C, sums, m, n, k);

@@ -239,20 +239,20 @@ __global__ __launch_bounds__(SK_WAVES * 64, DUMP ? 2 : 4) void gemm_skinny_kerne
 	store(sum);
 }
 
-// Scratch of the K-split path (partial 32x32 tiles and arrival counters): one allocation per device on first use.
+// Scratch of the K-split path (partial 32x32 tiles and arrival counters): one allocation per device on first use, in two parts: the null
+// stream's, which may not be queried while some other stream is being captured and so never shares, and one that serves the other
+// streams one at a time.
 static_assert(GEMM_SPLIT_SCRATCH_FLOATS == SK_MAX_SPLIT_UNITS * 2 * 16 * 64 && GEMM_SPLIT_MAX_UNITS == SK_MAX_SPLIT_STRIPS, "one scratch, two users");
 struct skinny_scratch {
 	float* partials	   = nullptr;
 	unsigned* counters = nullptr;
 	hipStream_t user   = nullptr; // stream of the last K-split launch
-	bool has_user	   = false;
 };
-// launching = true: a K-split launch on `s` is about to use the scratch.  It serves one stream at a time: if the previous such
-// launch went to another stream that has not drained, hipErrorNotReady comes back (NH_ERR_BUSY at the C ABI).  Not checked for
-// capturing streams or after a launch on the null stream (neither may be queried safely).
+// launching = true: a K-split launch on `s` is about to use the scratch.  If the previous such launch of its part went to another stream
+// that has not drained, hipErrorNotReady comes back (NH_ERR_BUSY at the C ABI).  Not checked for capturing streams.
 static hipError_t get_skinny_scratch(skinny_scratch* out, bool launching = false, hipStream_t s = nullptr) {
 	static std::mutex lock;
-	static skinny_scratch per_device[64];
+	static skinny_scratch per_device[64][2];
 	int dev		 = 0;
 	hipError_t e = hipGetDevice(&dev);
 	if (e != hipSuccess) {
@@ -262,35 +262,34 @@ static hipError_t get_skinny_scratch(skinny_scratch* out, bool launching = false
 		return hipErrorInvalidDevice;
 	}
 	std::lock_guard<std::mutex> g(lock);
-	skinny_scratch& sc = per_device[dev];
-	if (!sc.partials) {
+	if (!per_device[dev][0].partials) {
 		void* p			   = nullptr;
 		const size_t tiles = static_cast<size_t>(SK_MAX_SPLIT_UNITS) * 2 * 16 * 64 * 4; // two 32-row activation strips at most
-		const size_t bytes = tiles + SK_MAX_SPLIT_STRIPS * 4;
-		e				   = hipMalloc(&p, bytes);
+		const size_t part  = tiles + SK_MAX_SPLIT_STRIPS * 4;
+		e				   = hipMalloc(&p, 2 * part);
 		if (e != hipSuccess) {
 			return e;
 		}
-		e = hipMemset(p, 0, bytes);
+		e = hipMemset(p, 0, 2 * part);
 		if (e != hipSuccess) {
 			(void)hipFree(p);
 			return e;
 		}
-		sc.partials = static_cast<float*>(p);
-		sc.counters = reinterpret_cast<unsigned*>(static_cast<uint8_t*>(p) + tiles);
+		for (int i = 0; i < 2; ++i) {
+			uint8_t* base				= static_cast<uint8_t*>(p) + i * part;
+			per_device[dev][i].partials = reinterpret_cast<float*>(base);
+			per_device[dev][i].counters = reinterpret_cast<unsigned*>(base + tiles);
+		}
 	}
+	skinny_scratch& sc = per_device[dev][s != nullptr];
 	if (launching && !stream_is_capturing(s)) {
-		if (sc.has_user && sc.user != s && sc.user != nullptr && !stream_is_capturing(sc.user)) {
-			const hipError_t q = query_stream_any_capture_mode(sc.user);
-			if (q == hipErrorNotReady) {
-				return q;
-			}
-			if (q != hipSuccess) {
-				(void)hipGetLastError();
+		if (sc.user != s && sc.user != nullptr) {
+			e = stream_drained(sc.user);
+			if (e != hipSuccess) {
+				return e;
 			}
 		}
-		sc.user		= s;
-		sc.has_user = true;
+		sc.user = s;
 	}
 	*out = sc;
 	return hipSuccess;

@@ -27,8 +27,8 @@ constexpr int GEMM_SPLIT_MIN_TRIPS = 2; // K goes over more workgroups only whil
 constexpr int GEMM_STREAM_TILE_MIN_COLUMN_BLOCKS = 192; // 128-row column blocks from which the tile kernel also takes the few-row (batched decode) shapes
 
 // The MFMA tile kernel's cut: TM activation strips per wave; KS sets of four waves per workgroup, each on a share of K (grids
-// that would leave SIMDs short of their four waves); with non-temporal weights also K over kz workgroups per tile (grids short
-// of one workgroup per CU), their tiles added through the scratch by the last to arrive.
+// that would leave SIMDs short of their four waves); also K over kz workgroups per tile (grids short of one workgroup per CU), their
+// tiles added through the scratch by the last to arrive.
 struct gemm_tile_cut {
 	int tm, ks, kz;
 	unsigned grid_x, grid_y;
@@ -55,6 +55,28 @@ inline gemm_tile_cut plan_gemm_tile(int64_t M, int64_t N, int64_t K, bool stream
 		}
 	}
 	return c;
+}
+
+// More than 64 rows against a matrix whose tiles are short of a workgroup per CU, with K long enough: the tile kernel with K over workgroups
+// until there is about one per CU.  The streaming kernel, which has the shape otherwise, takes the activations out of L2 once per weight
+// strip, where four strips share them here; the hand-off costs 3 to 4 us, so every K set has to keep five groups.  Measured, us, this /
+// the streaming kernel: [8192 x 28672] at 128 rows 91 / 129, [8192 x 8192] at 96 / 128 rows 31 / 36 and 31 / 38, [4096 x 8192] at 200 rows
+// 28.5 / 34.3, [4096 x 14336] at 117 rows (seven groups, K over four) 28.5 / 31.1, [5120 x 5120] at 160 rows (five) 21.4 / 22.3; with four
+// groups [4096 x 4096] at 200 rows 18.4 / 18.0, [2048 x 8192] at 256 rows 19.8 / 18.1; with two [4096 x 4096] at 117 rows 14.9 / 12.5.
+constexpr int GEMM_TILE_SPLIT_MIN_GROUPS = 5;
+inline bool plan_gemm_tile_split(int64_t M, int64_t N, int64_t K, gemm_tile_cut* cut) {
+	gemm_tile_cut c		  = plan_gemm_tile(M, N, K, false);
+	const int groups	  = static_cast<int>(K / GROUP_K);
+	const int64_t wgs	  = static_cast<int64_t>(c.grid_x) * c.grid_y;
+	while (c.ks == 4 && wgs * c.kz * 2 <= 256 && groups % (c.ks * c.kz * 2) == 0 && groups / (c.ks * c.kz * 2) >= GEMM_TILE_SPLIT_MIN_GROUPS &&
+		wgs * c.kz * 2 * c.tm * 4096 <= GEMM_SPLIT_SCRATCH_FLOATS && wgs <= GEMM_SPLIT_MAX_UNITS) {
+		c.kz *= 2;
+	}
+	if (c.tm != 2 || c.kz == 1 || wgs * c.kz <= 128) {
+		return false;
+	}
+	*cut = c;
+	return true;
 }
 
 // The weight-streaming MFMA kernel's cut: MS activation strips per workgroup, K of a strip over `splits` workgroups.
@@ -165,6 +187,8 @@ inline gemm_plan plan_gemm(int64_t M, int64_t N, int64_t K) {
 	if (stream_tile) {
 		p.kernel = MM_GEMM_TILE_STREAM;
 		p.tile	 = plan_gemm_tile(M, N, K, true);
+	} else if (M > GEMM_SKINNY_MAX_M && tile_workgroups <= 256 && plan_gemm_tile_split(M, N, K, &p.tile)) {
+		p.kernel = MM_GEMM_TILE;
 	} else if (M <= GEMM_SKINNY_MAX_M || tile_workgroups <= 256) {
 		p.kernel = MM_GEMM_SKINNY;
 		p.skinny = plan_gemm_skinny(M, N, K);

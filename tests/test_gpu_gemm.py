@@ -203,3 +203,20 @@ def test_gemm_extreme_quants(q8, oracle):
     w = oracle.pack_blocks(np.full(n * nb, one), np.full((n, k), 127, dtype=np.int8))
     c = to_host(q8.gemm(to_dev(w), to_dev(a), m, n, k, tiled=False))
     assert np.array_equal(c, np.full((m, n), -127.0 * 127.0 * k, dtype=np.float32))
+
+
+# more than 64 rows with K over two and four workgroups per tile: ragged last strips, an odd number of them, a ragged last weight strip
+@pytest.mark.parametrize("m,n,k", [(66, 4200, 5120), (160, 2800, 5120), (66, 4096, 10240)])
+def test_tile_kernel_with_k_over_workgroups(q8, oracle, m, n, k):
+    plan = q8.plan_mul_mat(m, n, k)
+    assert plan["kernel"] == "gemm_tile" and plan["k_splits"] == (4 if k == 10240 else 2)
+    w, x = oracle.fill_weights(m, n, k), oracle.fill_activations(n, m * k).reshape(m, k)
+    want = oracle.gemm(w, oracle.quantize_rows(x), m, n, k, threads=8)
+    wt, at = q8.tile(to_dev(w), n, k), q8.quantize_row_q8_0(to_dev(x), tiled=True)
+    got = to_host(q8.gemm(wt, at, m, n, k, tiled=True))
+    for i in range(m):
+        assert rel_l2(got[i], want[i]) <= REL_L2_TOL, i
+    res = oracle.fill_activations(5, m * n).reshape(m, n)
+    acc = to_dev(res.copy())
+    q8.gemm_residual(wt, at, acc, m, n, k, out=acc)
+    assert np.array_equal(to_host(acc), got + res)  # one fp32 add after a sum that does not depend on the order of arrival

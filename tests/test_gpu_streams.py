@@ -1,4 +1,4 @@
-"""GPU: mat-mats of up to 32 rows beside work on other streams: never refused, never wrong, whichever of them splits K over workgroups."""
+"""GPU: mat-mats that split K over workgroups beside work on other streams: never refused, never wrong."""
 import numpy as np
 import pytest
 import torch
@@ -7,7 +7,8 @@ from helpers import REL_L2_TOL, rel_l2, to_dev, to_host
 
 pytestmark = pytest.mark.gpu
 
-M, N, K = 4, 4096, 4096  # K over two workgroups per strip
+# the kernel for up to 32 rows, K over two workgroups per strip; the tile kernel for more than 64, K over two per tile
+SHAPES = [(4, 4096, 4096), (66, 4224, 5120)]
 NV, KV = 4096, 14336  # a mat-vec with K over four
 
 
@@ -25,8 +26,9 @@ def _busy(stream, call):
 
 
 # the stream that is kept busy: mat-vecs or mat-mats on a side stream, mat-mats on the null stream
+@pytest.mark.parametrize("M,N,K", SHAPES, ids=["4 rows", "66 rows"])
 @pytest.mark.parametrize("busy_with", ["mat-vec", "mat-mat", "mat-mat on the null stream"])
-def test_mat_mat_beside_another_stream(q8, oracle, busy_with):
+def test_mat_mat_beside_another_stream(q8, oracle, busy_with, M, N, K):
     lib = q8._lib.lib()
     assert lib.nh_q8_0_prepare() == 0
     w, wv = oracle.fill_weights(1, N, K), q8.fill_weight_blocks(2, NV, KV)
