@@ -24,10 +24,10 @@ __device__ __forceinline__ v2u scale_slot(v2u four, int t) {
 	return v2u{ (t & 1) ? (dword >> 16) : (dword & 0xFFFFu), 0u };
 }
 
-template<int MS, bool DUMP, int GC>
-__global__ __launch_bounds__(SK_WAVES * 64, DUMP ? 2 : 4) void gemm_skinny_kernel(const uint8_t* __restrict__ W, const uint8_t* __restrict__ A, float* C, const float* R, int32_t* __restrict__ sums,
+template<int MS, bool DUMP, int GC, int WAVES>
+__global__ __launch_bounds__(WAVES * 64, DUMP ? 2 : 4) void gemm_skinny_kernel(const uint8_t* __restrict__ W, const uint8_t* __restrict__ A, float* C, const float* R, int32_t* __restrict__ sums,
 	float* __restrict__ partials, unsigned* __restrict__ counters, int M, int N, int groups, int split_shift) {
-	__shared__ float red[MS * 16][SK_WAVES][64];
+	__shared__ float red[MS * 16][WAVES][64];
 	__shared__ int last_flag;
 
 	const int tid	 = threadIdx.x;
@@ -39,7 +39,7 @@ __global__ __launch_bounds__(SK_WAVES * 64, DUMP ? 2 : 4) void gemm_skinny_kerne
 	const int mg	 = static_cast<int>(blockIdx.y); // group of MS activation strips (more than 32 * MS rows: the weights are read once per group, from cache after the first)
 	const int unit	 = mg * static_cast<int>(gridDim.x >> split_shift) + strip; // index of this (row group, weight strip) in the split scratch
 	int g0, g1; // this wave's share of the strip's K range
-	wave_k_range(groups, split_shift, split, SK_WAVES, wave, g0, g1);
+	wave_k_range(groups, split_shift, split, WAVES, wave, g0, g1);
 	const int r		 = lane & 31;
 	const int half	 = lane >> 5;
 
@@ -153,7 +153,7 @@ __global__ __launch_bounds__(SK_WAVES * 64, DUMP ? 2 : 4) void gemm_skinny_kerne
 	// ---- the waves' partial sums through LDS; a wave finishes OWN of every lane's MS * 16 values ----
 	// (One wave finishing them all, behind a tree of barriers, and reading the residual value by value behind its own stores was a chain
 	// of 16 * MS memory latencies: [4096 x 4096] at 117 rows 23.1 us with a residual against 13.9 without; now 13.9 and 12.6.)
-	constexpr int OWN = MS * 16 / SK_WAVES;
+	constexpr int OWN = MS * 16 / WAVES;
 	const int n		  = strip * STRIP_ROWS + r;
 	const auto row_of = [&](int v) { return (mg * MS + (v >> 4)) * STRIP_ROWS + 8 * ((v & 15) >> 2) + 4 * half + (v & 3); };
 	float add[OWN]; // R may be C: every element is read here and written below by the same thread
@@ -174,8 +174,14 @@ __global__ __launch_bounds__(SK_WAVES * 64, DUMP ? 2 : 4) void gemm_skinny_kerne
 #pragma unroll
 	for (int o = 0; o < OWN; ++o) {
 		const auto& p = red[wave * OWN + o];
-		static_assert(SK_WAVES == 8, "a fixed tree over eight partial sums");
-		own[o] = ((p[0][lane] + p[4][lane]) + (p[2][lane] + p[6][lane])) + ((p[1][lane] + p[5][lane]) + (p[3][lane] + p[7][lane]));
+		static_assert(WAVES == 8 || WAVES == 16, "a fixed tree over the waves' partial sums");
+		const auto eight = [&](int w) {
+			return ((p[w + 0][lane] + p[w + 4][lane]) + (p[w + 2][lane] + p[w + 6][lane])) + ((p[w + 1][lane] + p[w + 5][lane]) + (p[w + 3][lane] + p[w + 7][lane]));
+		};
+		own[o] = eight(0);
+		if constexpr (WAVES == 16) {
+			own[o] += eight(8);
+		}
 	}
 	auto store = [&](const float (&v)[OWN]) {
 #pragma unroll
@@ -314,7 +320,7 @@ hipError_t prepare_gemm_scratch() {
 	return e != hipSuccess ? e : prepare_gemm_rows_scratch();
 }
 
-template<int MS> static hipError_t launch_skinny_t(int splits, const uint8_t* w, const uint8_t* a, float* C, const float* R, int32_t* sums, int m, int n, int groups, hipStream_t s) {
+template<int MS> static hipError_t launch_skinny_t(int splits, int waves, const uint8_t* w, const uint8_t* a, float* C, const float* R, int32_t* sums, int m, int n, int groups, hipStream_t s) {
 	const int strips   = (n + STRIP_ROWS - 1) / STRIP_ROWS;
 	const int m_groups = ((m + STRIP_ROWS - 1) / STRIP_ROWS + MS - 1) / MS;
 	skinny_scratch sc;
@@ -328,12 +334,17 @@ template<int MS> static hipError_t launch_skinny_t(int splits, const uint8_t* w,
 	while ((1 << shift) < splits) {
 		++shift;
 	}
-	const dim3 grid(static_cast<unsigned>(strips * splits), static_cast<unsigned>(m_groups)), block(SK_WAVES * 64);
+	const dim3 grid(static_cast<unsigned>(strips * splits), static_cast<unsigned>(m_groups)), block(static_cast<unsigned>(64 * waves));
 	if (sums) {
-		gemm_skinny_kernel<MS, true, 1><<<grid, block, 0, s>>>(w, a, C, R, sums, sc.partials, sc.counters, m, n, groups, shift);
+		gemm_skinny_kernel<MS, true, 1, SK_WAVES><<<grid, dim3(SK_WAVES * 64), 0, s>>>(w, a, C, R, sums, sc.partials, sc.counters, m, n, groups, shift);
 		return hipGetLastError();
 	}
-	return launch_kernel(KIND_GEMM, gemm_skinny_kernel<MS, false, 2>, grid, block, 0, s, w, a, C, R, sums, sc.partials, sc.counters, m, n, groups, shift);
+	if constexpr (MS == 1) { // two strips per workgroup are only cut into 256 workgroups and more
+		if (waves == SK_WIDE_WAVES) {
+			return launch_kernel(KIND_GEMM, gemm_skinny_kernel<1, false, 2, SK_WIDE_WAVES>, grid, block, 0, s, w, a, C, R, sums, sc.partials, sc.counters, m, n, groups, shift);
+		}
+	}
+	return launch_kernel(KIND_GEMM, gemm_skinny_kernel<MS, false, 2, SK_WAVES>, grid, block, 0, s, w, a, C, R, sums, sc.partials, sc.counters, m, n, groups, shift);
 }
 
 hipError_t launch_gemm_skinny(const void* W, const void* Aq, float* C, int32_t* sums, int64_t M, int64_t N, int64_t K, hipStream_t s, const float* residual) {
@@ -342,9 +353,9 @@ hipError_t launch_gemm_skinny(const void* W, const void* Aq, float* C, int32_t* 
 	const int groups = static_cast<int>(K / GROUP_K);
 	const gemm_skinny_cut cut = plan_gemm_skinny(M, N, K); // activation strips per workgroup, workgroups per strip: q8_0_plan.h
 	if (cut.ms == 1) {
-		return launch_skinny_t<1>(cut.splits, w, a, C, residual, sums, static_cast<int>(M), static_cast<int>(N), groups, s);
+		return launch_skinny_t<1>(cut.splits, cut.waves, w, a, C, residual, sums, static_cast<int>(M), static_cast<int>(N), groups, s);
 	}
-	return launch_skinny_t<2>(cut.splits, w, a, C, residual, sums, static_cast<int>(M), static_cast<int>(N), groups, s);
+	return launch_skinny_t<2>(cut.splits, cut.waves, w, a, C, residual, sums, static_cast<int>(M), static_cast<int>(N), groups, s);
 }
 
 } // namespace nh

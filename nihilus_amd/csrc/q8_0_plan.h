@@ -21,6 +21,7 @@ enum mul_mat_kernel : int {
 };
 
 constexpr int SK_WAVES			  = 8; // waves per workgroup of the weight-streaming MFMA kernel
+constexpr int SK_WIDE_WAVES		  = 16; // the same in grids of 129 to 255 workgroups (plan_gemm_skinny)
 constexpr int SK_MAX_SPLIT_UNITS  = 2048; // strips * splits when splits > 1
 constexpr int SK_MAX_SPLIT_STRIPS = 512;
 constexpr int GEMM_SPLIT_MIN_TRIPS = 2; // K goes over more workgroups only while each K set keeps this many 128-quant groups
@@ -79,9 +80,9 @@ inline bool plan_gemm_tile_split(int64_t M, int64_t N, int64_t K, gemm_tile_cut*
 	return true;
 }
 
-// The weight-streaming MFMA kernel's cut: MS activation strips per workgroup, K of a strip over `splits` workgroups.
+// The weight-streaming MFMA kernel's cut: MS activation strips per workgroup, K of a strip over `splits` workgroups of `waves` waves.
 struct gemm_skinny_cut {
-	int ms, splits;
+	int ms, splits, waves;
 };
 inline gemm_skinny_cut plan_gemm_skinny(int64_t M, int64_t N, int64_t K) {
 	gemm_skinny_cut c{};
@@ -92,15 +93,22 @@ inline gemm_skinny_cut plan_gemm_skinny(int64_t M, int64_t N, int64_t K) {
 	c.ms				= (m_strips <= 1 || strips * ((m_strips + 1) / 2) < 256) ? 1 : 2;
 	const int64_t units = strips * ((m_strips + c.ms - 1) / c.ms);
 	c.splits			= 1;
+	// 129 to 255 units and a K that eight waves would split: two workgroups each leave some CUs two and some one or none, and the launch
+	// takes as long as the ones with two.  One workgroup of sixteen waves per unit has the same waves on every CU it uses and nothing to hand
+	// over.  Measured, us, split / this: [1024 x 8192] at 200 rows 13.6 / 11.9, [1024 x 4096] at 224 rows 9.5 / 7.7, [3072 x 12288] at 40 rows
+	// 20.6 / 18.0, [768 x 4096] at 180 rows 9.0 / 7.6, [4064 x 4096] at 50 rows 11.0 / 9.3, [2080 x 4096] at 64 rows 9.8 / 9.1, [640 x 14336] at
+	// 256 rows 20.1 / 19.4.  Outside it does not pay: at 128 units, which the split makes into a workgroup per CU, 7.4 / 7.6 ([1024 x 4096] at
+	// 117 rows) and 9.6 / 12.2 (K = 8192); at 256, 12.8 / 12.5 ([4096 x 4096] at 117 rows) and 8.5 / 8.8 (at 64).
+	c.waves = (units > 128 && units < 256 && groups >= 4 * SK_WAVES) ? SK_WIDE_WAVES : SK_WAVES;
 	// The hand-off between workgroups is expensive here (a partial tile of 16 values per lane and strip, an arrival counter,
 	// the last arriver reading every share): K goes over several workgroups only until every CU has one (and every wave
 	// keeps at least two groups, one step of the kernel's walk: [4096 x 4096] at M = 32 12.1 -> 10.8 us, [1024 x 8192] at M = 64
 	// 14.9 -> 13.2 us against keeping four), or when a wave would otherwise walk more than sixteen groups.  Measured on
 	// [8192 x 28672] at M = 16: 68 us with eight workgroups per strip, 51 us with two.
-	while (units * c.splits < 256 && groups >= 4 * SK_WAVES * c.splits && units * c.splits * 2 <= SK_MAX_SPLIT_UNITS && units <= SK_MAX_SPLIT_STRIPS) {
+	while (c.waves == SK_WAVES && units * c.splits < 256 && groups >= 4 * SK_WAVES * c.splits && units * c.splits * 2 <= SK_MAX_SPLIT_UNITS && units <= SK_MAX_SPLIT_STRIPS) {
 		c.splits *= 2;
 	}
-	while (groups > 16 * SK_WAVES * c.splits && units * c.splits * 2 <= SK_MAX_SPLIT_UNITS && units <= SK_MAX_SPLIT_STRIPS) {
+	while (groups > 16 * c.waves * c.splits && units * c.splits * 2 <= SK_MAX_SPLIT_UNITS && units <= SK_MAX_SPLIT_STRIPS) {
 		c.splits *= 2;
 	}
 	return c;

@@ -220,3 +220,21 @@ def test_tile_kernel_with_k_over_workgroups(q8, oracle, m, n, k):
     acc = to_dev(res.copy())
     q8.gemm_residual(wt, at, acc, m, n, k, out=acc)
     assert np.array_equal(to_host(acc), got + res)  # one fp32 add after a sum that does not depend on the order of arrival
+
+
+# the streaming kernel with sixteen waves per workgroup (129 to 255 workgroups): a ragged weight strip, groups that the waves do not share
+# evenly, the longest K that needs no split and the first that does
+@pytest.mark.parametrize("m,n,k,splits", [(33, 2050, 4096, 1), (250, 544, 4608, 1), (33, 2080, 32768, 1), (33, 2080, 33280, 2)])
+def test_streaming_kernel_with_sixteen_waves(q8, oracle, m, n, k, splits):
+    plan = q8.plan_mul_mat(m, n, k)
+    assert plan["kernel"] == "gemm_skinny" and plan["activation_strips"] == 1 and plan["k_splits"] == splits
+    w, x = oracle.fill_weights(m, n, k), oracle.fill_activations(n, m * k).reshape(m, k)
+    want = oracle.gemm(w, oracle.quantize_rows(x), m, n, k, threads=8)
+    wt, at = q8.tile(to_dev(w), n, k), q8.quantize_row_q8_0(to_dev(x), tiled=True)
+    got = to_host(q8.gemm(wt, at, m, n, k, tiled=True))
+    for i in range(m):
+        assert rel_l2(got[i], want[i]) <= REL_L2_TOL, i
+    res = oracle.fill_activations(5, m * n).reshape(m, n)
+    acc = to_dev(res.copy())
+    q8.gemm_residual(wt, at, acc, m, n, k, out=acc)
+    assert np.array_equal(to_host(acc), got + res)
