@@ -418,7 +418,8 @@ hipError_t launch_decode_layer(const void* w_o, const float* attn, const float* 
 		return launch_gemv_tiled_multi(w_next, y_next, n_next, count_next, l_out, true, n_embd, s, next_norm_w, eps);
 	}
 	gemv_scratch sc;
-	const hipError_t e = get_gemv_scratch(&sc, true, s);
+	scratch_hold hold;
+	const hipError_t e = get_gemv_scratch(&sc, &hold, s);
 	if (e != hipSuccess) {
 		return e;
 	}

@@ -7,6 +7,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <mutex>
+
 namespace nh {
 
 constexpr int QK			= 32; // quants per block (Q_SIZE, common/data_types.hpp:28)
@@ -293,6 +295,11 @@ inline hipError_t query_stream_any_capture_mode(hipStream_t s) {
 	return q;
 }
 
+// A launcher's hold on a piece of hand-off scratch, from being given it until its launches are enqueued.  Who gets the scratch is decided
+// by asking the previous user's stream whether it has drained: between the answer and the launch that rests on it nobody else may ask, or
+// two threads with a stream each are both given it.  Recursive: a call of several launches holds it around launchers that take it too.
+using scratch_hold = std::unique_lock<std::recursive_mutex>;
+
 // hipErrorNotReady when `prev` still has work in flight; anything else (a destroyed stream, a capturing one) counts as drained
 inline hipError_t stream_drained(hipStream_t prev) {
 	if (stream_is_capturing(prev)) {
@@ -403,7 +410,7 @@ hipError_t prepare_gemv_scratch();
 hipError_t prepare_gemm_scratch();
 constexpr int64_t GEMM_SPLIT_SCRATCH_FLOATS = 2048 * 2 * 16 * 64; // partial tiles of a K split over workgroups
 constexpr int GEMM_SPLIT_MAX_UNITS			  = 512; // arrival counters
-hipError_t acquire_gemm_split_scratch(float** partials, unsigned** counters, hipStream_t s);
+hipError_t acquire_gemm_split_scratch(float** partials, unsigned** counters, scratch_hold* hold, hipStream_t s);
 hipError_t launch_gemm_skinny(const void* W, const void* Aq, float* C, int32_t* sums, int64_t M, int64_t N, int64_t K, hipStream_t s, const float* residual = nullptr);
 
 } // namespace nh

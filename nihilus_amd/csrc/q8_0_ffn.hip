@@ -231,7 +231,8 @@ hipError_t launch_ffn_decode(const void* w_gate, const void* w_up, const void* w
 		return hipGetLastError();
 	}
 	gemv_scratch sc;
-	const hipError_t e = get_gemv_scratch(&sc, true, s);
+	scratch_hold hold;
+	const hipError_t e = get_gemv_scratch(&sc, &hold, s);
 	if (e != hipSuccess) {
 		return e;
 	}

@@ -628,7 +628,8 @@ template<int TM, bool STREAM> static hipError_t launch_gemm_tiled_t(const gemm_t
 		if (cut.kz > 1) {
 			float* partials	   = nullptr;
 			unsigned* counters = nullptr;
-			const hipError_t e = acquire_gemm_split_scratch(&partials, &counters, s);
+			scratch_hold hold;
+			const hipError_t e = acquire_gemm_split_scratch(&partials, &counters, &hold, s);
 			if (e != hipSuccess) {
 				return e;
 			}

@@ -298,8 +298,9 @@ namespace {
 		hipStream_t user = nullptr; // stream of the last launch that used this part
 	};
 	constexpr size_t ROWS_SCRATCH_WORDS = static_cast<size_t>(GEMV_MAX_SPLIT_UNITS) * STRIP_ROWS;
-	hipError_t get_rows_scratch(rows_scratch* out, bool launching, hipStream_t s) {
-		static std::mutex lock;
+	// hold == nullptr: make it if need be; otherwise a launch on `s` is about to use it, and the caller keeps *hold until it is enqueued
+	hipError_t get_rows_scratch(rows_scratch* out, scratch_hold* hold, hipStream_t s) {
+		static std::recursive_mutex locks[64];
 		static rows_scratch per_device[64][2];
 		int dev		 = 0;
 		hipError_t e = hipGetDevice(&dev);
@@ -309,7 +310,7 @@ namespace {
 		if (dev < 0 || dev >= 64) {
 			return hipErrorInvalidDevice;
 		}
-		std::lock_guard<std::mutex> g(lock);
+		scratch_hold g(locks[dev]);
 		if (!per_device[dev][0].tagged) {
 			void* p = nullptr;
 			e		= hipMalloc(&p, 2 * ROWS_SCRATCH_WORDS * 8);
@@ -325,7 +326,7 @@ namespace {
 			per_device[dev][1].tagged = static_cast<uint64_t*>(p) + ROWS_SCRATCH_WORDS;
 		}
 		rows_scratch& sc = per_device[dev][s != nullptr];
-		if (launching) {
+		if (hold) {
 			if (sc.user != s && sc.user != nullptr) {
 				e = stream_drained(sc.user);
 				if (e != hipSuccess) {
@@ -338,21 +339,25 @@ namespace {
 			}
 		}
 		*out = sc;
+		if (hold) {
+			*hold = std::move(g);
+		}
 		return hipSuccess;
 	}
 } // namespace
 
 hipError_t prepare_gemm_rows_scratch() {
 	rows_scratch sc;
-	return get_rows_scratch(&sc, false, nullptr);
+	return get_rows_scratch(&sc, nullptr, nullptr);
 }
 
 // 1 <= M <= 32, K > 0; splits: plan_gemm_rows_splits
 hipError_t launch_gemm_rows(const void* W, const void* Aq, float* C, const float* residual, int64_t M, int64_t N, int64_t K, int splits, hipStream_t s) {
 	const int64_t strips = (N + STRIP_ROWS - 1) / STRIP_ROWS;
 	rows_scratch sc;
+	scratch_hold hold;
 	if (splits > 1) {
-		const hipError_t e = get_rows_scratch(&sc, true, s);
+		const hipError_t e = get_rows_scratch(&sc, &hold, s);
 		if (e != hipSuccess) {
 			return e;
 		}

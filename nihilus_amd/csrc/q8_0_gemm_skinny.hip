@@ -254,10 +254,10 @@ struct skinny_scratch {
 	unsigned* counters = nullptr;
 	hipStream_t user   = nullptr; // stream of the last K-split launch
 };
-// launching = true: a K-split launch on `s` is about to use the scratch.  If the previous such launch of its part went to another stream
+// hold == nullptr: make it if need be.  Otherwise a K-split launch on `s` is about to use it, and the caller keeps *hold until it is enqueued.  If the previous such launch of its part went to another stream
 // that has not drained, hipErrorNotReady comes back (NH_ERR_BUSY at the C ABI).  Not checked for capturing streams.
-static hipError_t get_skinny_scratch(skinny_scratch* out, bool launching = false, hipStream_t s = nullptr) {
-	static std::mutex lock;
+static hipError_t get_skinny_scratch(skinny_scratch* out, scratch_hold* hold = nullptr, hipStream_t s = nullptr) {
+	static std::recursive_mutex locks[64];
 	static skinny_scratch per_device[64][2];
 	int dev		 = 0;
 	hipError_t e = hipGetDevice(&dev);
@@ -267,7 +267,7 @@ static hipError_t get_skinny_scratch(skinny_scratch* out, bool launching = false
 	if (dev < 0 || dev >= 64) {
 		return hipErrorInvalidDevice;
 	}
-	std::lock_guard<std::mutex> g(lock);
+	scratch_hold g(locks[dev]);
 	if (!per_device[dev][0].partials) {
 		void* p			   = nullptr;
 		const size_t tiles = static_cast<size_t>(SK_MAX_SPLIT_UNITS) * 2 * 16 * 64 * 4; // two 32-row activation strips at most
@@ -288,7 +288,7 @@ static hipError_t get_skinny_scratch(skinny_scratch* out, bool launching = false
 		}
 	}
 	skinny_scratch& sc = per_device[dev][s != nullptr];
-	if (launching && !stream_is_capturing(s)) {
+	if (hold && !stream_is_capturing(s)) {
 		if (sc.user != s && sc.user != nullptr) {
 			e = stream_drained(sc.user);
 			if (e != hipSuccess) {
@@ -298,14 +298,17 @@ static hipError_t get_skinny_scratch(skinny_scratch* out, bool launching = false
 		sc.user = s;
 	}
 	*out = sc;
+	if (hold) {
+		*hold = std::move(g);
+	}
 	return hipSuccess;
 }
 
 // The same scratch for the tile kernel's K split over workgroups (GEMM_SPLIT_SCRATCH_FLOATS floats of tiles, GEMM_SPLIT_MAX_UNITS
 // counters that every launch leaves at zero); same one-stream rule.
-hipError_t acquire_gemm_split_scratch(float** partials, unsigned** counters, hipStream_t s) {
+hipError_t acquire_gemm_split_scratch(float** partials, unsigned** counters, scratch_hold* hold, hipStream_t s) {
 	skinny_scratch sc;
-	const hipError_t e = get_skinny_scratch(&sc, true, s);
+	const hipError_t e = get_skinny_scratch(&sc, hold, s);
 	if (e != hipSuccess) {
 		return e;
 	}
@@ -324,8 +327,9 @@ template<int MS> static hipError_t launch_skinny_t(int splits, int waves, const 
 	const int strips   = (n + STRIP_ROWS - 1) / STRIP_ROWS;
 	const int m_groups = ((m + STRIP_ROWS - 1) / STRIP_ROWS + MS - 1) / MS;
 	skinny_scratch sc;
+	scratch_hold hold;
 	if (splits > 1) {
-		const hipError_t e = get_skinny_scratch(&sc, true, s);
+		const hipError_t e = get_skinny_scratch(&sc, &hold, s);
 		if (e != hipSuccess) {
 			return e;
 		}

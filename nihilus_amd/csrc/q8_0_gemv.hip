@@ -218,16 +218,20 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_tiled_kernel(gemv_segmen
 
 namespace {
 	struct scratch_state {
+		std::recursive_mutex lock;
 		gemv_scratch sc;
 		hipStream_t user = nullptr; // stream of the last launch that used the scratch
 		bool has_user	 = false;
 	};
-	std::mutex scratch_lock;
 	scratch_state scratch_per_device[64];
-	int published_spin_limit = PUBLISHED_SPIN_LIMIT;
+	// beside the state: whoever reads the error must not wait for another thread's launch
+	std::atomic<unsigned*> error_word_per_device[64];
+	std::atomic<int> published_spin_limit{ PUBLISHED_SPIN_LIMIT };
 } // namespace
 
-hipError_t get_gemv_scratch(gemv_scratch* out, bool next_epoch, hipStream_t s) {
+// hold == nullptr: the scratch alone (made if need be).  Otherwise it is about to be used by launches on `s`: with a fresh epoch, and the
+// caller keeps *hold until they are enqueued.
+hipError_t get_gemv_scratch(gemv_scratch* out, scratch_hold* hold, hipStream_t s) {
 	int dev		 = 0;
 	hipError_t e = hipGetDevice(&dev);
 	if (e != hipSuccess) {
@@ -236,9 +240,9 @@ hipError_t get_gemv_scratch(gemv_scratch* out, bool next_epoch, hipStream_t s) {
 	if (dev < 0 || dev >= 64) {
 		return hipErrorInvalidDevice;
 	}
-	std::lock_guard<std::mutex> g(scratch_lock);
 	scratch_state& st = scratch_per_device[dev];
-	gemv_scratch& sc  = st.sc;
+	scratch_hold g(st.lock);
+	gemv_scratch& sc = st.sc;
 	if (!sc.tagged) {
 		void* p			   = nullptr;
 		const size_t blocks_end = static_cast<size_t>(GEMV_MAX_SPLIT_UNITS) * STRIP_ROWS * 8 + 2 * FFN_MAX_HIDDEN * 4 + (FFN_MAX_HIDDEN / STRIP_ROWS) * PUBLISHED_WORDS * 8 + (FFN_MAX_HIDDEN / QK) * BLOCK_BYTES;
@@ -269,8 +273,9 @@ hipError_t get_gemv_scratch(gemv_scratch* out, bool next_epoch, hipStream_t s) {
 		sc.row_tagged[1] = sc.row_tagged[0] + CHAIN_MAX_EMBD;
 		sc.x_words_next	 = reinterpret_cast<uint64_t*>(static_cast<uint8_t*>(p) + next_at);
 		sc.error_word = static_cast<unsigned*>(word);
+		error_word_per_device[dev].store(sc.error_word, std::memory_order_release);
 	}
-	if (next_epoch) {
+	if (hold) {
 		if (!stream_is_capturing(s)) {
 			if (st.has_user && st.user != s && st.user != nullptr) {
 				e = stream_drained(st.user);
@@ -286,8 +291,11 @@ hipError_t get_gemv_scratch(gemv_scratch* out, bool next_epoch, hipStream_t s) {
 			++sc.epoch;
 		}
 	}
-	sc.spin_limit = published_spin_limit;
+	sc.spin_limit = published_spin_limit.load(std::memory_order_relaxed);
 	*out		  = sc;
+	if (hold) {
+		*hold = std::move(g);
+	}
 	return hipSuccess;
 }
 
@@ -297,8 +305,7 @@ unsigned read_device_error(bool clear) {
 		(void)hipGetLastError();
 		return DEVICE_ERROR_NONE;
 	}
-	std::lock_guard<std::mutex> g(scratch_lock);
-	unsigned* word = scratch_per_device[dev].sc.error_word;
+	unsigned* word = error_word_per_device[dev].load(std::memory_order_acquire);
 	if (!word) {
 		return DEVICE_ERROR_NONE;
 	}
@@ -316,8 +323,7 @@ bool set_in_kernel_waits(bool enabled) {
 }
 
 void set_published_spin_limit(int limit) {
-	std::lock_guard<std::mutex> g(scratch_lock);
-	published_spin_limit = limit < 1 ? 1 : (limit > PUBLISHED_SPIN_LIMIT ? PUBLISHED_SPIN_LIMIT : limit);
+	published_spin_limit.store(limit < 1 ? 1 : (limit > PUBLISHED_SPIN_LIMIT ? PUBLISHED_SPIN_LIMIT : limit), std::memory_order_relaxed);
 }
 
 hipError_t prepare_gemv_scratch() {
@@ -344,14 +350,14 @@ __global__ void clear_tags_kernel(uint64_t* __restrict__ p, int n) {
 // Calls that overlap on one GPU share the array and would race on it, like the calls that share the allocated scratch: the
 // same one-stream-at-a-time rule applies (hipErrorNotReady while the previous user's stream, a different one, has work in
 // flight; the query allocates nothing).
-static hipError_t get_noalloc_scratch(gemv_scratch* out, hipStream_t s) {
+static hipError_t get_noalloc_scratch(gemv_scratch* out, scratch_hold* hold, hipStream_t s) {
 	struct state {
+		std::recursive_mutex lock;
 		uint64_t* ptr  = nullptr;
 		unsigned epoch = 0;
 		hipStream_t user = nullptr; // stream of the last launch that used the array
 		bool has_user	 = false;
 	};
-	static std::mutex lock;
 	static state per_device[64];
 	int dev		 = 0;
 	hipError_t e = hipGetDevice(&dev);
@@ -361,8 +367,8 @@ static hipError_t get_noalloc_scratch(gemv_scratch* out, hipStream_t s) {
 	if (dev < 0 || dev >= 64) {
 		return hipErrorInvalidDevice;
 	}
-	std::lock_guard<std::mutex> g(lock);
 	state& st = per_device[dev];
+	scratch_hold g(st.lock);
 	if (!stream_is_capturing(s)) {
 		if (st.has_user && st.user != s && st.user != nullptr) {
 			e = stream_drained(st.user); // also covers the first use's tag clearing, which went to that stream
@@ -397,6 +403,7 @@ static hipError_t get_noalloc_scratch(gemv_scratch* out, hipStream_t s) {
 	*out		= gemv_scratch{};
 	out->tagged = st.ptr;
 	out->epoch	= st.epoch;
+	*hold		= std::move(g);
 	return hipSuccess;
 }
 
@@ -479,10 +486,11 @@ static hipError_t launch_gemv_tiled_any(const void* const* W, float* const* y, c
 		p.tiles	 = (p.groups + GEMV_WAVES - 1) / GEMV_WAVES;
 	}
 	gemv_scratch sc;
+	scratch_hold hold;
 	if (p.splits == 1 && norm_w && x_is_f32 && dump_mode == DUMP_NONE && !noalloc && gemv_shares_x(p, 1) && !stream_is_capturing(s) && in_kernel_waits_enabled()) {
 		// the normalised, quantized row goes from the first strip's workgroups to the others through the scratch, tagged with a
 		// fresh epoch; not under capture, where a replay could not renew the epoch: there every workgroup works the row out
-		const hipError_t e = get_gemv_scratch(&sc, true, s);
+		const hipError_t e = get_gemv_scratch(&sc, &hold, s);
 		if (e != hipSuccess) {
 			return e;
 		}
@@ -491,7 +499,7 @@ static hipError_t launch_gemv_tiled_any(const void* const* W, float* const* y, c
 		if (noalloc && p.strips * p.splits > NOALLOC_MAX_SPLIT_UNITS) {
 			return hipErrorInvalidValue; // the caller checks gemv_noalloc_fits first
 		}
-		const hipError_t e = noalloc ? get_noalloc_scratch(&sc, s) : get_gemv_scratch(&sc, true, s);
+		const hipError_t e = noalloc ? get_noalloc_scratch(&sc, &hold, s) : get_gemv_scratch(&sc, &hold, s);
 		if (e != hipSuccess) {
 			return e;
 		}

@@ -145,8 +145,9 @@ hipError_t launch_gemv_group(const gemv_group_op* ops, int count, hipStream_t s)
 		return hipErrorInvalidValue;
 	}
 	gemv_scratch sc;
+	scratch_hold hold;
 	if (units > 0) {
-		const hipError_t e = get_gemv_scratch(&sc, true, s);
+		const hipError_t e = get_gemv_scratch(&sc, &hold, s);
 		if (e != hipSuccess) {
 			return e;
 		}

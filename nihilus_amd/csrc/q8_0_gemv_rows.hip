@@ -212,8 +212,9 @@ hipError_t launch_gemv_rows(const void* W, const float* x, float* y, int64_t M, 
 	}
 	p.tiles = tiles_for(p.splits);
 	gemv_scratch sc;
+	scratch_hold hold;
 	if (p.splits > 1) {
-		const hipError_t e = get_gemv_scratch(&sc, true, s);
+		const hipError_t e = get_gemv_scratch(&sc, &hold, s);
 		if (e != hipSuccess) {
 			return e;
 		}

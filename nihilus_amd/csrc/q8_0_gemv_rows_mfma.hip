@@ -208,8 +208,9 @@ hipError_t launch_gemv_rows_mfma(const void* W, const float* x, float* y, int64_
 	const int rows	  = M <= 8 ? 8 : 16;
 	const gemv_plan p = plan_gemv_rows_mfma(strips, K, rows, stream_is_capturing(s));
 	gemv_scratch sc;
+	scratch_hold hold;
 	if (p.splits > 1) {
-		const hipError_t e = get_gemv_scratch(&sc, true, s);
+		const hipError_t e = get_gemv_scratch(&sc, &hold, s);
 		if (e != hipSuccess) {
 			return e;
 		}

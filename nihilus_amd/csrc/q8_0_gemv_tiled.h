@@ -491,7 +491,7 @@ struct gemv_scratch {
 	// the second normalised, quantized row of the launch
 	uint64_t* row_tagged[2] = { nullptr, nullptr }; // [CHAIN_MAX_EMBD] each: attn_out + residual, then down + residual
 	uint64_t* x_words_next	= nullptr; // [CHAIN_MAX_EMBD / 32][PUBLISHED_WORDS]
-	unsigned epoch	   = 0; // with next_epoch = true: a value no earlier launch on this device has used
+	unsigned epoch	   = 0; // with a hold: a value no earlier launch on this device has used
 	unsigned* error_word = nullptr; // 4 bytes of pinned host memory the device can write: non-zero once a kernel has given up a bounded wait
 	int spin_limit	   = PUBLISHED_SPIN_LIMIT; // polls before a consumer of published blocks gives up (lowered only by tests)
 };
@@ -500,7 +500,7 @@ struct gemv_scratch {
 // stream has not drained, hipErrorNotReady comes back (NH_ERR_BUSY at the C ABI) instead of a launch that would corrupt both.
 // The check is skipped for capturing streams and when the previous user was the null stream (which may not be queried while
 // another stream captures).
-hipError_t get_gemv_scratch(gemv_scratch* out, bool next_epoch = false, hipStream_t s = nullptr);
+hipError_t get_gemv_scratch(gemv_scratch* out, scratch_hold* hold = nullptr, hipStream_t s = nullptr);
 // Reads the current device's error word (DEVICE_ERROR_NONE if no scratch exists yet); clear = true also resets it.
 unsigned read_device_error(bool clear);
 void set_published_spin_limit(int limit);

@@ -114,13 +114,14 @@ hipError_t launch_mul_mat_f32act(const void* W_tiled, const float* x, float* y, 
 	// capturing stream (the hand-off's epoch would be the same in every replay).
 	int shift		   = 0;
 	gemv_scratch sc;
+	scratch_hold hold;
 	if (M == 1 && !stream_is_capturing(s)) {
 		const gemv_plan p = plan_gemv(strips, K);
 		if (p.splits > 1) {
 			while ((1 << shift) < p.splits) {
 				++shift;
 			}
-			const hipError_t e = get_gemv_scratch(&sc, true, s);
+			const hipError_t e = get_gemv_scratch(&sc, &hold, s);
 			if (e != hipSuccess) {
 				return e;
 			}

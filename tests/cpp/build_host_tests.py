@@ -18,10 +18,11 @@ REFERENCE_MODE_BIN = os.path.join(HERE, "test_reference_mode_compiles")  # the h
 LAUNCH_FLOOR_BIN = os.path.join(HERE, "launch_floor_probe")  # cost of a dispatch that does nothing (a HIP program of its own, no library)
 READ_PROBE_BIN = os.path.join(HERE, "read_probe")  # what a bare read of a matrix's bytes costs (a HIP program of its own, no library)
 COISSUE_PROBE_BIN = os.path.join(HERE, "coissue_probe")  # whether the matrix pipe and the VALU of a SIMD overlap (a HIP program of its own, no library)
+SCRATCH_BIN = os.path.join(HERE, "scratch_hand_out")  # the hand-off scratch between two threads, against a stand-in for the HIP runtime (no GPU, no checker)
 TIME_MEGA_BIN = os.path.join(HERE, "time_mega_dispatch")  # decode token timed through the dispatch point (links the library only, not the checker)
 
 
-def _build_one(src: str, out: str, with_checker: bool = True) -> str:
+def _build_one(src: str, out: str, with_checker: bool = True, extra: tuple[str, ...] = ()) -> str:
     from nihilus_amd.build import PKG_DIR, hipcc
 
     cxx = os.path.join(os.path.dirname(hipcc()), "amdclang++")
@@ -32,6 +33,7 @@ def _build_one(src: str, out: str, with_checker: bool = True) -> str:
         cxx, "-std=c++23", "-O2", "-Wall", "-Wextra", "-I", os.path.join(ROOT, "include"), os.path.join(HERE, src), "-o", out,
         "-L", PKG_DIR, "-lnihilus_q8_hip", "-Wl,-rpath,$ORIGIN/../../nihilus_amd", "-Wl,-rpath,/opt/rocm/lib",
     ]
+    cmd += extra
     if with_checker:
         cmd += ["-L", oracle_dir, "-lq8_0_oracle", "-Wl,-rpath,$ORIGIN/../../oracle"]
     res = subprocess.run(cmd, capture_output=True, text=True)
@@ -59,6 +61,7 @@ def build_host_tests() -> str:
     _build_one("test_mega_dispatch.cpp", MEGA_TEST_BIN)
     _build_one("time_mega_dispatch.cpp", TIME_MEGA_BIN, with_checker=False)
     _build_one("test_reference_mode_compiles.cpp", REFERENCE_MODE_BIN)
+    _build_one("scratch_hand_out.cpp", SCRATCH_BIN, with_checker=False, extra=("-isystem", "/opt/rocm/include", "-pthread", "-rdynamic"))
     return _build_one("test_mul_mat_dispatch.cpp", HOST_TEST_BIN)
 
 
