@@ -43,6 +43,11 @@ __device__ __forceinline__ int dot16(v4i a, v4i b) {
 	return dot4(a.w, b.w, s);
 }
 typedef float v16f __attribute__((ext_vector_type(16)));
+// fp16 scale of block t (0..3) from a row's four packed scales, as the f16 MFMA's k = 0 slot: {d_t, 0, 0, 0}
+__device__ __forceinline__ v2u scale_slot(v2u four, int t) {
+	const uint32_t dword = (t < 2) ? four.x : four.y;
+	return v2u{ (t & 1) ? (dword >> 16) : (dword & 0xFFFFu), 0u };
+}
 // One result tile (rows m0 + 8 (e / 4) + 4 half + e % 4, column n0 + r) to C, + R if given.  R may be C: an element is read and written by
 // the same thread.  The sixteen reads are issued together: written one by one behind stores that they may alias, they were a chain of
 // sixteen memory latencies.

@@ -75,14 +75,14 @@ __device__ __forceinline__ void rows_chunk_n(const uint8_t* __restrict__ w_strip
 		}
 	}
 	__builtin_amdgcn_sched_barrier(0);
-	// ---- 3. the scales, [block][row]: as fp32, or (32 rows) as the scale MFMA's operand {d in half-word t, zeros} ----
+	// ---- 3. the scales, [block][row]: as fp32, or (32 rows) as the fp16 bits that the scale MFMA takes ----
 	if (lane / R < CNT) {
 		if constexpr (rows_scale_mfma<R>) {
-			v2u* out   = reinterpret_cast<v2u*>(a_scales) + (lane / R) * GROUP_BLOCKS * R + sr;
-			out[0]	   = v2u{ sc.x & 0xFFFFu, 0u };
-			out[R]	   = v2u{ sc.x & 0xFFFF0000u, 0u };
-			out[2 * R] = v2u{ 0u, sc.y & 0xFFFFu };
-			out[3 * R] = v2u{ 0u, sc.y & 0xFFFF0000u };
+			uint32_t* out = reinterpret_cast<uint32_t*>(a_scales) + (lane / R) * GROUP_BLOCKS * R + sr;
+			out[0]		  = sc.x & 0xFFFFu;
+			out[R]		  = sc.x >> 16;
+			out[2 * R]	  = sc.y & 0xFFFFu;
+			out[3 * R]	  = sc.y >> 16;
 		} else {
 			float* out = reinterpret_cast<float*>(a_scales) + (lane / R) * GROUP_BLOCKS * R + sr;
 			out[0]	   = half_bits_to_float(static_cast<uint16_t>(sc.x & 0xFFFFu));
@@ -100,14 +100,15 @@ __device__ __forceinline__ void rows_chunk_n(const uint8_t* __restrict__ w_strip
 		for (int j = 0; j < GROUP_BLOCKS; ++j) {
 			const v4i a = *reinterpret_cast<const v4i*>(a_tiles + c * rows_group_bytes<R> + j * (32 * R) + half * (16 * R) + (r & (R - 1)) * 16);
 			if constexpr (rows_scale_mfma<R>) {
-				// the products d_x * d_w on the matrix pipe: the weights' four scales as loaded are the operand, the activation's picks
-				// block j's; the k = 4..7 slots (lanes 32..63) hold zeros
-				const v2u dx = reinterpret_cast<const v2u*>(a_scales)[(c * GROUP_BLOCKS + j) * R + (r & (R - 1))];
+				// the products d_x * d_w on the matrix pipe, block j's scales in the k = 0 slot.  Both operands are zero in every other slot
+				// (k = 4..7: lanes 32..63): a zero on one side only would make a NaN of the other side's infinity.
+				const uint32_t d = reinterpret_cast<const uint32_t*>(a_scales)[(c * GROUP_BLOCKS + j) * R + (r & (R - 1))];
+				const v2u dx	 = v2u{ half ? 0u : d, 0u };
 #pragma unroll
 				for (int k = 0; k < MATS; ++k) {
 					const v16i zi	 = { 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0 };
 					const rq_v16f zf = { 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0 };
-					const v2u dw	 = half ? v2u{ 0u, 0u } : dd[k][c];
+					const v2u dw	 = scale_slot(half ? v2u{ 0u, 0u } : dd[k][c], j);
 					const v16i s	 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, q[k][c][j], zi, 0, 0, 0);
 					const rq_v16f p	 = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(rq_v4h, dx), __builtin_bit_cast(rq_v4h, dw), zf, 0, 0, 0);
 #pragma unroll
@@ -167,7 +168,7 @@ __device__ __forceinline__ void rows_chunk(const uint8_t* __restrict__ w_strip, 
 // The workgroup's LDS: the waves' activation tiles and scales, then (behind a barrier) the partial sums in the same place.
 template<int R, int T, int MATS> struct rows_lds {
 	static constexpr int TILES	= T * rows_group_bytes<R>; // per wave
-	static constexpr int SCALES = T * GROUP_BLOCKS * R * (rows_scale_mfma<R> ? 8 : 4); // per wave
+	static constexpr int SCALES = T * GROUP_BLOCKS * R * 4; // per wave
 	static constexpr int STAGE	= ROWS_WAVES * (TILES + SCALES);
 	static constexpr int RED	= MATS * (R / 2) * ROWS_WAVES * 64 * 4;
 	static constexpr int BYTES	= STAGE > RED ? STAGE : RED;

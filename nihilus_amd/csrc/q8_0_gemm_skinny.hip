@@ -18,12 +18,6 @@ namespace nh {
 typedef _Float16 sk_v4h __attribute__((ext_vector_type(4)));
 typedef float sk_v16f __attribute__((ext_vector_type(16)));
 
-// fp16 scale of block t (0..3) from a row's four packed scales, as the f16 MFMA's k = 0 slot: {d_t, 0, 0, 0}
-__device__ __forceinline__ v2u scale_slot(v2u four, int t) {
-	const uint32_t dword = (t < 2) ? four.x : four.y;
-	return v2u{ (t & 1) ? (dword >> 16) : (dword & 0xFFFFu), 0u };
-}
-
 template<int MS, bool DUMP, int GC, int WAVES>
 __global__ __launch_bounds__(WAVES * 64, DUMP ? 2 : 4) void gemm_skinny_kernel(const uint8_t* __restrict__ W, const uint8_t* __restrict__ A, float* C, const float* R, int32_t* __restrict__ sums,
 	float* __restrict__ partials, unsigned* __restrict__ counters, int M, int N, int groups, int split_shift) {

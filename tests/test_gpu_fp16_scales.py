@@ -139,6 +139,31 @@ def test_mfma_kernels_read_extreme_scales(q8, oracle, m, n, k):
 
 
 @gpu
+@pytest.mark.parametrize("m", [1, 8, 9, 16, 17, 31, 32, 33, 70])
+def test_infinite_scales_stay_where_they_are(q8, oracle, m):
+    # an infinite scale (a block maximum above 127 * 65504) makes its own row or column infinite, in every form of the mat-mat alike,
+    # and leaves the others finite: every quant is 1, so no product is 0 * inf
+    n, k = 70, 512
+    w_d, a_d = np.full((n, k // 32), 0x3C00, dtype=np.uint16), np.full((m, k // 32), 0x3C00, dtype=np.uint16)
+    w_d[5, 2], w_d[40, 13], a_d[m // 2, 7] = 0x7C00, 0xFC00, 0x7C00
+    w = oracle.pack_blocks(w_d, np.ones((n, k // 32, 32), dtype=np.int8))
+    aq = oracle.pack_blocks(a_d, np.ones((m, k // 32, 32), dtype=np.int8))
+    want = np.full((m, n), k, dtype=np.float32)
+    want[m // 2], want[:, 5] = np.inf, np.inf
+    want[:, 40] = -np.inf
+    want[m // 2, 40] = np.nan  # inf - inf
+    wt, at = q8.tile(to_dev(w), n, k), q8.tile(to_dev(aq), m, k)
+    assert np.array_equal(to_host(q8.gemm(wt, at, m, n, k, tiled=True)), want, equal_nan=True)
+    # the pair with SiLU * up: gate and up as computed (at 17 to 32 rows the other user of the same inner loop)
+    n = 128
+    wg = oracle.pack_blocks(np.concatenate([w_d, np.full((n - 70, k // 32), 0x3C00, dtype=np.uint16)]), np.ones((n, k // 32, 32), dtype=np.int8))
+    tg = q8.tile(to_dev(wg), n, k)
+    _, gate, up = q8.gate_up_silu(tg, tg, at, m, n, k, debug=True)
+    for got in (gate, up):
+        assert np.array_equal(to_host(got)[:, :70], want, equal_nan=True)
+
+
+@gpu
 @pytest.mark.parametrize("m", [8, 32])
 @pytest.mark.parametrize("n,k", [(4096, 4096), (14336, 4096)])
 def test_crossover_rows_at_the_prefill_weights(q8, oracle, m, n, k):
