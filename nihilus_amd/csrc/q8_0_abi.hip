@@ -693,6 +693,7 @@ int nh_q8_0_debug_plan_mul_mat(int64_t M, int64_t N, int64_t K, int32_t* host_pl
 	}
 	host_plan[0] = p.kernel;
 	host_plan[1] = p.quantize_launch;
+	host_plan[7] = nh::plan_gemm(M, N, K).rows ? 1 : 0;
 	switch (p.kernel) {
 		case nh::MM_GEMV:
 		case nh::MM_GEMV_ROWS_MFMA:
@@ -701,8 +702,9 @@ int nh_q8_0_debug_plan_mul_mat(int64_t M, int64_t N, int64_t K, int32_t* host_pl
 			host_plan[4] = p.gemv_row_parts;
 			break;
 		case nh::MM_GEMM_SKINNY:
-			host_plan[2] = p.gemm.rows_splits > 0 ? 1 : p.gemm.skinny.ms;
-			host_plan[3] = p.gemm.rows_splits > 0 ? p.gemm.rows_splits : p.gemm.skinny.splits;
+			host_plan[2] = p.gemm.skinny.ms;
+			host_plan[3] = p.gemm.skinny.splits;
+			host_plan[4] = p.gemm.skinny.waves;
 			break;
 		case nh::MM_GEMM_TILE_STREAM:
 		case nh::MM_GEMM_TILE:

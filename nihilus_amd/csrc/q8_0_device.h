@@ -404,12 +404,14 @@ hipError_t launch_gemm_gate_up_silu(const void* w_gate, const void* w_up, const 
 // Tiled operands, M <= GEMM_SKINNY_MAX_M (or a tile-kernel grid of at most one workgroup per CU): the streaming MFMA kernel
 // of batched decode (q8_0_gemm_skinny.hip), which walks larger M in groups of 64 rows.
 constexpr int64_t GEMM_SKINNY_MAX_M = 64;
-// Tiled operands, 1 <= M <= 32: the streaming mat-vec's shape with the int8 MFMA as inner product (q8_0_gemm_rows.hip), K of a strip over
-// `splits` workgroups, and the same for a gate / up pair with SiLU * up and the quantizer behind it (n_ff % 128 == 0).
-// hipErrorNotReady: another stream's launch may still be handing sums over (the streaming kernel of q8_0_gemm_skinny.hip takes the shape too).
+// Tiled operands, 1 <= M <= 32: the streaming mat-vec's shape with the int8 MFMA as inner product (q8_0_gemm_rows.hip), cut as the plan
+// says, and the same for a gate / up pair with SiLU * up and the quantizer behind it (n_ff % 128 == 0, K not over workgroups).
+// hipErrorNotReady: another stream's launch may still be handing sums over (the streaming kernel of q8_0_gemm_skinny.hip takes the shape
+// too, and gives the same bits).
+struct gemm_skinny_cut;
 hipError_t prepare_gemm_rows_scratch();
-hipError_t launch_gemm_rows(const void* W, const void* Aq, float* C, const float* residual, int64_t M, int64_t N, int64_t K, int splits, hipStream_t s);
-hipError_t launch_gemm_rows_gate_up(const void* w_gate, const void* w_up, const void* aq, void* act_out, float* gate_dbg, float* up_dbg, int64_t M, int64_t n_ff, int64_t K, hipStream_t s);
+hipError_t launch_gemm_rows(const void* W, const void* Aq, float* C, const float* residual, int64_t M, int64_t N, int64_t K, const gemm_skinny_cut& cut, hipStream_t s);
+hipError_t launch_gemm_rows_gate_up(const void* w_gate, const void* w_up, const void* aq, void* act_out, float* gate_dbg, float* up_dbg, int64_t M, int64_t n_ff, int64_t K, int waves, hipStream_t s);
 // Make this device's K-split scratch buffers now (otherwise: on the first launch that needs one).
 hipError_t prepare_gemv_scratch();
 hipError_t prepare_gemm_scratch();

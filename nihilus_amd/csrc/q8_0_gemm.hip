@@ -662,7 +662,7 @@ hipError_t launch_gemm_gate_up_silu(const void* w_gate, const void* w_up, const 
 		return hipSuccess;
 	}
 	if (gate_up_rows_suits(M, n_ff, K)) {
-		return launch_gemm_rows_gate_up(w_gate, w_up, aq, act_out, gate_dbg, up_dbg, M, n_ff, K, s);
+		return launch_gemm_rows_gate_up(w_gate, w_up, aq, act_out, gate_dbg, up_dbg, M, n_ff, K, plan_gemm_skinny(M, n_ff, K).waves, s);
 	}
 	gemm_tile_cut cut{};
 	if (plan_gate_up_fused(M, n_ff, K, &cut)) {
@@ -722,10 +722,10 @@ hipError_t launch_gemm(const void* W, const void* Aq, float* C, int32_t* sums, i
 		const gemm_plan plan = plan_gemm(M, N, K); // which kernel and how it cuts the work: q8_0_plan.h
 		if (plan.kernel == MM_GEMM_SKINNY) {
 			// (a launch that hands K parts' sums over by epoch cannot be replayed from a graph, and is refused while another stream's is
-			// under way: the streaming kernel, with counters or without a K split, takes those calls)
-			if (plan.rows_splits == 1 || (plan.rows_splits > 1 && !stream_is_capturing(s))) {
-				const hipError_t e = launch_gemm_rows(W, Aq, C, residual, M, N, K, plan.rows_splits, s);
-				if (e != hipErrorNotReady || plan.rows_splits == 1) {
+			// under way: the streaming kernel, whose cut and order of additions are the same, takes those calls)
+			if (plan.rows && (plan.skinny.splits == 1 || !stream_is_capturing(s))) {
+				const hipError_t e = launch_gemm_rows(W, Aq, C, residual, M, N, K, plan.skinny, s);
+				if (e != hipErrorNotReady) {
 					return e;
 				}
 			}

@@ -165,78 +165,89 @@ __device__ __forceinline__ void rows_chunk(const uint8_t* __restrict__ w_strip, 
 	}
 }
 
-// The workgroup's LDS: the waves' activation tiles and scales, then (behind a barrier) the partial sums in the same place.
-template<int R, int T, int MATS> struct rows_lds {
+// The workgroup's LDS: the waves' activation tiles and scales, then (behind a barrier) the last set's partial sums in the same place; the
+// first of two sets' behind them.
+template<int R, int T, int MATS, int SETS> struct rows_lds {
 	static constexpr int TILES	= T * rows_group_bytes<R>; // per wave
 	static constexpr int SCALES = T * GROUP_BLOCKS * R * 4; // per wave
-	static constexpr int STAGE	= ROWS_WAVES * (TILES + SCALES);
-	static constexpr int RED	= MATS * (R / 2) * ROWS_WAVES * 64 * 4;
-	static constexpr int BYTES	= STAGE > RED ? STAGE : RED;
+	static constexpr int STAGE	= SK_WAVES * (TILES + SCALES);
+	static constexpr int RED	= MATS * (R / 2) * SK_WAVES * 64 * 4;
+	static constexpr int FIRST	= STAGE > RED ? STAGE : RED;
+	static constexpr int BYTES	= FIRST + (SETS - 1) * RED;
+	static_assert(SK_WAVES * TILES <= 65536, "the memory -> LDS transfers address the tiles with 16 bits");
+	static_assert(SETS == 1 || SETS == 2);
 };
 
-// A workgroup's K part of a strip, all waves' partial sums left in LDS: red[matrix][value][wave][lane]
-template<int R, int T, int MATS>
+// A workgroup's K part of a strip, all waves' partial sums left in LDS: [matrix][value][wave][lane].  With two sets the eight waves walk
+// the ranges that sixteen would have, one after the other: as many additions in a row as sixteen waves make, with no more than eight
+// waves' registers, LDS or launch.
+template<int R, int T, int MATS, int SETS>
 __device__ __forceinline__ void rows_strip(const uint8_t* __restrict__ w_strip, const uint8_t* __restrict__ w_strip2, const uint8_t* __restrict__ A, uint8_t* lds, int groups, int split_shift, int split,
 	int lane, int wave) {
-	using L = rows_lds<R, T, MATS>;
-	int g0, g1;
-	wave_k_range(groups, split_shift, split, ROWS_WAVES, wave, g0, g1);
+	using L = rows_lds<R, T, MATS, SETS>;
 	uint8_t* a_tiles = lds + wave * L::TILES;
-	uint8_t* a_scales = lds + ROWS_WAVES * L::TILES + wave * L::SCALES;
-	float acc[MATS][R / 2];
+	uint8_t* a_scales = lds + SK_WAVES * L::TILES + wave * L::SCALES;
+	for (int set = 0; set < SETS; ++set) {
+		int g0, g1;
+		wave_k_range(groups, split_shift, split, SETS * SK_WAVES, set * SK_WAVES + wave, g0, g1);
+		float acc[MATS][R / 2];
 #pragma unroll
-	for (int k = 0; k < MATS; ++k) {
+		for (int k = 0; k < MATS; ++k) {
 #pragma unroll
-		for (int e = 0; e < R / 2; ++e) {
-			acc[k][e] = 0.0f;
+			for (int e = 0; e < R / 2; ++e) {
+				acc[k][e] = 0.0f;
+			}
 		}
-	}
-	for (int gc = g0; gc < g1; gc += T) {
-		rows_chunk<R, T, MATS>(w_strip, w_strip2, A, a_tiles, a_scales, gc, min(T, g1 - gc), lane, acc);
-		__builtin_amdgcn_wave_barrier(); // the next chunk overwrites this wave's tiles
-	}
-	__syncthreads(); // everybody is through with the tiles
-	float* red = reinterpret_cast<float*>(lds);
+		for (int gc = g0; gc < g1; gc += T) {
+			rows_chunk<R, T, MATS>(w_strip, w_strip2, A, a_tiles, a_scales, gc, min(T, g1 - gc), lane, acc);
+			__builtin_amdgcn_wave_barrier(); // the next chunk overwrites this wave's tiles
+		}
+		const bool last = set == SETS - 1;
+		if (last) {
+			__syncthreads(); // everybody is through with the tiles
+		}
+		float* red = reinterpret_cast<float*>(lds + (last ? 0 : L::FIRST));
 #pragma unroll
-	for (int k = 0; k < MATS; ++k) {
+		for (int k = 0; k < MATS; ++k) {
 #pragma unroll
-		for (int e = 0; e < R / 2; ++e) {
-			red[((k * (R / 2) + e) * ROWS_WAVES + wave) * 64 + lane] = acc[k][e];
+			for (int e = 0; e < R / 2; ++e) {
+				red[((k * (R / 2) + e) * SK_WAVES + wave) * 64 + lane] = acc[k][e];
+			}
 		}
 	}
 	__syncthreads();
 }
-// output (row m, strip column l) of matrix k: the waves' partial sums in wave order
-template<int R> __device__ __forceinline__ float rows_total(const uint8_t* lds, int k, int m, int l) {
-	const float* red = reinterpret_cast<const float*>(lds);
+// output (row m, strip column l) of matrix k: the waves' partial sums in the streaming kernel's order (q8_0_gemm_skinny.hip), of which this
+// is the form for few rows: the same cut, the same chains of additions, the same tree over them, so the same bits.  (One wave after the
+// other, and longer chains, were also up to 35 % further from the sums in 64 bits.)
+template<int R, int T, int MATS, int SETS> __device__ __forceinline__ float rows_total(const uint8_t* lds, int k, int m, int l) {
 	const int e = 4 * (m >> 3) + (m & 3), at = 32 * ((m >> 2) & 1) + l;
-	float total = 0.0f;
-#pragma unroll
-	for (int w = 0; w < ROWS_WAVES; ++w) {
-		total += red[((k * (R / 2) + e) * ROWS_WAVES + w) * 64 + at];
-	}
-	return total;
+	const auto eight = [&](const uint8_t* red) {
+		const float* p = reinterpret_cast<const float*>(red) + (k * (R / 2) + e) * (SK_WAVES * 64) + at;
+		return ((p[64 * 0] + p[64 * 4]) + (p[64 * 2] + p[64 * 6])) + ((p[64 * 1] + p[64 * 5]) + (p[64 * 3] + p[64 * 7]));
+	};
+	return SETS == 1 ? eight(lds) : eight(lds + rows_lds<R, T, MATS, SETS>::FIRST) + eight(lds);
 }
 
 } // namespace
 
-template<int R, int T>
-__global__ __launch_bounds__(ROWS_WAVES * 64, 4) void gemm_rows_kernel(const uint8_t* __restrict__ W, const uint8_t* __restrict__ A, float* C, const float* residual, uint64_t* __restrict__ tagged,
+template<int R, int T, int SETS>
+__global__ __launch_bounds__(SK_WAVES * 64, 4) void gemm_rows_kernel(const uint8_t* __restrict__ W, const uint8_t* __restrict__ A, float* C, const float* residual, uint64_t* __restrict__ tagged,
 	unsigned epoch, int M, int N, int groups, int split_shift) {
-	__shared__ __align__(16) uint8_t lds[rows_lds<R, T, 1>::BYTES];
+	__shared__ __align__(16) uint8_t lds[rows_lds<R, T, 1, SETS>::BYTES];
 	const int tid	= threadIdx.x;
 	const int lane	= tid & 63;
 	const int wave	= __builtin_amdgcn_readfirstlane(tid >> 6);
 	const int strip = static_cast<int>(blockIdx.x >> split_shift);
 	const int split = static_cast<int>(blockIdx.x) & ((1 << split_shift) - 1);
-	rows_strip<R, T, 1>(W + macro_offset(strip, 0, groups), nullptr, A, lds, groups, split_shift, split, lane, wave);
+	rows_strip<R, T, 1, SETS>(W + macro_offset(strip, 0, groups), nullptr, A, lds, groups, split_shift, split, lane, wave);
 #pragma unroll
-	for (int o = 0; o < R * STRIP_ROWS; o += ROWS_WAVES * 64) {
+	for (int o = 0; o < R * STRIP_ROWS; o += SK_WAVES * 64) {
 		const int m = (o + tid) >> 5, l = tid & 31;
 		if (m >= M || m >= R) {
 			continue;
 		}
-		const float total = rows_total<R>(lds, 0, m, l);
+		const float total = rows_total<R, T, 1, SETS>(lds, 0, m, l);
 		const int n		  = strip * STRIP_ROWS + l;
 		float* cm		  = C + static_cast<int64_t>(m) * N;
 		const float* rm	  = residual ? residual + static_cast<int64_t>(m) * N : nullptr; // may be cm: read before the write, by the same thread
@@ -252,23 +263,23 @@ __global__ __launch_bounds__(ROWS_WAVES * 64, 4) void gemm_rows_kernel(const uin
 
 // The gate and up strips of the same 32 rows against one activation, then silu(g) * u and quantize_row_q8_0: the 32 values of an
 // activation row are one block of the down projection's operand and sit in one half-wave.
-template<int R, int T>
-__global__ __launch_bounds__(ROWS_WAVES * 64, 4) void gemm_rows_gate_up_kernel(const uint8_t* __restrict__ W_gate, const uint8_t* __restrict__ W_up, const uint8_t* __restrict__ A,
+template<int R, int T, int SETS>
+__global__ __launch_bounds__(SK_WAVES * 64, 4) void gemm_rows_gate_up_kernel(const uint8_t* __restrict__ W_gate, const uint8_t* __restrict__ W_up, const uint8_t* __restrict__ A,
 	uint8_t* __restrict__ act_out, float* __restrict__ gate_out, float* __restrict__ up_out, int M, int N, int groups) {
-	__shared__ __align__(16) uint8_t lds[rows_lds<R, T, 2>::BYTES];
+	__shared__ __align__(16) uint8_t lds[rows_lds<R, T, 2, SETS>::BYTES];
 	const int tid	= threadIdx.x;
 	const int lane	= tid & 63;
 	const int wave	= __builtin_amdgcn_readfirstlane(tid >> 6);
 	const int strip = static_cast<int>(blockIdx.x);
-	rows_strip<R, T, 2>(W_gate + macro_offset(strip, 0, groups), W_up + macro_offset(strip, 0, groups), A, lds, groups, 0, 0, lane, wave);
+	rows_strip<R, T, 2, SETS>(W_gate + macro_offset(strip, 0, groups), W_up + macro_offset(strip, 0, groups), A, lds, groups, 0, 0, lane, wave);
 	uint8_t* macro = act_out + macro_offset(0, strip / GROUP_BLOCKS, N / GROUP_K);
 	const int t	   = strip % GROUP_BLOCKS;
 #pragma unroll
-	for (int o = 0; o < STRIP_ROWS * STRIP_ROWS; o += ROWS_WAVES * 64) {
+	for (int o = 0; o < STRIP_ROWS * STRIP_ROWS; o += SK_WAVES * 64) {
 		const int m = (o + tid) >> 5, l = tid & 31;
 		float v = 0.0f; // rows past M are the operand's padding: zero blocks
 		if (m < M && m < R) {
-			const float g = rows_total<R>(lds, 0, m, l), u = rows_total<R>(lds, 1, m, l);
+			const float g = rows_total<R, T, 2, SETS>(lds, 0, m, l), u = rows_total<R, T, 2, SETS>(lds, 1, m, l);
 			v = silu_mul(g, u);
 			if (gate_out) {
 				gate_out[static_cast<int64_t>(m) * N + strip * STRIP_ROWS + l] = g;
@@ -352,45 +363,41 @@ hipError_t prepare_gemm_rows_scratch() {
 	return get_rows_scratch(&sc, nullptr, nullptr);
 }
 
-// 1 <= M <= 32, K > 0; splits: plan_gemm_rows_splits
-hipError_t launch_gemm_rows(const void* W, const void* Aq, float* C, const float* residual, int64_t M, int64_t N, int64_t K, int splits, hipStream_t s) {
-	const int64_t strips = (N + STRIP_ROWS - 1) / STRIP_ROWS;
+template<int SETS> static hipError_t launch_rows_t(const uint8_t* w, const uint8_t* a, float* C, const float* residual, int m, int n, int groups, int splits, const rows_scratch& sc, hipStream_t s) {
+	int shift = 0;
+	while ((1 << shift) < splits) {
+		++shift;
+	}
+	const dim3 grid(static_cast<unsigned>((n + STRIP_ROWS - 1) / STRIP_ROWS * splits)), block(SK_WAVES * 64);
+	auto launch = [&](auto kernel) { return launch_kernel(KIND_GEMM, kernel, grid, block, 0, s, w, a, C, residual, sc.tagged, sc.epoch, m, n, groups, shift); };
+	return m <= 8 ? launch(gemm_rows_kernel<8, 2, SETS>) : m <= 16 ? launch(gemm_rows_kernel<16, 2, SETS>) : launch(gemm_rows_kernel<32, 2, SETS>);
+}
+
+// 1 <= M <= 32, K > 0; cut: plan_gemm_skinny, where gemm_rows_fits
+hipError_t launch_gemm_rows(const void* W, const void* Aq, float* C, const float* residual, int64_t M, int64_t N, int64_t K, const gemm_skinny_cut& cut, hipStream_t s) {
 	rows_scratch sc;
 	scratch_hold hold;
-	if (splits > 1) {
+	if (cut.splits > 1) {
 		const hipError_t e = get_rows_scratch(&sc, &hold, s);
 		if (e != hipSuccess) {
 			return e;
 		}
 	}
-	int shift = 0;
-	while ((1 << shift) < splits) {
-		++shift;
-	}
-	const dim3 grid(static_cast<unsigned>(strips * splits)), block(ROWS_WAVES * 64);
 	const uint8_t *w = static_cast<const uint8_t*>(W), *a = static_cast<const uint8_t*>(Aq);
 	const int m = static_cast<int>(M), n = static_cast<int>(N), groups = static_cast<int>(K / GROUP_K);
-	if (M <= 8) {
-		return launch_kernel(KIND_GEMM, gemm_rows_kernel<8, 2>, grid, block, 0, s, w, a, C, residual, sc.tagged, sc.epoch, m, n, groups, shift);
-	}
-	if (M <= 16) {
-		return launch_kernel(KIND_GEMM, gemm_rows_kernel<16, 2>, grid, block, 0, s, w, a, C, residual, sc.tagged, sc.epoch, m, n, groups, shift);
-	}
-	return launch_kernel(KIND_GEMM, gemm_rows_kernel<32, 2>, grid, block, 0, s, w, a, C, residual, sc.tagged, sc.epoch, m, n, groups, shift);
+	return cut.waves == SK_WAVES ? launch_rows_t<1>(w, a, C, residual, m, n, groups, cut.splits, sc, s) : launch_rows_t<2>(w, a, C, residual, m, n, groups, cut.splits, sc, s);
 }
 
-hipError_t launch_gemm_rows_gate_up(const void* w_gate, const void* w_up, const void* aq, void* act_out, float* gate_dbg, float* up_dbg, int64_t M, int64_t n_ff, int64_t K, hipStream_t s) {
-	const dim3 grid(static_cast<unsigned>(n_ff / STRIP_ROWS)), block(ROWS_WAVES * 64);
+template<int SETS> static hipError_t launch_rows_gate_up_t(const uint8_t* wg, const uint8_t* wu, const uint8_t* a, uint8_t* out, float* gate_dbg, float* up_dbg, int m, int n, int groups, hipStream_t s) {
+	auto launch = [&](auto kernel) { return launch_kernel(KIND_GEMM, kernel, dim3(static_cast<unsigned>(n / STRIP_ROWS)), dim3(SK_WAVES * 64), 0, s, wg, wu, a, out, gate_dbg, up_dbg, m, n, groups); };
+	return m <= 8 ? launch(gemm_rows_gate_up_kernel<8, 1, SETS>) : m <= 16 ? launch(gemm_rows_gate_up_kernel<16, 1, SETS>) : launch(gemm_rows_gate_up_kernel<32, 1, SETS>);
+}
+
+hipError_t launch_gemm_rows_gate_up(const void* w_gate, const void* w_up, const void* aq, void* act_out, float* gate_dbg, float* up_dbg, int64_t M, int64_t n_ff, int64_t K, int waves, hipStream_t s) {
 	const uint8_t *wg = static_cast<const uint8_t*>(w_gate), *wu = static_cast<const uint8_t*>(w_up), *a = static_cast<const uint8_t*>(aq);
 	uint8_t* out = static_cast<uint8_t*>(act_out);
 	const int m = static_cast<int>(M), n = static_cast<int>(n_ff), groups = static_cast<int>(K / GROUP_K);
-	if (M <= 8) {
-		return launch_kernel(KIND_GEMM, gemm_rows_gate_up_kernel<8, 1>, grid, block, 0, s, wg, wu, a, out, gate_dbg, up_dbg, m, n, groups);
-	}
-	if (M <= 16) {
-		return launch_kernel(KIND_GEMM, gemm_rows_gate_up_kernel<16, 1>, grid, block, 0, s, wg, wu, a, out, gate_dbg, up_dbg, m, n, groups);
-	}
-	return launch_kernel(KIND_GEMM, gemm_rows_gate_up_kernel<32, 1>, grid, block, 0, s, wg, wu, a, out, gate_dbg, up_dbg, m, n, groups);
+	return waves == SK_WAVES ? launch_rows_gate_up_t<1>(wg, wu, a, out, gate_dbg, up_dbg, m, n, groups, s) : launch_rows_gate_up_t<2>(wg, wu, a, out, gate_dbg, up_dbg, m, n, groups, s);
 }
 
 } // namespace nh

@@ -82,8 +82,12 @@ inline bool plan_gemm_tile_split(int64_t M, int64_t N, int64_t K, gemm_tile_cut*
 
 // The weight-streaming MFMA kernel's cut: MS activation strips per workgroup, K of a strip over `splits` workgroups of `waves` waves.
 struct gemm_skinny_cut {
-	int ms, splits, waves;
+	int ms, splits, waves; // waves: 8 or 16, the shares of K that a workgroup adds
 };
+constexpr int64_t GEMM_ROWS_MAX = 32;
+inline int gemm_rows_operand(int64_t M) { // operand rows the rows kernel is instantiated for
+	return M <= 8 ? 8 : M <= 16 ? 16 : 32;
+}
 inline gemm_skinny_cut plan_gemm_skinny(int64_t M, int64_t N, int64_t K) {
 	gemm_skinny_cut c{};
 	const int groups	 = static_cast<int>(K / GROUP_K);
@@ -92,44 +96,54 @@ inline gemm_skinny_cut plan_gemm_skinny(int64_t M, int64_t N, int64_t K) {
 	// without them: 64 rows against 128 weight strips are better off as 256 workgroups of one strip each.
 	c.ms				= (m_strips <= 1 || strips * ((m_strips + 1) / 2) < 256) ? 1 : 2;
 	const int64_t units = strips * ((m_strips + c.ms - 1) / c.ms);
-	c.splits			= 1;
+	// K goes over sets of eight waves.  The hand-off between workgroups is expensive here (a partial tile of 16 values per lane and strip, an
+	// arrival counter, the last arriver reading every share): only until every CU has a workgroup (and every wave
+	// keeps at least two groups, one step of the kernel's walk: [4096 x 4096] at M = 32 12.1 -> 10.8 us, [1024 x 8192] at M = 64
+	// 14.9 -> 13.2 us against keeping four), or when a wave would otherwise walk more than sixteen groups.  Measured on
+	// [8192 x 28672] at M = 16: 68 us with eight sets per strip, 51 us with two.
+	const auto sets_for = [&](int waves) {
+		int sets = 1;
+		while (waves == SK_WAVES && units * sets < 256 && groups >= 4 * SK_WAVES * sets && units * sets * 2 <= SK_MAX_SPLIT_UNITS && units <= SK_MAX_SPLIT_STRIPS) {
+			sets *= 2;
+		}
+		while (groups > 16 * waves * sets && units * sets * 2 <= SK_MAX_SPLIT_UNITS && units <= SK_MAX_SPLIT_STRIPS) {
+			sets *= 2;
+		}
+		return sets;
+	};
+	if (M <= GEMM_ROWS_MAX) {
+		// Up to 32 rows: one cut for the rows kernel (q8_0_gemm_rows.hip) and for the streaming kernel, which takes its calls where the hand-off's
+		// tags cannot be used, so that both add the same sums in the same order.  The rows kernel's hand-off is cheaper: until the launch has
+		// a workgroup per CU, while every wave keeps a group ([4096 x 4096] at 4 rows 5.7 us with 256 workgroups, 6.0 with 512;
+		// [4096 x 14336] 12.6 and 13.3; [1024 x 4096] 4.6 us with 128).  Where the rule above makes more sets than that, a workgroup takes
+		// two of them (sixteen waves; in the rows kernel eight, one set after the other): no more additions in a row than there, and nothing
+		// more to hand over.  One set instead, [6144 x 6144] at 8 / 32 rows: 8.7 / 11.5 us against 9.0 / 12.1, but [8192 x 28672] 2.0e-7 from
+		// the sums in 64 bits where two sets are 1.5e-7, and [5120 x 5120] 9.9e-8 against 8.2e-8.  (Sixteen waves in the rows kernel too:
+		// 9.0 / 12.8 us.)
+		const int sets = sets_for(SK_WAVES);
+		c.waves		   = SK_WAVES;
+		c.splits	   = 1;
+		while (strips * c.splits * 2 <= 256 && groups >= 2 * SK_WAVES * c.splits && strips * gemm_rows_operand(M) * c.splits * 2 <= GEMV_MAX_SPLIT_UNITS) {
+			c.splits *= 2;
+		}
+		if (sets > c.splits) {
+			c.waves	 = SK_WIDE_WAVES;
+			c.splits = sets / 2;
+		}
+		return c;
+	}
 	// 129 to 255 units and a K that eight waves would split: two workgroups each leave some CUs two and some one or none, and the launch
 	// takes as long as the ones with two.  One workgroup of sixteen waves per unit has the same waves on every CU it uses and nothing to hand
 	// over.  Measured, us, split / this: [1024 x 8192] at 200 rows 13.6 / 11.9, [1024 x 4096] at 224 rows 9.5 / 7.7, [3072 x 12288] at 40 rows
 	// 20.6 / 18.0, [768 x 4096] at 180 rows 9.0 / 7.6, [4064 x 4096] at 50 rows 11.0 / 9.3, [2080 x 4096] at 64 rows 9.8 / 9.1, [640 x 14336] at
 	// 256 rows 20.1 / 19.4.  Outside it does not pay: at 128 units, which the split makes into a workgroup per CU, 7.4 / 7.6 ([1024 x 4096] at
 	// 117 rows) and 9.6 / 12.2 (K = 8192); at 256, 12.8 / 12.5 ([4096 x 4096] at 117 rows) and 8.5 / 8.8 (at 64).
-	c.waves = (units > 128 && units < 256 && groups >= 4 * SK_WAVES) ? SK_WIDE_WAVES : SK_WAVES;
-	// The hand-off between workgroups is expensive here (a partial tile of 16 values per lane and strip, an arrival counter,
-	// the last arriver reading every share): K goes over several workgroups only until every CU has one (and every wave
-	// keeps at least two groups, one step of the kernel's walk: [4096 x 4096] at M = 32 12.1 -> 10.8 us, [1024 x 8192] at M = 64
-	// 14.9 -> 13.2 us against keeping four), or when a wave would otherwise walk more than sixteen groups.  Measured on
-	// [8192 x 28672] at M = 16: 68 us with eight workgroups per strip, 51 us with two.
-	while (c.waves == SK_WAVES && units * c.splits < 256 && groups >= 4 * SK_WAVES * c.splits && units * c.splits * 2 <= SK_MAX_SPLIT_UNITS && units <= SK_MAX_SPLIT_STRIPS) {
-		c.splits *= 2;
-	}
-	while (groups > 16 * c.waves * c.splits && units * c.splits * 2 <= SK_MAX_SPLIT_UNITS && units <= SK_MAX_SPLIT_STRIPS) {
-		c.splits *= 2;
-	}
+	c.waves	 = (units > 128 && units < 256 && groups >= 4 * SK_WAVES) ? SK_WIDE_WAVES : SK_WAVES;
+	c.splits = sets_for(c.waves);
 	return c;
 }
 
-// The same for up to 32 rows (q8_0_gemm_rows.hip): workgroups of ROWS_WAVES waves, a strip's K over `splits` of them.
-constexpr int ROWS_WAVES		= 8;
-constexpr int64_t GEMM_ROWS_MAX = 32;
-inline int gemm_rows_operand(int64_t M) { // operand rows the kernel is instantiated for
-	return M <= 8 ? 8 : M <= 16 ? 16 : 32;
-}
-// Until the launch has a workgroup per CU, while every wave keeps a group.  ([4096 x 4096] at 4 rows 5.7 us with 256 workgroups, 6.0 with
-// 512; [4096 x 14336] 12.6 and 13.3; [1024 x 4096] 4.6 us with 128, 8.0 with 32 (the kernel it replaced there).)
-inline int plan_gemm_rows_splits(int64_t M, int64_t N, int64_t K) {
-	const int64_t strips = (N + STRIP_ROWS - 1) / STRIP_ROWS, groups = K / GROUP_K;
-	int splits			 = 1;
-	while (strips * splits * 2 <= 256 && groups >= 2 * ROWS_WAVES * splits && strips * gemm_rows_operand(M) * splits * 2 <= GEMV_MAX_SPLIT_UNITS) {
-		splits *= 2;
-	}
-	return splits;
-}
+// Up to 32 rows the kernel of q8_0_gemm_rows.hip, with the cut above, where it is the faster one.
 // Measured against the kernels that had these shapes (weights rotated, kernel times, us):
 //   rows                4            16            32
 //   [4096 x 4096]    5.7 /  9.8    6.3 /  9.1    8.7 /  9.4   (streaming kernel with eight waves' operand tiles from L2)
@@ -149,12 +163,17 @@ inline bool gemm_rows_suits(int64_t M, int64_t N, int64_t K) {
 	return column_blocks < GEMM_STREAM_TILE_MIN_COLUMN_BLOCKS || (M <= 16 && K <= 4096);
 }
 
+// whether the rows kernel's tagged sums hold this cut
+inline bool gemm_rows_fits(int64_t M, int64_t N, const gemm_skinny_cut& cut) {
+	return cut.splits == 1 || (N + STRIP_ROWS - 1) / STRIP_ROWS * gemm_rows_operand(M) * cut.splits <= GEMV_MAX_SPLIT_UNITS;
+}
+
 // A mat-mat on tiled, already quantized operands (nh_q8_0_gemm_tiled, and the second half of nh_q8_0_mul_mat wherever the activations are quantized by a launch of their own).
 struct gemm_plan {
 	int kernel; // MM_GEMM_SKINNY, MM_GEMM_TILE_STREAM or MM_GEMM_TILE (MM_NOTHING for an empty problem)
 	gemm_tile_cut tile; // when a tile kernel runs
 	gemm_skinny_cut skinny; // when the streaming kernel runs
-	int rows_splits; // > 0: it runs as the form for up to 32 rows, with a strip's K over this many workgroups
+	bool rows; // the streaming kernel's form for up to 32 rows, with the same cut
 };
 inline gemm_plan plan_gemm(int64_t M, int64_t N, int64_t K) {
 	gemm_plan p{};
@@ -200,9 +219,7 @@ inline gemm_plan plan_gemm(int64_t M, int64_t N, int64_t K) {
 	} else if (M <= GEMM_SKINNY_MAX_M || tile_workgroups <= 256) {
 		p.kernel = MM_GEMM_SKINNY;
 		p.skinny = plan_gemm_skinny(M, N, K);
-		if (gemm_rows_suits(M, N, K)) {
-			p.rows_splits = plan_gemm_rows_splits(M, N, K);
-		}
+		p.rows	 = gemm_rows_suits(M, N, K) && gemm_rows_fits(M, N, p.skinny);
 	} else {
 		p.kernel = MM_GEMM_TILE;
 		p.tile	 = plan_gemm_tile(M, N, K, false);
@@ -220,7 +237,7 @@ inline bool gate_up_rows_suits(int64_t M, int64_t n_ff, int64_t K) {
 	if (M <= 0 || M > GEMM_ROWS_MAX || n_ff <= 0 || K <= 0 || n_ff % GROUP_K != 0 || K % GROUP_K != 0) {
 		return false;
 	}
-	return plan_gemm_rows_splits(M, n_ff, K) == 1 && (M <= 16 || gemm_rows_suits(M, n_ff, K));
+	return plan_gemm_skinny(M, n_ff, K).splits == 1 && (M <= 16 || gemm_rows_suits(M, n_ff, K));
 }
 // The tile kernel's fused form, K sets included, wherever its grid has the chip's SIMDs two waves each, or about one where the matrices are
 // small enough that the launches saved count for more than idle CUs.  Whole calls, us, fused / three launches:

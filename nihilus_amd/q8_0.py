@@ -49,11 +49,11 @@ def plan_mul_mat(m: int, n: int, k: int) -> dict:
 
     raw = (ctypes.c_int32 * 8)()
     _lib.check("nh_q8_0_debug_plan_mul_mat", _lib.lib().nh_q8_0_debug_plan_mul_mat(m, n, k, raw))
-    plan = {"kernel": KERNEL_NAMES[raw[0]], "quantize_launch": bool(raw[1])}
+    plan = {"kernel": KERNEL_NAMES[raw[0]], "quantize_launch": bool(raw[1]), "gemm_rows": bool(raw[7])}
     if raw[0] in (1, 6):
         plan.update(k_splits=raw[2], groups_per_wave=raw[3], row_parts=raw[4])
     elif raw[0] == 3:
-        plan.update(activation_strips=raw[2], k_splits=raw[3])
+        plan.update(activation_strips=raw[2], k_splits=raw[3], waves=raw[4])
     elif raw[0] in (4, 5):
         plan.update(activation_strips=raw[2], k_sets=raw[3], k_splits=raw[4], grid=(raw[5], raw[6]))
     return plan

@@ -14,8 +14,10 @@ def _gemm(oracle, w, aq, m, n, k):  # the threaded checker takes block counts th
 # rows at either side of the 8-, 16- and 32-row operands; N with a ragged last strip; K of one group, fewer groups than waves, a last chunk
 # of one group, and long enough for two and four workgroups per strip
 @pytest.mark.parametrize("m", [1, 2, 8, 9, 16, 17, 31, 32])
-@pytest.mark.parametrize("n,k", [(33, 128), (100, 128 * 7), (8200, 128 * 17), (257, 128 * 35), (1024, 4096), (4096, 128 * 21)])
+# ... and for two sets of shares per workgroup (129 to 255 strips, or more than 128 groups), evenly shared and not
+@pytest.mark.parametrize("n,k", [(33, 128), (100, 128 * 7), (8200, 128 * 17), (257, 128 * 35), (1024, 4096), (4096, 128 * 21), (4100, 4096), (5120, 128 * 37), (8200, 128 * 131)])
 def test_gemm_rows(q8, oracle, m, n, k):
+    assert q8.plan_mul_mat(m, n, k)["gemm_rows"]
     w = oracle.fill_weights(m + n, n, k)
     x = oracle.fill_activations(m + k, m * k).reshape(m, k)
     aq = oracle.quantize_rows(x)
@@ -32,7 +34,7 @@ def test_gemm_rows(q8, oracle, m, n, k):
 
 # [2 x n_ff x k] with a strip's K uncut (>= 129 strips, or a short K), several chunks per wave and ragged rows
 @pytest.mark.parametrize("m", [1, 8, 11, 16, 23, 32])
-@pytest.mark.parametrize("n_ff,k", [(128, 128), (4224, 128 * 9), (8192, 2048)])
+@pytest.mark.parametrize("n_ff,k", [(128, 128), (4224, 128 * 9), (8192, 2048), (4224, 128 * 34)])
 def test_gate_up_rows(q8, oracle, m, n_ff, k):
     lib = q8._lib.lib()
     assert lib.nh_q8_0_gate_up_silu_workspace_bytes(m, n_ff, k) == 0
@@ -50,6 +52,32 @@ def test_gate_up_rows(q8, oracle, m, n_ff, k):
     assert np.array_equal(whole[:m], oracle.silu_mul_quantize_rows(gate, up))
     assert not whole[m:].any()
     assert np.array_equal(to_host(q8.gate_up_silu(tg, tu, at, m, n_ff, k)), to_host(act))
+
+
+# A captured call, whose hand-off cannot be the eager call's, runs the streaming kernel: the same sums in the same order, so the same bits.
+# Two and four workgroups per strip, K shared unevenly, ragged strips; 100 strips with two sets of shares in each of two workgroups; and one workgroup.
+@pytest.mark.parametrize("m", [3, 16, 17])
+@pytest.mark.parametrize("n,k,splits,waves", [(4096, 4096, 2, 8), (1024, 4096, 4, 8), (257, 128 * 35, 4, 8), (4090, 128 * 21, 2, 8), (3200, 8192, 2, 16), (5120, 5120, 1, 16)])
+def test_captured_and_eager_calls_have_the_same_bits(q8, oracle, m, n, k, splits, waves):
+    import torch
+
+    plan = q8.plan_mul_mat(17, n, k)  # (fewer rows would report the kernel that mul_mat quantizes in)
+    assert plan["kernel"] == "gemm_skinny" and (plan["k_splits"], plan["waves"]) == (splits, waves) and q8.plan_mul_mat(m, n, k)["gemm_rows"]
+    wt = q8.tile(q8.fill_weight_blocks(n + m, n, k), n, k)
+    xs = [q8.fill_activations(30 + i, m * k).reshape(m, k) for i in range(3)]
+    at = q8.quantize_row_q8_0(xs[0], tiled=True)
+    c = torch.empty((m, n), dtype=torch.float32, device="cuda")
+    q8._lib.check("nh_q8_0_prepare", q8._lib.lib().nh_q8_0_prepare())
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        q8._lib.check("gemm", q8._lib.lib().nh_q8_0_gemm_tiled(wt.data_ptr(), at.data_ptr(), c.data_ptr(), m, n, k, torch.cuda.current_stream().cuda_stream))
+    for x in xs:
+        at.copy_(q8.quantize_row_q8_0(x, tiled=True))
+        c.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(to_host(c).view(np.uint32), to_host(q8.gemm(wt, at, m, n, k, tiled=True)).view(np.uint32))
 
 
 def test_gemm_rows_in_a_graph(q8, oracle):

@@ -98,3 +98,12 @@ def test_empty_and_rejected_shapes():
         q8_0.plan_mul_mat(4, 4096, 100)
     with pytest.raises(q8_0._lib.Q8Error):
         q8_0.plan_mul_mat(-1, 4096, 4096)
+
+
+def test_up_to_32_rows_every_wave_keeps_its_share_of_the_sums():
+    # sets of eight waves that K goes over, in one workgroup or several: what bounds the additions in a row, and so the rounding error.
+    # 129 to 255 strips and long K: two sets in one workgroup
+    for (m, n, k), sets in {(4, 8192, 28672): 2, (24, 5120, 5120): 2, (24, 6144, 6144): 2, (24, 3200, 8192): 4, (32, 4096, 14336): 2, (8, 14336, 4096): 1, (24, 1024, 4096): 4}.items():
+        p = q8_0.plan_mul_mat(m, n, k)
+        assert p["kernel"] == "gemm_skinny" and p["gemm_rows"] and p["k_splits"] * p["waves"] == 8 * sets, (m, n, k, p)
+    assert not q8_0.plan_mul_mat(33, 5120, 5120)["gemm_rows"] and not q8_0.plan_mul_mat(24, 28672, 8192)["gemm_rows"]
