@@ -107,7 +107,7 @@ int nh_q8_0_clear_error(void);
  * previous setting (1 or 0); 1 by default.  Takes effect for calls made afterwards; needs no GPU. */
 int nh_q8_0_set_in_kernel_waits(int enabled);
 /* Allocates, for the current device, the three internal scratch buffers that K-split launches hand partial sums through
- * (about 2.6, 32 and 4 MiB; otherwise made by the first launch that needs one).  After it no launch entry point of this library
+ * (about 2.6, 64 and 4 MiB; otherwise made by the first launch that needs one).  After it no launch entry point of this library
  * allocates device memory: call it once per device before capturing launches into a HIP graph or entering a serving loop.
  * No counterpart in the reference, whose kernels never allocate (infra/model.hpp:241 owns the arena). */
 int nh_q8_0_prepare(void);

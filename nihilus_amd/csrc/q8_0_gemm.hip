@@ -629,7 +629,7 @@ template<int TM, bool STREAM> static hipError_t launch_gemm_tiled_t(const gemm_t
 			float* partials	   = nullptr;
 			unsigned* counters = nullptr;
 			scratch_hold hold;
-			const hipError_t e = acquire_gemm_split_scratch(&partials, &counters, &hold, s);
+			const hipError_t e = acquire_gemm_split_scratch(&partials, &counters, STREAM, &hold, s);
 			if (e != hipSuccess) {
 				return e;
 			}

@@ -239,20 +239,23 @@ __global__ __launch_bounds__(WAVES * 64, DUMP ? 2 : 4) void gemm_skinny_kernel(c
 	store(sum);
 }
 
-// Scratch of the K-split path (partial 32x32 tiles and arrival counters): one allocation per device on first use, in two parts: the null
-// stream's, which may not be queried while some other stream is being captured and so never shares, and one that serves the other
-// streams one at a time.
-static_assert(GEMM_SPLIT_SCRATCH_FLOATS == SK_MAX_SPLIT_UNITS * 2 * 16 * 64 && GEMM_SPLIT_MAX_UNITS == SK_MAX_SPLIT_STRIPS, "one scratch, two users");
+// Scratch of the K-split paths (partial tiles and arrival counters): one allocation per device on first use, in two pairs: one for the
+// launches of this kernel and of the tile kernel for up to 64 rows, one for the tile kernel's with more rows (which need no scratch if they
+// must: they would have the others refused).  Of a pair one is the null stream's, which may not be queried while some other stream is
+// being captured and so never shares, and one serves the other streams one at a time.
+static_assert(GEMM_SPLIT_SCRATCH_FLOATS == SK_MAX_SPLIT_UNITS * 2 * 16 * 64 && GEMM_SPLIT_MAX_UNITS == SK_MAX_SPLIT_STRIPS, "scratch of one size");
 struct skinny_scratch {
 	float* partials	   = nullptr;
 	unsigned* counters = nullptr;
 	hipStream_t user   = nullptr; // stream of the last K-split launch
 };
-// hold == nullptr: make it if need be.  Otherwise a K-split launch on `s` is about to use it, and the caller keeps *hold until it is enqueued.  If the previous such launch of its part went to another stream
-// that has not drained, hipErrorNotReady comes back (NH_ERR_BUSY at the C ABI).  Not checked for capturing streams.
-static hipError_t get_skinny_scratch(skinny_scratch* out, scratch_hold* hold = nullptr, hipStream_t s = nullptr) {
+// hold == nullptr: make it if need be.  Otherwise a K-split launch on `s` is about to use it, and the caller keeps *hold until it is
+// enqueued.  If the previous such launch of its part went to another stream that has not drained, hipErrorNotReady comes back.  Not
+// checked for capturing streams.
+static hipError_t get_skinny_scratch(skinny_scratch* out, bool few_rows = true, scratch_hold* hold = nullptr, hipStream_t s = nullptr) {
+	constexpr int PARTS = 4;
 	static std::recursive_mutex locks[64];
-	static skinny_scratch per_device[64][2];
+	static skinny_scratch per_device[64][PARTS];
 	int dev		 = 0;
 	hipError_t e = hipGetDevice(&dev);
 	if (e != hipSuccess) {
@@ -266,22 +269,22 @@ static hipError_t get_skinny_scratch(skinny_scratch* out, scratch_hold* hold = n
 		void* p			   = nullptr;
 		const size_t tiles = static_cast<size_t>(SK_MAX_SPLIT_UNITS) * 2 * 16 * 64 * 4; // two 32-row activation strips at most
 		const size_t part  = tiles + SK_MAX_SPLIT_STRIPS * 4;
-		e				   = hipMalloc(&p, 2 * part);
+		e				   = hipMalloc(&p, PARTS * part);
 		if (e != hipSuccess) {
 			return e;
 		}
-		e = hipMemset(p, 0, 2 * part);
+		e = hipMemset(p, 0, PARTS * part);
 		if (e != hipSuccess) {
 			(void)hipFree(p);
 			return e;
 		}
-		for (int i = 0; i < 2; ++i) {
+		for (int i = 0; i < PARTS; ++i) {
 			uint8_t* base				= static_cast<uint8_t*>(p) + i * part;
 			per_device[dev][i].partials = reinterpret_cast<float*>(base);
 			per_device[dev][i].counters = reinterpret_cast<unsigned*>(base + tiles);
 		}
 	}
-	skinny_scratch& sc = per_device[dev][s != nullptr];
+	skinny_scratch& sc = per_device[dev][2 * !few_rows + (s != nullptr)];
 	if (hold && !stream_is_capturing(s)) {
 		if (sc.user != s && sc.user != nullptr) {
 			e = stream_drained(sc.user);
@@ -300,9 +303,9 @@ static hipError_t get_skinny_scratch(skinny_scratch* out, scratch_hold* hold = n
 
 // The same scratch for the tile kernel's K split over workgroups (GEMM_SPLIT_SCRATCH_FLOATS floats of tiles, GEMM_SPLIT_MAX_UNITS
 // counters that every launch leaves at zero); same one-stream rule.
-hipError_t acquire_gemm_split_scratch(float** partials, unsigned** counters, scratch_hold* hold, hipStream_t s) {
+hipError_t acquire_gemm_split_scratch(float** partials, unsigned** counters, bool few_rows, scratch_hold* hold, hipStream_t s) {
 	skinny_scratch sc;
-	const hipError_t e = get_skinny_scratch(&sc, hold, s);
+	const hipError_t e = get_skinny_scratch(&sc, few_rows, hold, s);
 	if (e != hipSuccess) {
 		return e;
 	}
@@ -323,7 +326,7 @@ template<int MS> static hipError_t launch_skinny_t(int splits, int waves, const 
 	skinny_scratch sc;
 	scratch_hold hold;
 	if (splits > 1) {
-		const hipError_t e = get_skinny_scratch(&sc, &hold, s);
+		const hipError_t e = get_skinny_scratch(&sc, true, &hold, s);
 		if (e != hipSuccess) {
 			return e;
 		}

@@ -195,6 +195,21 @@ std::vector<entry_point> entry_points() {
 	return all;
 }
 
+// A mat-mat on one stream never has the mat-mat on another one refused where their scratch is not the same: (rows, N, K) running, (rows, N, K) called.
+struct shape {
+	int64_t m, n, k;
+};
+const std::pair<shape, shape> side_by_side[] = {
+	{ { 96, 8192, 8192 }, { 64, 1024, 8192 } }, // the tile kernel with K over workgroups beside the streaming kernel with K over workgroups
+	{ { 96, 8192, 8192 }, { 40, 1024, 4096 } },
+	{ { 96, 8192, 8192 }, { 96, 8192, 8192 } }, // the second one takes a form without scratch
+	{ { 128, 8192, 28672 }, { 128, 8192, 28672 } },
+	{ { 66, 4096, 10240 }, { 66, 4096, 10240 } },
+	{ { 4, 4096, 4096 }, { 40, 1024, 4096 } }, // the rows kernel beside the streaming kernel
+	{ { 4, 4096, 4096 }, { 4, 4096, 4096 } }, // the second one runs on the streaming kernel
+	{ { 40, 1024, 4096 }, { 96, 8192, 8192 } },
+};
+
 int failures = 0;
 void expect(bool ok, const std::string& name, const char* what) {
 	if (!ok) {
@@ -246,6 +261,24 @@ int main() {
 		expect(launches.size() == want.size() && !launches.empty() && launches.back().kernel == want.back(), e.name, "another form on an idle GPU");
 		reset();
 	}
+	uintptr_t next_stream = 0x100; // streams that no earlier call has used: the library asks whether a stream is idle, not what it runs
+	for (const auto& [one, two] : side_by_side) {
+		const hipStream_t s1 = reinterpret_cast<hipStream_t>(next_stream += 0x10), s2 = reinterpret_cast<hipStream_t>(next_stream += 0x10);
+		const auto call = [](const shape& x, void* s) { return nh_q8_0_gemm_tiled(operand<void>(0), operand<void>(1), operand<float>(2), x.m, x.n, x.k, s); };
+		const std::string name = std::to_string(two.m) + " rows [" + std::to_string(two.n) + " x " + std::to_string(two.k) + "] beside " + std::to_string(one.m) + " rows [" + std::to_string(one.n) + " x " +
+			std::to_string(one.k) + "]";
+		reset();
+		expect(call(one, s1) == NH_OK, name, "the first call failed");
+		expect(call(two, s2) == NH_OK, name, "the second call failed");
+		reset();
+	}
+	// ... and is refused, with nothing launched, where the form that is left needs scratch that a third stream is using
+	reset();
+	const hipStream_t s1 = reinterpret_cast<hipStream_t>(next_stream += 0x10), s2 = reinterpret_cast<hipStream_t>(next_stream += 0x10), s3 = reinterpret_cast<hipStream_t>(next_stream += 0x10);
+	const auto four_rows = [](void* s) { return nh_q8_0_gemm_tiled(operand<void>(0), operand<void>(1), operand<float>(2), 4, 4096, 4096, s); };
+	expect(four_rows(s1) == NH_OK && four_rows(s2) == NH_OK, "4 rows on three streams", "the first two are served");
+	const size_t before = launches.size();
+	expect(four_rows(s3) == NH_ERR_BUSY && launches.size() == before, "4 rows on three streams", "the third is refused");
 	if (failures == 0) {
 		std::printf("scratch hand-out ok\n");
 	}
