@@ -230,7 +230,13 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 	uint8_t* lds	   = lds_raw + kr * SET_BYTES;
 	// the host launches KS > 1, and K over gridDim.z workgroups, only when they divide
 	const int g_len	   = SPLIT ? groups / (KS * static_cast<int>(gridDim.z)) : groups / KS;
-	const int g_base   = SPLIT ? (static_cast<int>(blockIdx.z) * KS + kr) * g_len : kr * g_len;
+	// which share of K: with K over workgroups in the shapes that the streaming kernel can take too, the one that makes the sums below the
+	// tree that kernel adds its eight or sixteen waves' shares in (0 4 2 6 / 1 5 3 7, then the same of 8 to 15)
+	constexpr bool TREE = SPLIT && !STREAM;
+	static_assert(!TREE || KS == 4);
+	const int z		  = SPLIT ? static_cast<int>(blockIdx.z) : 0;
+	const int share	  = TREE ? 8 * (z >> 1) + (z & 1) + 4 * (kr & 1) + 2 * (kr >> 1) : z * KS + kr;
+	const int g_base  = share * g_len;
 	const int half	   = lane >> 5;
 	const int m_strips = (M + 31) / 32;
 	const int n_strips = (N + 31) / 32;
@@ -447,11 +453,14 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 				for (int i = 0; i < TM; ++i) {
 #pragma unroll
 					for (int e = 0; e < PER; ++e) {
-						float v = 0.0f;
+						float part[KS], v;
 #pragma unroll
 						for (int src = 0; src < KS; ++src) {
-							const float part = src == q ? acc[i][q * PER + e] : slot(q, src)[(i * PER + e) * 64];
-							v				 = src == 0 ? part : v + part;
+							part[src] = src == q ? acc[i][q * PER + e] : slot(q, src)[(i * PER + e) * 64];
+							v		  = src == 0 ? part[src] : v + part[src];
+						}
+						if constexpr (TREE) {
+							v = (part[0] + part[1]) + (part[2] + part[3]);
 						}
 						mine[i * PER + e] = v;
 					}
@@ -489,15 +498,20 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 			for (int j = 0; j < TM * PER; ++j) {
 				mine[j] = 0.0f;
 			}
-			for (int z = 0; z < kz_count; ++z) {
-				float got[TM * PER];
+			constexpr int STEP = TREE ? 2 : 1; // (an even number of workgroups)
+			for (int z0 = 0; z0 < kz_count; z0 += STEP) {
+				float got[STEP][TM * PER];
 #pragma unroll
-				for (int j = 0; j < TM * PER; ++j) {
-					got[j] = __hip_atomic_load(&tile[static_cast<int64_t>(z) * TILE_FLOATS + j * 64], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+				for (int u = 0; u < STEP; ++u) {
+#pragma unroll
+					for (int j = 0; j < TM * PER; ++j) {
+						got[u][j] = __hip_atomic_load(&tile[static_cast<int64_t>(z0 + u) * TILE_FLOATS + j * 64], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+					}
 				}
 #pragma unroll
 				for (int j = 0; j < TM * PER; ++j) {
-					mine[j] = z == 0 ? got[j] : mine[j] + got[j];
+					const float v = TREE ? got[0][j] + got[STEP - 1][j] : got[0][j];
+					mine[j]		  = z0 == 0 ? v : mine[j] + v;
 				}
 			}
 		}
@@ -729,10 +743,10 @@ hipError_t launch_gemm(const void* W, const void* Aq, float* C, int32_t* sums, i
 					return e;
 				}
 			}
-			return launch_gemm_skinny(W, Aq, C, sums, M, N, K, s, residual);
+			return launch_gemm_skinny(W, Aq, C, sums, M, N, K, plan.skinny, s, residual);
 		}
 		// K over workgroups with more than 64 rows: where the scratch is another stream's for now, or the launch goes into a graph that may be
-		// replayed beside another (the scratch would be both's), the streaming kernel, which seldom needs any
+		// replayed beside another (the scratch would be both's), the streaming kernel, which gives the same bits without any
 		const bool split_rows = plan.kernel == MM_GEMM_TILE && plan.tile.kz > 1;
 		if (!split_rows || !stream_is_capturing(s)) {
 			const hipError_t e = launch_gemm_tiled(plan.tile, w, a, C, residual, sums, m, n, k, s, plan.kernel == MM_GEMM_TILE_STREAM);
@@ -740,7 +754,7 @@ hipError_t launch_gemm(const void* W, const void* Aq, float* C, int32_t* sums, i
 				return e;
 			}
 		}
-		return launch_gemm_skinny(W, Aq, C, sums, M, N, K, s, residual);
+		return launch_gemm_skinny(W, Aq, C, sums, M, N, K, plan.skinny, s, residual);
 	} else {
 		if (sums) {
 			gemm_kernel<false, true><<<grid, dim3(GEMM_THREADS), 0, s>>>(w, a, C, sums, m, n, k);

@@ -189,7 +189,7 @@ __device__ __forceinline__ void rows_strip(const uint8_t* __restrict__ w_strip, 
 	uint8_t* a_scales = lds + SK_WAVES * L::TILES + wave * L::SCALES;
 	for (int set = 0; set < SETS; ++set) {
 		int g0, g1;
-		wave_k_range(groups, split_shift, split, SETS * SK_WAVES, set * SK_WAVES + wave, g0, g1);
+		wave_k_range(groups, split_shift + (SETS - 1), split * SETS + set, SK_WAVES, wave, g0, g1);
 		float acc[MATS][R / 2];
 #pragma unroll
 		for (int k = 0; k < MATS; ++k) {

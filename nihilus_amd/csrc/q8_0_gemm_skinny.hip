@@ -33,7 +33,12 @@ __global__ __launch_bounds__(WAVES * 64, DUMP ? 2 : 4) void gemm_skinny_kernel(c
 	const int mg	 = static_cast<int>(blockIdx.y); // group of MS activation strips (more than 32 * MS rows: the weights are read once per group, from cache after the first)
 	const int unit	 = mg * static_cast<int>(gridDim.x >> split_shift) + strip; // index of this (row group, weight strip) in the split scratch
 	int g0, g1; // this wave's share of the strip's K range
-	wave_k_range(groups, split_shift, split, WAVES, wave, g0, g1);
+	// sixteen waves: the shares that two workgroups of eight would have
+	if constexpr (WAVES == SK_WIDE_WAVES) {
+		wave_k_range(groups, split_shift + 1, 2 * split + (wave >> 3), SK_WAVES, wave & 7, g0, g1);
+	} else {
+		wave_k_range(groups, split_shift, split, WAVES, wave, g0, g1);
+	}
 	const int r		 = lane & 31;
 	const int half	 = lane >> 5;
 
@@ -340,19 +345,17 @@ template<int MS> static hipError_t launch_skinny_t(int splits, int waves, const 
 		gemm_skinny_kernel<MS, true, 1, SK_WAVES><<<grid, dim3(SK_WAVES * 64), 0, s>>>(w, a, C, R, sums, sc.partials, sc.counters, m, n, groups, shift);
 		return hipGetLastError();
 	}
-	if constexpr (MS == 1) { // two strips per workgroup are only cut into 256 workgroups and more
-		if (waves == SK_WIDE_WAVES) {
-			return launch_kernel(KIND_GEMM, gemm_skinny_kernel<1, false, 2, SK_WIDE_WAVES>, grid, block, 0, s, w, a, C, R, sums, sc.partials, sc.counters, m, n, groups, shift);
-		}
+	if (waves == SK_WIDE_WAVES) {
+		return launch_kernel(KIND_GEMM, gemm_skinny_kernel<MS, false, 2, SK_WIDE_WAVES>, grid, block, 0, s, w, a, C, R, sums, sc.partials, sc.counters, m, n, groups, shift);
 	}
 	return launch_kernel(KIND_GEMM, gemm_skinny_kernel<MS, false, 2, SK_WAVES>, grid, block, 0, s, w, a, C, R, sums, sc.partials, sc.counters, m, n, groups, shift);
 }
 
-hipError_t launch_gemm_skinny(const void* W, const void* Aq, float* C, int32_t* sums, int64_t M, int64_t N, int64_t K, hipStream_t s, const float* residual) {
+// cut: plan_gemm_skinny, or the stand-in for a tile kernel's (q8_0_plan.h)
+hipError_t launch_gemm_skinny(const void* W, const void* Aq, float* C, int32_t* sums, int64_t M, int64_t N, int64_t K, const gemm_skinny_cut& cut, hipStream_t s, const float* residual) {
 	const uint8_t* w = static_cast<const uint8_t*>(W);
 	const uint8_t* a = static_cast<const uint8_t*>(Aq);
 	const int groups = static_cast<int>(K / GROUP_K);
-	const gemm_skinny_cut cut = plan_gemm_skinny(M, N, K); // activation strips per workgroup, workgroups per strip: q8_0_plan.h
 	if (cut.ms == 1) {
 		return launch_skinny_t<1>(cut.splits, cut.waves, w, a, C, residual, sums, static_cast<int>(M), static_cast<int>(N), groups, s);
 	}

@@ -58,28 +58,6 @@ inline gemm_tile_cut plan_gemm_tile(int64_t M, int64_t N, int64_t K, bool stream
 	return c;
 }
 
-// More than 64 rows against a matrix whose tiles are short of a workgroup per CU, with K long enough: the tile kernel with K over workgroups
-// until there is about one per CU.  The streaming kernel, which has the shape otherwise, takes the activations out of L2 once per weight
-// strip, where four strips share them here; the hand-off costs 3 to 4 us, so every K set has to keep five groups.  Measured, us, this /
-// the streaming kernel: [8192 x 28672] at 128 rows 91 / 129, [8192 x 8192] at 96 / 128 rows 31 / 36 and 31 / 38, [4096 x 8192] at 200 rows
-// 28.5 / 34.3, [4096 x 14336] at 117 rows (seven groups, K over four) 28.5 / 31.1, [5120 x 5120] at 160 rows (five) 21.4 / 22.3; with four
-// groups [4096 x 4096] at 200 rows 18.4 / 18.0, [2048 x 8192] at 256 rows 19.8 / 18.1; with two [4096 x 4096] at 117 rows 14.9 / 12.5.
-constexpr int GEMM_TILE_SPLIT_MIN_GROUPS = 5;
-inline bool plan_gemm_tile_split(int64_t M, int64_t N, int64_t K, gemm_tile_cut* cut) {
-	gemm_tile_cut c		  = plan_gemm_tile(M, N, K, false);
-	const int groups	  = static_cast<int>(K / GROUP_K);
-	const int64_t wgs	  = static_cast<int64_t>(c.grid_x) * c.grid_y;
-	while (c.ks == 4 && wgs * c.kz * 2 <= 256 && groups % (c.ks * c.kz * 2) == 0 && groups / (c.ks * c.kz * 2) >= GEMM_TILE_SPLIT_MIN_GROUPS &&
-		wgs * c.kz * 2 * c.tm * 4096 <= GEMM_SPLIT_SCRATCH_FLOATS && wgs <= GEMM_SPLIT_MAX_UNITS) {
-		c.kz *= 2;
-	}
-	if (c.tm != 2 || c.kz == 1 || wgs * c.kz <= 128) {
-		return false;
-	}
-	*cut = c;
-	return true;
-}
-
 // The weight-streaming MFMA kernel's cut: MS activation strips per workgroup, K of a strip over `splits` workgroups of `waves` waves.
 struct gemm_skinny_cut {
 	int ms, splits, waves; // waves: 8 or 16, the shares of K that a workgroup adds
@@ -143,6 +121,37 @@ inline gemm_skinny_cut plan_gemm_skinny(int64_t M, int64_t N, int64_t K) {
 	return c;
 }
 
+// More than 64 rows against a matrix whose tiles are short of a workgroup per CU, with K long enough: the tile kernel with K over workgroups
+// until there is about one per CU.  The streaming kernel, which has the shape otherwise, takes the activations out of L2 once per weight
+// strip, where four strips share them here; the hand-off costs 3 to 4 us, so every K set has to keep five groups.  Measured, us, this /
+// the streaming kernel: [8192 x 28672] at 128 rows 91 / 129, [8192 x 8192] at 96 / 128 rows 31 / 36 and 31 / 38, [4096 x 8192] at 200 rows
+// 28.5 / 34.3, [4096 x 14336] at 117 rows (seven groups, K over four) 28.5 / 31.1, [5120 x 5120] at 160 rows (five) 21.4 / 22.3; with four
+// groups [4096 x 4096] at 200 rows 18.4 / 18.0, [2048 x 8192] at 256 rows 19.8 / 18.1; with two [4096 x 4096] at 117 rows 14.9 / 12.5.
+//
+// A captured call, and one that finds the hand-off scratch in use on another stream, runs on the streaming kernel with as many shares of K in
+// one workgroup of eight or sixteen waves (`twin`), which add to the same bits and need no scratch: hence two or four workgroups along
+// K, and as many as give no fewer shares than the streaming kernel's own cut.
+constexpr int GEMM_TILE_SPLIT_MIN_GROUPS = 5, GEMM_TILE_SPLIT_MAX = 4;
+inline bool plan_gemm_tile_split(int64_t M, int64_t N, int64_t K, gemm_tile_cut* cut, gemm_skinny_cut* twin) {
+	gemm_tile_cut c			  = plan_gemm_tile(M, N, K, false);
+	const gemm_skinny_cut own = plan_gemm_skinny(M, N, K);
+	const int groups		  = static_cast<int>(K / GROUP_K);
+	const int64_t wgs		  = static_cast<int64_t>(c.grid_x) * c.grid_y;
+	const auto can_double	  = [&] {
+		return c.ks == 4 && c.kz < GEMM_TILE_SPLIT_MAX && groups % (c.ks * c.kz * 2) == 0 && groups / (c.ks * c.kz * 2) >= GEMM_TILE_SPLIT_MIN_GROUPS &&
+			wgs * c.kz * 2 * c.tm * 4096 <= GEMM_SPLIT_SCRATCH_FLOATS && wgs <= GEMM_SPLIT_MAX_UNITS;
+	};
+	while (can_double() && (wgs * c.kz * 2 <= 256 || c.ks * c.kz < own.splits * own.waves)) {
+		c.kz *= 2;
+	}
+	if (c.tm != 2 || c.kz == 1 || wgs * c.kz <= 128 || c.ks * c.kz < own.splits * own.waves) {
+		return false;
+	}
+	*cut  = c;
+	*twin = gemm_skinny_cut{ own.ms, 1, c.ks * c.kz };
+	return true;
+}
+
 // Up to 32 rows the kernel of q8_0_gemm_rows.hip, with the cut above, where it is the faster one.
 // Measured against the kernels that had these shapes (weights rotated, kernel times, us):
 //   rows                4            16            32
@@ -172,7 +181,7 @@ inline bool gemm_rows_fits(int64_t M, int64_t N, const gemm_skinny_cut& cut) {
 struct gemm_plan {
 	int kernel; // MM_GEMM_SKINNY, MM_GEMM_TILE_STREAM or MM_GEMM_TILE (MM_NOTHING for an empty problem)
 	gemm_tile_cut tile; // when a tile kernel runs
-	gemm_skinny_cut skinny; // when the streaming kernel runs
+	gemm_skinny_cut skinny; // when the streaming kernel runs, and when it stands in for the tile kernel with K over workgroups
 	bool rows; // the streaming kernel's form for up to 32 rows, with the same cut
 };
 inline gemm_plan plan_gemm(int64_t M, int64_t N, int64_t K) {
@@ -214,7 +223,7 @@ inline gemm_plan plan_gemm(int64_t M, int64_t N, int64_t K) {
 	if (stream_tile) {
 		p.kernel = MM_GEMM_TILE_STREAM;
 		p.tile	 = plan_gemm_tile(M, N, K, true);
-	} else if (M > GEMM_SKINNY_MAX_M && tile_workgroups <= 256 && plan_gemm_tile_split(M, N, K, &p.tile)) {
+	} else if (M > GEMM_SKINNY_MAX_M && tile_workgroups <= 256 && plan_gemm_tile_split(M, N, K, &p.tile, &p.skinny)) {
 		p.kernel = MM_GEMM_TILE;
 	} else if (M <= GEMM_SKINNY_MAX_M || tile_workgroups <= 256) {
 		p.kernel = MM_GEMM_SKINNY;

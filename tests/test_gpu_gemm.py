@@ -238,3 +238,32 @@ def test_streaming_kernel_with_sixteen_waves(q8, oracle, m, n, k, splits):
     acc = to_dev(res.copy())
     q8.gemm_residual(wt, at, acc, m, n, k, out=acc)
     assert np.array_equal(to_host(acc), got + res)
+
+
+# A captured call has the streaming kernel in place of the tile kernel with K over workgroups (whose scratch a replay could not have to itself):
+# eight or sixteen shares of K in one workgroup, added in the same order, so the same bits.  Two and four workgroups along K, odd numbers
+# of strips, ragged ones, and the shape whose streaming form alone would have taken K over workgroups too.
+@pytest.mark.parametrize("m,n,k,splits", [(66, 4200, 5120, 2), (160, 2800, 5120, 2), (66, 4096, 10240, 4), (117, 4096, 14336, 4), (128, 8192, 28672, 4), (96, 8192, 8192, 2)])
+def test_captured_and_eager_calls_with_k_over_workgroups_have_the_same_bits(q8, oracle, m, n, k, splits):
+    import torch
+
+    plan = q8.plan_mul_mat(m, n, k)
+    assert plan["kernel"] == "gemm_tile" and plan["k_splits"] == splits
+    wt = q8.tile(q8.fill_weight_blocks(m + n, n, k), n, k)
+    xs = [q8.fill_activations(50 + i, m * k).reshape(m, k) for i in range(3)]
+    res = q8.fill_activations(60, m * n).reshape(m, n)
+    at = q8.quantize_row_q8_0(xs[0], tiled=True)
+    c = torch.empty((m, n), dtype=torch.float32, device="cuda")
+    lib = q8._lib.lib()
+    q8._lib.check("nh_q8_0_prepare", lib.nh_q8_0_prepare())
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        q8._lib.check("gemm", lib.nh_q8_0_gemm_tiled_residual(wt.data_ptr(), at.data_ptr(), c.data_ptr(), c.data_ptr(), m, n, k, torch.cuda.current_stream().cuda_stream))
+    for x in xs:
+        at.copy_(q8.quantize_row_q8_0(x, tiled=True))
+        c.copy_(res)
+        graph.replay()
+        torch.cuda.synchronize()
+        eager = q8.gemm_residual(wt, at, res, m, n, k)
+        assert np.array_equal(to_host(c).view(np.uint32), to_host(eager).view(np.uint32))
