@@ -50,23 +50,29 @@ __device__ __forceinline__ v2u scale_slot(v2u four, int t) {
 }
 // One result tile (rows m0 + 8 (e / 4) + 4 half + e % 4, column n0 + r) to C, + R if given.  R may be C: an element is read and written by
 // the same thread.  The sixteen reads are issued together: written one by one behind stores that they may alias, they were a chain of
-// sixteen memory latencies.
-__device__ __forceinline__ void store_tile(const v16f& v, int m0, int n0, int half, int r, float* C, const float* R, int M, int N) {
+// sixteen memory latencies.  (One branch around them: a launch without a residual runs and fetches none of it.)
+__device__ __forceinline__ void store_tile(v16f v, int m0, int n0, int half, int r, float* C, const float* R, int M, int N) {
 	const int n = n0 + r;
 	if (n >= N) {
 		return;
 	}
-	float add[16];
+	if (R) {
+		float add[16];
 #pragma unroll
-	for (int e = 0; e < 16; ++e) {
-		const int m = m0 + 8 * (e >> 2) + 4 * half + (e & 3);
-		add[e]		= (R && m < M) ? R[static_cast<int64_t>(m) * N + n] : 0.0f;
+		for (int e = 0; e < 16; ++e) {
+			const int m = m0 + 8 * (e >> 2) + 4 * half + (e & 3);
+			add[e]		= m < M ? R[static_cast<int64_t>(m) * N + n] : 0.0f;
+		}
+#pragma unroll
+		for (int e = 0; e < 16; ++e) {
+			v[e] += add[e];
+		}
 	}
 #pragma unroll
 	for (int e = 0; e < 16; ++e) {
 		const int m = m0 + 8 * (e >> 2) + 4 * half + (e & 3);
 		if (m < M) {
-			C[static_cast<int64_t>(m) * N + n] = R ? v[e] + add[e] : v[e];
+			C[static_cast<int64_t>(m) * N + n] = v[e];
 		}
 	}
 }

@@ -439,11 +439,13 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 		// the residual of this wave's rows, requested together and before the sums are: R may be C, every element is read here and written
 		// below by the same thread
 		float add[TM * PER];
+		if (!GATE_UP && R) {
 #pragma unroll
-		for (int j = 0; j < TM * PER; ++j) {
-			const int ee = kr * PER + j % PER;
-			const int m	 = (ms0 + j / PER) * 32 + 8 * (ee >> 2) + 4 * half + (ee & 3);
-			add[j]		 = (!GATE_UP && R && m < M && n < N) ? R[static_cast<int64_t>(m) * N + n] : 0.0f;
+			for (int j = 0; j < TM * PER; ++j) {
+				const int ee = kr * PER + j % PER;
+				const int m	 = (ms0 + j / PER) * 32 + 8 * (ee >> 2) + 4 * half + (ee & 3);
+				add[j]		 = (m < M && n < N) ? R[static_cast<int64_t>(m) * N + n] : 0.0f;
+			}
 		}
 		__syncthreads();
 #pragma unroll
@@ -516,12 +518,18 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 			}
 		}
 		if constexpr (!GATE_UP) {
+			if (R) {
+#pragma unroll
+				for (int j = 0; j < TM * PER; ++j) {
+					mine[j] += add[j];
+				}
+			}
 #pragma unroll
 			for (int j = 0; j < TM * PER; ++j) {
 				const int ee = kr * PER + j % PER;
 				const int m	 = (ms0 + j / PER) * 32 + 8 * (ee >> 2) + 4 * half + (ee & 3);
 				if (m < M && n < N) {
-					C[static_cast<int64_t>(m) * N + n] = R ? mine[j] + add[j] : mine[j];
+					C[static_cast<int64_t>(m) * N + n] = mine[j];
 				}
 			}
 			return;

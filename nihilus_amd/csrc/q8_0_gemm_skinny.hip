@@ -156,10 +156,12 @@ __global__ __launch_bounds__(WAVES * 64, DUMP ? 2 : 4) void gemm_skinny_kernel(c
 	const int n		  = strip * STRIP_ROWS + r;
 	const auto row_of = [&](int v) { return (mg * MS + (v >> 4)) * STRIP_ROWS + 8 * ((v & 15) >> 2) + 4 * half + (v & 3); };
 	float add[OWN]; // R may be C: every element is read here and written below by the same thread
+	if (R) {
 #pragma unroll
-	for (int o = 0; o < OWN; ++o) {
-		const int m = row_of(wave * OWN + o);
-		add[o]		= (R && m < M && n < N) ? R[static_cast<int64_t>(m) * N + n] : 0.0f;
+		for (int o = 0; o < OWN; ++o) {
+			const int m = row_of(wave * OWN + o);
+			add[o]		= (m < M && n < N) ? R[static_cast<int64_t>(m) * N + n] : 0.0f;
+		}
 	}
 #pragma unroll
 	for (int i = 0; i < MS; ++i) {
@@ -182,12 +184,18 @@ __global__ __launch_bounds__(WAVES * 64, DUMP ? 2 : 4) void gemm_skinny_kernel(c
 			own[o] += eight(8);
 		}
 	}
-	auto store = [&](const float (&v)[OWN]) {
+	auto store = [&](float (&v)[OWN]) {
+		if (R) {
+#pragma unroll
+			for (int o = 0; o < OWN; ++o) {
+				v[o] += add[o];
+			}
+		}
 #pragma unroll
 		for (int o = 0; o < OWN; ++o) {
 			const int m = row_of(wave * OWN + o);
 			if (m < M && n < N) {
-				C[static_cast<int64_t>(m) * N + n] = R ? v[o] + add[o] : v[o];
+				C[static_cast<int64_t>(m) * N + n] = v[o];
 			}
 		}
 	};
