@@ -425,6 +425,6 @@ constexpr int64_t GEMM_SPLIT_SCRATCH_FLOATS = 2048 * 2 * 16 * 64; // partial til
 constexpr int GEMM_SPLIT_MAX_UNITS			  = 512; // arrival counters
 // few_rows: the launches of up to 64 rows, which share theirs with the streaming kernel's
 hipError_t acquire_gemm_split_scratch(float** partials, unsigned** counters, bool few_rows, scratch_hold* hold, hipStream_t s);
-hipError_t launch_gemm_skinny(const void* W, const void* Aq, float* C, int32_t* sums, int64_t M, int64_t N, int64_t K, const gemm_skinny_cut& cut, hipStream_t s, const float* residual = nullptr);
+hipError_t launch_gemm_skinny(const void* W, const void* Aq, float* C, int64_t M, int64_t N, int64_t K, const gemm_skinny_cut& cut, hipStream_t s, const float* residual = nullptr);
 
 } // namespace nh

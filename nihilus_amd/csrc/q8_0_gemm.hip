@@ -751,7 +751,7 @@ hipError_t launch_gemm(const void* W, const void* Aq, float* C, int32_t* sums, i
 					return e;
 				}
 			}
-			return launch_gemm_skinny(W, Aq, C, sums, M, N, K, plan.skinny, s, residual);
+			return launch_gemm_skinny(W, Aq, C, M, N, K, plan.skinny, s, residual);
 		}
 		// K over workgroups with more than 64 rows: where the scratch is another stream's for now, or the launch goes into a graph that may be
 		// replayed beside another (the scratch would be both's), the streaming kernel, which gives the same bits without any
@@ -762,7 +762,7 @@ hipError_t launch_gemm(const void* W, const void* Aq, float* C, int32_t* sums, i
 				return e;
 			}
 		}
-		return launch_gemm_skinny(W, Aq, C, sums, M, N, K, plan.skinny, s, residual);
+		return launch_gemm_skinny(W, Aq, C, M, N, K, plan.skinny, s, residual);
 	} else {
 		if (sums) {
 			gemm_kernel<false, true><<<grid, dim3(GEMM_THREADS), 0, s>>>(w, a, C, sums, m, n, k);

@@ -2,10 +2,13 @@
 // SiLU * up and the quantizer behind it in the same launch, gfx950.
 //
 // What bounds it is HBM and, at these sizes, latency: the weights are read once, so the kernel is the streaming mat-vec again -- a
-// workgroup per (32-row weight strip, K part), its waves splitting the K range, every weight load of a wave's share in flight
-// before anything is waited for, one reduction at the end -- with the int8 MFMA as the inner product.  The weight tile as loaded is
-// the B operand; the activation rows are the A operand.  Eight waves per workgroup and at most 128 registers: two workgroups per
-// CU, so that one streams while the other reduces and leaves.
+// workgroup per (32-row weight strip, K part), its waves splitting the K range, a chunk of two groups (one of each matrix in the gate /
+// up form) at a time with every load of it in flight before anything is waited for, one reduction at the end -- with the int8 MFMA as the
+// inner product.  The weight tile as loaded is the B operand; the activation rows are the A operand.  Eight waves per workgroup and at
+// most 128 registers: two workgroups per CU, so that one streams while the other reduces and leaves.
+//
+// K is cut, and the sums are added, as in the streaming kernel (q8_0_gemm_skinny.hip), which runs a call that is being captured or finds
+// the hand-off's scratch in use on another stream: the result does not depend on which of the two ran.
 //
 // The activations come memory -> LDS without registers, and only the rows that exist: a 128-quant group of R rows (R = 8, 16 or 32) is
 // R / 8 transfers of 1 KiB (lane l fetches the 16 bytes of one (block, k half, row)), so that eight rows cost a quarter of the weight
@@ -141,27 +144,11 @@ __device__ __forceinline__ void rows_chunk_n(const uint8_t* __restrict__ w_strip
 template<int R, int T, int MATS>
 __device__ __forceinline__ void rows_chunk(const uint8_t* __restrict__ w_strip, const uint8_t* __restrict__ w_strip2, const uint8_t* __restrict__ a_strip, uint8_t* a_tiles, uint8_t* a_scales, int gc,
 	int cnt, int lane, float (&acc)[MATS][R / 2]) {
-	switch (cnt) { // wave-uniform; 0: an idle wave (still takes part in the reduction)
-		case 1:
-			rows_chunk_n<R, T, MATS, 1>(w_strip, w_strip2, a_strip, a_tiles, a_scales, gc, lane, acc);
-			break;
-		case 2:
-			if constexpr (T >= 2) {
-				rows_chunk_n<R, T, MATS, 2>(w_strip, w_strip2, a_strip, a_tiles, a_scales, gc, lane, acc);
-			}
-			break;
-		case 3:
-			if constexpr (T >= 3) {
-				rows_chunk_n<R, T, MATS, 3>(w_strip, w_strip2, a_strip, a_tiles, a_scales, gc, lane, acc);
-			}
-			break;
-		case 4:
-			if constexpr (T >= 4) {
-				rows_chunk_n<R, T, MATS, 4>(w_strip, w_strip2, a_strip, a_tiles, a_scales, gc, lane, acc);
-			}
-			break;
-		default:
-			break;
+	static_assert(T == 1 || T == 2);
+	if (T == 2 && cnt == 2) { // wave-uniform
+		rows_chunk_n<R, T, MATS, T>(w_strip, w_strip2, a_strip, a_tiles, a_scales, gc, lane, acc);
+	} else {
+		rows_chunk_n<R, T, MATS, 1>(w_strip, w_strip2, a_strip, a_tiles, a_scales, gc, lane, acc);
 	}
 }
 

@@ -18,8 +18,8 @@ namespace nh {
 typedef _Float16 sk_v4h __attribute__((ext_vector_type(4)));
 typedef float sk_v16f __attribute__((ext_vector_type(16)));
 
-template<int MS, bool DUMP, int GC, int WAVES>
-__global__ __launch_bounds__(WAVES * 64, DUMP ? 2 : 4) void gemm_skinny_kernel(const uint8_t* __restrict__ W, const uint8_t* __restrict__ A, float* C, const float* R, int32_t* __restrict__ sums,
+template<int MS, int GC, int WAVES>
+__global__ __launch_bounds__(WAVES * 64, 4) void gemm_skinny_kernel(const uint8_t* __restrict__ W, const uint8_t* __restrict__ A, float* C, const float* R,
 	float* __restrict__ partials, unsigned* __restrict__ counters, int M, int N, int groups, int split_shift) {
 	__shared__ float red[MS * 16][WAVES][64];
 	__shared__ int last_flag;
@@ -89,7 +89,7 @@ __global__ __launch_bounds__(WAVES * 64, DUMP ? 2 : 4) void gemm_skinny_kernel(c
 			b.d[i] = *reinterpret_cast<const v2u*>(am + MACRO_D_OFFSET + a_d_off[i]);
 		}
 	};
-	auto compute = [&](int g, const w_regs& w, const a_regs& a) {
+	auto compute = [&](const w_regs& w, const a_regs& a) {
 		// lanes 32..63 feed the k = 4..7 slots of the scale MFMA: zero
 		const v2u wdz = half ? v2u{ 0u, 0u } : w.d;
 #pragma unroll
@@ -100,22 +100,11 @@ __global__ __launch_bounds__(WAVES * 64, DUMP ? 2 : 4) void gemm_skinny_kernel(c
 				const sk_v16f zf = { 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0 };
 				const v16i zi	 = { 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0 };
 				const v16i s	 = __builtin_amdgcn_mfma_i32_32x32x32_i8(a.q[i][j], w.q[j], zi, 0, 0, 0);
-				if constexpr (DUMP) {
-					const int n = strip * STRIP_ROWS + r;
+				const v2u as	 = scale_slot(half ? v2u{ 0u, 0u } : a.d[i], j);
+				const sk_v16f p	 = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(sk_v4h, as), __builtin_bit_cast(sk_v4h, ws), zf, 0, 0, 0);
 #pragma unroll
-					for (int e = 0; e < 16; ++e) {
-						const int m = (mg * MS + i) * 32 + 8 * (e >> 2) + 4 * half + (e & 3);
-						if (m < M && n < N) {
-							sums[(static_cast<int64_t>(m) * N + n) * (groups * GROUP_BLOCKS) + (g * GROUP_BLOCKS + j)] = s[e];
-						}
-					}
-				} else {
-					const v2u as	= scale_slot(half ? v2u{ 0u, 0u } : a.d[i], j);
-					const sk_v16f p = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(sk_v4h, as), __builtin_bit_cast(sk_v4h, ws), zf, 0, 0, 0);
-#pragma unroll
-					for (int e = 0; e < 16; ++e) {
-						acc[i][e] = fmaf(static_cast<float>(s[e]), p[e], acc[i][e]);
-					}
+				for (int e = 0; e < 16; ++e) {
+					acc[i][e] = fmaf(static_cast<float>(s[e]), p[e], acc[i][e]);
 				}
 			}
 		}
@@ -141,14 +130,10 @@ __global__ __launch_bounds__(WAVES * 64, DUMP ? 2 : 4) void gemm_skinny_kernel(c
 #pragma unroll
 		for (int c = 0; c < GC; ++c) {
 			if (c == 0 || g + c < g1) {
-				compute(g + c, w[c], a[c]);
+				compute(w[c], a[c]);
 			}
 		}
 	}
-	if constexpr (DUMP) {
-		return;
-	}
-
 	// ---- the waves' partial sums through LDS; a wave finishes OWN of every lane's MS * 16 values ----
 	// (One wave finishing them all, behind a tree of barriers, and reading the residual value by value behind its own stores was a chain
 	// of 16 * MS memory latencies: [4096 x 4096] at 117 rows 23.1 us with a residual against 13.9 without; now 13.9 and 12.6.)
@@ -333,7 +318,7 @@ hipError_t prepare_gemm_scratch() {
 	return e != hipSuccess ? e : prepare_gemm_rows_scratch();
 }
 
-template<int MS> static hipError_t launch_skinny_t(int splits, int waves, const uint8_t* w, const uint8_t* a, float* C, const float* R, int32_t* sums, int m, int n, int groups, hipStream_t s) {
+template<int MS> static hipError_t launch_skinny_t(int splits, int waves, const uint8_t* w, const uint8_t* a, float* C, const float* R, int m, int n, int groups, hipStream_t s) {
 	const int strips   = (n + STRIP_ROWS - 1) / STRIP_ROWS;
 	const int m_groups = ((m + STRIP_ROWS - 1) / STRIP_ROWS + MS - 1) / MS;
 	skinny_scratch sc;
@@ -349,25 +334,21 @@ template<int MS> static hipError_t launch_skinny_t(int splits, int waves, const 
 		++shift;
 	}
 	const dim3 grid(static_cast<unsigned>(strips * splits), static_cast<unsigned>(m_groups)), block(static_cast<unsigned>(64 * waves));
-	if (sums) {
-		gemm_skinny_kernel<MS, true, 1, SK_WAVES><<<grid, dim3(SK_WAVES * 64), 0, s>>>(w, a, C, R, sums, sc.partials, sc.counters, m, n, groups, shift);
-		return hipGetLastError();
-	}
 	if (waves == SK_WIDE_WAVES) {
-		return launch_kernel(KIND_GEMM, gemm_skinny_kernel<MS, false, 2, SK_WIDE_WAVES>, grid, block, 0, s, w, a, C, R, sums, sc.partials, sc.counters, m, n, groups, shift);
+		return launch_kernel(KIND_GEMM, gemm_skinny_kernel<MS, 2, SK_WIDE_WAVES>, grid, block, 0, s, w, a, C, R, sc.partials, sc.counters, m, n, groups, shift);
 	}
-	return launch_kernel(KIND_GEMM, gemm_skinny_kernel<MS, false, 2, SK_WAVES>, grid, block, 0, s, w, a, C, R, sums, sc.partials, sc.counters, m, n, groups, shift);
+	return launch_kernel(KIND_GEMM, gemm_skinny_kernel<MS, 2, SK_WAVES>, grid, block, 0, s, w, a, C, R, sc.partials, sc.counters, m, n, groups, shift);
 }
 
 // cut: plan_gemm_skinny, or the stand-in for a tile kernel's (q8_0_plan.h)
-hipError_t launch_gemm_skinny(const void* W, const void* Aq, float* C, int32_t* sums, int64_t M, int64_t N, int64_t K, const gemm_skinny_cut& cut, hipStream_t s, const float* residual) {
+hipError_t launch_gemm_skinny(const void* W, const void* Aq, float* C, int64_t M, int64_t N, int64_t K, const gemm_skinny_cut& cut, hipStream_t s, const float* residual) {
 	const uint8_t* w = static_cast<const uint8_t*>(W);
 	const uint8_t* a = static_cast<const uint8_t*>(Aq);
 	const int groups = static_cast<int>(K / GROUP_K);
 	if (cut.ms == 1) {
-		return launch_skinny_t<1>(cut.splits, cut.waves, w, a, C, residual, sums, static_cast<int>(M), static_cast<int>(N), groups, s);
+		return launch_skinny_t<1>(cut.splits, cut.waves, w, a, C, residual, static_cast<int>(M), static_cast<int>(N), groups, s);
 	}
-	return launch_skinny_t<2>(cut.splits, cut.waves, w, a, C, residual, sums, static_cast<int>(M), static_cast<int>(N), groups, s);
+	return launch_skinny_t<2>(cut.splits, cut.waves, w, a, C, residual, static_cast<int>(M), static_cast<int>(N), groups, s);
 }
 
 } // namespace nh
