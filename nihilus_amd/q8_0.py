@@ -16,10 +16,20 @@ QK = 32
 BLOCK_BYTES = 34
 
 
-def _stream() -> int:
-    # The current device's current stream as the handle the library takes: 0.2 us.  torch.cuda.current_stream() makes a Stream object to
-    # ask for it, 2.7 us of a call whose launch takes 3.5.  (Every caller holds a GPU tensor by now, so torch's GPU side is set up.)
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+# The current device's current stream as the handle the library takes, in 0.2 us: torch.cuda.current_stream() makes a Stream object to ask
+# for it, 2.7 us of a call whose launch takes 3.5.  The names are torch's own, not its public interface: a build without them takes
+# the public way.  (Every caller holds a GPU tensor by now, so torch's GPU side is set up.)
+def _public_stream() -> int:
+    return torch.cuda.current_stream().cuda_stream
+
+
+if hasattr(torch._C, "_cuda_getCurrentRawStream") and hasattr(torch._C, "_cuda_getDevice"):
+
+    def _stream() -> int:
+        return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+else:
+    _stream = _public_stream
 
 
 def _dev(t: torch.Tensor, dtype: torch.dtype, name: str) -> torch.Tensor:

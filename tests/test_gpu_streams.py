@@ -1,4 +1,5 @@
-"""GPU: mat-mats that split K over workgroups beside work on other streams: never refused, never wrong."""
+"""GPU: mat-mats that split K over workgroups beside work on other streams, where a form without that hand-off is left: not refused, not
+wrong, and the same bits.  (Which calls are refused, and that a refused one launches nothing: tests/test_scratch_hand_out.py, on the CPU.)"""
 import numpy as np
 import pytest
 import torch
@@ -7,8 +8,9 @@ from helpers import REL_L2_TOL, rel_l2, to_dev, to_host
 
 pytestmark = pytest.mark.gpu
 
-# the kernel for up to 32 rows, K over two workgroups per strip; the tile kernel for more than 64, K over two per tile
-SHAPES = [(4, 4096, 4096), (66, 4224, 5120)]
+# the kernel for up to 32 rows, K over two workgroups per strip; the tile kernel for more than 64, K over two and over four per tile (the
+# streaming kernel, with its own cut, would have had to hand sums over for the last one too)
+SHAPES = [(4, 4096, 4096), (66, 4224, 5120), (66, 8192, 18432)]
 NV, KV = 4096, 14336  # a mat-vec with K over four
 
 
@@ -26,7 +28,7 @@ def _busy(stream, call):
 
 
 # the stream that is kept busy: mat-vecs or mat-mats on a side stream, mat-mats on the null stream
-@pytest.mark.parametrize("M,N,K", SHAPES, ids=["4 rows", "66 rows"])
+@pytest.mark.parametrize("M,N,K", SHAPES, ids=["4 rows", "66 rows", "66 rows, long K"])
 @pytest.mark.parametrize("busy_with", ["mat-vec", "mat-mat", "mat-mat on the null stream"])
 def test_mat_mat_beside_another_stream(q8, oracle, busy_with, M, N, K):
     lib = q8._lib.lib()
@@ -62,6 +64,14 @@ def test_mat_mat_beside_another_stream(q8, oracle, busy_with, M, N, K):
     torch.cuda.synchronize()
     for o in outs + ([c_busy] if busy_with != "mat-vec" else []):
         assert rel_l2(to_host(o), want) <= REL_L2_TOL
+        assert np.array_equal(to_host(o), to_host(c))  # c: computed with nothing else running
     assert np.array_equal(to_host(y), y_want)
     if not running:
         pytest.skip("the busy stream drained before the others were tried: nothing overlapped")
+
+
+def test_current_stream_handle(q8):
+    # the handle the wrappers pass on is torch's, on the default stream and on another, by the short way and by the public one
+    for s in (torch.cuda.default_stream(), torch.cuda.Stream()):
+        with torch.cuda.stream(s):
+            assert q8._stream() == q8._public_stream() == s.cuda_stream
