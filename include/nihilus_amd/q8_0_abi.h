@@ -263,7 +263,8 @@ int nh_q8_0_gemm_tiled_residual(const void* W_tiled, const void* Aq_tiled, const
  * mat-mats against one activation image and applies SiLU * up and the quantizer to them in registers, so the two fp32 [M x N_ff]
  * intermediates are never written and no separate quantize launch runs (nh_q8_0_gate_up_silu_workspace_bytes == 0 for such a
  * shape).  Other shapes run nh_q8_0_gemm_tiled twice into `workspace` and nh_q8_0_silu_mul_quantize_tiled.  Either way the bytes are
- * those of that three-call sequence (where that sums K in the same order; else the fp32 sums differ in their last bits, and single quants with them).  W_gate, W_up: [N_ff x K] tiled; Aq: [M x K] tiled; act: [M x N_ff] tiled; N_ff, K % 128 == 0. */
+ * those of that three-call sequence wherever one launch adds up K in the mat-mats' order, which it does for most shapes; elsewhere the
+ * fp32 sums differ in their last bits, and single quants with them.  W_gate, W_up: [N_ff x K] tiled; Aq: [M x K] tiled; act: [M x N_ff] tiled; N_ff, K % 128 == 0. */
 int64_t nh_q8_0_gate_up_silu_workspace_bytes(int64_t M, int64_t N_ff, int64_t K);
 int nh_q8_0_gemm_tiled_gate_up_silu(const void* W_gate_tiled, const void* W_up_tiled, const void* Aq_tiled, void* act_tiled_out, void* workspace, int64_t workspace_bytes, int64_t M, int64_t N_ff,
 	int64_t K, void* stream);

@@ -14,6 +14,8 @@
 // shuffle.  Result lanes: register i of lane l is C[m = 8*(i/4) + 4*(l/32) + i%4][n = l % 32].
 #include "q8_0_plan.h"
 
+#include <type_traits>
+
 namespace nh {
 
 constexpr int GEMM_WAVES_M = 2; // waves along M in a workgroup
@@ -203,11 +205,13 @@ template<typename T, bool NT> __device__ __forceinline__ T load_sv(gptr_u8 p, ui
 // operand layout (through an LDS image of the tile, one 16-byte store per lane).  With several K sets the sets' tiles are summed first, as
 // in the plain kernel, and each set finishes the rows it has summed.  The two fp32 [M x N] intermediates are never
 // written, the activation is read once for both matrices, and two launches (the second mat-mat and the SiLU * up quantizer) are gone.
-// The arithmetic per value is that of the stand-alone kernels (same fp32 sums, silu_mul, quantize_row_q8_0), so the bytes are theirs.
+// The arithmetic per value is that of the stand-alone kernels (silu_mul, quantize_row_q8_0), and where they add up K in more shares than
+// the launch has sets, the sets take the shares in PASSES, each ending in the sum over the sets (gate_up_cut in q8_0_plan.h: 2.5 us a pass,
+// with the next pass's first group on its way meanwhile; fetched behind the sum it was 4).
 // C / C2 (optional, inspection): the fp32 gate / up tiles as the launch computed them.
-template<int TM, bool DUMP, int KS, bool STREAM, bool SPLIT, bool GATE_UP>
+template<int TM, bool DUMP, int KS, bool STREAM, bool SPLIT, bool GATE_UP, bool PASSES = false>
 __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, const uint8_t* __restrict__ A, float* C, const float* R, int32_t* __restrict__ sums, int M, int N, int groups,
-	float* __restrict__ partials, unsigned* __restrict__ counters, const uint8_t* __restrict__ W2, uint8_t* __restrict__ act_out, float* __restrict__ C2) {
+	float* __restrict__ partials, unsigned* __restrict__ counters, const uint8_t* __restrict__ W2, uint8_t* __restrict__ act_out, float* __restrict__ C2, int passes = 1, bool tree = false) {
 	static_assert(!SPLIT || (KS > 1 && !DUMP), "K over several workgroups continues the K sets' sum");
 	static_assert(!GATE_UP || (!DUMP && !SPLIT), "the fused gate/up form leaves a workgroup's tile quantized");
 	constexpr int DATA_BYTES  = TM * MACRO_BYTES;
@@ -218,7 +222,9 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 	constexpr int XCH_BYTES	   = GATE_UP ? 2 * TM * 16 * 64 * 4 : 0;
 	constexpr int FUSE_BYTES   = GATE_UP ? XCH_BYTES + 2 * TM * (TILE_BYTES + 64) : 0;
 	constexpr int LDS_BASE	   = KS * SET_BYTES > PARK_BYTES ? KS * SET_BYTES : PARK_BYTES;
-	constexpr int LDS_BYTES	   = LDS_BASE > FUSE_BYTES ? LDS_BASE : FUSE_BYTES;
+	constexpr int SAVE_AT	   = LDS_BASE > FUSE_BYTES ? LDS_BASE : FUSE_BYTES; // the passes' sums so far, every value where its lane put it
+	constexpr int LDS_BYTES	   = SAVE_AT + (PASSES ? 4 * TM * 16 * 64 * 4 : 0);
+	static_assert(!PASSES || (GATE_UP && KS > 1));
 	__shared__ __align__(16) uint8_t lds_raw[LDS_BYTES];
 	typedef _Float16 v4h __attribute__((ext_vector_type(4)));
 
@@ -229,14 +235,31 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 	const int kr	   = wave_all >> 2; // which K range
 	uint8_t* lds	   = lds_raw + kr * SET_BYTES;
 	// the host launches KS > 1, and K over gridDim.z workgroups, only when they divide
-	const int g_len	   = SPLIT ? groups / (KS * static_cast<int>(gridDim.z)) : groups / KS;
+	int g_len = SPLIT ? groups / (KS * static_cast<int>(gridDim.z)) : groups / KS;
 	// which share of K: with K over workgroups in the shapes that the streaming kernel can take too, the one that makes the sums below the
 	// tree that kernel adds its eight or sixteen waves' shares in (0 4 2 6 / 1 5 3 7, then the same of 8 to 15)
 	constexpr bool TREE = SPLIT && !STREAM;
 	static_assert(!TREE || KS == 4);
 	const int z		  = SPLIT ? static_cast<int>(blockIdx.z) : 0;
 	const int share	  = TREE ? 8 * (z >> 1) + (z & 1) + 4 * (kr & 1) + 2 * (kr >> 1) : z * KS + kr;
-	const int g_base  = share * g_len;
+	const int g_base  = PASSES ? 0 : share * g_len;
+	// passes: passes * KS shares of K, cut as wave_k_range does; the sets take them in the order that makes the sums below the mat-mat's.
+	// This set's first group and number of groups in this pass, and its first group in the next one; g_len: the most groups any set has.
+	int g0 = 0, live = 0, after = 0;
+	auto begin_pass = [&](int pass) {
+		const auto share_of = [&](int p) { return tree ? p + 4 * (kr & 1) + 2 * (kr >> 1) : p * KS + kr; };
+		int g1, unused;
+		wave_k_range(groups, 0, 0, passes * KS, share_of(pass), g0, g1);
+		live  = g1 - g0;
+		g_len = (groups + passes * KS - 1) / (passes * KS);
+		after = g1 - 1;
+		if (pass + 1 < passes) {
+			wave_k_range(groups, 0, 0, passes * KS, share_of(pass + 1), after, unused);
+		}
+	};
+	if constexpr (PASSES) {
+		begin_pass(0);
+	}
 	const int half	   = lane >> 5;
 	const int m_strips = (M + 31) / 32;
 	const int n_strips = (N + 31) / 32;
@@ -273,7 +296,7 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 		uint32_t d;
 	};
 	auto fetch_a = [&](int g, a_regs& r) {
-		const int64_t adv = static_cast<int64_t>(g) * MACRO_BYTES;
+		const int64_t adv = static_cast<int64_t>(g0 + g) * MACRO_BYTES;
 		uint32_t l16 = lane16;
 		asm volatile("" : "+v"(l16));
 		const uint32_t l4 = l16 >> 2;
@@ -294,7 +317,7 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 		*reinterpret_cast<uint32_t*>(lds + stage * sc_stage + sc_dst + (l16 >> 2)) = r.d;
 	};
 	auto fetch_w = [&](int g, w_regs& r) {
-		const int64_t at = w_off + static_cast<int64_t>(g) * MACRO_BYTES;
+		const int64_t at = w_off + static_cast<int64_t>(g0 + g) * MACRO_BYTES;
 		const gptr_u8 p	 = scalar_base(Wm, at);
 		uint32_t l16 = lane16;
 		asm volatile("" : "+v"(l16));
@@ -308,7 +331,8 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 	// load number p of a group's set (PIECES of them: TM activation tiles, their scale dword, four weight tiles, their scales);
 	// the same loads as fetch_a and fetch_w, which the prologue issues in one go
 	constexpr int PIECES = TM + 2 + GROUP_BLOCKS;
-	auto fetch_piece = [&](int p, int g, a_regs& ra, w_regs& rw) {
+	auto fetch_piece = [&](int p, int in_pass, a_regs& ra, w_regs& rw) {
+		const int g	 = g0 + in_pass;
 		uint32_t l16 = lane16;
 		asm volatile("" : "+v"(l16));
 		if (p < TM) {
@@ -328,7 +352,7 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 		acc[i] = v16f{ 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0 };
 	}
 	const int a_sc_rel = half ? DATA_BYTES : MACRO_D_OFFSET + 8 * (lane & 31);
-	const int last	   = g_len - 1;
+	int last		   = PASSES ? live - 1 : g_len - 1;
 
 	w_regs wa, wb;
 	a_regs pre;
@@ -345,17 +369,21 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 	// loads, so every wait the compiler places is a count (a load under a condition makes it wait for everything
 	// outstanding instead).
 	auto trip = [&](int g, w_regs& cur, w_regs& nxt) {
-		const int gn = min(g + 1, last);
-		if (half) {
+		// (with another pass to come: its first group, on its way while this pass is summed)
+		const int gn = PASSES ? (g < last ? g + 1 : after - g0) : min(g + 1, last);
+		// (past the end of a set's share, where another set has one group more: zero scales on both sides add nothing)
+		const bool zero = PASSES ? half || g >= live : half;
+		if (zero) {
 			cur.d = v2u{ 0u, 0u };
 		}
+		const int sc_rel = PASSES && zero ? DATA_BYTES : a_sc_rel;
 		const uint8_t* stage = lds + (g & 1) * STAGE_BYTES;
 		// the operand of unit u + 1 is read from LDS before unit u's arithmetic starts: one exposed LDS latency per trip, not eight
 		constexpr int UNITS = GROUP_BLOCKS * TM;
 		auto read_a = [&](int u, v4i& a, uint32_t& sc) {
 			const int t = u / TM, i = u % TM;
 			a  = *reinterpret_cast<const v4i*>(stage + i * MACRO_BYTES + t * TILE_BYTES + 16 * lane);
-			sc = *reinterpret_cast<const uint16_t*>(stage + (half ? 0 : i * MACRO_BYTES) + a_sc_rel + 2 * t);
+			sc = *reinterpret_cast<const uint16_t*>(stage + (zero ? 0 : i * MACRO_BYTES) + sc_rel + 2 * t);
 		};
 		v4i a_cur;
 		uint32_t s_cur;
@@ -404,142 +432,195 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 		stash_a((g + 1) & 1, pre);
 		__syncthreads();
 	};
-	for (int g = 0; g < g_len; g += 2) {
-		trip(g, wa, wb);
-		if (g + 1 < g_len) {
-			trip(g + 1, wb, wa);
-		}
-	}
 	constexpr int PER = 16 / KS; // values of a lane's 16 per strip that a K set finishes: registers PER * kr .. PER * kr + PER - 1
 	float mine[TM * PER]; // this wave's share of the workgroup's tile (SPLIT: of its part of K)
-	if constexpr (KS > 1 && !DUMP) {
-		// The K sets' tiles are summed by all of them at once: set q keeps PER = 16 / KS of a lane's 16 values per strip (with
-		// four sets: rows 8q .. 8q+7 of every 32-row strip), parks the other sets' shares in LDS, and after one barrier adds what
-		// the others parked for it, in set order (s0 + s1 + s2 + s3 whatever q is, so the result does not depend on who adds),
-		// and stores its own rows.  One set adding the others' whole tiles in turn took 12 % of the launch at M=512, N=K=4096.
-		__syncthreads(); // every set is through with its stages
-		float* park = reinterpret_cast<float*>(lds_raw);
-		auto slot	= [&](int q, int src) { // where set src parks its share of part q (src != q), this wave's strip
-			return park + ((((q * 4 + wave) * (KS - 1)) + (src < q ? src : src - 1)) * (PER * TM)) * 64 + lane;
-		};
+	for (int pass = 0;; ++pass) {
+		for (int g = 0; g < g_len; g += 2) {
+			trip(g, wa, wb);
+			if (g + 1 < g_len) {
+				trip(g + 1, wb, wa);
+			}
+		}
+		if constexpr (KS > 1 && !DUMP) {
+			// The K sets' tiles are summed by all of them at once: set q keeps PER = 16 / KS of a lane's 16 values per strip (with
+			// four sets: rows 8q .. 8q+7 of every 32-row strip), parks the other sets' shares in LDS, and after one barrier adds what
+			// the others parked for it, in set order (s0 + s1 + s2 + s3 whatever q is, so the result does not depend on who adds),
+			// and stores its own rows.  One set adding the others' whole tiles in turn took 12 % of the launch at M=512, N=K=4096.
+			__syncthreads(); // every set is through with its stages
+			float* park = reinterpret_cast<float*>(lds_raw);
+			int own		= lane;
+			if constexpr (PASSES) {
+				asm volatile("" : "+v"(own)); // the addresses are worked out here, not kept in registers that the trips need
+			}
+			auto slot	= [&](int q, int src) { // where set src parks its share of part q (src != q), this wave's strip
+				return park + ((((q * 4 + wave) * (KS - 1)) + (src < q ? src : src - 1)) * (PER * TM)) * 64 + own;
+			};
 #pragma unroll
-		for (int q = 0; q < KS; ++q) {
-			if (q != kr) {
-				float* dst = slot(q, kr);
+			for (int q = 0; q < KS; ++q) {
+				if (q != kr) {
+					float* dst = slot(q, kr);
 #pragma unroll
-				for (int i = 0; i < TM; ++i) {
+					for (int i = 0; i < TM; ++i) {
 #pragma unroll
-					for (int e = 0; e < PER; ++e) {
-						dst[(i * PER + e) * 64] = acc[i][q * PER + e];
+						for (int e = 0; e < PER; ++e) {
+							dst[(i * PER + e) * 64] = acc[i][q * PER + e];
+						}
 					}
 				}
 			}
-		}
-		const int n = ns * 32 + (lane & 31);
-		// the residual of this wave's rows, requested together and before the sums are: R may be C, every element is read here and written
-		// below by the same thread
-		float add[TM * PER];
-		if (!GATE_UP && R) {
+			float* save = reinterpret_cast<float*>(lds_raw + (PASSES ? SAVE_AT : 0)) + wave_all * (TM * PER * 64) + own;
+			const int n = ns * 32 + (lane & 31);
+			// the residual of this wave's rows, requested together and before the sums are: R may be C, every element is read here and written
+			// below by the same thread
+			float add[TM * PER];
+			if (!GATE_UP && R) {
 #pragma unroll
-			for (int j = 0; j < TM * PER; ++j) {
-				const int ee = kr * PER + j % PER;
-				const int m	 = (ms0 + j / PER) * 32 + 8 * (ee >> 2) + 4 * half + (ee & 3);
-				add[j]		 = (m < M && n < N) ? R[static_cast<int64_t>(m) * N + n] : 0.0f;
+				for (int j = 0; j < TM * PER; ++j) {
+					const int ee = kr * PER + j % PER;
+					const int m	 = (ms0 + j / PER) * 32 + 8 * (ee >> 2) + 4 * half + (ee & 3);
+					add[j]		 = (m < M && n < N) ? R[static_cast<int64_t>(m) * N + n] : 0.0f;
+				}
 			}
-		}
-		__syncthreads();
+			__syncthreads();
+			if constexpr (PASSES) { // (an earlier pass's are in LDS: nothing for the compiler to keep through the trips)
 #pragma unroll
-		for (int q = 0; q < KS; ++q) {
-			if (q == kr) {
+				for (int j = 0; j < TM * PER; ++j) {
+					mine[j] = 0.0f;
+				}
+			}
 #pragma unroll
-				for (int i = 0; i < TM; ++i) {
+			for (int q = 0; q < KS; ++q) {
+				if (q == kr) {
 #pragma unroll
-					for (int e = 0; e < PER; ++e) {
-						float part[KS], v;
+					for (int i = 0; i < TM; ++i) {
 #pragma unroll
-						for (int src = 0; src < KS; ++src) {
-							part[src] = src == q ? acc[i][q * PER + e] : slot(q, src)[(i * PER + e) * 64];
-							v		  = src == 0 ? part[src] : v + part[src];
+						for (int e = 0; e < PER; ++e) {
+							float part[KS], v;
+#pragma unroll
+							for (int src = 0; src < KS; ++src) {
+								part[src] = src == q ? acc[i][q * PER + e] : slot(q, src)[(i * PER + e) * 64];
+							}
+							if constexpr (PASSES && KS == 2) { // one set after the other, two of them in each pass
+								if (pass > 0) {
+									part[0] = save[(i * PER + e) * 64] + part[0];
+								}
+							}
+							v = part[0];
+#pragma unroll
+							for (int src = 1; src < KS; ++src) {
+								v += part[src];
+							}
+							if constexpr (KS == 4) {
+								if (TREE || (PASSES && tree)) {
+									v = (part[0] + part[1]) + (part[2] + part[3]);
+								}
+							}
+							if constexpr (PASSES && KS == 4) { // two workgroups' sums, or the two halves of the tree
+								if (pass > 0) {
+									v = save[(i * PER + e) * 64] + v;
+								}
+							}
+							mine[i * PER + e] = v;
 						}
-						if constexpr (TREE) {
-							v = (part[0] + part[1]) + (part[2] + part[3]);
-						}
-						mine[i * PER + e] = v;
 					}
 				}
 			}
-		}
-		if constexpr (SPLIT) {
-			// K over gridDim.z workgroups: every one leaves its tile in the scratch (each wave its own rows, as it holds them),
-			// counts itself in, and the last to arrive adds the tiles in z order -- whoever that is -- and stores
-			__shared__ int last_flag;
-			const int kz_count = static_cast<int>(gridDim.z);
-			const int unit	   = static_cast<int>(blockIdx.y * gridDim.x + blockIdx.x);
-			constexpr int TILE_FLOATS = 4 * KS * TM * PER * 64; // = TM * 4096: a workgroup's tile
-			float* tile = partials + (static_cast<int64_t>(unit) * kz_count) * TILE_FLOATS + wave_all * (TM * PER * 64) + lane;
-			float* dst	= tile + static_cast<int64_t>(blockIdx.z) * TILE_FLOATS;
+			if constexpr (SPLIT) {
+				// K over gridDim.z workgroups: every one leaves its tile in the scratch (each wave its own rows, as it holds them),
+				// counts itself in, and the last to arrive adds the tiles in z order -- whoever that is -- and stores
+				__shared__ int last_flag;
+				const int kz_count = static_cast<int>(gridDim.z);
+				const int unit	   = static_cast<int>(blockIdx.y * gridDim.x + blockIdx.x);
+				constexpr int TILE_FLOATS = 4 * KS * TM * PER * 64; // = TM * 4096: a workgroup's tile
+				float* tile = partials + (static_cast<int64_t>(unit) * kz_count) * TILE_FLOATS + wave_all * (TM * PER * 64) + lane;
+				float* dst	= tile + static_cast<int64_t>(blockIdx.z) * TILE_FLOATS;
 #pragma unroll
-			for (int j = 0; j < TM * PER; ++j) {
-				__hip_atomic_store(&dst[j * 64], mine[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-			}
-			wait_stores_acknowledged();
-			__syncthreads();
-			if (tid == 0) {
-				const unsigned prev = __hip_atomic_fetch_add(&counters[unit], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-				const int last		= (prev == static_cast<unsigned>(kz_count - 1));
-				if (last) {
-					__hip_atomic_store(&counters[unit], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); // ready for the next launch
+				for (int j = 0; j < TM * PER; ++j) {
+					__hip_atomic_store(&dst[j * 64], mine[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 				}
-				last_flag = last;
-			}
-			__syncthreads();
-			if (!last_flag) {
-				return;
-			}
+				wait_stores_acknowledged();
+				__syncthreads();
+				if (tid == 0) {
+					const unsigned prev = __hip_atomic_fetch_add(&counters[unit], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+					const int last		= (prev == static_cast<unsigned>(kz_count - 1));
+					if (last) {
+						__hip_atomic_store(&counters[unit], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); // ready for the next launch
+					}
+					last_flag = last;
+				}
+				__syncthreads();
+				if (!last_flag) {
+					return;
+				}
 #pragma unroll
-			for (int j = 0; j < TM * PER; ++j) {
-				mine[j] = 0.0f;
-			}
-			constexpr int STEP = TREE ? 2 : 1; // (an even number of workgroups)
-			for (int z0 = 0; z0 < kz_count; z0 += STEP) {
-				float got[STEP][TM * PER];
+				for (int j = 0; j < TM * PER; ++j) {
+					mine[j] = 0.0f;
+				}
+				constexpr int STEP = TREE ? 2 : 1; // (an even number of workgroups)
+				for (int z0 = 0; z0 < kz_count; z0 += STEP) {
+					float got[STEP][TM * PER];
 #pragma unroll
-				for (int u = 0; u < STEP; ++u) {
+					for (int u = 0; u < STEP; ++u) {
+#pragma unroll
+						for (int j = 0; j < TM * PER; ++j) {
+							got[u][j] = __hip_atomic_load(&tile[static_cast<int64_t>(z0 + u) * TILE_FLOATS + j * 64], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+						}
+					}
 #pragma unroll
 					for (int j = 0; j < TM * PER; ++j) {
-						got[u][j] = __hip_atomic_load(&tile[static_cast<int64_t>(z0 + u) * TILE_FLOATS + j * 64], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+						const float v = TREE ? got[0][j] + got[STEP - 1][j] : got[0][j];
+						mine[j]		  = z0 == 0 ? v : mine[j] + v;
+					}
+				}
+			}
+			if constexpr (!GATE_UP) {
+				if (R) {
+#pragma unroll
+					for (int j = 0; j < TM * PER; ++j) {
+						mine[j] += add[j];
 					}
 				}
 #pragma unroll
 				for (int j = 0; j < TM * PER; ++j) {
-					const float v = TREE ? got[0][j] + got[STEP - 1][j] : got[0][j];
-					mine[j]		  = z0 == 0 ? v : mine[j] + v;
+					const int ee = kr * PER + j % PER;
+					const int m	 = (ms0 + j / PER) * 32 + 8 * (ee >> 2) + 4 * half + (ee & 3);
+					if (m < M && n < N) {
+						C[static_cast<int64_t>(m) * N + n] = mine[j];
+					}
 				}
+				return;
 			}
-		}
-		if constexpr (!GATE_UP) {
-			if (R) {
+			__syncthreads(); // the sets have read each other's sums: the exchange below (or the next pass's stages) goes to the same place
+			if constexpr (PASSES) {
+				if (pass + 1 < passes) {
 #pragma unroll
-				for (int j = 0; j < TM * PER; ++j) {
-					mine[j] += add[j];
+					for (int j = 0; j < TM * PER; ++j) {
+						save[j * 64] = mine[j];
+					}
+#pragma unroll
+					for (int i = 0; i < TM; ++i) {
+						acc[i] = v16f{ 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0 };
+					}
+					if ((tid & 255) < 8) {
+						*reinterpret_cast<uint32_t*>(lds + ((tid & 255) >> 2) * STAGE_BYTES + DATA_BYTES + 4 * (tid & 3)) = 0u; // the zero scales again
+					}
+					if (g_len & 1) {
+						wa = wb;
+					}
+					stash_a(0, pre);
+					begin_pass(pass + 1);
+					last = live - 1;
+					__syncthreads();
+					continue;
 				}
 			}
+		} else {
 #pragma unroll
 			for (int j = 0; j < TM * PER; ++j) {
-				const int ee = kr * PER + j % PER;
-				const int m	 = (ms0 + j / PER) * 32 + 8 * (ee >> 2) + 4 * half + (ee & 3);
-				if (m < M && n < N) {
-					C[static_cast<int64_t>(m) * N + n] = mine[j];
-				}
+				mine[j] = acc[j / PER][j % PER];
 			}
-			return;
 		}
-		__syncthreads(); // the sets have read each other's sums: the exchange below goes to the same place
-	} else {
-#pragma unroll
-		for (int j = 0; j < TM * PER; ++j) {
-			mine[j] = acc[j / PER][j % PER];
-		}
+		break;
 	}
 	if constexpr (GATE_UP) {
 		// Every wave is through with the stages (the last trip ended in a barrier).  The gate wave and the up wave of a strip (and K set)
@@ -630,10 +711,10 @@ __global__ __launch_bounds__(256 * KS, 4) void gemm_tiled_kernel(const uint8_t* 
 }
 
 // the fused gate / up form (GATE_UP above): N = rows of each of the two matrices; gate_out / up_out optional
-template<int TM, int KS, bool STREAM>
+template<int TM, int KS, bool STREAM, bool PASSES>
 __global__ __launch_bounds__(256 * KS, 4) void gemm_gate_up_kernel(const uint8_t* __restrict__ W_gate, const uint8_t* __restrict__ W_up, const uint8_t* __restrict__ A, uint8_t* __restrict__ act_out,
-	float* __restrict__ gate_out, float* __restrict__ up_out, int M, int N, int groups) {
-	gemm_tiled_body<TM, false, KS, STREAM, false, true>(W_gate, A, gate_out, nullptr, nullptr, M, N, groups, nullptr, nullptr, W_up, act_out, up_out);
+	float* __restrict__ gate_out, float* __restrict__ up_out, int M, int N, int groups, int passes, bool tree) {
+	gemm_tiled_body<TM, false, KS, STREAM, false, true, PASSES>(W_gate, A, gate_out, nullptr, nullptr, M, N, groups, nullptr, nullptr, W_up, act_out, up_out, passes, tree);
 }
 
 // Executes a cut made by plan_gemm_tile (q8_0_plan.h): TM activation strips per wave, KS sets of four waves per workgroup,
@@ -684,24 +765,30 @@ hipError_t launch_gemm_gate_up_silu(const void* w_gate, const void* w_up, const 
 		return hipSuccess;
 	}
 	if (gate_up_rows_suits(M, n_ff, K)) {
-		return launch_gemm_rows_gate_up(w_gate, w_up, aq, act_out, gate_dbg, up_dbg, M, n_ff, K, plan_gemm_skinny(M, n_ff, K).waves, s);
+		return launch_gemm_rows_gate_up(w_gate, w_up, aq, act_out, gate_dbg, up_dbg, M, n_ff, K, gate_up_rows_waves(M, n_ff, K), s);
 	}
-	gemm_tile_cut cut{};
+	gate_up_cut cut{};
 	if (plan_gate_up_fused(M, n_ff, K, &cut)) {
-		const uint8_t* wg = static_cast<const uint8_t*>(w_gate);
-		const uint8_t* wu = static_cast<const uint8_t*>(w_up);
-		const uint8_t* a  = static_cast<const uint8_t*>(aq);
-		uint8_t* out	  = static_cast<uint8_t*>(act_out);
-		const int m = static_cast<int>(M), n = static_cast<int>(n_ff), groups = static_cast<int>(K / GROUP_K);
-		const dim3 grid(cut.grid_x, cut.grid_y);
-		auto launch = [&](auto kernel, int ks) { return launch_kernel(KIND_GEMM, kernel, grid, dim3(256 * ks), 0, s, wg, wu, a, out, gate_dbg, up_dbg, m, n, groups); };
-		if (cut.tm == 1) { // 17 to 32 rows on matrices of 192 column blocks and more (the rows kernel has the others): four K sets are never cut
-			return cut.ks == 2 ? launch(gemm_gate_up_kernel<1, 2, true>, 2) : launch(gemm_gate_up_kernel<1, 1, true>, 1);
+		const gemm_tile_cut& t = cut.tile;
+		const dim3 grid(t.grid_x, t.grid_y);
+		auto launch = [&](auto kernel) {
+			return launch_kernel(KIND_GEMM, kernel, grid, dim3(static_cast<unsigned>(256 * t.ks)), 0, s, static_cast<const uint8_t*>(w_gate), static_cast<const uint8_t*>(w_up), static_cast<const uint8_t*>(aq),
+				static_cast<uint8_t*>(act_out), gate_dbg, up_dbg, static_cast<int>(M), static_cast<int>(n_ff), static_cast<int>(K / GROUP_K), cut.passes, cut.tree);
+		};
+		if (t.tm == 1) { // 17 to 32 rows on matrices of 192 column blocks and more (the rows kernel has the others): four K sets are never cut
+			return t.ks == 1 ? launch(gemm_gate_up_kernel<1, 1, true, false>) : cut.passes > 1 ? launch(gemm_gate_up_kernel<1, 2, true, true>) : launch(gemm_gate_up_kernel<1, 2, true, false>);
 		}
-		if (cut.grid_y == 1) { // up to 64 rows: the weights are read once
-			return cut.ks == 4 ? launch(gemm_gate_up_kernel<2, 4, true>, 4) : cut.ks == 2 ? launch(gemm_gate_up_kernel<2, 2, true>, 2) : launch(gemm_gate_up_kernel<2, 1, true>, 1);
-		}
-		return cut.ks == 4 ? launch(gemm_gate_up_kernel<2, 4, false>, 4) : cut.ks == 2 ? launch(gemm_gate_up_kernel<2, 2, false>, 2) : launch(gemm_gate_up_kernel<2, 1, false>, 1);
+		auto launch_t = [&](auto stream) { // up to 64 rows the weights are read once
+			constexpr bool STREAM = decltype(stream)::value;
+			if (t.ks == 1) {
+				return launch(gemm_gate_up_kernel<2, 1, STREAM, false>);
+			}
+			if (t.ks == 2) {
+				return cut.passes > 1 ? launch(gemm_gate_up_kernel<2, 2, STREAM, true>) : launch(gemm_gate_up_kernel<2, 2, STREAM, false>);
+			}
+			return cut.passes > 1 ? launch(gemm_gate_up_kernel<2, 4, STREAM, true>) : launch(gemm_gate_up_kernel<2, 4, STREAM, false>);
+		};
+		return t.grid_y == 1 ? launch_t(std::true_type{}) : launch_t(std::false_type{});
 	}
 	float* gate = gate_dbg ? gate_dbg : workspace;
 	float* up	= up_dbg ? up_dbg : workspace + M * n_ff;

@@ -248,23 +248,57 @@ inline bool gate_up_rows_suits(int64_t M, int64_t n_ff, int64_t K) {
 	}
 	return plan_gemm_skinny(M, n_ff, K).splits == 1 && (M <= 16 || gemm_rows_suits(M, n_ff, K));
 }
+// Its shares of K, eight or sixteen: the streaming kernel's, or no fewer than the tile kernel has where it takes the mat-mats ([8192 x 8192] at
+// 16 rows: 9.4e-8 from the sums in 64 bits there, 1.1e-7 here with eight).
+inline int gate_up_rows_waves(int64_t M, int64_t n_ff, int64_t K) {
+	const gemm_plan g = plan_gemm(M, n_ff, K);
+	if (g.kernel == MM_GEMM_TILE_STREAM) {
+		return g.tile.ks * g.tile.kz > SK_WAVES ? SK_WIDE_WAVES : SK_WAVES;
+	}
+	return plan_gemm_skinny(M, n_ff, K).waves;
+}
 // The tile kernel's fused form, K sets included, wherever its grid has the chip's SIMDs two waves each, or about one where the matrices are
 // small enough that the launches saved count for more than idle CUs.  Whole calls, us, fused / three launches:
 //   rows      [2 x 14336 x 4096]   [2 x 28672 x 8192]   [2 x 11008 x 4096]   [2 x 8192 x 8192]   [2 x 5632 x 2048]   [2 x 4096 x 1024]
-//   64        30.8 / 43.1          105 / 114            26.6 / 43.2                              16.2 / 19.5
-//   117, 128  51.7 / 57.0                                                    54.5 / 82.5
-//   256                                                                                                              11.6 / 20.8
-// and below two waves per SIMD: [2 x 5632 x 4096] at 40 rows (1408 waves, 46 Mi weights) 24.7 / 29.0, but [2 x 6144 x 8192] at 64 rows
-// (1536 waves, 101 Mi) 42.0 / 39.4.
-constexpr int64_t GATE_UP_MIN_WAVES = 2048, GATE_UP_MIN_WAVES_SMALL = 1100, GATE_UP_SMALL_WEIGHTS = 48ll << 20;
-inline bool plan_gate_up_fused(int64_t M, int64_t n_ff, int64_t K, gemm_tile_cut* cut = nullptr) {
+//   64        34.8 / 43.5          114 / 116            31.1 / 47.9                              19.4 / 22.4         11.8 / 13.8
+//   117, 128  56.5 / 62                                 52 / 54              60 / 86             20.5 / 31           15.4 / 19.7
+//   256                                                                      102 / 111           30 / 35             13.0 / 25.5
+// and below two waves per SIMD: [2 x 5632 x 4096] at 40 rows (1408 waves, 46 Mi weights) faster, but [2 x 6144 x 8192] at 64 rows
+// (1536 waves, 101 Mi) not.
+//
+// The mat-mats it stands for have K in up to four times as many shares (grids of half the size, and K over workgroups), and fewer shares
+// are longer sums: [8192 x 8192] at 64 rows 9.4e-8 from the sums in 64 bits with sixteen, 1.5e-7 with four.  So the sets take as many, in two passes,
+// adding them in the mat-mats' order (same bytes), or in four with two sets (their tree of eight has no room for a second sum: the last
+// bits differ).  A pass costs 2.5 us; two of four sets are the most that pays ([2 x 8192 x 8192] at 64 rows: four would be 53 us, three
+// launches are 52).  K of at most 1024, 32 blocks, has nothing to gain: one pass, whatever the mat-mats do.
+struct gate_up_cut {
+	gemm_tile_cut tile;
+	int passes; // passes * ks shares of K, ks at a time
+	bool tree; // eight shares in two passes, added as the streaming kernel adds them
+};
+constexpr int64_t GATE_UP_MIN_WAVES = 2048, GATE_UP_MIN_WAVES_SMALL = 1100, GATE_UP_SMALL_WEIGHTS = 48ll << 20, GATE_UP_SHORT_K = 1024;
+inline bool plan_gate_up_fused(int64_t M, int64_t n_ff, int64_t K, gate_up_cut* cut = nullptr) {
 	if (M <= 0 || n_ff <= 0 || K <= 0 || n_ff % GROUP_K != 0 || K % GROUP_K != 0) {
 		return false;
 	}
-	const gemm_tile_cut c = plan_gemm_tile(M, 2 * n_ff, K, false); // grid_x = n_ff / 64 workgroups of two gate and two up strips
-	const int64_t waves	  = int64_t{ 4 } * c.ks * c.grid_x * c.grid_y;
-	if (waves < (2 * n_ff * K <= GATE_UP_SMALL_WEIGHTS ? GATE_UP_MIN_WAVES_SMALL : GATE_UP_MIN_WAVES) && !(c.ks == 1 && plan_gemm(M, n_ff, K).kernel == MM_GEMM_TILE)) {
+	gate_up_cut c{ {}, 1, false };
+	c.tile			  = plan_gemm_tile(M, 2 * n_ff, K, false); // grid_x = n_ff / 64 workgroups of two gate and two up strips
+	const gemm_plan g = plan_gemm(M, n_ff, K);
+	const int64_t waves = int64_t{ 4 } * c.tile.ks * c.tile.grid_x * c.tile.grid_y;
+	if (c.tile.ks == 1 && g.kernel == MM_GEMM_TILE) {
+		// a prompt: one set of waves per workgroup has all of K (the mat-mats alone may have two)
+	} else if (waves < (2 * n_ff * K <= GATE_UP_SMALL_WEIGHTS ? GATE_UP_MIN_WAVES_SMALL : GATE_UP_MIN_WAVES)) {
 		return false;
+	} else {
+		const bool tree	 = g.kernel == MM_GEMM_SKINNY || (g.kernel == MM_GEMM_TILE && g.tile.kz > 1);
+		const int shares = g.kernel == MM_GEMM_SKINNY ? g.skinny.splits * g.skinny.waves : g.tile.ks * g.tile.kz;
+		if (K > GATE_UP_SHORT_K) {
+			c.passes = shares / c.tile.ks;
+			c.tree	 = tree && c.tile.ks == 4;
+			if (c.passes > 1 && (c.tile.ks == 1 || c.passes > (c.tile.ks == 4 ? 2 : 4))) {
+				return false;
+			}
+		}
 	}
 	if (cut) {
 		*cut = c;

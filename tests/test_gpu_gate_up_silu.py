@@ -106,3 +106,41 @@ def test_gate_up_silu_k_sets(q8, oracle, m, n_ff, k):
     whole = to_host(q8.untile(act, padded, n_ff)).reshape(padded, -1)
     assert np.array_equal(whole[:m], oracle.silu_mul_quantize_rows(gate, up)) and not whole[m:].any()
     assert np.array_equal(to_host(q8.gate_up_silu(tg, tu, aq, m, n_ff, k)), to_host(act))
+
+
+# One launch, the bytes of the three it stands for: four K sets in two passes as two workgroups' sums (40 rows: K over two workgroups per
+# tile in the mat-mats) and as the streaming kernel's tree, with even shares, with shares that differ by a group, and for mat-mats with K
+# over workgroups; two K sets in two passes, of two row strips and of one; one pass.  Infinite scales at the ends of the shares: what
+# stands for the group that a smaller share does not have must add nothing to them.
+@pytest.mark.parametrize("m,n_ff,k", [(40, 12800, 4096), (64, 4608, 2048), (64, 4608, 2560), (97, 2304, 4608), (66, 4224, 5120), (64, 24576, 2048), (33, 24576, 2048), (24, 24576, 2048), (100, 12288, 512)])
+def test_gate_up_silu_has_the_bytes_of_three_launches(q8, oracle, m, n_ff, k):
+    assert q8._lib.lib().nh_q8_0_gate_up_silu_workspace_bytes(m, n_ff, k) == 0
+    tg, tu = (q8.tile(q8.fill_weight_blocks(s + m, n_ff, k), n_ff, k) for s in (31, 32))
+    aq = oracle.quantize_rows(oracle.fill_activations(m + k, m * k).reshape(m, k))
+    aq = aq.reshape(m, k // 32, 34)
+    last = np.cumsum([len(share) for share in np.array_split(np.arange(k // 128), 8)]) * 4 - 1  # the last block of each eighth of K
+    for row, block in enumerate(last):
+        aq[row, block, :2] = [0x00, 0x7C]
+    at = q8.tile(to_dev(aq.reshape(-1)), m, k)
+    gate, up = q8.gemm(tg, at, m, n_ff, k, tiled=True), q8.gemm(tu, at, m, n_ff, k, tiled=True)
+    act, g, u = q8.gate_up_silu(tg, tu, at, m, n_ff, k, debug=True)
+    assert np.array_equal(to_host(g), to_host(gate), equal_nan=True) and np.array_equal(to_host(u), to_host(up), equal_nan=True)
+    assert np.isinf(to_host(g)[:8]).mean() > 0.99 and np.isfinite(to_host(g)[8:]).all()  # (a block sum of 0 makes a NaN)
+    assert np.array_equal(to_host(act), to_host(q8.silu_mul_quantize(gate, up, tiled=True)))
+    assert np.array_equal(to_host(act), to_host(q8.gate_up_silu(tg, tu, at, m, n_ff, k)))
+
+
+# eight shares of K, two K sets at a time (the mat-mats add them in another order)
+@pytest.mark.parametrize("m,n_ff,k", [(48, 18432, 2048), (33, 17664, 2560)])
+def test_gate_up_silu_in_four_passes(q8, oracle, m, n_ff, k):
+    assert q8._lib.lib().nh_q8_0_gate_up_silu_workspace_bytes(m, n_ff, k) == 0
+    wg = oracle.fill_weights(m, n_ff, k)
+    tg, x = q8.tile(to_dev(wg), n_ff, k), oracle.fill_activations(m + k, m * k).reshape(m, k)
+    act, gate, up = q8.gate_up_silu(tg, tg, q8.quantize_row_q8_0(to_dev(x), tiled=True), m, n_ff, k, debug=True)
+    gate, up = to_host(gate), to_host(up)
+    assert np.array_equal(gate, up)
+    want = oracle.gemm(wg, oracle.quantize_rows(x), m, n_ff, k, threads=8)
+    assert all(rel_l2(gate[i], want[i]) <= REL_L2_TOL for i in range(m))
+    padded = (m + 31) // 32 * 32
+    whole = to_host(q8.untile(act, padded, n_ff)).reshape(padded, -1)
+    assert np.array_equal(whole[:m], oracle.silu_mul_quantize_rows(gate, up)) and not whole[m:].any()
