@@ -20,9 +20,14 @@
  *   use or by nh_q8_0_prepare): nh_q8_0_gemv_tiled*, nh_q8_0_gemv_tiled_group_f32, nh_q8_0_mul_mat*, nh_q8_0_mul_mat_batch,
  *   nh_q8_0_mul_mat_f32_activations (each when the shape makes them split K over workgroups), nh_q8_0_gemm_tiled*,
  *   and nh_q8_0_ffn_f32 and nh_q8_0_decode_layer_f32 always.  That scratch serves ONE stream at a time per GPU: enqueue such calls on one stream, or let
- *   the other stream drain first.  A call that would use the scratch while a launch from a different stream may still be
- *   running returns NH_ERR_BUSY and launches nothing (not detected: work on a capturing stream, work that followed a
- *   launch on the NULL stream, and replays of captured graphs, which the caller must keep from overlapping).
+ *   the other stream drain first.  Any number of host threads may make such calls: a launch is enqueued before the scratch is given out again.
+ *   A call that would use the scratch while a launch from a different stream may still be
+ *   running returns NH_ERR_BUSY and launches nothing (not detected: work on a capturing stream, a mat-vec's, FFN's or block's launch that
+ *   followed one on the NULL stream, and replays of captured graphs, which the caller must keep from overlapping).
+ *   The mat-mats have scratch of their own: (a) for up to 32 rows, (b) for up to 64 and for more against small matrices, (c) for more than
+ *   64 with K over workgroups; each once for the NULL stream and once for the others.  A call that would use (c) and finds it in use, or is
+ *   being captured, runs as a slower form without scratch; one that would use (a) does the same where that needs none, and
+ *   otherwise uses (b).  The result has the same bits either way.
  *   The check queries the other stream; it does so in the relaxed capture mode, so it may run while a third stream of the
  *   calling thread is being captured in the global mode without disturbing that capture.
  *   A kernel that waits for another workgroup's data does so for a bounded time; if it gives up, the output holds NaN and

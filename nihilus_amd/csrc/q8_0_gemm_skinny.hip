@@ -1,4 +1,5 @@
-// Batched-decode mat-mat for a handful of activation rows (M <= 64): C[m][n] = dot(W row n, Aq row m), gfx950.
+// Batched-decode mat-mat for some dozens of activation rows, and for more on small grids: C[m][n] = dot(W row n, Aq row m), gfx950.  (Up to 32
+// rows the kernel of q8_0_gemm_rows.hip has the shapes; this one runs those of its calls that cannot use its hand-off, to the same bits.)
 //
 // With so few rows the weights are read once and nothing is reused enough to leave the HBM roofline, so this is the
 // streaming mat-vec again -- one workgroup per (32-row weight strip, K split), waves splitting the strip's K range,
@@ -136,7 +137,7 @@ __global__ __launch_bounds__(WAVES * 64, 4) void gemm_skinny_kernel(const uint8_
 	}
 	// ---- the waves' partial sums through LDS; a wave finishes OWN of every lane's MS * 16 values ----
 	// (One wave finishing them all, behind a tree of barriers, and reading the residual value by value behind its own stores was a chain
-	// of 16 * MS memory latencies: [4096 x 4096] at 117 rows 23.1 us with a residual against 13.9 without; now 13.9 and 12.6.)
+	// of 16 * MS memory latencies: [4096 x 4096] at 117 rows 17.2 us with a residual and 14.6 without; now 12.3 and 12.2.)
 	constexpr int OWN = MS * 16 / WAVES;
 	const int n		  = strip * STRIP_ROWS + r;
 	const auto row_of = [&](int v) { return (mg * MS + (v >> 4)) * STRIP_ROWS + 8 * ((v & 15) >> 2) + 4 * half + (v & 3); };

@@ -468,7 +468,7 @@ __device__ __forceinline__ void split_k_finish(uint64_t* __restrict__ tagged, un
 
 // Scratch of the K-split path (tagged partial sums) and of the fused FFN launch (the gate and up
 // projections' outputs and one "published" word per producer strip): one allocation per device, made on first use and
-// kept for the life of the process.  Calls that overlap on one GPU (different streams) and both use it race on it.
+// kept for the life of the process.  It serves one stream at a time (get_gemv_scratch).
 constexpr int GEMV_MAX_SPLIT_UNITS	= 8192; // strips * splits when splits > 1
 constexpr int GEMV_MAX_SPLIT_STRIPS = 512;
 constexpr int FFN_MAX_HIDDEN		= 65536; // rows of the gate / up projections in a fused FFN launch

@@ -22,7 +22,7 @@ __device__ __forceinline__ int64_t tiled_d_offset(int64_t row, int64_t b, int64_
 // One wave per macro-tile (32 rows x 4 blocks), a workgroup's four waves on consecutive groups of a strip.  Lane (row r, half h) takes 68
 // contiguous bytes of its row, blocks 2h and 2h + 1 of the group, and owns what they become: 16 bytes of either half of tiles 2h and
 // 2h + 1 and a dword of the scale table; per store instruction 32 lanes fill 512 contiguous bytes.  It is a copy and bounded by memory:
-// [14336 x 4096] 25 us = 4.9 TB/s read and written, a plain copy on this card 5.1.  A thread per four quants (half-word loads, dword
+// [14336 x 4096] from memory 24.6 us = 5.1 TB/s read and written, a plain copy of as many bytes 5.0 (of 4 GiB 4.8).  A thread per four quants (half-word loads, dword
 // stores, divisions of a 64-bit index) was bounded by its instructions: 57 us, 2.2 TB/s; [1024 x 4096] 8.3 us against 5.7.
 constexpr int TILE_WAVES = 4;
 __global__ __launch_bounds__(TILE_WAVES * 64) void tile_kernel(const uint8_t* __restrict__ blocks, uint8_t* __restrict__ tiled, int64_t rows, int groups, int wg_per_strip) {

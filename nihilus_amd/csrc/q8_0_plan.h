@@ -1,5 +1,7 @@
 // Which kernel a mul_mat call runs, and how that kernel cuts the work: decided here, on the host, in one place, from the
-// shape alone.  The launchers execute the plan they get from these functions and decide nothing themselves, so a test can
+// shape alone.  The launchers execute the plan they get from these functions and decide nothing themselves -- but for a call that is being
+// captured, or finds the hand-off scratch of its form in use on another stream, which runs as the form without it that the plan has
+// for it: in the mat-mats the same additions in the same order -- so a test can
 // ask (nh_q8_0_debug_plan_mul_mat, no GPU needed) what a shape will run and pin it.
 //
 // The rules are measurements, not a model: each threshold below names the shapes it was fitted on.  A shape between the
@@ -152,18 +154,20 @@ inline bool plan_gemm_tile_split(int64_t M, int64_t N, int64_t K, gemm_tile_cut*
 	return true;
 }
 
-// Up to 32 rows the kernel of q8_0_gemm_rows.hip, with the cut above, where it is the faster one.
-// Measured against the kernels that had these shapes (weights rotated, kernel times, us):
+// Up to 32 rows the kernel of q8_0_gemm_rows.hip, with the cut above, where it is the faster one.  Measured against the kernels that had these
+// shapes (weights rotated, kernel times, us):
 //   rows                4            16            32
 //   [4096 x 4096]    5.7 /  9.8    6.3 /  9.1    8.7 /  9.4   (streaming kernel with eight waves' operand tiles from L2)
 //   [1024 x 4096]    4.6 /  8.0    5.0 /  8.2    6.9 /  8.8
 //   [4096 x 14336]  12.3 / 18.1   13.2 / 17.9   15.8 / 18.4
 //   [14336 x 4096]  11.0 / 13.9   12.1 / 14.7   14.4 / 15.8
-//   [8192 x 8192]                               14.9 / 17.8   (tile kernel, K over workgroups)
 //   [128256 x 4096] 80.7 / 83.9   86.1 / 88.1  106   / 91     (tile kernel)
 //   [28672 x 8192]  39.1 / 39.4   41.5 / 39.6   47   / 40
-// Every wave takes its own copy of the activations out of L2, M / 32 times the weight bytes, which the tile kernel shares over four
-// strips: that decides large matrices from 17 rows on, and long K from 9.
+// Every wave takes its own copy of the activations out of L2 (requests per weight line, [4096 x 14336]: 1.27 at 4 rows, 1.53 at 16, 2.07 at
+// 32), which the tile kernel shares over four strips (1.29 to 1.36): from 192 column blocks on, where that fills the chip by itself, this kernel has K up to 4096
+// and 16 rows.  The line lies between the two K measured.  plan_gemm asks the tile kernel first for 16 to 32 rows against 64 column blocks and
+// 64 Mi weights and more, by a rule drawn against the kernel before this one; not measured against this one but at [8192 x 8192], 32 rows:
+// 14.9 / 17.8.
 inline bool gemm_rows_suits(int64_t M, int64_t N, int64_t K) {
 	const int64_t column_blocks = (N + 127) / 128;
 	if (M > GEMM_ROWS_MAX) {
