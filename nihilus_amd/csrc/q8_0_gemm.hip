@@ -775,7 +775,7 @@ hipError_t launch_gemm_gate_up_silu(const void* w_gate, const void* w_up, const 
 			return launch_kernel(KIND_GEMM, kernel, grid, dim3(static_cast<unsigned>(256 * t.ks)), 0, s, static_cast<const uint8_t*>(w_gate), static_cast<const uint8_t*>(w_up), static_cast<const uint8_t*>(aq),
 				static_cast<uint8_t*>(act_out), gate_dbg, up_dbg, static_cast<int>(M), static_cast<int>(n_ff), static_cast<int>(K / GROUP_K), cut.passes, cut.tree);
 		};
-		if (t.tm == 1) { // 17 to 32 rows on matrices of 192 column blocks and more (the rows kernel has the others): four K sets are never cut
+		if (t.tm == 1) { // 17 to 32 rows on matrices of 192 column blocks and more (the rows kernel has the others)
 			return t.ks == 1 ? launch(gemm_gate_up_kernel<1, 1, true, false>) : cut.passes > 1 ? launch(gemm_gate_up_kernel<1, 2, true, true>) : launch(gemm_gate_up_kernel<1, 2, true, false>);
 		}
 		auto launch_t = [&](auto stream) { // up to 64 rows the weights are read once

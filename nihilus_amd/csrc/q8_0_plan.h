@@ -289,6 +289,9 @@ inline bool plan_gate_up_fused(int64_t M, int64_t n_ff, int64_t K, gate_up_cut* 
 	c.tile			  = plan_gemm_tile(M, 2 * n_ff, K, false); // grid_x = n_ff / 64 workgroups of two gate and two up strips
 	const gemm_plan g = plan_gemm(M, n_ff, K);
 	const int64_t waves = int64_t{ 4 } * c.tile.ks * c.tile.grid_x * c.tile.grid_y;
+	if (c.tile.tm == 1 && c.tile.ks > 2) {
+		return false; // no such form: K above 32768, which the rows kernel would have to hand over
+	}
 	if (c.tile.ks == 1 && g.kernel == MM_GEMM_TILE) {
 		// a prompt: one set of waves per workgroup has all of K (the mat-mats alone may have two)
 	} else if (waves < (2 * n_ff * K <= GATE_UP_SMALL_WEIGHTS ? GATE_UP_MIN_WAVES_SMALL : GATE_UP_MIN_WAVES)) {

@@ -107,3 +107,10 @@ def test_up_to_32_rows_every_wave_keeps_its_share_of_the_sums():
         p = q8_0.plan_mul_mat(m, n, k)
         assert p["kernel"] == "gemm_skinny" and p["gemm_rows"] and p["k_splits"] * p["waves"] == 8 * sets, (m, n, k, p)
     assert not q8_0.plan_mul_mat(33, 5120, 5120)["gemm_rows"] and not q8_0.plan_mul_mat(24, 28672, 8192)["gemm_rows"]
+
+
+@pytest.mark.parametrize("m,n_ff,k", [(26, 9600, 36864), (29, 8320, 45056), (18, 9088, 176128), (32, 16128, 160768)])
+def test_gate_up_of_one_strip_never_asks_for_four_k_sets(m, n_ff, k):
+    # the fused kernel for one strip of rows has one and two K sets; K above 32768, which the kernel for up to 32 rows would have to hand over,
+    # asks for more on grids this small: three launches, through the workspace
+    assert q8_0._lib.lib().nh_q8_0_gate_up_silu_workspace_bytes(m, n_ff, k) == 2 * m * n_ff * 4
