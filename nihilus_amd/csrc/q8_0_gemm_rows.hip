@@ -145,10 +145,17 @@ template<int R, int T, int MATS>
 __device__ __forceinline__ void rows_chunk(const uint8_t* __restrict__ w_strip, const uint8_t* __restrict__ w_strip2, const uint8_t* __restrict__ a_strip, uint8_t* a_tiles, uint8_t* a_scales, int gc,
 	int cnt, int lane, float (&acc)[MATS][R / 2]) {
 	static_assert(T == 1 || T == 2);
-	if (T == 2 && cnt == 2) { // wave-uniform
-		rows_chunk_n<R, T, MATS, T>(w_strip, w_strip2, a_strip, a_tiles, a_scales, gc, lane, acc);
-	} else {
-		rows_chunk_n<R, T, MATS, 1>(w_strip, w_strip2, a_strip, a_tiles, a_scales, gc, lane, acc);
+	switch (cnt) { // wave-uniform (an if with an else instead: 4.16 -> 4.23 us at [8123 x 1280], 5.29 -> 5.50 at 24 rows)
+		case 1:
+			rows_chunk_n<R, T, MATS, 1>(w_strip, w_strip2, a_strip, a_tiles, a_scales, gc, lane, acc);
+			break;
+		case 2:
+			if constexpr (T == 2) {
+				rows_chunk_n<R, T, MATS, 2>(w_strip, w_strip2, a_strip, a_tiles, a_scales, gc, lane, acc);
+			}
+			break;
+		default:
+			break;
 	}
 }
 
