@@ -98,8 +98,9 @@ inline gemm_skinny_cut plan_gemm_skinny(int64_t M, int64_t N, int64_t K) {
 		// [4096 x 14336] 12.6 and 13.3; [1024 x 4096] 4.6 us with 128).  Where the rule above makes more sets than that, a workgroup takes
 		// two of them (sixteen waves; in the rows kernel eight, one set after the other): no more additions in a row than there, and nothing
 		// more to hand over.  One set instead, [6144 x 6144] at 8 / 32 rows: 8.7 / 11.5 us against 9.0 / 12.1, but [8192 x 28672] 2.0e-7 from
-		// the sums in 64 bits where two sets are 1.5e-7, and [5120 x 5120] 9.9e-8 against 8.2e-8.  (Sixteen waves in the rows kernel too:
-		// 9.0 / 12.8 us.)
+		// the sums in 64 bits where two sets are 1.5e-7, and [5120 x 5120] 9.9e-8 against 8.2e-8.  Few strips with a long K pay most for the
+		// second set: [1037 x 16640] 7.3 / 10.5 us at 4 / 24 rows with one, 8.2 / 11.7 with two.  (Sixteen waves in the rows kernel too, at
+		// [6144 x 6144]: 9.0 / 12.8 us.)
 		const int sets = sets_for(SK_WAVES);
 		c.waves		   = SK_WAVES;
 		c.splits	   = 1;
