@@ -12,6 +12,13 @@ import torch
 
 from . import _lib
 
+# The calls of a step on several rows as native functions (csrc/py_calls.cpp).  They return the result, a status, or None for whatever is not
+# a plain call, which then goes the way below.  Without the module (a torch that it was not built against) every call goes that way.
+try:
+    from . import _calls
+except ImportError:
+    _calls = None
+
 QK = 32
 BLOCK_BYTES = 34
 
@@ -36,6 +43,12 @@ def _dev(t: torch.Tensor, dtype: torch.dtype, name: str) -> torch.Tensor:
     if not (t.is_cuda and t.dtype == dtype and t.is_contiguous()):
         raise TypeError(f"{name} must be a contiguous {dtype} tensor on the GPU")
     return t
+
+
+def _native(result, fn: str):
+    if type(result) is int:
+        _lib.check(fn, result)
+    return result
 
 
 def blocks_bytes(rows: int, k: int) -> int:
@@ -275,6 +288,8 @@ def debug_fused_quantize(x: torch.Tensor, norm_weight: torch.Tensor | None = Non
 
 def rms_norm_quantize(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, tiled: bool = False) -> torch.Tensor:
     """quantize_row_q8_0((x * 1/rms(x)) * norm_weight) for fp32 [M, K] (or [K]) rows, one kernel; output as quantize_row_q8_0."""
+    if tiled and _calls is not None and (out := _native(_calls.rms_norm_quantize(x, norm_weight, eps), "nh_q8_0_rms_norm_quantize_tiled")) is not None:
+        return out
     x, nw = _dev(x, torch.float32, "x"), _dev(norm_weight, torch.float32, "norm_weight")
     x2 = x.reshape(1, -1) if x.dim() == 1 else x
     m, k = x2.shape
@@ -290,6 +305,8 @@ def rms_norm_quantize(x: torch.Tensor, norm_weight: torch.Tensor, eps: float, ti
 
 
 def gemm(w: torch.Tensor, aq: torch.Tensor, m: int, n: int, k: int, tiled: bool) -> torch.Tensor:
+    if tiled and _calls is not None and (out := _native(_calls.gemm(w, aq, m, n, k, None), "nh_q8_0_gemm_tiled")) is not None:
+        return out
     w, aq = _dev(w, torch.uint8, "w"), _dev(aq, torch.uint8, "aq")
     size = tiled_bytes if tiled else blocks_bytes
     if w.numel() != size(n, k) or aq.numel() != size(m, k):
@@ -302,6 +319,8 @@ def gemm(w: torch.Tensor, aq: torch.Tensor, m: int, n: int, k: int, tiled: bool)
 
 def gemm_residual(w_tiled: torch.Tensor, aq_tiled: torch.Tensor, residual: torch.Tensor, m: int, n: int, k: int, out: torch.Tensor | None = None) -> torch.Tensor:
     """C = W . Aq + residual on tiled operands in one launch (out may be the residual tensor itself: in-place accumulate)."""
+    if out is None and residual is not None and _calls is not None and (c := _native(_calls.gemm(w_tiled, aq_tiled, m, n, k, residual), "nh_q8_0_gemm_tiled_residual")) is not None:
+        return c
     w, aq, residual = _dev(w_tiled, torch.uint8, "w_tiled"), _dev(aq_tiled, torch.uint8, "aq_tiled"), _dev(residual, torch.float32, "residual")
     if w.numel() != tiled_bytes(n, k) or aq.numel() != tiled_bytes(m, k) or residual.numel() != m * n:
         raise ValueError("operand sizes do not match m x n x k")
@@ -315,6 +334,8 @@ def gemm_residual(w_tiled: torch.Tensor, aq_tiled: torch.Tensor, residual: torch
 def gate_up_silu(w_gate: torch.Tensor, w_up: torch.Tensor, aq_tiled: torch.Tensor, m: int, n_ff: int, k: int, debug: bool = False):
     """Tiled Q8_0 activation of the down projection: quantize(silu(W_gate . Aq) * (W_up . Aq)) (nh_q8_0_gemm_tiled_gate_up_silu).
     debug=True also returns the fp32 gate and up outputs the call computed."""
+    if not debug and _calls is not None and (out := _native(_calls.gate_up_silu(w_gate, w_up, aq_tiled, m, n_ff, k), "nh_q8_0_gemm_tiled_gate_up_silu")) is not None:
+        return out
     lib = _lib.lib()
     out = torch.empty(tiled_bytes(m, n_ff), dtype=torch.uint8, device=aq_tiled.device)
     if debug:
@@ -332,6 +353,10 @@ def gate_up_silu(w_gate: torch.Tensor, w_up: torch.Tensor, aq_tiled: torch.Tenso
 
 def mul_mat(w_tiled: torch.Tensor, x: torch.Tensor, n: int, k: int, workspace: torch.Tensor | None = None, residual: torch.Tensor | None = None) -> torch.Tensor:
     """fp32 activations [M, K] x tiled Q8_0 weight [N, K] -> fp32 [M, N]: quantize + GEMV/GEMM (+ residual [M, N] if given)."""
+    if workspace is None and _calls is not None:
+        y = _native(_calls.mul_mat(w_tiled, x, n, k, residual), "nh_q8_0_mul_mat" if residual is None else "nh_q8_0_mul_mat_residual")
+        if y is not None:
+            return y
     w_tiled, x = _dev(w_tiled, torch.uint8, "w_tiled"), _dev(x, torch.float32, "x")
     x2 = x.reshape(1, -1) if x.dim() == 1 else x
     m = x2.shape[0]
