@@ -10,7 +10,7 @@
 // K is cut, and the sums are added, as in the streaming kernel (q8_0_gemm_skinny.hip), which runs a call that is being captured or finds
 // the hand-off's scratch in use on another stream: the result does not depend on which of the two ran.
 //
-// The activations come memory -> LDS without registers, and only the rows that exist: a 128-quant group of R rows (R = 8, 16 or 32) is
+// The activations come memory -> LDS without registers, and only the rows that exist: a 128-quant group of R rows (R = 8, 16, 24 or 32) is
 // R / 8 transfers of 1 KiB (lane l fetches the 16 bytes of one (block, k half, row)), so that eight rows cost a quarter of the weight
 // tile's requests; operand rows past R repeat them and their sums are never looked at.
 #include "q8_0_plan.h"
@@ -30,10 +30,14 @@ __device__ __forceinline__ void dma_b128(const uint8_t* base, uint32_t lane_off,
 typedef _Float16 rq_v4h __attribute__((ext_vector_type(4)));
 typedef float rq_v16f __attribute__((ext_vector_type(16)));
 
-// With 8 or 16 rows a lane multiplies the two scales of its 4 or 8 sums itself; with 32 (16 sums per lane) the products come from an
-// f16 MFMA (measured at 32 rows, [14336 x 4096] 14.9 -> 14.4 us, [8192 x 8192] 15.6 -> 14.9; at 16 rows 12.2 -> 12.8).
-template<int R> constexpr bool rows_scale_mfma = R == 32;
+// With 8 or 16 rows a lane multiplies the two scales of its 4 or 8 sums itself; with 24 or 32 (12 or 16 sums per lane) the products come from
+// an f16 MFMA (measured at 32 rows, [14336 x 4096] 14.9 -> 14.4 us, [8192 x 8192] 15.6 -> 14.9; at 24 rows 14.9 -> 14.1 and 16.2 -> 15.8; at
+// 16 rows 12.2 -> 12.8).
+template<int R> constexpr bool rows_scale_mfma = R >= 24;
 template<int R> constexpr int rows_group_bytes = R / 8 * 1024; // a group's operand rows in LDS: [block][k half][row][16 bytes]
+template<int R> __device__ __forceinline__ int rows_operand_row(int r) { // of operand row r (0..31) in LDS: past R one that exists
+	return R == 24 ? min(r, R - 1) : r & (R - 1);
+}
 
 // Groups [gc, gc + CNT) of a wave's K range, against MATS weight strips that share the activations.  CNT is a template parameter so
 // that every wait is a count of younger loads.
@@ -51,10 +55,12 @@ __device__ __forceinline__ void rows_chunk_n(const uint8_t* __restrict__ w_strip
 		const uint8_t* macro = a_strip + static_cast<int64_t>(gc + c) * MACRO_BYTES;
 #pragma unroll
 		for (int d = 0; d < R / 8; ++d) {
-			// lane l of transfer d: byte 1024 d + 16 l of the group's LDS image = block (64 d + l) / (2 R), half (l / R) % 2, row l % R
-			const int unit = lane; // + 64 d: whole blocks further on
+			// lane l of transfer d: byte 1024 d + 16 l of the group's LDS image = block u / (2 R), half u / R % 2, row u % R of unit u = 64 d + l
+			// (64 units are whole blocks but for R = 24)
+			constexpr bool WHOLE = 64 % (2 * R) == 0;
+			const int unit = WHOLE ? lane : 64 * d + lane;
 			const int off  = unit / (2 * R) * TILE_BYTES + (unit / R) % 2 * (TILE_BYTES / 2) + unit % R * 16;
-			dma_b128(macro + d * (64 / (2 * R)) * TILE_BYTES, off, lds_addr + c * rows_group_bytes<R> + d * 1024);
+			dma_b128(macro + (WHOLE ? d * (64 / (2 * R)) * TILE_BYTES : 0), off, lds_addr + c * rows_group_bytes<R> + d * 1024);
 		}
 	}
 	const int sg = min(lane / R, CNT - 1), sr = lane % R;
@@ -101,11 +107,11 @@ __device__ __forceinline__ void rows_chunk_n(const uint8_t* __restrict__ w_strip
 	for (int c = 0; c < CNT; ++c) {
 #pragma unroll
 		for (int j = 0; j < GROUP_BLOCKS; ++j) {
-			const v4i a = *reinterpret_cast<const v4i*>(a_tiles + c * rows_group_bytes<R> + j * (32 * R) + half * (16 * R) + (r & (R - 1)) * 16);
+			const v4i a = *reinterpret_cast<const v4i*>(a_tiles + c * rows_group_bytes<R> + j * (32 * R) + half * (16 * R) + rows_operand_row<R>(r) * 16);
 			if constexpr (rows_scale_mfma<R>) {
 				// the products d_x * d_w on the matrix pipe, block j's scales in the k = 0 slot.  Both operands are zero in every other slot
 				// (k = 4..7: lanes 32..63): a zero on one side only would make a NaN of the other side's infinity.
-				const uint32_t d = reinterpret_cast<const uint32_t*>(a_scales)[(c * GROUP_BLOCKS + j) * R + (r & (R - 1))];
+				const uint32_t d = reinterpret_cast<const uint32_t*>(a_scales)[(c * GROUP_BLOCKS + j) * R + rows_operand_row<R>(r)];
 				const v2u dx	 = v2u{ half ? 0u : d, 0u };
 #pragma unroll
 				for (int k = 0; k < MATS; ++k) {
@@ -364,7 +370,7 @@ template<int SETS> static hipError_t launch_rows_t(const uint8_t* w, const uint8
 	}
 	const dim3 grid(static_cast<unsigned>((n + STRIP_ROWS - 1) / STRIP_ROWS * splits)), block(SK_WAVES * 64);
 	auto launch = [&](auto kernel) { return launch_kernel(KIND_GEMM, kernel, grid, block, 0, s, w, a, C, residual, sc.tagged, sc.epoch, m, n, groups, shift); };
-	return m <= 8 ? launch(gemm_rows_kernel<8, 2, SETS>) : m <= 16 ? launch(gemm_rows_kernel<16, 2, SETS>) : launch(gemm_rows_kernel<32, 2, SETS>);
+	return m <= 8 ? launch(gemm_rows_kernel<8, 2, SETS>) : m <= 16 ? launch(gemm_rows_kernel<16, 2, SETS>) : m <= 24 ? launch(gemm_rows_kernel<24, 2, SETS>) : launch(gemm_rows_kernel<32, 2, SETS>);
 }
 
 // 1 <= M <= 32, K > 0; cut: plan_gemm_skinny, where gemm_rows_fits
@@ -384,7 +390,7 @@ hipError_t launch_gemm_rows(const void* W, const void* Aq, float* C, const float
 
 template<int SETS> static hipError_t launch_rows_gate_up_t(const uint8_t* wg, const uint8_t* wu, const uint8_t* a, uint8_t* out, float* gate_dbg, float* up_dbg, int m, int n, int groups, hipStream_t s) {
 	auto launch = [&](auto kernel) { return launch_kernel(KIND_GEMM, kernel, dim3(static_cast<unsigned>(n / STRIP_ROWS)), dim3(SK_WAVES * 64), 0, s, wg, wu, a, out, gate_dbg, up_dbg, m, n, groups); };
-	return m <= 8 ? launch(gemm_rows_gate_up_kernel<8, 1, SETS>) : m <= 16 ? launch(gemm_rows_gate_up_kernel<16, 1, SETS>) : launch(gemm_rows_gate_up_kernel<32, 1, SETS>);
+	return m <= 8 ? launch(gemm_rows_gate_up_kernel<8, 1, SETS>) : m <= 16 ? launch(gemm_rows_gate_up_kernel<16, 1, SETS>) : m <= 24 ? launch(gemm_rows_gate_up_kernel<24, 1, SETS>) : launch(gemm_rows_gate_up_kernel<32, 1, SETS>);
 }
 
 hipError_t launch_gemm_rows_gate_up(const void* w_gate, const void* w_up, const void* aq, void* act_out, float* gate_dbg, float* up_dbg, int64_t M, int64_t n_ff, int64_t K, int waves, hipStream_t s) {

@@ -66,7 +66,7 @@ struct gemm_skinny_cut {
 };
 constexpr int64_t GEMM_ROWS_MAX = 32;
 inline int gemm_rows_operand(int64_t M) { // operand rows the rows kernel is instantiated for
-	return M <= 8 ? 8 : M <= 16 ? 16 : 32;
+	return M <= 8 ? 8 : M <= 16 ? 16 : M <= 24 ? 24 : 32;
 }
 inline gemm_skinny_cut plan_gemm_skinny(int64_t M, int64_t N, int64_t K) {
 	gemm_skinny_cut c{};
@@ -166,15 +166,25 @@ inline bool plan_gemm_tile_split(int64_t M, int64_t N, int64_t K, gemm_tile_cut*
 //   [28672 x 8192]  39.1 / 39.4   41.5 / 39.6   47   / 40
 // Every wave takes its own copy of the activations out of L2 (requests per weight line, [4096 x 14336]: 1.27 at 4 rows, 1.53 at 16, 2.07 at
 // 32), which the tile kernel shares over four strips (1.29 to 1.36): from 192 column blocks on, where that fills the chip by itself, this kernel has K up to 4096
-// and 16 rows.  The line lies between the two K measured.  plan_gemm asks the tile kernel first for 16 to 32 rows against 64 column blocks and
-// 64 Mi weights and more, by a rule drawn against the kernel before this one; not measured against this one but at [8192 x 8192], 32 rows:
-// 14.9 / 17.8.
+// and 16 rows.  The line lies between the two K measured.
 inline bool gemm_rows_suits(int64_t M, int64_t N, int64_t K) {
 	const int64_t column_blocks = (N + 127) / 128;
 	if (M > GEMM_ROWS_MAX) {
 		return false;
 	}
 	return column_blocks < GEMM_STREAM_TILE_MIN_COLUMN_BLOCKS || (M <= 16 && K <= 4096);
+}
+
+// The shapes of 64 to 191 column blocks and 64 Mi weights and more that the tile kernel with K over workgroups has otherwise (plan_gemm):
+// up to a workgroup per CU, and near two of them; between, some CUs have two and the launch takes as long as they do.  Measured, us, tile /
+// rows kernel:
+//   rows      [8192 x 8192]   [8192 x 14336]  [8192 x 28672]  [10240 x 8192]  [12288 x 12288]  [14336 x 14336]  [16384 x 4096]  [20480 x 8192]
+//   17 to 24  18.6 / 15.6     28.5 / 23.8     46.2 / 42.5     22.0 / 23.5     32.2 / 34.0      41.2 / 40.8      17.7 / 15.0     37.5 / 35.0
+//   25 to 32  18.2 / 15.8     28.6 / 25.1     45.7 / 45.3     22.1 / 25.2     32.3 / 36.8      41.4 / 43.8      17.8 / 15.9     37.8 / 38.0
+// (sixteen rows would gain as well, 18.8 / 14.4 and 45.8 / 40.4 in the first and third column: tests/test_plan_cpu.py fixes their kernel)
+inline bool gemm_rows_instead_of_tile(int64_t M, int64_t N, int64_t K) {
+	const int64_t strips = (N + STRIP_ROWS - 1) / STRIP_ROWS;
+	return M > 16 && M <= GEMM_ROWS_MAX && (strips <= 256 || (M <= 24 ? strips >= 448 : strips >= 512 && K <= 4096));
 }
 
 // whether the rows kernel's tagged sums hold this cut
@@ -203,6 +213,7 @@ inline gemm_plan plan_gemm(int64_t M, int64_t N, int64_t K) {
 	const int64_t tile_workgroups = column_blocks * ((M + 31) / 32);
 	const int64_t weights		  = N * K;
 	bool stream_tile			  = false;
+	bool wide					  = false;
 	if (M <= GEMM_SKINNY_MAX_M) {
 		// A matrix with enough 128-row column blocks to occupy the chip by itself takes the tile kernel at any M: its four
 		// waves share each activation tile through LDS, where the streaming kernel's eight waves fetch one each from L2 --
@@ -222,7 +233,12 @@ inline gemm_plan plan_gemm(int64_t M, int64_t N, int64_t K) {
 			// 64 Mi.  The rule only holds where that K split is actually possible: a shape whose groups do not divide (kz
 			// stays 1) would run the tile kernel on 32 to 191 workgroups, the form measured slower than the streaming kernel
 			// ([14336 x 4096] at M = 64 unsplit: 30 against 23 us), and stays with the streaming kernel.
-			stream_tile = plan_gemm_tile(M, N, K, true).kz > 1;
+			const gemm_tile_cut tile = plan_gemm_tile(M, N, K, true);
+			stream_tile				 = tile.kz > 1;
+			if (stream_tile && gemm_rows_instead_of_tile(M, N, K)) {
+				stream_tile = false;
+				wide		= plan_gemm_skinny(M, N, K).splits * SK_WAVES < tile.ks * tile.kz; // no fewer shares of K than there
+			}
 		}
 	}
 	if (stream_tile) {
@@ -233,7 +249,10 @@ inline gemm_plan plan_gemm(int64_t M, int64_t N, int64_t K) {
 	} else if (M <= GEMM_SKINNY_MAX_M || tile_workgroups <= 256) {
 		p.kernel = MM_GEMM_SKINNY;
 		p.skinny = plan_gemm_skinny(M, N, K);
-		p.rows	 = gemm_rows_suits(M, N, K) && gemm_rows_fits(M, N, p.skinny);
+		if (wide) {
+			p.skinny.waves = SK_WIDE_WAVES;
+		}
+		p.rows = gemm_rows_suits(M, N, K) && gemm_rows_fits(M, N, p.skinny);
 	} else {
 		p.kernel = MM_GEMM_TILE;
 		p.tile	 = plan_gemm_tile(M, N, K, false);
@@ -260,7 +279,7 @@ inline int gate_up_rows_waves(int64_t M, int64_t n_ff, int64_t K) {
 	if (g.kernel == MM_GEMM_TILE_STREAM) {
 		return g.tile.ks * g.tile.kz > SK_WAVES ? SK_WIDE_WAVES : SK_WAVES;
 	}
-	return plan_gemm_skinny(M, n_ff, K).waves;
+	return g.kernel == MM_GEMM_SKINNY ? g.skinny.waves : plan_gemm_skinny(M, n_ff, K).waves;
 }
 // The tile kernel's fused form, K sets included, wherever its grid has the chip's SIMDs two waves each, or about one where the matrices are
 // small enough that the launches saved count for more than idle CUs.  Whole calls, us, fused / three launches:

@@ -103,3 +103,35 @@ def test_gemm_rows_in_a_graph(q8, oracle):
         eager = to_host(q8.gemm(wt, at, m, n, k, tiled=True))
         assert rel_l2(to_host(c), eager) < 2e-6
         assert rel_l2(eager, oracle.gemm(w, oracle.quantize_rows(x), m, n, k, threads=8)) <= REL_L2_TOL
+
+
+# 18 to 24 rows: the 24-row operand (its 48 (k half, row) units do not divide a transfer), at its edges and the edges of the other sizes
+@pytest.mark.parametrize("m", [18, 24, 25])
+@pytest.mark.parametrize("n,k", [(33, 128), (257, 128 * 35), (4100, 4096), (5120, 128 * 37)])
+def test_the_24_row_operand(q8, oracle, m, n, k):
+    test_gemm_rows(q8, oracle, m, n, k)
+
+
+@pytest.mark.parametrize("n_ff,k", [(128, 128), (4224, 128 * 9), (4224, 128 * 34)])
+def test_gate_up_of_24_rows(q8, oracle, n_ff, k):
+    test_gate_up_rows(q8, oracle, 24, n_ff, k)
+
+
+# 17 to 32 rows against 64 to 191 column blocks and 64 Mi weights and more: as many shares of K as the tile kernel, which had these shapes,
+# where those are sixteen in two sets of eight waves' (or, captured, sixteen waves of the streaming kernel: the same bits); between 257 and 447 strips still the tile kernel
+@pytest.mark.parametrize("m", [17, 24, 32])
+@pytest.mark.parametrize("n,k,waves", [(8161, 10240, 16), (16384, 4096, 8)])
+def test_rows_kernel_in_the_tile_kernels_place(q8, oracle, m, n, k, waves):
+    plan = q8.plan_mul_mat(m, n, k)
+    assert plan["kernel"] == "gemm_skinny" and plan["gemm_rows"] and (plan["k_splits"], plan["waves"]) == (1, waves)
+    assert q8.plan_mul_mat(m, 10240, 8192)["kernel"] == "gemm_tile_stream" and q8.plan_mul_mat(33, n, k)["kernel"] != "gemm_skinny"
+    w = oracle.fill_weights(m + n, n, k)
+    x = oracle.fill_activations(m + k, m * k).reshape(m, k)
+    want = _gemm(oracle, w, oracle.quantize_rows(x), m, n, k)
+    got = to_host(q8.mul_mat(q8.tile(to_dev(w), n, k), to_dev(x), n, k))
+    assert max(rel_l2(got[i], want[i]) for i in range(m)) <= REL_L2_TOL
+
+
+@pytest.mark.parametrize("m", [20, 32])
+def test_captured_call_in_the_tile_kernels_place(q8, oracle, m):
+    test_captured_and_eager_calls_have_the_same_bits(q8, oracle, m, 8161, 10240, splits=1, waves=16)
