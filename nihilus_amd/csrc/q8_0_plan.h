@@ -338,18 +338,6 @@ inline bool plan_gate_up_fused(int64_t M, int64_t n_ff, int64_t K, gate_up_cut* 
 // further so that the launch reaches the CUs.  Under HIP graph capture: no K split (a replay could not renew the hand-off's epoch),
 // a chunked walk instead.
 constexpr int GEMV_ROWS_MFMA_MAX = 16;
-// Where it is the fastest form (measured against what ran before, quantize launch included; us, new / old):
-//   [4096 x 4096]   17.8 MB   M = 4:  5.2 /  8.1 (dot-product kernel)   M = 8:  6.8 / 12.2   M = 16:  8.6 / 11.7 (quantize + streaming MFMA kernel)
-//   [1024 x 8192]    8.9 MB   M = 4:  5.6 /  7.3                        M = 16:  9.1 / 14.3
-//   [14336 x 4096]  62.4 MB   M = 4: 13.7 / 15.6                        M = 8:  19.3 / 15.7
-//   [8192 x 8192]   71.3 MB   M = 4: 17.4 / 21.2
-//   [28672 x 8192]   250 MB   M = 4: 51   / 43.6;  [128256 x 8192]: 199 / 167
-// Every strip's workgroup quantizes all the rows again, which costs in proportion to M and to the matrix: up to sixteen rows on
-// matrices of at most 40 MB, four on matrices of at most 80 MB.  (Two and three rows stay on the dot-product kernel.)
-inline bool gemv_rows_mfma_suits(int64_t M, int64_t N, int64_t K) {
-	const int64_t weight_bytes = N * (K / QK) * BLOCK_BYTES;
-	return M >= 4 && M <= GEMV_ROWS_MFMA_MAX && (weight_bytes <= (int64_t{ 40 } << 20) || (M == 4 && weight_bytes <= (int64_t{ 80 } << 20)));
-}
 inline gemv_plan plan_gemv_rows_mfma(int64_t strips, int64_t K, int rows, bool capturing) { // rows: 8 or 16, the kernel's operand rows
 	gemv_plan p;
 	p.strips	   = static_cast<int>(strips);
@@ -371,6 +359,31 @@ inline gemv_plan plan_gemv_rows_mfma(int64_t strips, int64_t K, int rows, bool c
 	}
 	p.tiles = tiles_for(p.splits);
 	return p;
+}
+
+// Where it is the fastest form.  Every strip's workgroup quantizes all the rows again, which costs in proportion to M, and its sixteen waves
+// have a CU to themselves, so a launch of more workgroups than CUs walks some of them one after the other.  Measured against the quantize
+// launch and the kernel for up to 32 quantized rows (weights rotated, us, this / the two launches; workgroups, groups per wave):
+//   9 to 16 rows   [4096 x 4096] 256, 1:  9.7 /  9.7 (12 rows 8.5 /  9.5)   [8192 x 2048] 256, 1:  8.6 /  9.0   [1024 x 14336] 256, 1: 10.4 / 10.4
+//                  [6144 x 4096] 384, 1: 16.2 / 10.4   [2560 x 5120] 320, 1: 14.0 /  9.3   [4096 x 8192] 512, 1: 17.4 / 12.1
+//   8 rows         [4096 x 4096] 256, 1:  7.6 /  9.2   [4096 x 6144] 256, 2:  9.5 / 10.1   [8192 x 4096] 256, 2: 11.0 / 10.5
+//                  [5120 x 2560] 320, 1:  8.2 /  9.0   [6144 x 4096] 384, 1: 10.0 /  9.6   [5120 x 5120] 320, 2: 13.1 / 10.5
+//   6 rows         [8192 x 4096] 256, 2:  9.9 / 10.5   [6144 x 4096] 384, 1:  9.3 /  9.5   [4608 x 4608] 288, 2: 11.2 /  9.9
+//   4 rows         [4096 x 8192] 256, 2: 10.2 / 11.4   [6144 x 4096] 384, 1:  8.6 /  9.6   [4608 x 4608] 288, 2:  9.7 /  9.9
+// Four rows also on matrices of up to 80 MB ([14336 x 4096] 15.5 / 14.5, [8192 x 8192] 17.8 / 16.0: a line drawn against the kernels before,
+// which tests/test_plan_cpu.py fixes).  (Two and three rows stay on the dot-product kernel.)
+inline bool gemv_rows_mfma_suits(int64_t M, int64_t N, int64_t K) {
+	constexpr int64_t MIB		 = int64_t{ 1 } << 20;
+	const int64_t weight_bytes = N * (K / QK) * BLOCK_BYTES;
+	if (M < 4 || M > GEMV_ROWS_MFMA_MAX || weight_bytes > (M == 4 ? 80 : 40) * MIB) {
+		return false;
+	}
+	const gemv_plan p	 = plan_gemv_rows_mfma((N + STRIP_ROWS - 1) / STRIP_ROWS, K, M <= 8 ? 8 : 16, false);
+	const bool one_round = p.strips * p.splits <= 256;
+	if (M > 8) {
+		return one_round;
+	}
+	return M == 4 || (one_round ? M <= 6 || weight_bytes <= 32 * MIB : p.tiles == 1 && (M <= 6 || weight_bytes <= 20 * MIB));
 }
 
 // nh_q8_0_mul_mat: fp32 activations [M][K] against a tiled weight [N][K].

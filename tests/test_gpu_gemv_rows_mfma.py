@@ -88,3 +88,19 @@ def test_captured_stream_takes_the_unsplit_walk(q8, oracle, m):
         eager = to_host(q8.mul_mat(wt, x_d, n, k))  # the split form, with a fresh epoch, between the replays
         assert rel_l2(got, eager) < 2e-6, rep  # same arithmetic, another cut of K
         assert rel_l2(got, _want(oracle, w, x, n, k)) <= REL_L2_TOL, rep
+
+
+# either side of the line to the quantize launch and the kernel for up to 32 quantized rows: a workgroup per CU or more, one or two groups per wave
+@pytest.mark.parametrize("m,n,k,fused", [(9, 4096, 4096, True), (9, 4128, 4096, False), (16, 8192, 2048, True), (16, 6144, 4096, False), (8, 4096, 6144, True), (8, 8192, 4096, False), (6, 8192, 4096, True),
+                                         (6, 5120, 5120, False), (8, 5120, 2560, True), (5, 6144, 4096, True), (7, 6144, 4096, False), (4, 5120, 5120, True)])
+def test_the_line_to_the_quantize_launch(q8, oracle, m, n, k, fused):
+    plan = q8.plan_mul_mat(m, n, k)
+    assert (plan["kernel"] == "gemv_rows_mfma") == fused and plan["quantize_launch"] != fused
+    rng = np.random.default_rng(m + n)
+    w = random_blocks(rng, n, k, 0.02)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    res = rng.standard_normal((m, n)).astype(np.float32)
+    wt = q8.tile(to_dev(w), n, k)
+    y, want = to_host(q8.mul_mat(wt, to_dev(x), n, k)), _want(oracle, w, x, n, k)
+    assert max(rel_l2(y[i], want[i]) for i in range(m)) <= REL_L2_TOL
+    assert np.array_equal(to_host(q8.mul_mat(wt, to_dev(x), n, k, residual=to_dev(res))), y + res)
