@@ -163,15 +163,16 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_kernel(const uint8_t* __res
 //     in the int8 MFMA's own accumulator layout: no conversion, broadcast or cross-lane move of a scale, ever;
 //   * only the operand that is shared goes through LDS.  A workgroup is four waves; wave w owns weight strip
 //     4*blockIdx.x + w and loads its tiles straight from global memory into registers (one coalesced 16-byte-per-lane
-//     load per tile, already an MFMA operand, a whole 128-quant group ahead of use); all four waves share the same
+//     load per tile, already an MFMA operand, into the registers of the tile it follows as soon as the last MFMA on that one is
+//     issued: half a 128-quant group and more ahead of use, in 16 registers and not 32); all four waves share the same
 //     TM activation strips, copied global -> LDS one group ahead (double-buffered, one barrier per group, the copy
-//     spread over the four waves) and read back as conflict-free 16-byte-per-lane operand images plus one half-word
-//     read per scale;
+//     spread over the four waves) and read back as conflict-free 16-byte-per-lane operand images plus one 8-byte read of a
+//     group's four scales per strip;
 //   * every global address is a wave-uniform base in scalar registers plus a 32-bit lane offset (the addressing mode of
 //     global_load with a scalar base): no 64-bit address arithmetic on the VALU, which is the pipe the fold saturates,
 //     and ~10 fewer registers than per-lane pointers (the difference between spilling and not at two activation strips);
 //   * latency is hidden by occupancy, not by a software pipeline: one result-register set per tile keeps the kernel
-//     at <= 128 VGPRs, four workgroups per CU, four waves per SIMD.  (A two-result-set, software-pipelined variant
+//     at <= 128 VGPRs (112), four workgroups per CU, four waves per SIMD.  (A two-result-set, software-pipelined variant
 //     at two waves per SIMD measured 8 % slower: with so few waves the SIMD falls back to the lone-wave issue rate
 //     whenever one of them waits.)
 // a 64-bit offset that the compiler may keep in scalar registers (it is the same for every lane of the wave)
@@ -214,9 +215,8 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 	float* __restrict__ partials, unsigned* __restrict__ counters, const uint8_t* __restrict__ W2, uint8_t* __restrict__ act_out, float* __restrict__ C2, int passes = 1, bool tree = false) {
 	static_assert(!SPLIT || (KS > 1 && !DUMP), "K over several workgroups continues the K sets' sum");
 	static_assert(!GATE_UP || (!DUMP && !SPLIT), "the fused gate/up form leaves a workgroup's tile quantized");
-	constexpr int DATA_BYTES  = TM * MACRO_BYTES;
-	constexpr int STAGE_BYTES = DATA_BYTES + 16;
-	constexpr int SET_BYTES	   = 2 * STAGE_BYTES + 256; // + 256: where waves that copy no scale table put theirs
+	constexpr int STAGE_BYTES = TM * MACRO_BYTES; // the activation strips' macro-tiles of a group, as in memory
+	constexpr int SET_BYTES	  = 2 * STAGE_BYTES + 256; // + 256: where waves that copy no scale table put theirs
 	constexpr int PARK_BYTES   = KS > 1 ? KS * 4 * (KS - 1) * (16 * TM / KS) * 64 * 4 : 0; // the final sum over the K sets, below
 	// GATE_UP epilogue: two up tiles per activation strip as fp32, then per gate wave TM tile images and TM x 32 scales
 	constexpr int XCH_BYTES	   = GATE_UP ? 2 * TM * 16 * 64 * 4 : 0;
@@ -234,30 +234,41 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 	const int wave	   = wave_all & 3; // which of the workgroup's four weight strips
 	const int kr	   = wave_all >> 2; // which K range
 	uint8_t* lds	   = lds_raw + kr * SET_BYTES;
-	// the host launches KS > 1, and K over gridDim.z workgroups, only when they divide
-	int g_len = SPLIT ? groups / (KS * static_cast<int>(gridDim.z)) : groups / KS;
-	// which share of K: with K over workgroups in the shapes that the streaming kernel can take too, the one that makes the sums below the
-	// tree that kernel adds its eight or sixteen waves' shares in (0 4 2 6 / 1 5 3 7, then the same of 8 to 15)
+	// Which share of K a set has, of KS * gridDim.z (or, in PASSES, KS in each pass).  With K over workgroups in the shapes that the streaming kernel
+	// can take too, the one that makes the sums below the tree that kernel adds its eight or sixteen waves' shares in (0 4 2 6 / 1 5 3 7,
+	// then the same of 8 to 15), and its cut of K.  The shares differ by a group where K does not divide: every set of a workgroup walks as
+	// many groups as the longest (they meet at a barrier behind each), the last of a shorter one with zero scales.
 	constexpr bool TREE = SPLIT && !STREAM;
 	static_assert(!TREE || KS == 4);
-	const int z		  = SPLIT ? static_cast<int>(blockIdx.z) : 0;
-	const int share	  = TREE ? 8 * (z >> 1) + (z & 1) + 4 * (kr & 1) + 2 * (kr >> 1) : z * KS + kr;
-	const int g_base  = PASSES ? 0 : share * g_len;
-	// passes: passes * KS shares of K, cut as wave_k_range does; the sets take them in the order that makes the sums below the mat-mat's.
-	// This set's first group and number of groups in this pass, and its first group in the next one; g_len: the most groups any set has.
-	int g0 = 0, live = 0, after = 0;
+	const int z	= SPLIT ? static_cast<int>(blockIdx.z) : 0;
+	const int zs = SPLIT ? static_cast<int>(gridDim.z) : 1;
+	// this set's first group and number of groups (in this pass), and its first group in the next pass; g_len: the most groups any set has
+	int g0 = 0, live = groups, g_len = groups, after = 0;
 	auto begin_pass = [&](int pass) {
-		const auto share_of = [&](int p) { return tree ? p + 4 * (kr & 1) + 2 * (kr >> 1) : p * KS + kr; };
+		const int shares	= KS * (PASSES ? passes : zs);
+		const auto share_of = [&](int p) {
+			if (TREE) {
+				return 8 * (z >> 1) + (z & 1) + 4 * (kr & 1) + 2 * (kr >> 1);
+			}
+			return PASSES && tree ? p + 4 * (kr & 1) + 2 * (kr >> 1) : (PASSES ? p : z) * KS + kr;
+		};
+		const auto range = [&](int share, int& from, int& to) {
+			if (TREE) {
+				wave_k_range(groups, shares >> 4, share >> 3, 8, share & 7, from, to);
+			} else {
+				wave_k_range(groups, 0, 0, shares, share, from, to);
+			}
+		};
 		int g1, unused;
-		wave_k_range(groups, 0, 0, passes * KS, share_of(pass), g0, g1);
+		range(share_of(pass), g0, g1);
 		live  = g1 - g0;
-		g_len = (groups + passes * KS - 1) / (passes * KS);
+		g_len = (groups + shares - 1) / shares;
 		after = g1 - 1;
-		if (pass + 1 < passes) {
-			wave_k_range(groups, 0, 0, passes * KS, share_of(pass + 1), after, unused);
+		if (PASSES && pass + 1 < passes) {
+			range(share_of(pass + 1), after, unused);
 		}
 	};
-	if constexpr (PASSES) {
+	if constexpr (KS > 1) {
 		begin_pass(0);
 	}
 	const int half	   = lane >> 5;
@@ -266,12 +277,9 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 	const int ms0	   = blockIdx.y * TM;
 	const int ns	   = GATE_UP ? blockIdx.x * 2 + (wave & 1) : blockIdx.x * 4 + wave;
 	const uint8_t* Wm  = (GATE_UP && wave >= 2) ? W2 : W; // wave-uniform
-	if ((tid & 255) < 8) {
-		*reinterpret_cast<uint32_t*>(lds + ((tid & 255) >> 2) * STAGE_BYTES + DATA_BYTES + 4 * (tid & 3)) = 0u;
-	}
 	// every address below is a wave-uniform part (scalar registers, advanced by scalar adds) plus one of three lane constants
-	const uint32_t lane16 = 16u * lane;
-	const int64_t w_off	  = uniform_i64(macro_offset(min(ns, n_strips - 1), g_base, groups));
+	uint32_t lane16 = 16u * lane;
+	const int64_t w_off	  = uniform_i64(macro_offset(min(ns, n_strips - 1), 0, groups));
 	struct w_regs {
 		v4i q[GROUP_BLOCKS];
 		v2u d;
@@ -283,12 +291,12 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 #pragma unroll
 	for (int j = 0; j < TM; ++j) {
 		const int u = TM * wave + j;
-		a_off[j]	= uniform_i64(macro_offset(min(ms0 + u / 4, m_strips - 1), g_base, groups) + (u % 4) * TILE_BYTES);
+		a_off[j]	= uniform_i64(macro_offset(min(ms0 + u / 4, m_strips - 1), 0, groups) + (u % 4) * TILE_BYTES);
 		a_dst[j]	= (u / 4) * MACRO_BYTES + (u % 4) * TILE_BYTES; // + 16 * lane at the store
 	}
 	// every wave copies a dword per lane of a scale table (waves >= TM: strip TM-1's again, stored nowhere), so that all waves
 	// issue the same loads
-	const int64_t sc_off  = uniform_i64(macro_offset(min(ms0 + min(wave, TM - 1), m_strips - 1), g_base, groups) + MACRO_D_OFFSET);
+	const int64_t sc_off  = uniform_i64(macro_offset(min(ms0 + min(wave, TM - 1), m_strips - 1), 0, groups) + MACRO_D_OFFSET);
 	const uint32_t sc_dst = wave < TM ? wave * MACRO_BYTES + MACRO_D_OFFSET : 2 * STAGE_BYTES; // + 4 * lane at the store
 	const uint32_t sc_stage = wave < TM ? STAGE_BYTES : 0; // the spare area is not staged
 	struct a_regs {
@@ -297,53 +305,60 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 	};
 	auto fetch_a = [&](int g, a_regs& r) {
 		const int64_t adv = static_cast<int64_t>(g0 + g) * MACRO_BYTES;
-		uint32_t l16 = lane16;
-		asm volatile("" : "+v"(l16));
-		const uint32_t l4 = l16 >> 2;
+		asm volatile("" : "+v"(lane16));
+		const uint32_t l4 = lane16 >> 2;
 #pragma unroll
 		for (int j = 0; j < TM; ++j) {
-			r.q[j] = load_sv<v4i, false>(scalar_base(A, a_off[j] + adv), l16);
+			r.q[j] = load_sv<v4i, false>(scalar_base(A, a_off[j] + adv), lane16);
 		}
 		r.d = load_sv<uint32_t, false>(scalar_base(A, sc_off + adv), l4);
 	};
 	auto stash_a = [&](int stage, const a_regs& r) {
 		uint8_t* p	 = lds + stage * STAGE_BYTES;
-		uint32_t l16 = lane16;
-		asm volatile("" : "+v"(l16)); // wave-uniform offsets stay in scalar registers, added here, instead of one more lane constant each
+		asm volatile("" : "+v"(lane16)); // wave-uniform offsets stay in scalar registers, added here, instead of one more lane constant each
 #pragma unroll
 		for (int j = 0; j < TM; ++j) {
-			*reinterpret_cast<v4i*>(p + a_dst[j] + l16) = r.q[j];
+			*reinterpret_cast<v4i*>(p + a_dst[j] + lane16) = r.q[j];
 		}
-		*reinterpret_cast<uint32_t*>(lds + stage * sc_stage + sc_dst + (l16 >> 2)) = r.d;
+		*reinterpret_cast<uint32_t*>(lds + stage * sc_stage + sc_dst + (lane16 >> 2)) = r.d;
 	};
 	auto fetch_w = [&](int g, w_regs& r) {
 		const int64_t at = w_off + static_cast<int64_t>(g0 + g) * MACRO_BYTES;
 		const gptr_u8 p	 = scalar_base(Wm, at);
-		uint32_t l16 = lane16;
-		asm volatile("" : "+v"(l16));
-		const uint32_t l8 = (l16 & 0x1F0u) >> 1; // the widening of a lane offset has to stay beside its loads for scalar base + 32-bit lane offset to be picked as the addressing mode
+		asm volatile("" : "+v"(lane16));
+		const uint32_t l8 = (lane16 & 0x1F0u) >> 1; // the widening of a lane offset has to stay beside its loads for scalar base + 32-bit lane offset to be picked as the addressing mode
+		r.d = load_sv<v2u, STREAM>(scalar_base(Wm, at + MACRO_D_OFFSET), l8);
+		__builtin_amdgcn_sched_barrier(0); // in the trips' order: their waits are counts of what was requested behind
 #pragma unroll
 		for (int k = 0; k < GROUP_BLOCKS; ++k) {
-			r.q[k] = load_sv<v4i, STREAM>(p + k * TILE_BYTES, l16);
+			r.q[k] = load_sv<v4i, STREAM>(p + k * TILE_BYTES, lane16);
 		}
-		r.d = load_sv<v2u, STREAM>(scalar_base(Wm, at + MACRO_D_OFFSET), l8);
 	};
-	// load number p of a group's set (PIECES of them: TM activation tiles, their scale dword, four weight tiles, their scales);
+	// load number p of a group's set (PIECES of them: TM activation tiles, their scale dword, the weights' scales, four weight tiles);
 	// the same loads as fetch_a and fetch_w, which the prologue issues in one go
 	constexpr int PIECES = TM + 2 + GROUP_BLOCKS;
+	constexpr int UNITS	 = GROUP_BLOCKS * TM; // of a trip: (block t, activation strip i) in the order u = TM * t + i
+	// IN_PLACE: a weight tile goes to the registers of the one it replaces.  In PASSES there are two sets of registers instead, taken in turn:
+	// with sets of half the trips, [2 x 14336 x 4096] at 117 rows takes 57.2 us with two and 60.1 in place, on the slower of the cards measured.
+	constexpr bool IN_PLACE = !PASSES;
+	// the unit in front of whose arithmetic a piece is requested (UNITS: behind the last one): spread over the trip, in place not before the last
+	// unit that multiplies the tile it replaces (every piece as early as that allows instead: at 512 rows 0.2 % faster, at 117 0.3 % slower)
+	constexpr auto piece_unit = [](int p) {
+		const int spread = (UNITS * (p + 1) + PIECES - 1) / PIECES - 1, free = !IN_PLACE || p < TM + 2 ? 0 : TM * (p - TM - 2 + 1);
+		return spread > free ? spread : free;
+	};
 	auto fetch_piece = [&](int p, int in_pass, a_regs& ra, w_regs& rw) {
-		const int g	 = g0 + in_pass;
-		uint32_t l16 = lane16;
-		asm volatile("" : "+v"(l16));
+		const int g = g0 + in_pass;
+		asm volatile("" : "+v"(lane16)); // in place: a copy for every load was one VALU instruction each
 		if (p < TM) {
-			ra.q[p] = load_sv<v4i, false>(scalar_base(A, a_off[p] + static_cast<int64_t>(g) * MACRO_BYTES), l16);
+			ra.q[p] = load_sv<v4i, false>(scalar_base(A, a_off[p] + static_cast<int64_t>(g) * MACRO_BYTES), lane16);
 		} else if (p == TM) {
-			ra.d = load_sv<uint32_t, false>(scalar_base(A, sc_off + static_cast<int64_t>(g) * MACRO_BYTES), l16 >> 2);
-		} else if (p < TM + 1 + GROUP_BLOCKS) {
-			const int k = p - TM - 1;
-			rw.q[k] = load_sv<v4i, STREAM>(scalar_base(Wm, w_off + static_cast<int64_t>(g) * MACRO_BYTES + k * TILE_BYTES), l16);
+			ra.d = load_sv<uint32_t, false>(scalar_base(A, sc_off + static_cast<int64_t>(g) * MACRO_BYTES), lane16 >> 2);
+		} else if (p == TM + 1) { // in front of the tiles: the trip's first unit needs it, and waits for what was requested before it
+			rw.d = load_sv<v2u, STREAM>(scalar_base(Wm, w_off + static_cast<int64_t>(g) * MACRO_BYTES + MACRO_D_OFFSET), (lane16 & 0x1F0u) >> 1);
 		} else {
-			rw.d = load_sv<v2u, STREAM>(scalar_base(Wm, w_off + static_cast<int64_t>(g) * MACRO_BYTES + MACRO_D_OFFSET), (l16 & 0x1F0u) >> 1);
+			const int k = p - TM - 2;
+			rw.q[k] = load_sv<v4i, STREAM>(scalar_base(Wm, w_off + static_cast<int64_t>(g) * MACRO_BYTES + k * TILE_BYTES), lane16);
 		}
 	};
 	v16f acc[TM];
@@ -351,10 +366,9 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 	for (int i = 0; i < TM; ++i) {
 		acc[i] = v16f{ 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0 };
 	}
-	const int a_sc_rel = half ? DATA_BYTES : MACRO_D_OFFSET + 8 * (lane & 31);
-	int last		   = PASSES ? live - 1 : g_len - 1;
+	int last = live - 1;
 
-	w_regs wa, wb;
+	w_regs wa, wb; // this trip's weights and, unless IN_PLACE, the next one's
 	a_regs pre;
 	fetch_a(0, pre);
 	fetch_w(0, wa);
@@ -372,39 +386,37 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 		// (with another pass to come: its first group, on its way while this pass is summed)
 		const int gn = PASSES ? (g < last ? g + 1 : after - g0) : min(g + 1, last);
 		// (past the end of a set's share, where another set has one group more: zero scales on both sides add nothing)
-		const bool zero = PASSES ? half || g >= live : half;
-		if (zero) {
-			cur.d = v2u{ 0u, 0u };
-		}
-		const int sc_rel = PASSES && zero ? DATA_BYTES : a_sc_rel;
+		const bool zero = KS > 1 ? half || g >= live : half;
+		const v2u wd = zero ? v2u{ 0u, 0u } : cur.d;
 		const uint8_t* stage = lds + (g & 1) * STAGE_BYTES;
+		asm volatile("" : "+v"(lane16));
+		const uint8_t* a_at = stage + lane16;
+		// the rows' scales of the group's four blocks, one 8-byte read per strip and trip (a half-word read per unit was eight)
+		v2u a_sc[TM];
+#pragma unroll
+		for (int i = 0; i < TM; ++i) {
+			const v2u d = *reinterpret_cast<const v2u*>(stage + i * MACRO_BYTES + MACRO_D_OFFSET + ((lane16 >> 1) & 0xF8u));
+			a_sc[i]		= zero ? v2u{ 0u, 0u } : d;
+		}
 		// the operand of unit u + 1 is read from LDS before unit u's arithmetic starts: one exposed LDS latency per trip, not eight
-		constexpr int UNITS = GROUP_BLOCKS * TM;
-		auto read_a = [&](int u, v4i& a, uint32_t& sc) {
-			const int t = u / TM, i = u % TM;
-			a  = *reinterpret_cast<const v4i*>(stage + i * MACRO_BYTES + t * TILE_BYTES + 16 * lane);
-			sc = *reinterpret_cast<const uint16_t*>(stage + (zero ? 0 : i * MACRO_BYTES) + sc_rel + 2 * t);
-		};
-		v4i a_cur;
-		uint32_t s_cur;
-		read_a(0, a_cur, s_cur);
+		auto read_a = [&](int u) { return *reinterpret_cast<const v4i*>(a_at + (u % TM) * MACRO_BYTES + (u / TM) * TILE_BYTES); };
+		v4i a_cur = read_a(0);
 #pragma unroll
 		for (int u = 0; u < UNITS; ++u) {
 			const int t = u / TM, i = u % TM;
 			v4i a_nxt		= a_cur;
-			uint32_t s_nxt	= s_cur;
 			if (u + 1 < UNITS) {
-				read_a(u + 1, a_nxt, s_nxt);
+				a_nxt = read_a(u + 1);
 			}
 			__builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-			for (int pc = u * PIECES / UNITS; pc < (u + 1) * PIECES / UNITS; ++pc) {
-				fetch_piece(pc, gn, pre, nxt);
+			for (int pc = 0; pc < PIECES; ++pc) {
+				if (piece_unit(pc) == u) {
+					fetch_piece(pc, gn, pre, nxt);
+				}
 			}
 			__builtin_amdgcn_sched_barrier(0);
-			const uint32_t wd = (t < 2) ? cur.d.x : cur.d.y;
-			const v2u w_sc	  = v2u{ (t & 1) ? (wd >> 16) : (wd & 0xFFFFu), 0u };
-			const v2u a_sc	  = v2u{ s_cur, 0u };
+			const v2u w_slot  = scale_slot(wd, t), a_slot = scale_slot(a_sc[i], t);
 			const v16i zi	  = { 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0 };
 			const v16f zf	  = { 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0 };
 			const v16i sv	  = __builtin_amdgcn_mfma_i32_32x32x32_i8(a_cur, cur.q[t], zi, 0, 0, 0);
@@ -414,11 +426,11 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 				for (int e = 0; e < 16; ++e) {
 					const int m = (ms0 + i) * 32 + 8 * (e >> 2) + 4 * half + (e & 3);
 					if (m < M && n < N) {
-						sums[(static_cast<int64_t>(m) * N + n) * (groups * GROUP_BLOCKS) + (g_base + g) * GROUP_BLOCKS + t] = sv[e];
+						sums[(static_cast<int64_t>(m) * N + n) * (groups * GROUP_BLOCKS) + g * GROUP_BLOCKS + t] = sv[e];
 					}
 				}
 			} else {
-				const v16f pv = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(v4h, a_sc), __builtin_bit_cast(v4h, w_sc), zf, 0, 0, 0);
+				const v16f pv = __builtin_amdgcn_mfma_f32_32x32x8f16(__builtin_bit_cast(v4h, a_slot), __builtin_bit_cast(v4h, w_slot), zf, 0, 0, 0);
 #pragma unroll
 				for (int e = 0; e < 16; ++e) {
 					acc[i][e] = fmaf(static_cast<float>(sv[e]), pv[e], acc[i][e]);
@@ -427,17 +439,23 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 			}
 			__builtin_amdgcn_sched_barrier(0);
 			a_cur = a_nxt;
-			s_cur = s_nxt;
 		}
+#pragma unroll
+		for (int pc = 0; pc < PIECES; ++pc) {
+			if (piece_unit(pc) == UNITS) {
+				fetch_piece(pc, gn, pre, nxt);
+			}
+		}
+		__builtin_amdgcn_sched_barrier(0);
 		stash_a((g + 1) & 1, pre);
 		__syncthreads();
 	};
 	constexpr int PER = 16 / KS; // values of a lane's 16 per strip that a K set finishes: registers PER * kr .. PER * kr + PER - 1
 	float mine[TM * PER]; // this wave's share of the workgroup's tile (SPLIT: of its part of K)
 	for (int pass = 0;; ++pass) {
-		for (int g = 0; g < g_len; g += 2) {
-			trip(g, wa, wb);
-			if (g + 1 < g_len) {
+		for (int g = 0; g < g_len; g += IN_PLACE ? 1 : 2) {
+			trip(g, wa, IN_PLACE ? wa : wb);
+			if (!IN_PLACE && g + 1 < g_len) {
 				trip(g + 1, wb, wa);
 			}
 		}
@@ -601,10 +619,7 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 					for (int i = 0; i < TM; ++i) {
 						acc[i] = v16f{ 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0 };
 					}
-					if ((tid & 255) < 8) {
-						*reinterpret_cast<uint32_t*>(lds + ((tid & 255) >> 2) * STAGE_BYTES + DATA_BYTES + 4 * (tid & 3)) = 0u; // the zero scales again
-					}
-					if (g_len & 1) {
+					if (!IN_PLACE && (g_len & 1)) {
 						wa = wb;
 					}
 					stash_a(0, pre);

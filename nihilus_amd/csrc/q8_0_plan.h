@@ -45,8 +45,12 @@ inline gemm_tile_cut plan_gemm_tile(int64_t M, int64_t N, int64_t K, bool stream
 	c.tm	 = m_strips >= 2 ? 2 : 1;
 	c.grid_x = static_cast<unsigned>((n_strips + 3) / 4);
 	c.grid_y = static_cast<unsigned>((m_strips + c.tm - 1) / c.tm);
+	// K sets until every SIMD has four waves, while each keeps four groups.  K need not divide: the sets' shares differ by a group then.  Measured,
+	// us, with as many sets as divide / this: [4096 x 4224] at 350 / 512 rows 43.5 / 25.0 and 43.7 / 28.2, [4096 x 11136] 107.7 / 54.9 and 107.9 /
+	// 64.5, [4096 x 4352] (two sets / four) at 512 28.9 / 28.3, [2560 x 2688] at 512 28.5 / 18.4, [28672 x 3200] at 60 / 30 rows 36.7 / 26.9
+	// and 27.9 / 21.7
 	c.ks	 = 1;
-	while (c.ks < 4 && static_cast<int64_t>(c.grid_x) * c.grid_y * 4 * c.ks * 2 <= 4096 && groups % (c.ks * 2) == 0 && groups / (c.ks * 2) >= 4) {
+	while (c.ks < 4 && static_cast<int64_t>(c.grid_x) * c.grid_y * 4 * c.ks * 2 <= 4096 && groups / (c.ks * 2) >= 4) {
 		c.ks *= 2;
 	}
 	c.kz = 1;
@@ -131,6 +135,10 @@ inline gemm_skinny_cut plan_gemm_skinny(int64_t M, int64_t N, int64_t K) {
 // 28.5 / 34.3, [4096 x 14336] at 117 rows (seven groups, K over four) 28.5 / 31.1, [5120 x 5120] at 160 rows (five) 21.4 / 22.3; with four
 // groups [4096 x 4096] at 200 rows 18.4 / 18.0, [2048 x 8192] at 256 rows 19.8 / 18.1; with two [4096 x 4096] at 117 rows 14.9 / 12.5.
 //
+// K need not divide, if the longest share is at most a tenth over the average: [4096 x 11136] at 200 rows 47.5 / 36.1 (the streaming kernel / this),
+// [7936 x 28032] at 233 rows 271 / 172, [4992 x 13184] at 121 rows 55.5 / 39.6, [6784 x 6784] at 125 rows (seven groups where 6.6 would do)
+// 32.6 / 29.1; but [5376 x 5376] at 144 rows (six for 5.25) 25.6 / 28.4.
+//
 // A captured call, and one that finds the hand-off scratch in use on another stream, runs on the streaming kernel with as many shares of K in
 // one workgroup of eight or sixteen waves (`twin`), which add to the same bits and need no scratch: hence two or four workgroups along
 // K, and as many as give no fewer shares than the streaming kernel's own cut.
@@ -141,7 +149,8 @@ inline bool plan_gemm_tile_split(int64_t M, int64_t N, int64_t K, gemm_tile_cut*
 	const int groups		  = static_cast<int>(K / GROUP_K);
 	const int64_t wgs		  = static_cast<int64_t>(c.grid_x) * c.grid_y;
 	const auto can_double	  = [&] {
-		return c.ks == 4 && c.kz < GEMM_TILE_SPLIT_MAX && groups % (c.ks * c.kz * 2) == 0 && groups / (c.ks * c.kz * 2) >= GEMM_TILE_SPLIT_MIN_GROUPS &&
+		const int shares = c.ks * c.kz * 2, longest = (groups + shares - 1) / shares;
+		return c.ks == 4 && c.kz < GEMM_TILE_SPLIT_MAX && 10 * longest * shares <= 11 * groups && groups / (c.ks * c.kz * 2) >= GEMM_TILE_SPLIT_MIN_GROUPS &&
 			wgs * c.kz * 2 * c.tm * 4096 <= GEMM_SPLIT_SCRATCH_FLOATS && wgs <= GEMM_SPLIT_MAX_UNITS;
 	};
 	while (can_double() && (wgs * c.kz * 2 <= 256 || c.ks * c.kz < own.splits * own.waves)) {
@@ -300,14 +309,18 @@ struct gate_up_cut {
 	int passes; // passes * ks shares of K, ks at a time
 	bool tree; // eight shares in two passes, added as the streaming kernel adds them
 };
-constexpr int64_t GATE_UP_MIN_WAVES = 2048, GATE_UP_MIN_WAVES_SMALL = 1100, GATE_UP_SMALL_WEIGHTS = 48ll << 20, GATE_UP_SHORT_K = 1024;
+constexpr int64_t GATE_UP_MIN_WAVES = 2048, GATE_UP_MIN_WAVES_SMALL = 1100, GATE_UP_SMALL_WEIGHTS = 48ll << 20, GATE_UP_SHORT_K = 1024, GATE_UP_UNEVEN_MIN_GROUPS = 12;
 inline bool plan_gate_up_fused(int64_t M, int64_t n_ff, int64_t K, gate_up_cut* cut = nullptr) {
 	if (M <= 0 || n_ff <= 0 || K <= 0 || n_ff % GROUP_K != 0 || K % GROUP_K != 0) {
 		return false;
 	}
 	gate_up_cut c{ {}, 1, false };
 	c.tile			  = plan_gemm_tile(M, 2 * n_ff, K, false); // grid_x = n_ff / 64 workgroups of two gate and two up strips
+	const int groups  = static_cast<int>(K / GROUP_K);
 	const gemm_plan g = plan_gemm(M, n_ff, K);
+	while (g.kernel == MM_GEMM_TILE && c.tile.ks > 1 && groups % c.tile.ks != 0 && groups / c.tile.ks < GATE_UP_UNEVEN_MIN_GROUPS && int64_t{ 2 } * c.tile.ks * c.tile.grid_x * c.tile.grid_y >= 1024) {
+		c.tile.ks /= 2; // K does not divide, the sets' shares are short, and half as many sets already have a wave on every SIMD ([2 x 6016 x 2176] at 231 rows, one set / two: 32.5 / 35.3 us)
+	}
 	const int64_t waves = int64_t{ 4 } * c.tile.ks * c.tile.grid_x * c.tile.grid_y;
 	if (c.tile.tm == 1 && c.tile.ks > 2) {
 		return false; // no such form: K above 32768, which the rows kernel would have to hand over
@@ -318,11 +331,23 @@ inline bool plan_gate_up_fused(int64_t M, int64_t n_ff, int64_t K, gate_up_cut* 
 		return false;
 	} else {
 		const bool tree	 = g.kernel == MM_GEMM_SKINNY || (g.kernel == MM_GEMM_TILE && g.tile.kz > 1);
-		const int shares = g.kernel == MM_GEMM_SKINNY ? g.skinny.splits * g.skinny.waves : g.tile.ks * g.tile.kz;
+		int shares		 = g.kernel == MM_GEMM_SKINNY ? g.skinny.splits * g.skinny.waves : g.tile.ks * g.tile.kz;
+		if (g.kernel == MM_GEMM_TILE && g.tile.kz == 1) {
+			while (groups % shares != 0) { // K does not divide over the mat-mats' sets: a second pass for the last bits only ([2 x 11008 x 4352] at 100 rows 49.4 -> 55.1 us)
+				shares /= 2;
+			}
+			shares = shares > c.tile.ks ? shares : c.tile.ks;
+		}
 		if (K > GATE_UP_SHORT_K) {
 			c.passes = shares / c.tile.ks;
 			c.tree	 = tree && c.tile.ks == 4;
 			if (c.passes > 1 && (c.tile.ks == 1 || c.passes > (c.tile.ks == 4 ? 2 : 4))) {
+				return false;
+			}
+			// Passes of uneven sets: two, with the longest share at most a quarter over the average.  Fused / three launches, us: [2 x 11008 x 4224] at
+			// 48 rows (five groups for 4.1) 33.3 / 42.2, [2 x 6784 x 2816] at 50 rows (three for 2.75) 23.1 / 26.1, but [2 x 6912 x 3200] at 42 rows (four
+			// for 3.1) 27.5 / 26.3, [2 x 6400 x 2304] at 58 rows (three for 2.25) 23.3 / 21.9, and in four passes [2 x 5504 x 2176] at 140 rows 40.7 / 36.8.
+			if (c.passes > 1 && groups % c.tile.ks != 0 && (c.passes > 2 || 4 * ((groups + shares - 1) / shares * shares) > 5 * groups)) {
 				return false;
 			}
 		}
