@@ -310,7 +310,7 @@ struct gate_up_cut {
 	bool tree; // eight shares in two passes, added as the streaming kernel adds them
 };
 constexpr int64_t GATE_UP_MIN_WAVES = 2048, GATE_UP_MIN_WAVES_SMALL = 1100, GATE_UP_SMALL_WEIGHTS = 48ll << 20, GATE_UP_SHORT_K = 1024, GATE_UP_UNEVEN_MIN_GROUPS = 12;
-inline bool plan_gate_up_fused(int64_t M, int64_t n_ff, int64_t K, gate_up_cut* cut = nullptr) {
+inline bool plan_gate_up_with(bool even, int64_t M, int64_t n_ff, int64_t K, gate_up_cut* cut) { // even: no more sets than K divides over
 	if (M <= 0 || n_ff <= 0 || K <= 0 || n_ff % GROUP_K != 0 || K % GROUP_K != 0) {
 		return false;
 	}
@@ -318,6 +318,9 @@ inline bool plan_gate_up_fused(int64_t M, int64_t n_ff, int64_t K, gate_up_cut* 
 	c.tile			  = plan_gemm_tile(M, 2 * n_ff, K, false); // grid_x = n_ff / 64 workgroups of two gate and two up strips
 	const int groups  = static_cast<int>(K / GROUP_K);
 	const gemm_plan g = plan_gemm(M, n_ff, K);
+	while (even && groups % c.tile.ks != 0) {
+		c.tile.ks /= 2;
+	}
 	while (g.kernel == MM_GEMM_TILE && c.tile.ks > 1 && groups % c.tile.ks != 0 && groups / c.tile.ks < GATE_UP_UNEVEN_MIN_GROUPS && int64_t{ 2 } * c.tile.ks * c.tile.grid_x * c.tile.grid_y >= 1024) {
 		c.tile.ks /= 2; // K does not divide, the sets' shares are short, and half as many sets already have a wave on every SIMD ([2 x 6016 x 2176] at 231 rows, one set / two: 32.5 / 35.3 us)
 	}
@@ -325,7 +328,7 @@ inline bool plan_gate_up_fused(int64_t M, int64_t n_ff, int64_t K, gate_up_cut* 
 	if (c.tile.tm == 1 && c.tile.ks > 2) {
 		return false; // no such form: K above 32768, which the rows kernel would have to hand over
 	}
-	if (c.tile.ks == 1 && g.kernel == MM_GEMM_TILE) {
+	if (c.tile.ks == 1 && g.kernel == MM_GEMM_TILE && g.tile.kz == 1) {
 		// a prompt: one set of waves per workgroup has all of K (the mat-mats alone may have two)
 	} else if (waves < (2 * n_ff * K <= GATE_UP_SMALL_WEIGHTS ? GATE_UP_MIN_WAVES_SMALL : GATE_UP_MIN_WAVES)) {
 		return false;
@@ -356,6 +359,9 @@ inline bool plan_gate_up_fused(int64_t M, int64_t n_ff, int64_t K, gate_up_cut* 
 		*cut = c;
 	}
 	return true;
+}
+inline bool plan_gate_up_fused(int64_t M, int64_t n_ff, int64_t K, gate_up_cut* cut = nullptr) {
+	return plan_gate_up_with(false, M, n_ff, K, cut) || plan_gate_up_with(true, M, n_ff, K, cut);
 }
 
 // The MFMA mat-vec's cut (q8_0_gemv_rows_mfma.hip): K over workgroups until a wave owns at most two groups (one with the

@@ -114,3 +114,13 @@ def test_gate_up_of_one_strip_never_asks_for_four_k_sets(m, n_ff, k):
     # the fused kernel for one strip of rows has one and two K sets; K above 32768, which the kernel for up to 32 rows would have to hand over,
     # asks for more on grids this small: three launches, through the workspace
     assert q8_0._lib.lib().nh_q8_0_gate_up_silu_workspace_bytes(m, n_ff, k) == 2 * m * n_ff * 4
+
+
+def test_k_that_no_number_of_sets_divides():
+    # an odd number of 128-quant groups: the tile kernel takes as many K sets as for an even one, gate and up stay one launch
+    for k in (4096 - 128, 4096, 4096 + 128):
+        assert q8_0.plan_mul_mat(512, 4096, k)["k_sets"] == 4
+    size = q8_0._lib.lib().nh_q8_0_gate_up_silu_workspace_bytes
+    assert size(48, 11008, 4224) == 0 and size(100, 11008, 4224) == 0
+    # ... and three launches where the mat-mats have K over workgroups and the fused form would have one set, or ragged passes
+    assert size(65, 3712, 11648) > 0 and size(58, 6400, 2304) > 0
