@@ -182,6 +182,10 @@ PyObject* gate_up_silu(args& in) {
 	if (size < 0 || need < 0) {
 		return nullptr;
 	}
+	const int64_t w_size = nh_q8_0_tiled_bytes(n_ff, k);
+	if (size > 0 && (g->numel() < w_size || u->numel() < w_size || a->numel() < nh_q8_0_tiled_bytes(m, k))) {
+		return nullptr; // larger buffers than the operands are taken, as by the Python way
+	}
 	const at::Tensor out = bytes_like(*a, size);
 	at::Tensor workspace;
 	if (need > 0) {

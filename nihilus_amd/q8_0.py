@@ -45,6 +45,14 @@ def _dev(t: torch.Tensor, dtype: torch.dtype, name: str) -> torch.Tensor:
     return t
 
 
+def _holds(t: torch.Tensor, size: int, name: str) -> None:
+    """The library reads `size` bytes from t on the GPU, whatever t's own shape says."""
+    if not (t.is_cuda and t.is_contiguous()):
+        raise TypeError(f"{name} must be a contiguous tensor on the GPU")
+    if t.numel() * t.element_size() < size:
+        raise ValueError(f"{name} does not hold {size} bytes")
+
+
 def _native(result, fn: str):
     if type(result) is int:
         _lib.check(fn, result)
@@ -337,7 +345,11 @@ def gate_up_silu(w_gate: torch.Tensor, w_up: torch.Tensor, aq_tiled: torch.Tenso
     if not debug and _calls is not None and (out := _native(_calls.gate_up_silu(w_gate, w_up, aq_tiled, m, n_ff, k), "nh_q8_0_gemm_tiled_gate_up_silu")) is not None:
         return out
     lib = _lib.lib()
-    out = torch.empty(tiled_bytes(m, n_ff), dtype=torch.uint8, device=aq_tiled.device)
+    size = tiled_bytes(m, n_ff)
+    if size:
+        for name, t, rows in ("w_gate", w_gate, n_ff), ("w_up", w_up, n_ff), ("aq_tiled", aq_tiled, m):
+            _holds(t, lib.nh_q8_0_tiled_bytes(rows, k), name)  # (a size that the library refuses is negative, and left to it)
+    out = torch.empty(size, dtype=torch.uint8, device=aq_tiled.device)
     if debug:
         gate = torch.empty((m, n_ff), dtype=torch.float32, device=aq_tiled.device)
         up = torch.empty((m, n_ff), dtype=torch.float32, device=aq_tiled.device)

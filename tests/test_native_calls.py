@@ -25,6 +25,51 @@ def test_what_is_no_plain_call_is_left_to_python():
         q8_0.mul_mat(w, x, 1, 4)
 
 
+class _Memory:
+    """Stands for a uint8 tensor of n bytes on the GPU: what gate_up_silu asks of its operands, without one."""
+
+    is_cuda, device = True, "cpu"
+
+    def __init__(self, n):
+        self.numel = lambda: n
+
+    def is_contiguous(self):
+        return True
+
+    def element_size(self):
+        return 1
+
+    def data_ptr(self):
+        return 4096
+
+
+@pytest.mark.parametrize("debug", [False, True])
+def test_gate_up_refuses_operands_that_are_too_small(monkeypatch, debug):
+    # the launch reads what m, n_ff and k say, past the end of a smaller buffer: refused before it
+    m, n_ff, k = 40, 256, 384
+    real, launched = q8_0._lib.lib(), []
+
+    class Library:
+        nh_q8_0_tiled_bytes, nh_q8_0_gate_up_silu_workspace_bytes = real.nh_q8_0_tiled_bytes, real.nh_q8_0_gate_up_silu_workspace_bytes
+
+        def __getattr__(self, name):
+            return lambda *args: launched.append(name) or 0
+
+    monkeypatch.setattr(q8_0, "_calls", None)
+    monkeypatch.setattr(q8_0._lib, "lib", Library)
+    monkeypatch.setattr(q8_0, "_stream", lambda: 0)
+    w, a = q8_0.tiled_bytes(n_ff, k), q8_0.tiled_bytes(m, k)
+    for sizes in (w - 1, w, a), (w, w - 1, a), (w, w, a - 1), (w // 2, w // 2, a), (0, w, a):
+        with pytest.raises(ValueError, match="does not hold"):
+            q8_0.gate_up_silu(*map(_Memory, sizes), m, n_ff, k, debug=debug)
+    for wrong in (m + 32, n_ff, k), (m, n_ff + 128, k), (m, n_ff, k + 128):
+        with pytest.raises(ValueError, match="does not hold"):
+            q8_0.gate_up_silu(_Memory(w), _Memory(w), _Memory(a), *wrong, debug=debug)
+    assert not launched
+    q8_0.gate_up_silu(_Memory(w), _Memory(w + 5), _Memory(a), m, n_ff, k, debug=debug)  # buffers may be larger
+    assert len(launched) == 1
+
+
 class _Subclass(torch.Tensor):
     pass
 
@@ -102,3 +147,16 @@ def test_same_errors_either_way(q8, monkeypatch):
         got = q8.mul_mat(w, x, n, k)
     side.synchronize()
     assert torch.equal(got, want)
+
+
+@pytest.mark.gpu
+def test_gate_up_operands_that_are_too_small_either_way(q8, monkeypatch):
+    m, n_ff, k = 40, 256, 384
+    w = q8.tile(q8.fill_weight_blocks(3, n_ff, k), n_ff, k)
+    a = q8.quantize_row_q8_0(q8.fill_activations(4, m * k).reshape(m, k), tiled=True)
+    for call in (lambda: q8.gate_up_silu(w[:-1], w, a, m, n_ff, k), lambda: q8.gate_up_silu(w, w[:-1], a, m, n_ff, k), lambda: q8.gate_up_silu(w, w, a[:-1], m, n_ff, k),
+                 lambda: q8.gate_up_silu(w, w, a, m + 32, n_ff, k), lambda: q8.gate_up_silu(w, w, a, m, n_ff + 128, k), lambda: q8.gate_up_silu(w, w, a, m, n_ff, k + 128)):
+        native, python = _both(monkeypatch, call)
+        assert native == python and native[0] is ValueError
+    native, python = _both(monkeypatch, lambda: q8.gate_up_silu(torch.cat([w, w]), w, torch.cat([a, w]), m, n_ff, k))  # larger buffers are taken
+    assert native.tobytes() == python.tobytes() == q8.gate_up_silu(w, w, a, m, n_ff, k).cpu().numpy().tobytes()
