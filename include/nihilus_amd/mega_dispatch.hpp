@@ -342,7 +342,7 @@ namespace nihilus {
 			} else {
 				const int64_t ws_bytes = nh_q8_0_mul_mat_workspace_bytes(rows, n_embd);
 				void* ws			   = amd_detail::workspace<config_type>(amd_detail::slot_quantized, ws_bytes);
-				amd_detail::check<config_type>(nh_q8_0_mul_mat_residual(w, attn, residual, y, rows, n_embd, n_embd, ws, ws_bytes, nullptr),
+				amd_detail::check<config_type>(nh_q8_0_mul_mat_scratch(w, attn, residual, y, rows, n_embd, n_embd, ws, ws_bytes, nullptr),
 					"mega_attention_apply prompt_eval_time: attn_out mat-mat + residual");
 			}
 			amd_detail::after_launch<config_type>();

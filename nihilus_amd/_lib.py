@@ -55,6 +55,7 @@ SIGNATURES = {
     "nh_q8_0_debug_set_spin_limit": (_int, [_i64]),
     "nh_q8_0_set_in_kernel_waits": (_int, [_int]),
     "nh_q8_0_debug_plan_mul_mat": (_int, [_i64, _i64, _i64, _vp]),
+    "nh_q8_0_debug_plan_mul_mat_scratch": (_int, [_i64, _i64, _i64, _vp]),
     "nh_q8_0_gemv_tiled_residual_f32": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _vp]),
     "nh_q8_0_gemv_tiled_multi_f32": (_int, [C.POINTER(_vp), C.POINTER(_vp), C.POINTER(_i64), _i64, _vp, _i64, _vp]),
     "nh_q8_0_debug_fused_quantize": (_int, [_vp, _vp, _i64, _vp]),
@@ -64,6 +65,7 @@ SIGNATURES = {
     "nh_q8_0_mul_mat_workspace_bytes": (_i64, [_i64, _i64]),
     "nh_q8_0_mul_mat": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _vp, _i64, _vp]),
     "nh_q8_0_mul_mat_residual": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _i64, _vp]),
+    "nh_q8_0_mul_mat_scratch": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _i64, _vp]),
     "nh_q8_0_mul_mat_batch": (_int, [_vp, _i64, _vp, _i64, _vp]),
     "nh_profile_begin": (_int, [_int, _i64]),
     "nh_profile_shader_clock": (_int, [C.POINTER(C.c_double), _i64]),

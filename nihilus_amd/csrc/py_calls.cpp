@@ -131,7 +131,7 @@ PyObject* mul_mat(args& in) {
 	float* yp		   = static_cast<float*>(y.mutable_data_ptr());
 	void* ws		   = need > 0 ? workspace.mutable_data_ptr() : nullptr;
 	void* s			   = stream();
-	return finish(y, [&] { return residual ? nh_q8_0_mul_mat_residual(wp, xp, rp, yp, m, n, k, ws, need, s) : nh_q8_0_mul_mat(wp, xp, yp, m, n, k, ws, need, s); });
+	return finish(y, [&] { return nh_q8_0_mul_mat_scratch(wp, xp, rp, yp, m, n, k, ws, need, s); });
 }
 
 // gemm(w_tiled, aq_tiled, m, n, k, residual or None)

@@ -653,7 +653,8 @@ int64_t nh_q8_0_mul_mat_workspace_bytes(int64_t M, int64_t K) {
 	return (nh_q8_0_tiled_bytes(M, K) + 255) / 256 * 256;
 }
 
-static int mul_mat_common(const void* W_tiled, const float* x, const float* residual, float* y, int64_t M, int64_t N, int64_t K, void* workspace, int64_t workspace_bytes, void* stream) {
+static int mul_mat_common(const void* W_tiled, const float* x, const float* residual, float* y, int64_t M, int64_t N, int64_t K, void* workspace, int64_t workspace_bytes, void* stream,
+	bool scratch = false) {
 	NH_TRY(check_shape(M, N, K, true));
 	if (M == 0 || N == 0) {
 		return NH_OK;
@@ -664,7 +665,10 @@ static int mul_mat_common(const void* W_tiled, const float* x, const float* resi
 		NH_REQUIRE(x && (workspace || need == 0), NH_ERR_NULL_POINTER);
 		NH_REQUIRE(aligned16(workspace) && aligned16(x), NH_ERR_ALIGNMENT);
 	}
-	const nh::mul_mat_plan plan = nh::plan_mul_mat(M, N, K); // which kernel: q8_0_plan.h
+	nh::mul_mat_plan plan = nh::plan_mul_mat(M, N, K, scratch); // which kernel: q8_0_plan.h
+	if (scratch && plan.quantize_launch && plan.gemm.skinny.splits > 1 && nh::gemv_rows_mfma_suits(M, N, K) && nh::stream_is_capturing(as_stream(stream))) {
+		plan = nh::plan_mul_mat(M, N, K); // K over workgroups needs the library's hand-off scratch, which a capture may be without; this form does not
+	}
 	if (M == 1) { // quantize fused into the mat-vec: the workspace stays unused
 		return residual ? nh_q8_0_gemv_tiled_residual_f32(W_tiled, x, residual, y, N, K, stream) : nh_q8_0_gemv_tiled_f32(W_tiled, x, y, N, K, stream);
 	}
@@ -684,10 +688,10 @@ static int mul_mat_common(const void* W_tiled, const float* x, const float* resi
 	return residual ? nh_q8_0_gemm_tiled_residual(W_tiled, workspace, residual, y, M, N, K, stream) : nh_q8_0_gemm_tiled(W_tiled, workspace, y, M, N, K, stream);
 }
 
-int nh_q8_0_debug_plan_mul_mat(int64_t M, int64_t N, int64_t K, int32_t* host_plan) {
+static int debug_plan_common(int64_t M, int64_t N, int64_t K, int32_t* host_plan, bool scratch) {
 	NH_TRY(check_shape(M, N, K, true));
 	NH_REQUIRE(host_plan, NH_ERR_NULL_POINTER);
-	const nh::mul_mat_plan p = nh::plan_mul_mat(M, N, K);
+	const nh::mul_mat_plan p = nh::plan_mul_mat(M, N, K, scratch);
 	for (int i = 0; i < 8; ++i) {
 		host_plan[i] = 0;
 	}
@@ -720,6 +724,14 @@ int nh_q8_0_debug_plan_mul_mat(int64_t M, int64_t N, int64_t K, int32_t* host_pl
 	return NH_OK;
 }
 
+int nh_q8_0_debug_plan_mul_mat(int64_t M, int64_t N, int64_t K, int32_t* host_plan) {
+	return debug_plan_common(M, N, K, host_plan, false);
+}
+
+int nh_q8_0_debug_plan_mul_mat_scratch(int64_t M, int64_t N, int64_t K, int32_t* host_plan) {
+	return debug_plan_common(M, N, K, host_plan, true);
+}
+
 int nh_q8_0_mul_mat(const void* W_tiled, const float* x, float* y, int64_t M, int64_t N, int64_t K, void* workspace, int64_t workspace_bytes, void* stream) {
 	return mul_mat_common(W_tiled, x, nullptr, y, M, N, K, workspace, workspace_bytes, stream);
 }
@@ -728,6 +740,10 @@ int nh_q8_0_mul_mat_residual(const void* W_tiled, const float* x, const float* r
 	void* stream) {
 	NH_REQUIRE(residual || M == 0 || N == 0, NH_ERR_NULL_POINTER);
 	return mul_mat_common(W_tiled, x, residual, y, M, N, K, workspace, workspace_bytes, stream);
+}
+
+int nh_q8_0_mul_mat_scratch(const void* W_tiled, const float* x, const float* residual, float* y, int64_t M, int64_t N, int64_t K, void* scratch, int64_t scratch_bytes, void* stream) {
+	return mul_mat_common(W_tiled, x, residual, y, M, N, K, scratch, scratch_bytes, stream, true);
 }
 
 int nh_q8_0_debug_block_sums(const void* W, const void* Aq, int32_t* sums, int64_t M, int64_t N, int64_t K, int path, void* stream) {

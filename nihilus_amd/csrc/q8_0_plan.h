@@ -392,32 +392,36 @@ inline gemv_plan plan_gemv_rows_mfma(int64_t strips, int64_t K, int rows, bool c
 	return p;
 }
 
-// Where it is the fastest form.  Every strip's workgroup quantizes all the rows again, which costs in proportion to M, and its sixteen waves
-// have a CU to themselves, so a launch of more workgroups than CUs walks some of them one after the other.  Measured against the quantize
-// launch and the kernel for up to 32 quantized rows (weights rotated, us, this / the two launches; workgroups, groups per wave):
+// The matrices it takes: up to sixteen rows on at most 40 MB, four on at most 80 MB (two and three rows stay on the dot-product kernel).
+// nh_q8_0_mul_mat promises its callers that these leave their workspace untouched.
+inline bool gemv_rows_mfma_suits(int64_t M, int64_t N, int64_t K) {
+	return M >= 4 && M <= GEMV_ROWS_MFMA_MAX && N * (K / QK) * BLOCK_BYTES <= int64_t{ M == 4 ? 80 : 40 } << 20;
+}
+// Of those, the ones where it is the fastest form; the others run as a quantize launch and the kernel for up to 32 quantized rows where the
+// caller has no such promise (nh_q8_0_mul_mat_scratch).  Every strip's workgroup quantizes all the rows again, which costs in proportion to M, and its
+// sixteen waves have a CU to themselves, so a launch of more workgroups than CUs walks some of them one after the other.  Measured
+// against those two launches (weights rotated, us, this / the two launches; workgroups, groups per wave):
 //   9 to 16 rows   [4096 x 4096] 256, 1:  9.7 /  9.7 (12 rows 8.5 /  9.5)   [8192 x 2048] 256, 1:  8.6 /  9.0   [1024 x 14336] 256, 1: 10.4 / 10.4
 //                  [6144 x 4096] 384, 1: 16.2 / 10.4   [2560 x 5120] 320, 1: 14.0 /  9.3   [4096 x 8192] 512, 1: 17.4 / 12.1
 //   8 rows         [4096 x 4096] 256, 1:  7.6 /  9.2   [4096 x 6144] 256, 2:  9.5 / 10.1   [8192 x 4096] 256, 2: 11.0 / 10.5
 //                  [5120 x 2560] 320, 1:  8.2 /  9.0   [6144 x 4096] 384, 1: 10.0 /  9.6   [5120 x 5120] 320, 2: 13.1 / 10.5
 //   6 rows         [8192 x 4096] 256, 2:  9.9 / 10.5   [6144 x 4096] 384, 1:  9.3 /  9.5   [4608 x 4608] 288, 2: 11.2 /  9.9
 //   4 rows         [4096 x 8192] 256, 2: 10.2 / 11.4   [6144 x 4096] 384, 1:  8.6 /  9.6   [4608 x 4608] 288, 2:  9.7 /  9.9
-// Four rows also on matrices of up to 80 MB ([14336 x 4096] 15.5 / 14.5, [8192 x 8192] 17.8 / 16.0: a line drawn against the kernels before,
-// which tests/test_plan_cpu.py fixes).  (Two and three rows stay on the dot-product kernel.)
-inline bool gemv_rows_mfma_suits(int64_t M, int64_t N, int64_t K) {
-	constexpr int64_t MIB		 = int64_t{ 1 } << 20;
+// Over 500 random shapes of 5 to 16 rows on the far side of the line the two launches are faster, 1.1 (5, 6 rows) to 1.6 times (13 to 16), but for ten
+// within 6 %.  Four rows on matrices of up to 80 MB ([14336 x 4096] 15.5 / 14.5, [8192 x 8192] 17.8 / 16.0): a line drawn against the kernels
+// before, which tests/test_plan_cpu.py fixes.
+inline bool gemv_rows_mfma_fastest(int64_t M, int64_t N, int64_t K) {
+	constexpr int64_t MIB	   = int64_t{ 1 } << 20;
 	const int64_t weight_bytes = N * (K / QK) * BLOCK_BYTES;
-	if (M < 4 || M > GEMV_ROWS_MFMA_MAX || weight_bytes > (M == 4 ? 80 : 40) * MIB) {
-		return false;
-	}
-	const gemv_plan p	 = plan_gemv_rows_mfma((N + STRIP_ROWS - 1) / STRIP_ROWS, K, M <= 8 ? 8 : 16, false);
-	const bool one_round = p.strips * p.splits <= 256;
+	const gemv_plan p		   = plan_gemv_rows_mfma((N + STRIP_ROWS - 1) / STRIP_ROWS, K, M <= 8 ? 8 : 16, false);
+	const bool one_round	   = p.strips * p.splits <= 256;
 	if (M > 8) {
 		return one_round;
 	}
 	return M == 4 || (one_round ? M <= 6 || weight_bytes <= 32 * MIB : p.tiles == 1 && (M <= 6 || weight_bytes <= 20 * MIB));
 }
 
-// nh_q8_0_mul_mat: fp32 activations [M][K] against a tiled weight [N][K].
+// nh_q8_0_mul_mat: fp32 activations [M][K] against a tiled weight [N][K].  scratch: nh_q8_0_mul_mat_scratch, whose workspace any shape may write.
 struct mul_mat_plan {
 	int kernel; // mul_mat_kernel
 	int quantize_launch; // 1: the activations are quantized by a launch of their own into the caller's workspace
@@ -435,7 +439,7 @@ inline int plan_gemv_row_parts(const gemv_plan& p) {
 	}
 	return p.strips * 2 <= 256 ? (p.strips * 4 <= 256 ? 4 : 2) : 1;
 }
-inline mul_mat_plan plan_mul_mat(int64_t M, int64_t N, int64_t K) {
+inline mul_mat_plan plan_mul_mat(int64_t M, int64_t N, int64_t K, bool scratch = false) {
 	mul_mat_plan p{};
 	if (M <= 0 || N <= 0 || K <= 0) {
 		p.kernel = MM_NOTHING;
@@ -447,7 +451,7 @@ inline mul_mat_plan plan_mul_mat(int64_t M, int64_t N, int64_t K) {
 		p.gemv_row_parts = plan_gemv_row_parts(p.gemv);
 		return p;
 	}
-	if (gemv_rows_mfma_suits(M, N, K)) {
+	if (gemv_rows_mfma_suits(M, N, K) && (!scratch || gemv_rows_mfma_fastest(M, N, K))) {
 		p.kernel		 = MM_GEMV_ROWS_MFMA;
 		p.gemv			 = plan_gemv_rows_mfma((N + STRIP_ROWS - 1) / STRIP_ROWS, K, M <= 8 ? 8 : 16, false);
 		p.gemv_row_parts = 1;

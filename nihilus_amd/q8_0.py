@@ -74,12 +74,14 @@ def tiled_bytes(rows: int, k: int) -> int:
 KERNEL_NAMES = {0: "nothing", 1: "gemv", 2: "gemv_rows", 3: "gemm_skinny", 4: "gemm_tile_stream", 5: "gemm_tile", 6: "gemv_rows_mfma"}
 
 
-def plan_mul_mat(m: int, n: int, k: int) -> dict:
-    """Which kernel mul_mat runs for fp32 activations [m, k] against a tiled weight [n, k], and its cut (no GPU needed)."""
+def plan_mul_mat(m: int, n: int, k: int, own_workspace: bool = False) -> dict:
+    """Which kernel mul_mat runs for fp32 activations [m, k] against a tiled weight [n, k], and its cut (no GPU needed);
+    own_workspace: with a workspace of the caller's."""
     import ctypes
 
     raw = (ctypes.c_int32 * 8)()
-    _lib.check("nh_q8_0_debug_plan_mul_mat", _lib.lib().nh_q8_0_debug_plan_mul_mat(m, n, k, raw))
+    fn = "nh_q8_0_debug_plan_mul_mat" if own_workspace else "nh_q8_0_debug_plan_mul_mat_scratch"
+    _lib.check("nh_q8_0_debug_plan_mul_mat", getattr(_lib.lib(), fn)(m, n, k, raw))
     plan = {"kernel": KERNEL_NAMES[raw[0]], "quantize_launch": bool(raw[1]), "gemm_rows": bool(raw[7])}
     if raw[0] in (1, 6):
         plan.update(k_splits=raw[2], groups_per_wave=raw[3], row_parts=raw[4])
@@ -364,9 +366,12 @@ def gate_up_silu(w_gate: torch.Tensor, w_up: torch.Tensor, aq_tiled: torch.Tenso
 
 
 def mul_mat(w_tiled: torch.Tensor, x: torch.Tensor, n: int, k: int, workspace: torch.Tensor | None = None, residual: torch.Tensor | None = None) -> torch.Tensor:
-    """fp32 activations [M, K] x tiled Q8_0 weight [N, K] -> fp32 [M, N]: quantize + GEMV/GEMM (+ residual [M, N] if given)."""
+    """fp32 activations [M, K] x tiled Q8_0 weight [N, K] -> fp32 [M, N]: quantize + GEMV/GEMM (+ residual [M, N] if given).
+
+    A workspace of the caller's is written only where nh_q8_0_mul_mat says so; without one the call has its own."""
+    fn = "nh_q8_0_mul_mat" if residual is None else "nh_q8_0_mul_mat_residual"
     if workspace is None and _calls is not None:
-        y = _native(_calls.mul_mat(w_tiled, x, n, k, residual), "nh_q8_0_mul_mat" if residual is None else "nh_q8_0_mul_mat_residual")
+        y = _native(_calls.mul_mat(w_tiled, x, n, k, residual), fn)
         if y is not None:
             return y
     w_tiled, x = _dev(w_tiled, torch.uint8, "w_tiled"), _dev(x, torch.float32, "x")
@@ -374,9 +379,11 @@ def mul_mat(w_tiled: torch.Tensor, x: torch.Tensor, n: int, k: int, workspace: t
     m = x2.shape[0]
     if x2.shape[1] != k or w_tiled.numel() != tiled_bytes(n, k):
         raise ValueError("operand sizes do not match m x n x k")
-    need = _lib.lib().nh_q8_0_mul_mat_workspace_bytes(m, k)
+    lib = _lib.lib()
+    need = lib.nh_q8_0_mul_mat_workspace_bytes(m, k)
     _lib.check("nh_q8_0_mul_mat_workspace_bytes", need if need < 0 else 0)
-    if workspace is None and need > 0:  # (a few rows need none: an allocation of nothing was 1.4 us of the call)
+    own = workspace is None
+    if own and need > 0:  # (a few rows need none: an allocation of nothing was 1.4 us of the call)
         workspace = x.new_empty(need, dtype=torch.uint8)
     ws_ptr, ws_bytes = (None, 0) if workspace is None else (workspace.data_ptr(), workspace.numel())
     y = x.new_empty((m, n))
@@ -384,9 +391,14 @@ def mul_mat(w_tiled: torch.Tensor, x: torch.Tensor, n: int, k: int, workspace: t
         residual = _dev(residual, torch.float32, "residual")
         if residual.numel() != m * n:
             raise ValueError("residual must hold m x n floats")
-        _lib.check("nh_q8_0_mul_mat_residual", _lib.lib().nh_q8_0_mul_mat_residual(w_tiled.data_ptr(), x2.data_ptr(), residual.data_ptr(), y.data_ptr(), m, n, k, ws_ptr, ws_bytes, _stream()))
-        return y
-    _lib.check("nh_q8_0_mul_mat", _lib.lib().nh_q8_0_mul_mat(w_tiled.data_ptr(), x2.data_ptr(), y.data_ptr(), m, n, k, ws_ptr, ws_bytes, _stream()))
+    add = None if residual is None else residual.data_ptr()
+    if own:
+        status = lib.nh_q8_0_mul_mat_scratch(w_tiled.data_ptr(), x2.data_ptr(), add, y.data_ptr(), m, n, k, ws_ptr, ws_bytes, _stream())
+    elif residual is None:
+        status = lib.nh_q8_0_mul_mat(w_tiled.data_ptr(), x2.data_ptr(), y.data_ptr(), m, n, k, ws_ptr, ws_bytes, _stream())
+    else:
+        status = lib.nh_q8_0_mul_mat_residual(w_tiled.data_ptr(), x2.data_ptr(), add, y.data_ptr(), m, n, k, ws_ptr, ws_bytes, _stream())
+    _lib.check(fn, status)
     return y
 
 

@@ -124,3 +124,18 @@ def test_k_that_no_number_of_sets_divides():
     assert size(48, 11008, 4224) == 0 and size(100, 11008, 4224) == 0
     # ... and three launches where the mat-mats have K over workgroups and the fused form would have one set, or ragged passes
     assert size(65, 3712, 11648) > 0 and size(58, 6400, 2304) > 0
+
+
+def test_what_leaves_a_callers_workspace_untouched():
+    # nh_q8_0_mul_mat's promise: 4 to 16 rows on matrices of up to 40 MB, 4 rows up to 80 MB.  Without a workspace of the caller's the faster way
+    moved = 0
+    for n in (32, 1000, 1024, 2560, 4096, 4500, 5120, 6144, 8192, 14336, 28672, 128256):
+        for k in (128, 1024, 2048, 4096, 5120, 8192, 14336, 28672):
+            for m in range(4, 18):
+                promised = m <= 16 and n * (k // 32) * 34 <= (80 if m == 4 else 40) << 20
+                kept = q8_0.plan_mul_mat(m, n, k, own_workspace=True)
+                assert kept["quantize_launch"] != promised and (kept["kernel"] == "gemv_rows_mfma") == promised, (m, n, k)
+                moved += kept != q8_0.plan_mul_mat(m, n, k)
+                assert promised or kept == q8_0.plan_mul_mat(m, n, k)
+    assert moved > 100
+    assert q8_0.plan_mul_mat(16, 4096, 8192)["quantize_launch"] and not q8_0.plan_mul_mat(16, 4096, 8192, own_workspace=True)["quantize_launch"]
