@@ -245,8 +245,10 @@ inline gemm_plan plan_gemm(int64_t M, int64_t N, int64_t K) {
 			const gemm_tile_cut tile = plan_gemm_tile(M, N, K, true);
 			stream_tile				 = tile.kz > 1;
 			if (stream_tile && gemm_rows_instead_of_tile(M, N, K)) {
-				stream_tile = false;
-				wide		= plan_gemm_skinny(M, N, K).splits * SK_WAVES < tile.ks * tile.kz; // no fewer shares of K than there
+				gemm_skinny_cut cut = plan_gemm_skinny(M, N, K);
+				wide				= cut.splits * SK_WAVES < tile.ks * tile.kz; // no fewer shares of K than there
+				cut.waves			= wide ? SK_WIDE_WAVES : cut.waves;
+				stream_tile			= !gemm_rows_fits(M, N, cut); // K above 32768: the streaming kernel, 62.7 us at [8192 x 36864] and 24 rows, against 54.2
 			}
 		}
 	}

@@ -139,3 +139,9 @@ def test_what_leaves_a_callers_workspace_untouched():
                 assert promised or kept == q8_0.plan_mul_mat(m, n, k)
     assert moved > 100
     assert q8_0.plan_mul_mat(16, 4096, 8192)["quantize_launch"] and not q8_0.plan_mul_mat(16, 4096, 8192, own_workspace=True)["quantize_launch"]
+
+
+@pytest.mark.parametrize("m,n,k", [(24, 8192, 36864), (32, 8192, 36864), (20, 14336, 40960), (17, 8096, 45056)])
+def test_k_too_long_for_the_rows_kernel_stays_with_the_tile_kernel(m, n, k):
+    # the rows kernel's hand-off does not hold two sets of K of so many strips; the streaming kernel in its place is the slowest of the three
+    assert kernel(m, n, k) == "gemm_tile_stream"
