@@ -190,10 +190,20 @@ inline bool gemm_rows_suits(int64_t M, int64_t N, int64_t K) {
 //   rows      [8192 x 8192]   [8192 x 14336]  [8192 x 28672]  [10240 x 8192]  [12288 x 12288]  [14336 x 14336]  [16384 x 4096]  [20480 x 8192]
 //   17 to 24  18.6 / 15.6     28.5 / 23.8     46.2 / 42.5     22.0 / 23.5     32.2 / 34.0      41.2 / 40.8      17.7 / 15.0     37.5 / 35.0
 //   25 to 32  18.2 / 15.8     28.6 / 25.1     45.7 / 45.3     22.1 / 25.2     32.3 / 36.8      41.4 / 43.8      17.8 / 15.9     37.8 / 38.0
+// Near two workgroups per CU only while K is at most 15360: over 370 random shapes of 17 to 24 rows and 448 to 512 strips tile / rows is 0.97 to 1.3 up to
+// there, 0.96 to 1.0 at 16384 and 0.89 to 1.07 beyond ([14655 x 27648] at 17 rows 69.2 / 77.6).  25 to 32 rows on up to 256 strips with K above
+// 24576 only where the tile kernel has fewer than four workgroups along K, one per CU ([8192 x 27648] at 26 rows 55.9 / 44.4, but
+// [8192 x 32768] at 28 rows 48.8 / 51.9).
 // (sixteen rows would gain as well, 18.8 / 14.4 and 45.8 / 40.4 in the first and third column: tests/test_plan_cpu.py fixes their kernel)
-inline bool gemm_rows_instead_of_tile(int64_t M, int64_t N, int64_t K) {
+inline bool gemm_rows_instead_of_tile(int64_t M, int64_t N, int64_t K, const gemm_tile_cut& tile) {
 	const int64_t strips = (N + STRIP_ROWS - 1) / STRIP_ROWS;
-	return M > 16 && M <= GEMM_ROWS_MAX && (strips <= 256 || (M <= 24 ? strips >= 448 : strips >= 512 && K <= 4096));
+	if (M <= 16 || M > GEMM_ROWS_MAX) {
+		return false;
+	}
+	if (strips <= 256) {
+		return M <= 24 || K <= 24576 || tile.kz < 4;
+	}
+	return M <= 24 ? strips >= 448 && K <= 15360 : strips >= 512 && K <= 4096;
 }
 
 // whether the rows kernel's tagged sums hold this cut
@@ -244,7 +254,7 @@ inline gemm_plan plan_gemm(int64_t M, int64_t N, int64_t K) {
 			// ([14336 x 4096] at M = 64 unsplit: 30 against 23 us), and stays with the streaming kernel.
 			const gemm_tile_cut tile = plan_gemm_tile(M, N, K, true);
 			stream_tile				 = tile.kz > 1;
-			if (stream_tile && gemm_rows_instead_of_tile(M, N, K)) {
+			if (stream_tile && gemm_rows_instead_of_tile(M, N, K, tile)) {
 				gemm_skinny_cut cut = plan_gemm_skinny(M, N, K);
 				wide				= cut.splits * SK_WAVES < tile.ks * tile.kz; // no fewer shares of K than there
 				cut.waves			= wide ? SK_WIDE_WAVES : cut.waves;

@@ -145,3 +145,11 @@ def test_what_leaves_a_callers_workspace_untouched():
 def test_k_too_long_for_the_rows_kernel_stays_with_the_tile_kernel(m, n, k):
     # the rows kernel's hand-off does not hold two sets of K of so many strips; the streaming kernel in its place is the slowest of the three
     assert kernel(m, n, k) == "gemm_tile_stream"
+
+
+@pytest.mark.parametrize("m,n,k,rows", [(20, 14656, 15360, True), (20, 14656, 17408, False), (17, 16128, 27648, False), (24, 8192, 32768, True), (28, 8192, 24576, True), (26, 8192, 27648, True),
+                                        (28, 8192, 32768, False), (28, 8084, 26624, False)])
+def test_long_k_of_17_to_32_rows(m, n, k, rows):
+    # the rows kernel's line to the tile kernel with K over workgroups: two workgroups per CU with long K, and 25 rows and more where the tile
+    # kernel has a workgroup per CU, are faster there
+    assert q8_0.plan_mul_mat(m, n, k)["gemm_rows"] == rows and (kernel(m, n, k) == "gemm_tile_stream") != rows
