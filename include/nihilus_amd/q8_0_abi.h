@@ -375,6 +375,12 @@ int nh_q8_0_debug_ffn_gate_up(float* gate_out, float* up_out, int64_t N_ff, void
 int nh_q8_0_debug_plan_mul_mat(int64_t M, int64_t N, int64_t K, int32_t* host_plan);
 /* ... and nh_q8_0_mul_mat_scratch */
 int nh_q8_0_debug_plan_mul_mat_scratch(int64_t M, int64_t N, int64_t K, int32_t* host_plan);
+/* The same of nh_q8_0_gemm_tiled_gate_up_silu: [0] 0 three launches through the workspace (or an empty problem), 1 one launch of the kernel
+ * for few rows, 2 one launch of the MFMA tile kernel;
+ *   1: [1] shares of K that a workgroup adds;
+ *   2: [1] activation strips per wave, [2] K sets of four waves per workgroup, [3] passes over K, [4] 1 when the shares are added in the
+ *      streaming kernel's order, [5], [6] the grid (blocks of 64 rows of both matrices, groups of activation strips). */
+int nh_q8_0_debug_plan_gate_up_silu(int64_t M, int64_t N_ff, int64_t K, int32_t* host_plan);
 
 /* nh_q8_0_gemm_tiled_gate_up_silu with the fp32 outputs of the two mat-mats copied out as well (gate_out, up_out: [M][N_ff]), so that
  * the quantized activation can be compared with the CPU quantizer applied to exactly the sums the launch computed. */

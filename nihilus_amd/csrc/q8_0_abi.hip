@@ -732,6 +732,29 @@ int nh_q8_0_debug_plan_mul_mat_scratch(int64_t M, int64_t N, int64_t K, int32_t*
 	return debug_plan_common(M, N, K, host_plan, true);
 }
 
+int nh_q8_0_debug_plan_gate_up_silu(int64_t M, int64_t N_ff, int64_t K, int32_t* host_plan) {
+	NH_TRY(check_shape(M, N_ff, K, true));
+	NH_REQUIRE(N_ff % nh::GROUP_K == 0, NH_ERR_SHAPE);
+	NH_REQUIRE(host_plan, NH_ERR_NULL_POINTER);
+	for (int i = 0; i < 8; ++i) {
+		host_plan[i] = 0;
+	}
+	nh::gate_up_cut cut{};
+	if (nh::gate_up_rows_suits(M, N_ff, K)) {
+		host_plan[0] = 1;
+		host_plan[1] = nh::gate_up_rows_waves(M, N_ff, K);
+	} else if (nh::plan_gate_up_fused(M, N_ff, K, &cut)) {
+		host_plan[0] = 2;
+		host_plan[1] = cut.tile.tm;
+		host_plan[2] = cut.tile.ks;
+		host_plan[3] = cut.passes;
+		host_plan[4] = cut.tree;
+		host_plan[5] = static_cast<int32_t>(cut.tile.grid_x);
+		host_plan[6] = static_cast<int32_t>(cut.tile.grid_y);
+	}
+	return NH_OK;
+}
+
 int nh_q8_0_mul_mat(const void* W_tiled, const float* x, float* y, int64_t M, int64_t N, int64_t K, void* workspace, int64_t workspace_bytes, void* stream) {
 	return mul_mat_common(W_tiled, x, nullptr, y, M, N, K, workspace, workspace_bytes, stream);
 }

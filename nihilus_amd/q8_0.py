@@ -92,6 +92,19 @@ def plan_mul_mat(m: int, n: int, k: int, own_workspace: bool = False) -> dict:
     return plan
 
 
+def plan_gate_up_silu(m: int, n_ff: int, k: int) -> dict:
+    """How gate_up_silu runs: "three_launches", "rows" (the kernel for few rows) or "tile", and the cut (no GPU needed)."""
+    import ctypes
+
+    raw = (ctypes.c_int32 * 8)()
+    _lib.check("nh_q8_0_debug_plan_gate_up_silu", _lib.lib().nh_q8_0_debug_plan_gate_up_silu(m, n_ff, k, raw))
+    if raw[0] == 1:
+        return {"form": "rows", "waves": raw[1]}
+    if raw[0] == 2:
+        return {"form": "tile", "activation_strips": raw[1], "k_sets": raw[2], "passes": raw[3], "tree": bool(raw[4]), "grid": (raw[5], raw[6])}
+    return {"form": "three_launches"}
+
+
 def quantize_row_q8_0(x: torch.Tensor, tiled: bool = False) -> torch.Tensor:
     """x fp32 [M, K] (or [K]) -> uint8 blocks [M, K/32*34] (or the tiled byte stream)."""
     x = _dev(x, torch.float32, "x")
