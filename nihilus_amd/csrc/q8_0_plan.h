@@ -347,8 +347,10 @@ inline bool plan_gate_up_with(bool even, int64_t M, int64_t n_ff, int64_t K, gat
 	} else {
 		const bool tree	 = g.kernel == MM_GEMM_SKINNY || (g.kernel == MM_GEMM_TILE && g.tile.kz > 1);
 		int shares		 = g.kernel == MM_GEMM_SKINNY ? g.skinny.splits * g.skinny.waves : g.tile.ks * g.tile.kz;
-		if (g.kernel == MM_GEMM_TILE && g.tile.kz == 1) {
-			while (groups % shares != 0) { // K does not divide over the mat-mats' sets: a second pass for the last bits only ([2 x 11008 x 4352] at 100 rows 49.4 -> 55.1 us)
+		if (g.kernel != MM_GEMM_SKINNY && g.tile.kz == 1) {
+			// K does not divide over the mat-mats' sets: a second pass for the last bits only ([2 x 11008 x 4352] at 100 rows 49.4 -> 55.1 us, [2 x 24832 x 6912] at 40 rows
+			// 79.8 -> 88.2), or no single launch at all where there is one set ([2 x 41856 x 13184] at 21 rows 196 us, three launches 231)
+			while (groups % shares != 0) {
 				shares /= 2;
 			}
 			shares = shares > c.tile.ks ? shares : c.tile.ks;

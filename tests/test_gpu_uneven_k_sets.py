@@ -60,12 +60,14 @@ def test_the_zero_scales_hide_an_infinity(q8, oracle):
     assert np.array_equal(to_host(q8.gemm(wt, at, m, n, k, tiled=True)), want, equal_nan=True)
 
 
-# the fused gate / up, (m, n_ff, groups, activation strips, K sets, passes): two sets in one pass, four in two
-@pytest.mark.parametrize("m,n_ff,groups,strips,sets,passes", [(100, 11008, 33, 2, 2, 1), (48, 5504, 33, 2, 4, 2), (40, 5504, 21, 2, 4, 2)])
+# the fused gate / up, (m, n_ff, groups, activation strips, K sets, passes): two sets in one pass, of one and two strips, streamed weights or not, and
+# one set where the mat-mats have two uneven ones; four sets in two passes, and two in four
+@pytest.mark.parametrize("m,n_ff,groups,strips,sets,passes", [(100, 11008, 33, 2, 2, 1), (48, 5504, 33, 2, 4, 2), (40, 5504, 21, 2, 4, 2), (24, 24576, 33, 1, 2, 1), (40, 24576, 33, 2, 2, 1), (24, 24576, 15, 1, 2, 1),
+                                                              (40, 24576, 15, 2, 2, 1), (24, 33024, 9, 1, 1, 1), (58, 9216, 18, 2, 2, 4)])
 def test_uneven_k_sets_of_gate_up(q8, oracle, m, n_ff, groups, strips, sets, passes):
     k = 128 * groups
     plan = q8.plan_gate_up_silu(m, n_ff, k)
-    assert (plan["form"], plan["activation_strips"], plan["k_sets"], plan["passes"]) == ("tile", strips, sets, passes) and groups % (sets * passes)
+    assert (plan["form"], plan["activation_strips"], plan["k_sets"], plan["passes"]) == ("tile", strips, sets, passes) and (groups % (sets * passes) or sets == 1)
     assert q8._lib.lib().nh_q8_0_gate_up_silu_workspace_bytes(m, n_ff, k) == 0
     wg, wu = oracle.fill_weights(1 + m, n_ff, k), oracle.fill_weights(2 + m, n_ff, k)
     x = oracle.fill_activations(m + k, m * k).reshape(m, k)

@@ -153,3 +153,11 @@ def test_long_k_of_17_to_32_rows(m, n, k, rows):
     # the rows kernel's line to the tile kernel with K over workgroups: two workgroups per CU with long K, and 25 rows and more where the tile
     # kernel has a workgroup per CU, are faster there
     assert q8_0.plan_mul_mat(m, n, k)["gemm_rows"] == rows and (kernel(m, n, k) == "gemm_tile_stream") != rows
+
+
+@pytest.mark.parametrize("m,n_ff,groups,form", [(40, 24832, 54, (2, 2, 1)), (24, 29568, 38, (1, 2, 1)), (58, 25600, 18, (2, 2, 1)), (21, 41856, 103, (1, 1, 1)), (59, 40832, 103, (2, 1, 1)), (24, 33024, 9, (1, 1, 1))])
+def test_gate_up_takes_no_pass_for_uneven_sets_of_the_mat_mats(m, n_ff, groups, form):
+    # where the mat-mats' sets of K differ by a group, the one launch keeps its own number of sets and one pass
+    p = q8_0.plan_gate_up_silu(m, n_ff, 128 * groups)
+    assert (p["activation_strips"], p["k_sets"], p["passes"]) == form
+    assert q8_0._lib.lib().nh_q8_0_gate_up_silu_workspace_bytes(m, n_ff, 128 * groups) == 0
