@@ -354,6 +354,11 @@ inline bool plan_gate_up_with(bool even, int64_t M, int64_t n_ff, int64_t K, gat
 				shares /= 2;
 			}
 			shares = shares > c.tile.ks ? shares : c.tile.ks;
+		} else if (g.kernel == MM_GEMM_TILE && shares > 2 * c.tile.ks && groups % shares != 0 && groups % c.tile.ks == 0) {
+			// Sixteen shares that differ by a group, from K over workgroups: eight, if the streaming kernel would have no more, so that a pair which is one launch
+			// with a K that sixteen divide is one here too.  ([2 x 768 x 11264] at 484 rows: 56 us, the three launches 49 through a workspace.)
+			const gemm_skinny_cut own = plan_gemm_skinny(M, n_ff, K);
+			shares					  = shares / 2 >= own.splits * own.waves ? shares / 2 : shares;
 		}
 		if (K > GATE_UP_SHORT_K) {
 			c.passes = shares / c.tile.ks;

@@ -161,3 +161,11 @@ def test_gate_up_takes_no_pass_for_uneven_sets_of_the_mat_mats(m, n_ff, groups, 
     p = q8_0.plan_gate_up_silu(m, n_ff, 128 * groups)
     assert (p["activation_strips"], p["k_sets"], p["passes"]) == form
     assert q8_0._lib.lib().nh_q8_0_gate_up_silu_workspace_bytes(m, n_ff, 128 * groups) == 0
+
+
+@pytest.mark.parametrize("m,n_ff,groups", [(484, 768, 88), (331, 1024, 92), (902, 384, 120), (176, 1792, 108)])
+def test_gate_up_stays_one_launch_where_the_mat_mats_have_sixteen_uneven_shares(m, n_ff, groups):
+    assert q8_0.plan_mul_mat(m, n_ff, 128 * groups)["k_splits"] == 4 and groups % 16
+    p = q8_0.plan_gate_up_silu(m, n_ff, 128 * groups)
+    assert (p["form"], p["k_sets"], p["passes"], p["tree"]) == ("tile", 4, 2, True)
+    assert q8_0._lib.lib().nh_q8_0_gate_up_silu_workspace_bytes(m, n_ff, 128 * groups) == 0
