@@ -369,7 +369,10 @@ inline bool plan_gate_up_with(bool even, int64_t M, int64_t n_ff, int64_t K, gat
 			// Passes of uneven sets: two, with the longest share at most a quarter over the average.  Fused / three launches, us: [2 x 11008 x 4224] at
 			// 48 rows (five groups for 4.1) 33.3 / 42.2, [2 x 6784 x 2816] at 50 rows (three for 2.75) 23.1 / 26.1, but [2 x 6912 x 3200] at 42 rows (four
 			// for 3.1) 27.5 / 26.3, [2 x 6400 x 2304] at 58 rows (three for 2.25) 23.3 / 21.9, and in four passes [2 x 5504 x 2176] at 140 rows 40.7 / 36.8.
-			if (c.passes > 1 && groups % c.tile.ks != 0 && (c.passes > 2 || 4 * ((groups + shares - 1) / shares * shares) > 5 * groups)) {
+			// And with more than 64 rows a workgroup on more than half the CUs: over 630 random shapes the three launches take 1.09 to 1.7 times as long there, and
+			// 0.6 to 1.25 times (mean 0.98) with up to 128 workgroups ([2 x 4096 x 5504] at 67 rows 35.8 / 30.6).  Of up to 64 rows with 70 to 128: 0.91 to 1.24, mean 1.06.
+			const int64_t wgs = int64_t{ c.tile.grid_x } * c.tile.grid_y;
+			if (c.passes > 1 && groups % c.tile.ks != 0 && (c.passes > 2 || 4 * ((groups + shares - 1) / shares * shares) > 5 * groups || (c.tile.grid_y > 1 && wgs <= 128))) {
 				return false;
 			}
 		}

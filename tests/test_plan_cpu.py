@@ -169,3 +169,9 @@ def test_gate_up_stays_one_launch_where_the_mat_mats_have_sixteen_uneven_shares(
     p = q8_0.plan_gate_up_silu(m, n_ff, 128 * groups)
     assert (p["form"], p["k_sets"], p["passes"], p["tree"]) == ("tile", 4, 2, True)
     assert q8_0._lib.lib().nh_q8_0_gate_up_silu_workspace_bytes(m, n_ff, 128 * groups) == 0
+
+
+@pytest.mark.parametrize("m,n_ff,groups,form", [(67, 4096, 43, "three_launches"), (254, 2048, 114, "three_launches"), (131, 1536, 27, "three_launches"), (126, 4224, 43, "tile"), (354, 1536, 35, "tile"), (48, 5504, 33, "tile")])
+def test_uneven_passes_of_gate_up_need_more_than_half_the_cus(m, n_ff, groups, form):
+    p = q8_0.plan_gate_up_silu(m, n_ff, 128 * groups)
+    assert p["form"] == form and (form != "tile" or p["passes"] == 2)
