@@ -366,8 +366,9 @@ inline bool plan_gate_up_with(bool even, int64_t M, int64_t n_ff, int64_t K, gat
 			if (c.passes > 1 && (c.tile.ks == 1 || c.passes > (c.tile.ks == 4 ? 2 : 4))) {
 				return false;
 			}
-			// Passes of uneven sets: two, with the longest share at most a quarter over the average.  Fused / three launches, us: [2 x 11008 x 4224] at
-			// 48 rows (five groups for 4.1) 33.3 / 42.2, [2 x 6784 x 2816] at 50 rows (three for 2.75) 23.1 / 26.1, but [2 x 6912 x 3200] at 42 rows (four
+			// Passes of sets that K does not divide over: two, with the longest share at most a quarter over the average.  (Sets that do divide K have had their passes
+			// before and keep them, also where the shares of all passes differ: two sets in four, [2 x 9216 x 2304] at 58 rows, three groups for 2.25, 28.4 / 29.1.)
+			// Fused / three launches, us: [2 x 11008 x 4224] at 48 rows (five groups for 4.1) 33.3 / 42.2, [2 x 6784 x 2816] at 50 rows (three for 2.75) 23.1 / 26.1, but [2 x 6912 x 3200] at 42 rows (four
 			// for 3.1) 27.5 / 26.3, [2 x 6400 x 2304] at 58 rows (three for 2.25) 23.3 / 21.9, and in four passes [2 x 5504 x 2176] at 140 rows 40.7 / 36.8.
 			// And with more than 64 rows a workgroup on more than half the CUs: over 630 random shapes the three launches take 1.09 to 1.7 times as long there, and
 			// 0.6 to 1.25 times (mean 0.98) with up to 128 workgroups ([2 x 4096 x 5504] at 67 rows 35.8 / 30.6).  Of up to 64 rows with 70 to 128: 0.91 to 1.24, mean 1.06.
