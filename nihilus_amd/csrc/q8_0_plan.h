@@ -45,10 +45,10 @@ inline gemm_tile_cut plan_gemm_tile(int64_t M, int64_t N, int64_t K, bool stream
 	c.tm	 = m_strips >= 2 ? 2 : 1;
 	c.grid_x = static_cast<unsigned>((n_strips + 3) / 4);
 	c.grid_y = static_cast<unsigned>((m_strips + c.tm - 1) / c.tm);
-	// K sets until every SIMD has four waves, while each keeps four groups.  K need not divide: the sets' shares differ by a group then.  Measured,
-	// us, with as many sets as divide / this: [4096 x 4224] at 350 / 512 rows 43.5 / 25.0 and 43.7 / 28.2, [4096 x 11136] 107.7 / 54.9 and 107.9 /
-	// 64.5, [4096 x 4352] (two sets / four) at 512 28.9 / 28.3, [2560 x 2688] at 512 28.5 / 18.4, [28672 x 3200] at 60 / 30 rows 36.7 / 26.9
-	// and 27.9 / 21.7
+	// K sets until every SIMD has four waves, while each keeps four groups.  K need not divide: the sets' shares differ by a group then (a mat-mat of its
+	// own takes fewer where that does not pay, gemm_tile_mat_mat).  Measured, us, with as many sets as divide / this: [4096 x 4224] at 350 / 512 rows
+	// 43.5 / 25.0 and 43.7 / 28.2, [4096 x 11136] 107.7 / 54.9 and 107.9 / 64.5, [2560 x 2688] at 512 28.5 / 18.4, [28672 x 3200] at 60 / 30 rows
+	// 36.7 / 26.9 and 27.9 / 21.7
 	c.ks	 = 1;
 	while (c.ks < 4 && static_cast<int64_t>(c.grid_x) * c.grid_y * 4 * c.ks * 2 <= 4096 && groups / (c.ks * 2) >= 4) {
 		c.ks *= 2;
@@ -60,6 +60,23 @@ inline gemm_tile_cut plan_gemm_tile(int64_t M, int64_t N, int64_t K, bool stream
 			wgs * c.kz * 2 * c.tm * 4096 <= GEMM_SPLIT_SCRATCH_FLOATS && wgs <= GEMM_SPLIT_MAX_UNITS) {
 			c.kz *= 2;
 		}
+	}
+	return c;
+}
+
+// The tile kernel's cut for a mat-mat of its own (K not over workgroups).  Uneven sets walk as many trips as the longest, so short ones multiply up to a tenth
+// more for nothing, and behind two sets, or more workgroups than CUs, there are two waves on a SIMD already.  Measured, us:
+//   two even sets / four uneven   [4096 x 2304] at 512 rows 16.1 / 17.1, [8064 x 2816] at 200 22.9 / 25.5, [2048 x 3328] at 1000 22.8 / 23.1; of streamed weights
+//                                 [24832 x 3840] at 24 / 64 rows 27.0 / 34.5 and 32.0 / 38.1, [32000 x 4864] 29.4 / 30.5 and 38.4 / 39.8; but
+//                                 [4096 x 6912] at 512 43.2 / 40.9, [24832 x 5376] at 64 38.2 / 34.9.  One strip [32000 x 6400] at 24 38.4 / 40.0
+//   one set / two uneven          [60032 x 1152] at 64 rows 21.4 / 25.3, [16640 x 1920] at 117 25.3 / 26.9, [28672 x 2176] at 117 31.2 / 30.3; one strip
+//                                 [40064 x 1152] at 24 12.7 / 14.6, [60032 x 7296] 72.8 / 74.4
+inline gemm_tile_cut gemm_tile_mat_mat(gemm_tile_cut c, int groups) {
+	if (c.ks == 4 && c.kz == 1 && groups % 4 == 2 && (c.tm == 1 || groups < 40)) {
+		c.ks = 2;
+	}
+	if (c.ks == 2 && groups % 2 != 0 && static_cast<int64_t>(c.grid_x) * c.grid_y > 256 && (c.tm == 1 || groups < 24)) {
+		c.ks = 1;
 	}
 	return c;
 }
@@ -264,7 +281,7 @@ inline gemm_plan plan_gemm(int64_t M, int64_t N, int64_t K) {
 	}
 	if (stream_tile) {
 		p.kernel = MM_GEMM_TILE_STREAM;
-		p.tile	 = plan_gemm_tile(M, N, K, true);
+		p.tile	 = gemm_tile_mat_mat(plan_gemm_tile(M, N, K, true), static_cast<int>(K / GROUP_K));
 	} else if (M > GEMM_SKINNY_MAX_M && tile_workgroups <= 256 && plan_gemm_tile_split(M, N, K, &p.tile, &p.skinny)) {
 		p.kernel = MM_GEMM_TILE;
 	} else if (M <= GEMM_SKINNY_MAX_M || tile_workgroups <= 256) {
@@ -276,7 +293,7 @@ inline gemm_plan plan_gemm(int64_t M, int64_t N, int64_t K) {
 		p.rows = gemm_rows_suits(M, N, K) && gemm_rows_fits(M, N, p.skinny);
 	} else {
 		p.kernel = MM_GEMM_TILE;
-		p.tile	 = plan_gemm_tile(M, N, K, false);
+		p.tile	 = gemm_tile_mat_mat(plan_gemm_tile(M, N, K, false), static_cast<int>(K / GROUP_K));
 	}
 	return p;
 }

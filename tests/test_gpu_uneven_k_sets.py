@@ -15,7 +15,7 @@ def _gemm(oracle, w, aq, m, n, k):  # the threaded checker takes block counts th
 
 # (m, n, groups, kernel, K sets, workgroups along K): two and four sets, one and two activation strips, streamed weights or not, ragged rows and
 # columns, the fewest groups that are cut, and one, two and three sets with the longer share; then K over two and four workgroups as well
-SHAPES = [(700, 1536, 13, "gemm_tile", 2, 1), (700, 1500, 17, "gemm_tile", 4, 1), (701, 1536, 18, "gemm_tile", 4, 1), (300, 3400, 19, "gemm_tile", 4, 1), (24, 24577, 9, "gemm_tile_stream", 2, 1),
+SHAPES = [(700, 1536, 13, "gemm_tile", 2, 1), (700, 1500, 17, "gemm_tile", 4, 1), (701, 1536, 42, "gemm_tile", 4, 1), (300, 3400, 19, "gemm_tile", 4, 1), (24, 24577, 9, "gemm_tile_stream", 2, 1),
           (40, 24577, 17, "gemm_tile_stream", 4, 1), (200, 4090, 47, "gemm_tile", 4, 2), (120, 3840, 104 + 1, "gemm_tile", 4, 4)]
 
 

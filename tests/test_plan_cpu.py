@@ -175,3 +175,11 @@ def test_gate_up_stays_one_launch_where_the_mat_mats_have_sixteen_uneven_shares(
 def test_uneven_passes_of_gate_up_need_more_than_half_the_cus(m, n_ff, groups, form):
     p = q8_0.plan_gate_up_silu(m, n_ff, 128 * groups)
     assert p["form"] == form and (form != "tile" or p["passes"] == 2)
+
+
+@pytest.mark.parametrize("m,n,groups,sets", [(701, 1536, 18, 2), (512, 4096, 38, 2), (512, 4096, 42, 4), (512, 4096, 17, 4), (24, 24832, 30, 2), (64, 24832, 30, 2), (64, 24832, 42, 4), (24, 24832, 58, 2),
+                                             (24, 24832, 33, 4), (64, 60032, 9, 1), (117, 16640, 15, 1), (117, 28672, 25, 2), (24, 60032, 57, 1), (24, 60032, 56, 2)])
+def test_short_uneven_sets_of_the_mat_mats(m, n, groups, sets):
+    # two even sets stay two while four uneven ones would be short; with more workgroups than CUs one set stays one
+    p = q8_0.plan_mul_mat(m, n, 128 * groups)
+    assert p["kernel"].startswith("gemm_tile") and (p["k_sets"], p["k_splits"]) == (sets, 1)
