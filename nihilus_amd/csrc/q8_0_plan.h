@@ -155,6 +155,9 @@ inline gemm_skinny_cut plan_gemm_skinny(int64_t M, int64_t N, int64_t K) {
 // K need not divide, if the longest share is at most a tenth over the average: [4096 x 11136] at 200 rows 47.5 / 36.1 (the streaming kernel / this),
 // [7936 x 28032] at 233 rows 271 / 172, [4992 x 13184] at 121 rows 55.5 / 39.6, [6784 x 6784] at 125 rows (seven groups where 6.6 would do)
 // 32.6 / 29.1; but [5376 x 5376] at 144 rows (six for 5.25) 25.6 / 28.4.
+// Such a K also needs its workgroups to fit the CUs once or fill them nearly twice, and not the sixteen waves that the streaming kernel has for
+// 129 to 255 units: over 430 random shapes the streaming kernel takes 1.0 to 2.0 times as long then (two of 306 at 0.95 and 0.97), with 257 to 383
+// workgroups 0.78 to 1.08 times ([9580 x 6016] at 65 rows 35.9 / 42.7), with sixteen waves 0.76 to 1.2 times ([1380 x 11264] at 159 rows 16.7 / 22.0).
 //
 // A captured call, and one that finds the hand-off scratch in use on another stream, runs on the streaming kernel with as many shares of K in
 // one workgroup of eight or sixteen waves (`twin`), which add to the same bits and need no scratch: hence two or four workgroups along
@@ -174,6 +177,9 @@ inline bool plan_gemm_tile_split(int64_t M, int64_t N, int64_t K, gemm_tile_cut*
 		c.kz *= 2;
 	}
 	if (c.tm != 2 || c.kz == 1 || wgs * c.kz <= 128 || c.ks * c.kz < own.splits * own.waves) {
+		return false;
+	}
+	if (groups % (c.ks * c.kz) != 0 && ((wgs * c.kz > 256 && wgs * c.kz < 384) || own.waves != SK_WAVES)) {
 		return false;
 	}
 	*cut  = c;

@@ -183,3 +183,10 @@ def test_short_uneven_sets_of_the_mat_mats(m, n, groups, sets):
     # two even sets stay two while four uneven ones would be short; with more workgroups than CUs one set stays one
     p = q8_0.plan_mul_mat(m, n, 128 * groups)
     assert p["kernel"].startswith("gemm_tile") and (p["k_sets"], p["k_splits"]) == (sets, 1)
+
+
+@pytest.mark.parametrize("m,n,groups,splits", [(200, 4096, 87, 2), (120, 3840, 105, 4), (74, 9712, 46, 0), (358, 1636, 241, 0), (330, 1389, 242, 0), (86, 6255, 252, 4), (159, 1380, 88, 0), (96, 2139, 91, 0), (512, 4096, 33, 1)])
+def test_uneven_k_over_workgroups_has_no_second_round_of_few(m, n, groups, splits):
+    # more than 64 rows, K that the shares do not divide: over workgroups (splits) while they fit the CUs once or fill them nearly twice; else the streaming kernel (0)
+    p = q8_0.plan_mul_mat(m, n, 128 * groups)
+    assert (p["kernel"], p["k_splits"]) == ("gemm_tile", splits) if splits else p["kernel"] == "gemm_skinny"
