@@ -163,8 +163,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_kernel(const uint8_t* __res
 //     in the int8 MFMA's own accumulator layout: no conversion, broadcast or cross-lane move of a scale, ever;
 //   * only the operand that is shared goes through LDS.  A workgroup is four waves; wave w owns weight strip
 //     4*blockIdx.x + w and loads its tiles straight from global memory into registers (one coalesced 16-byte-per-lane
-//     load per tile, already an MFMA operand, into the registers of the tile it follows as soon as the last MFMA on that one is
-//     issued: half a 128-quant group and more ahead of use, in 16 registers and not 32); all four waves share the same
+//     load per tile, already an MFMA operand, a whole 128-quant group ahead of use); all four waves share the same
 //     TM activation strips, copied global -> LDS one group ahead (double-buffered, one barrier per group, the copy
 //     spread over the four waves) and read back as conflict-free 16-byte-per-lane operand images plus one 8-byte read of a
 //     group's four scales per strip;
@@ -172,7 +171,7 @@ __global__ __launch_bounds__(GEMM_THREADS) void gemm_kernel(const uint8_t* __res
 //     global_load with a scalar base): no 64-bit address arithmetic on the VALU, which is the pipe the fold saturates,
 //     and ~10 fewer registers than per-lane pointers (the difference between spilling and not at two activation strips);
 //   * latency is hidden by occupancy, not by a software pipeline: one result-register set per tile keeps the kernel
-//     at <= 128 VGPRs (112), four workgroups per CU, four waves per SIMD.  (A two-result-set, software-pipelined variant
+//     at <= 128 VGPRs, four workgroups per CU, four waves per SIMD.  (A two-result-set, software-pipelined variant
 //     at two waves per SIMD measured 8 % slower: with so few waves the SIMD falls back to the lone-wave issue rate
 //     whenever one of them waits.)
 // a 64-bit offset that the compiler may keep in scalar registers (it is the same for every lane of the wave)
@@ -338,15 +337,9 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 	// the same loads as fetch_a and fetch_w, which the prologue issues in one go
 	constexpr int PIECES = TM + 2 + GROUP_BLOCKS;
 	constexpr int UNITS	 = GROUP_BLOCKS * TM; // of a trip: (block t, activation strip i) in the order u = TM * t + i
-	// IN_PLACE: a weight tile goes to the registers of the one it replaces.  In PASSES there are two sets of registers instead, taken in turn:
-	// with sets of half the trips, [2 x 14336 x 4096] at 117 rows takes 57.2 us with two and 60.1 in place, on the slower of the cards measured.
-	constexpr bool IN_PLACE = !PASSES;
-	// the unit in front of whose arithmetic a piece is requested (UNITS: behind the last one): spread over the trip, in place not before the last
-	// unit that multiplies the tile it replaces (every piece as early as that allows instead: at 512 rows 0.2 % faster, at 117 0.3 % slower)
-	constexpr auto piece_unit = [](int p) {
-		const int spread = (UNITS * (p + 1) + PIECES - 1) / PIECES - 1, free = !IN_PLACE || p < TM + 2 ? 0 : TM * (p - TM - 2 + 1);
-		return spread > free ? spread : free;
-	};
+	// (The next trip's weights go to a second set of registers.  Into those of the tile each follows, once its last MFMA is issued, was 112 registers instead of 126
+	// and no faster: [14336 x 4096] at 3001 rows 426.1 us against 424.3, [4096 x 14336] at 512 rows 78.5 / 78.1, [128256 x 4096] at 24 rows
+	// 93.2 / 91.4, gate / up [2 x 41856 x 13184] at 21 rows 195.4 / 190.6; launches in random order.)
 	auto fetch_piece = [&](int p, int in_pass, a_regs& ra, w_regs& rw) {
 		const int g = g0 + in_pass;
 		asm volatile("" : "+v"(lane16)); // in place: a copy for every load was one VALU instruction each
@@ -368,7 +361,7 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 	}
 	int last = live - 1;
 
-	w_regs wa, wb; // this trip's weights and, unless IN_PLACE, the next one's
+	w_regs wa, wb;
 	a_regs pre;
 	fetch_a(0, pre);
 	fetch_w(0, wa);
@@ -410,10 +403,8 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 			}
 			__builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-			for (int pc = 0; pc < PIECES; ++pc) {
-				if (piece_unit(pc) == u) {
-					fetch_piece(pc, gn, pre, nxt);
-				}
+			for (int pc = u * PIECES / UNITS; pc < (u + 1) * PIECES / UNITS; ++pc) {
+				fetch_piece(pc, gn, pre, nxt);
 			}
 			__builtin_amdgcn_sched_barrier(0);
 			const v2u w_slot  = scale_slot(wd, t), a_slot = scale_slot(a_sc[i], t);
@@ -440,22 +431,15 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 			__builtin_amdgcn_sched_barrier(0);
 			a_cur = a_nxt;
 		}
-#pragma unroll
-		for (int pc = 0; pc < PIECES; ++pc) {
-			if (piece_unit(pc) == UNITS) {
-				fetch_piece(pc, gn, pre, nxt);
-			}
-		}
-		__builtin_amdgcn_sched_barrier(0);
 		stash_a((g + 1) & 1, pre);
 		__syncthreads();
 	};
 	constexpr int PER = 16 / KS; // values of a lane's 16 per strip that a K set finishes: registers PER * kr .. PER * kr + PER - 1
 	float mine[TM * PER]; // this wave's share of the workgroup's tile (SPLIT: of its part of K)
 	for (int pass = 0;; ++pass) {
-		for (int g = 0; g < g_len; g += IN_PLACE ? 1 : 2) {
-			trip(g, wa, IN_PLACE ? wa : wb);
-			if (!IN_PLACE && g + 1 < g_len) {
+		for (int g = 0; g < g_len; g += 2) {
+			trip(g, wa, wb);
+			if (g + 1 < g_len) {
 				trip(g + 1, wb, wa);
 			}
 		}
@@ -619,7 +603,7 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 					for (int i = 0; i < TM; ++i) {
 						acc[i] = v16f{ 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0 };
 					}
-					if (!IN_PLACE && (g_len & 1)) {
+					if (g_len & 1) {
 						wa = wb;
 					}
 					stash_a(0, pre);
