@@ -4,6 +4,8 @@ from __future__ import annotations
 import os
 import shutil
 import subprocess
+import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
@@ -30,9 +32,10 @@ HIPCC_FLAGS = [
     # result parked in an accumulation register would cost one extra copy instruction per value (doubling the VALU work)
     "-mllvm", "-amdgpu-mfma-vgpr-form",
 ]
-# The wrappers' native calls, a CPython module against torch's own headers and libraries (which are loaded with torch, before it).
+# The wrappers' native calls, a CPython module against torch's own headers and libraries (which are loaded with torch, before it).  Not part of
+# the library, whose other users need no torch, and the wrappers work without it.
 CALLS_SOURCE = "py_calls.cpp"
-CALLS_PATH = os.path.join(PKG_DIR, "_calls.so")
+CALLS_PATH = os.path.join(PKG_DIR, "_calls" + sysconfig.get_config_var("EXT_SUFFIX"))
 # the host pass does not know the packed-fp32 feature name and says so once per source: not an error
 NOISE = "is not a recognized feature for this target"
 
@@ -82,7 +85,6 @@ def build_library(verbose: bool = False, extra_flags: list[str] | None = None, i
         notes = list(pool.map(compile_one, SOURCES))
     objs = [os.path.join(OBJ_DIR, os.path.splitext(s)[0] + ".o") for s in SOURCES]
     notes.append(_run([hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB_PATH, *objs]))
-    notes.append(build_calls(include, incremental))
     if verbose:
         text = "\n".join(n for n in notes if n.strip())
         if text:
@@ -90,26 +92,38 @@ def build_library(verbose: bool = False, extra_flags: list[str] | None = None, i
     return LIB_PATH
 
 
-def build_calls(include: str, incremental: bool = False) -> str:
-    """Compile the CPython module behind the wrappers of nihilus_amd/q8_0.py (host code only), linked against the library beside it."""
-    import sysconfig
-
+def calls_tag() -> str:
+    """What the module of the native calls is built for: it reads torch's and CPython's structures by their layout, so by no other one."""
     import torch
 
+    return f"torch {torch.__version__} {sys.implementation.cache_tag}"
+
+
+def build_calls(incremental: bool = False) -> str:
+    """Compile the CPython module behind the wrappers of nihilus_amd/q8_0.py (host code only), linked against the library beside it."""
+    tag = calls_tag()
+    import torch
+
+    include = os.path.join(os.path.dirname(PKG_DIR), "include")
     path = os.path.join(CSRC, CALLS_SOURCE)
     if incremental and os.path.exists(CALLS_PATH) and os.path.getmtime(CALLS_PATH) > max(os.path.getmtime(path), _newest_header_mtime(include)):
-        return ""
+        with open(CALLS_PATH, "rb") as f:
+            if tag.encode() + b"\0" in f.read():
+                return ""
+    os.makedirs(OBJ_DIR, exist_ok=True)
     root = os.path.dirname(torch.__file__)
     rocm = os.path.dirname(os.path.dirname(os.path.realpath(hipcc())))
     system = [os.path.join(rocm, "include"), os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"), sysconfig.get_paths()["include"]]
     obj = os.path.join(OBJ_DIR, "py_calls.o")
-    note = _run([hipcc(), "-x", "c++", "-O2", "-std=c++20", "-fPIC", "-Wall", "-Wextra", "-DUSE_ROCM=1", "-D__HIP_PLATFORM_AMD__=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I", include,
-                 *(x for d in system for x in ("-isystem", d)), "-c", path, "-o", obj])
+    note = _run([hipcc(), "-x", "c++", "-O2", "-std=c++20", "-fPIC", "-Wall", "-Wextra", "-DUSE_ROCM=1", "-D__HIP_PLATFORM_AMD__=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+                 f'-DNH_BUILT_FOR="{tag}"', "-I", include, *(x for d in system for x in ("-isystem", d)), "-c", path, "-o", obj])
     return note + _run([hipcc(), "-shared", "-fPIC", "-o", CALLS_PATH, obj, "-L", os.path.join(root, "lib"), "-L", PKG_DIR, "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip", f"-l:{LIB_NAME}",
                         "-Wl,-rpath,$ORIGIN"])
 
 
 if __name__ == "__main__":
-    import sys
-
     print(build_library(verbose=True, incremental="--incremental" in sys.argv))
+    try:
+        print(build_calls("--incremental" in sys.argv) or CALLS_PATH)
+    except Exception as e:  # noqa: BLE001 -- no torch, or headers that do not fit: the library is whole, the wrappers take the Python way
+        print(f"the wrappers' native calls were not built: {e}", file=sys.stderr)

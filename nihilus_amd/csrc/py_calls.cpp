@@ -206,5 +206,9 @@ PyModuleDef module = { PyModuleDef_HEAD_INIT, "_calls", nullptr, -1, methods, nu
 } // namespace
 
 PyMODINIT_FUNC PyInit__calls() {
-	return PyModule_Create(&module);
+	PyObject* m = PyModule_Create(&module);
+	if (m && PyModule_AddStringConstant(m, "built_for", NH_BUILT_FOR) != 0) { // nihilus_amd/build.py
+		Py_CLEAR(m);
+	}
+	return m;
 }

@@ -11,13 +11,19 @@ from __future__ import annotations
 import torch
 
 from . import _lib
+from .build import calls_tag
 
 # The calls of a step on several rows as native functions (csrc/py_calls.cpp).  They return the result, a status, or None for whatever is not
-# a plain call, which then goes the way below.  Without the module (a torch that it was not built against) every call goes that way.
+# a plain call, which then goes the way below.  Without the module, or with one for another torch or CPython, every call goes that way.
+def _fitting(module):
+    return module if getattr(module, "built_for", None) == calls_tag() else None
+
+
 try:
     from . import _calls
 except ImportError:
     _calls = None
+_calls = _fitting(_calls)
 
 QK = 32
 BLOCK_BYTES = 34

@@ -3,15 +3,48 @@
 On the CPU: whatever is not a plain call on GPU tensors is left to the Python way.  On the GPU: the same bits either way over the forms the
 wrappers take, and the same errors for the ones they refuse.
 """
+import sys
+import types
+
 import numpy as np
 import pytest
 import torch
 
-from nihilus_amd import q8_0
+from nihilus_amd import build, q8_0
 
 
 def test_the_module_is_built():
     assert q8_0._calls is not None
+
+
+def test_the_module_is_for_this_torch_and_python():
+    tag = build.calls_tag()
+    assert q8_0._calls.built_for == tag and torch.__version__ in tag
+    assert q8_0._fitting(q8_0._calls) is q8_0._calls
+    for other in None, types.SimpleNamespace(), types.SimpleNamespace(built_for=tag.replace(torch.__version__, "0.0.1")):
+        assert q8_0._fitting(other) is None
+
+
+def test_the_library_is_built_without_torch(monkeypatch):
+    ran = []
+    monkeypatch.setattr(build, "_run", lambda cmd: ran.append(" ".join(cmd)) or "")
+    monkeypatch.setitem(sys.modules, "torch", None)  # import torch raises ImportError
+    build.build_library()
+    assert len(ran) == len(build.SOURCES) + 1 and not any(build.CALLS_SOURCE in c for c in ran)
+    with pytest.raises(ImportError):
+        build.build_calls()
+
+
+def test_an_old_module_is_built_again_for_another_torch(monkeypatch):
+    ran = []
+    monkeypatch.setattr(build, "_run", lambda cmd: ran.append(cmd) or "")
+    monkeypatch.setattr(build, "_newest_header_mtime", lambda include: 0.0)
+    monkeypatch.setattr(build.os.path, "getmtime", lambda path: 2.0 if path == build.CALLS_PATH else 1.0)
+    build.build_calls(incremental=True)
+    assert not ran
+    monkeypatch.setattr(build, "calls_tag", lambda: "torch 0.0.1 cpython-310")
+    build.build_calls(incremental=True)
+    assert len(ran) == 2
 
 
 def test_what_is_no_plain_call_is_left_to_python():
