@@ -142,6 +142,27 @@ def test_same_bits_either_way(q8, oracle, monkeypatch, m):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("m", [1, 5, 40])
+def test_plain_calls_are_native(q8, monkeypatch, m):
+    # every function takes its plain call itself: with one that left it to Python, the comparison above would be of Python with itself
+    n, k = 384, 1024
+    w = q8.tile(q8.fill_weight_blocks(3, n, k), n, k)
+    x, add, norm = q8.fill_activations(4, m * k).reshape(m, k), q8.fill_activations(5, m * n).reshape(m, n), q8.fill_activations(6, k)
+    a = q8.quantize_row_q8_0(x, tiled=True)
+    calls = q8._calls
+    for out in (calls.mul_mat(w, x, n, k, None), calls.mul_mat(w, x, n, k, add), calls.gemm(w, a, m, n, k, None), calls.gemm(w, a, m, n, k, add), calls.rms_norm_quantize(x, norm, 1e-5), calls.gate_up_silu(w, w, a, m, n, k)):
+        assert isinstance(out, torch.Tensor)
+
+    def refuse(*args):
+        raise AssertionError("the Python way")
+
+    monkeypatch.setattr(q8_0._lib, "lib", refuse)  # ... and the wrappers hand it over
+    for call in (lambda: q8.mul_mat(w, x, n, k), lambda: q8.mul_mat(w, x, n, k, residual=add), lambda: q8.gemm(w, a, m, n, k, tiled=True), lambda: q8.gemm_residual(w, a, add, m, n, k),
+                 lambda: q8.rms_norm_quantize(x, norm, 1e-5, tiled=True), lambda: q8.gate_up_silu(w, w, a, m, n, k)):
+        assert isinstance(call(), torch.Tensor)
+
+
+@pytest.mark.gpu
 def test_same_errors_either_way(q8, monkeypatch):
     n, k, m = 64, 256, 5
     w = q8.tile(q8.fill_weight_blocks(3, n, k), n, k)
