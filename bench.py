@@ -614,7 +614,7 @@ def side_workload(kind: str, steps: int, warmup: int) -> dict:
                 torch.cuda.synchronize()
                 sec = (time.perf_counter() - t0) / steps
                 wbytes = n * (k // 32) * 34
-                rows.append({"M": m, "N": n, "K": k, "kernel": _kernel_name(q8_0.plan_mul_mat(m, n, k)), "us": round(sec * 1e6, 2), "weight_GBs": round(wbytes / sec / 1e9, 1), "TOPs": round(2.0 * m * n * k / sec / 1e12, 2),
+                rows.append({"M": m, "N": n, "K": k, "kernel": _kernel_name(q8_0.plan_mul_mat(m, n, k, own_workspace=True)), "us": round(sec * 1e6, 2), "weight_GBs": round(wbytes / sec / 1e9, 1), "TOPs": round(2.0 * m * n * k / sec / 1e12, 2),
                              "pct_hbm": round(100 * wbytes / sec / 1e9 / HBM_PEAK_GBS, 1), "pct_mfma": round(100 * 2.0 * m * n * k / sec / 1e12 / INT8_MFMA_PEAK_TOPS, 2)})
         return {"metric": "Q8_0 mul_mat (quantize + mat-vec / mat-mat) time against M", "unit": "us", "n_gpus": 1, "steps": steps, "warmup": warmup, "higher_is_better": False,
                 "dtype": "int8 x int8 -> int32 block sums, fp32 scale-accumulate", "data": "synthetic",
@@ -652,7 +652,7 @@ def side_workload(kind: str, steps: int, warmup: int) -> dict:
                     fn()
                 torch.cuda.synchronize()
                 sec = (time.perf_counter() - t0) / steps
-                rows.append({"projection": name, "M": m, "N": n, "K": k, "kernel": _kernel_name(q8_0.plan_mul_mat(m, n, k)), "us": round(sec * 1e6, 2), "weight_GBs": round(wbytes / sec / 1e9, 1),
+                rows.append({"projection": name, "M": m, "N": n, "K": k, "kernel": _kernel_name(q8_0.plan_mul_mat(m, n, k, own_workspace=True)), "us": round(sec * 1e6, 2), "weight_GBs": round(wbytes / sec / 1e9, 1),
                              "pct_hbm": round(100 * wbytes / sec / 1e9 / HBM_PEAK_GBS, 1), "TOPs": round(2.0 * m * n * k / sec / 1e12, 2)})
             del ws
             torch.cuda.empty_cache()

@@ -384,7 +384,8 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 		const uint8_t* stage = lds + (g & 1) * STAGE_BYTES;
 		asm volatile("" : "+v"(lane16));
 		const uint8_t* a_at = stage + lane16;
-		// the rows' scales of the group's four blocks, one 8-byte read per strip and trip (a half-word read per unit was eight)
+		// the rows' scales of the group's four blocks, one 8-byte read per strip and trip (a half-word read per unit was eight: [8192 x 8192] at 512 rows
+		// 94.4 -> 92.3 us, [4096 x 14336] at 117 rows 30.4 -> 29.4, one strip [128256 x 4096] at 24 rows 90.8 -> 91.8)
 		v2u a_sc[TM];
 #pragma unroll
 		for (int i = 0; i < TM; ++i) {

@@ -84,7 +84,7 @@ __device__ __forceinline__ void rows_chunk_n(const uint8_t* __restrict__ w_strip
 		}
 	}
 	__builtin_amdgcn_sched_barrier(0);
-	// ---- 3. the scales, [block][row]: as fp32, or (32 rows) as the fp16 bits that the scale MFMA takes ----
+	// ---- 3. the scales, [block][row]: as fp32, or (24 and 32 rows) as the fp16 bits that the scale MFMA takes ----
 	if (lane / R < CNT) {
 		if constexpr (rows_scale_mfma<R>) {
 			uint32_t* out = reinterpret_cast<uint32_t*>(a_scales) + (lane / R) * GROUP_BLOCKS * R + sr;

@@ -272,7 +272,8 @@ inline gemm_plan plan_gemm(int64_t M, int64_t N, int64_t K) {
 			// 24.1 / 19.0 / 18.4; [14336 x 4096] M = 64: 20.5 against 22.9 (M = 32: 16.8 against 16.2, left where it was);
 			// [4096 x 14336] M = 64: 24.0 against 26.2 (M = 16: 19.8 against 18.0); [1024 x 8192] M = 64: 13.5 against 11.7;
 			// [4096 x 4096] M = 64: 13.6 against 10.3.  So: two row strips from 48 Mi weights on, one (16 rows or more) from
-			// 64 Mi.  The rule only holds where that K split is actually possible: a shape whose groups do not divide (kz
+			// 64 Mi (17 to 32 rows of those mostly go on to the rows kernel, which this line was drawn before:
+			// gemm_rows_instead_of_tile).  The rule only holds where that K split is actually possible: a shape whose groups do not divide (kz
 			// stays 1) would run the tile kernel on 32 to 191 workgroups, the form measured slower than the streaming kernel
 			// ([14336 x 4096] at M = 64 unsplit: 30 against 23 us), and stays with the streaming kernel.
 			const gemm_tile_cut tile = plan_gemm_tile(M, N, K, true);

@@ -1,7 +1,7 @@
 """Host-side wrappers of the Q8_0 path for callers that hold torch tensors.
 
 torch is used for device memory and streams only; every operation below is one call through the C ABI
-(``include/nihilus_amd/q8_0_abi.h``).  Names follow the reference: ``quantize_row_q8_0``
+(``include/nihilus_amd/q8_0_abi.h``), by ctypes or by the native functions of ``csrc/py_calls.cpp``.  Names follow the reference: ``quantize_row_q8_0``
 (cpu/avx_2.hpp:4439-4489), ``mul_mat`` (kernel_types::mul_mat, cpu/avx_2.hpp:1296-1444).  Q8_0 data is a
 ``torch.uint8`` tensor: "blocks" = rows of packed 34-byte block_q8_0, "tiled" = the device layout
 described in the ABI header.

@@ -34,8 +34,9 @@ def test_mat_vec_cut_of_the_decode_shapes():
 
 
 def test_four_to_sixteen_rows_on_small_matrices_take_the_mfma_mat_vec():
-    # no quantize launch, no workspace: up to 16 rows on matrices of at most 40 MB, 4 rows up to 80 MB; beyond that the quantize launch
-    # and the MFMA kernels (every strip's workgroup quantizing the rows again would cost more than the launch)
+    # no quantize launch, nothing in the workspace: 4 rows on matrices of up to 80 MB, 5 to 16 rows up to 40 MB while every workgroup has a CU (all of
+    # them with a workspace of the caller's); beyond that the quantize launch and the MFMA kernels (every strip's workgroup quantizing the rows again
+    # would cost more than the launch)
     for n, k in (L8B["q_o"], L8B["k_v"], L70B["k_v"]):
         for m in (4, 5, 8, 9, 16):
             p = q8_0.plan_mul_mat(m, n, k)
