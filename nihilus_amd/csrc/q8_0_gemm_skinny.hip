@@ -19,7 +19,16 @@ namespace nh {
 typedef _Float16 sk_v4h __attribute__((ext_vector_type(4)));
 typedef float sk_v16f __attribute__((ext_vector_type(16)));
 
-template<int MS, int GC, int WAVES>
+// NT: past the caches, for weights that no other workgroup reads
+template<bool NT, typename T> __device__ __forceinline__ T load_weights(const T* p) {
+	if constexpr (NT) {
+		return __builtin_nontemporal_load(p);
+	} else {
+		return *p;
+	}
+}
+
+template<int MS, int GC, int WAVES, bool NT>
 __global__ __launch_bounds__(WAVES * 64, 4) void gemm_skinny_kernel(const uint8_t* __restrict__ W, const uint8_t* __restrict__ A, float* C, const float* R,
 	float* __restrict__ partials, unsigned* __restrict__ counters, int M, int N, int groups, int split_shift) {
 	__shared__ float red[MS * 16][WAVES][64];
@@ -62,9 +71,9 @@ __global__ __launch_bounds__(WAVES * 64, 4) void gemm_skinny_kernel(const uint8_
 		const uint8_t* macro = w_strip + static_cast<int64_t>(g) * MACRO_BYTES;
 #pragma unroll
 		for (int j = 0; j < GROUP_BLOCKS; ++j) {
-			b.q[j] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(macro + j * TILE_BYTES + 16 * lane));
+			b.q[j] = load_weights<NT>(reinterpret_cast<const v4i*>(macro + j * TILE_BYTES + 16 * lane));
 		}
-		b.d = __builtin_nontemporal_load(reinterpret_cast<const v2u*>(macro + MACRO_D_OFFSET + 8 * r));
+		b.d = load_weights<NT>(reinterpret_cast<const v2u*>(macro + MACRO_D_OFFSET + 8 * r));
 	};
 	// Activation rows beyond M are zero padding in the tiled operand.  Their lanes all read the strip's last row instead of
 	// their own (zeros as well, since a strip with any padding ends in it): one cache line per load instead of one per four
@@ -335,10 +344,16 @@ template<int MS> static hipError_t launch_skinny_t(int splits, int waves, const 
 		++shift;
 	}
 	const dim3 grid(static_cast<unsigned>(strips * splits), static_cast<unsigned>(m_groups)), block(static_cast<unsigned>(64 * waves));
+	// The groups of rows read the same weights: past the caches each would take them from memory again ([896 x 6400] at 316 rows 17.1 -> 11.4 us, [4319 x 4224]
+	// at 35 rows 13.9 -> 11.5, [4096 x 4096] at 200 rows 18.4 -> 16.8, [1024 x 4096] at 512 / 250 / 117 rows 10.6 -> 9.6, 7.3 -> 6.6, 7.1 -> 6.7).  Not with one
+	// group ([8192 x 4096] at 40 rows 12.3 as it is, 13.2 through the caches), nor with two whose workgroups are on one XCD (workgroups go to the eight in turn) at
+	// the same time: the second finds the first's lines on their way ([4096 x 4096] at 64 rows 8.1 / 8.25, at 117 rows the same).
+	const bool nt = m_groups == 1 || (m_groups == 2 && (strips * splits) % 8 == 0);
+	const auto launch = [&](auto kernel) { return launch_kernel(KIND_GEMM, kernel, grid, block, 0, s, w, a, C, R, sc.partials, sc.counters, m, n, groups, shift); };
 	if (waves == SK_WIDE_WAVES) {
-		return launch_kernel(KIND_GEMM, gemm_skinny_kernel<MS, 2, SK_WIDE_WAVES>, grid, block, 0, s, w, a, C, R, sc.partials, sc.counters, m, n, groups, shift);
+		return nt ? launch(gemm_skinny_kernel<MS, 2, SK_WIDE_WAVES, true>) : launch(gemm_skinny_kernel<MS, 2, SK_WIDE_WAVES, false>);
 	}
-	return launch_kernel(KIND_GEMM, gemm_skinny_kernel<MS, 2, SK_WAVES>, grid, block, 0, s, w, a, C, R, sc.partials, sc.counters, m, n, groups, shift);
+	return nt ? launch(gemm_skinny_kernel<MS, 2, SK_WAVES, true>) : launch(gemm_skinny_kernel<MS, 2, SK_WAVES, false>);
 }
 
 // cut: plan_gemm_skinny, or the stand-in for a tile kernel's (q8_0_plan.h)
