@@ -32,6 +32,13 @@ HIPCC_FLAGS = [
     # result parked in an accumulation register would cost one extra copy instruction per value (doubling the VALU work)
     "-mllvm", "-amdgpu-mfma-vgpr-form",
 ]
+# The first six dwords of a kernel's arguments (three pointers) arrive in scalar registers with the wave instead of being read from memory by it, a miss of
+# the scalar cache in front of the first address: norm + quantize of 4 rows 3.02 -> 2.76 us, [1024 x 4096] at 4 rows 4.17 -> 3.98, mul_mat of 16 rows
+# [4096 x 4096] 10.2 -> 9.7, of 2 and 4 rows 6.25 -> 6.07 and 6.12, of 5 rows the same.  (Ten and sixteen dwords: the same, but 5 and 8 rows 0.6 % slower.)
+PRELOAD_FLAGS = ["-mllvm", "-amdgpu-kernarg-preload-count=6"]
+# not where a launch is many short waves, each of which then starts later: embedding rows of 4 tokens 1.83 us without, 1.99 with; [14336 x 4096] into the
+# device layout 25.0 / 25.8
+NO_PRELOAD = ("q8_0_get_rows.hip", "q8_0_layout.hip")
 # The wrappers' native calls, a CPython module against torch's own headers and libraries (which are loaded with torch, before it).  Not part of
 # the library, whose other users need no torch, and the wrappers work without it.
 CALLS_SOURCE = "py_calls.cpp"
@@ -77,9 +84,10 @@ def build_library(verbose: bool = False, extra_flags: list[str] | None = None, i
     def compile_one(src: str) -> str:
         path = os.path.join(CSRC, src)
         obj = os.path.join(OBJ_DIR, os.path.splitext(src)[0] + ".o")
+        preload = PRELOAD_FLAGS if src.endswith(".hip") and src not in NO_PRELOAD else []
         if incremental and not extra_flags and os.path.exists(obj) and os.path.getmtime(obj) > max(os.path.getmtime(path), headers):
             return ""
-        return _run([hipcc(), *flags, "-c", path, "-o", obj])
+        return _run([hipcc(), *flags, *preload, "-c", path, "-o", obj])
 
     with ThreadPoolExecutor(max_workers=max(1, jobs)) as pool:
         notes = list(pool.map(compile_one, SOURCES))
