@@ -32,10 +32,10 @@ HIPCC_FLAGS = [
     # result parked in an accumulation register would cost one extra copy instruction per value (doubling the VALU work)
     "-mllvm", "-amdgpu-mfma-vgpr-form",
 ]
-# The first six dwords of a kernel's arguments (three pointers) arrive in scalar registers with the wave instead of being read from memory by it, a miss of
-# the scalar cache in front of the first address: norm + quantize of 4 rows 3.02 -> 2.76 us, [1024 x 4096] at 4 rows 4.17 -> 3.98, mul_mat of 16 rows
-# [4096 x 4096] 10.2 -> 9.7, of 2 and 4 rows 6.25 -> 6.07 and 6.12, of 5 rows the same.  (Ten and sixteen dwords: the same, but 5 and 8 rows 0.6 % slower.)
-PRELOAD_FLAGS = ["-mllvm", "-amdgpu-kernarg-preload-count=6"]
+# A kernel's first arguments (up to sixteen dwords) arrive in scalar registers with the wave instead of being read from memory by it, a miss of the scalar
+# cache in front of the first address; kernels name what that address takes first.  norm + quantize of 4 rows 3.02 -> 2.77 us, [1024 x 4096] at 4 rows
+# 4.17 -> 3.99, mul_mat of 4 / 16 rows [4096 x 4096] 6.3 -> 5.9 and 10.2 -> 9.5, [1024 x 4096] at 512 rows 10.3 -> 10.1.
+PRELOAD_FLAGS = ["-mllvm", "-amdgpu-kernarg-preload-count=16"]
 # not where a launch is many short waves, each of which then starts later: embedding rows of 4 tokens 1.83 us without, 1.99 with; [14336 x 4096] into the
 # device layout 25.0 / 25.8
 NO_PRELOAD = ("q8_0_get_rows.hip", "q8_0_layout.hip")

@@ -171,6 +171,12 @@ template<int TILES, bool LOOP, bool NORM, bool PAIR = false> __global__ __launch
 	int g0, g1;
 	wave_k_range(a.groups_c, a.split_shift, split, GEMV_WAVES, wave, g0, g1);
 
+	// thread t stores row t of the strip; its residual (which may be that output) is requested here, a memory latency ahead of its use
+	const int row = gstrip * STRIP_ROWS + tid;
+	float res	  = 0.0f;
+	if (a.residual && tid < STRIP_ROWS && row < a.n_out) {
+		res = a.residual[row];
+	}
 	const uint8_t* w_strip = a.w_down + macro_offset(gstrip, 0, a.groups_c);
 	const int row_l		   = gstrip * STRIP_ROWS + (lane & 31);
 	float acc			   = 0.0f;
@@ -192,16 +198,15 @@ template<int TILES, bool LOOP, bool NORM, bool PAIR = false> __global__ __launch
 			total += red[w][tid] + red[w][32 + tid];
 		}
 	}
-	const int row = gstrip * STRIP_ROWS + tid;
 	if (splits == 1) {
 		if (tid < STRIP_ROWS && row < a.n_out) {
-			a.y[row] = a.residual ? total + a.residual[row] : total;
+			a.y[row] = a.residual ? total + res : total;
 		}
 		return;
 	}
 	// K split over several workgroups: as in the plain mat-vec
 	if (tid < STRIP_ROWS) {
-		split_k_finish(a.tagged, a.epoch, gstrip, splits, split, tid, total, a.y, row, a.n_out, a.residual);
+		split_k_finish(a.tagged, a.epoch, gstrip, splits, split, tid, total, a.y, row, a.n_out, a.residual != nullptr, res);
 	}
 }
 

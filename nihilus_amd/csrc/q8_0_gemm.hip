@@ -705,15 +705,15 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 }
 
 template<int TM, bool DUMP, int KS = 1, bool STREAM = false, bool SPLIT = false>
-__global__ __launch_bounds__(256 * KS, 4) void gemm_tiled_kernel(const uint8_t* __restrict__ W, const uint8_t* __restrict__ A, float* C, const float* R, int32_t* __restrict__ sums, int M, int N,
-	int groups, float* __restrict__ partials, unsigned* __restrict__ counters) {
+__global__ __launch_bounds__(256 * KS, 4) void gemm_tiled_kernel(const uint8_t* __restrict__ W, const uint8_t* __restrict__ A, int M, int N, int groups, float* C, const float* R,
+	int32_t* __restrict__ sums, float* __restrict__ partials, unsigned* __restrict__ counters) {
 	gemm_tiled_body<TM, DUMP, KS, STREAM, SPLIT, false>(W, A, C, R, sums, M, N, groups, partials, counters, nullptr, nullptr, nullptr);
 }
 
 // the fused gate / up form (GATE_UP above): N = rows of each of the two matrices; gate_out / up_out optional
 template<int TM, int KS, bool STREAM, bool PASSES>
-__global__ __launch_bounds__(256 * KS, 4) void gemm_gate_up_kernel(const uint8_t* __restrict__ W_gate, const uint8_t* __restrict__ W_up, const uint8_t* __restrict__ A, uint8_t* __restrict__ act_out,
-	float* __restrict__ gate_out, float* __restrict__ up_out, int M, int N, int groups, int passes, bool tree) {
+__global__ __launch_bounds__(256 * KS, 4) void gemm_gate_up_kernel(const uint8_t* __restrict__ W_gate, const uint8_t* __restrict__ W_up, const uint8_t* __restrict__ A, int M, int N, int groups,
+	int passes, bool tree, uint8_t* __restrict__ act_out, float* __restrict__ gate_out, float* __restrict__ up_out) {
 	gemm_tiled_body<TM, false, KS, STREAM, false, true, PASSES>(W_gate, A, gate_out, nullptr, nullptr, M, N, groups, nullptr, nullptr, W_up, act_out, up_out, passes, tree);
 }
 
@@ -723,7 +723,7 @@ template<int TM, bool STREAM> static hipError_t launch_gemm_tiled_t(const gemm_t
 	const int groups = k / GROUP_K;
 	const dim3 grid(cut.grid_x, cut.grid_y);
 	if (sums) {
-		gemm_tiled_kernel<TM, true><<<grid, dim3(256), 0, s>>>(w, a, C, R, sums, m, n, groups, nullptr, nullptr);
+		gemm_tiled_kernel<TM, true><<<grid, dim3(256), 0, s>>>(w, a, m, n, groups, C, R, sums, nullptr, nullptr);
 		return hipGetLastError();
 	}
 	const int ks = cut.ks;
@@ -736,17 +736,17 @@ template<int TM, bool STREAM> static hipError_t launch_gemm_tiled_t(const gemm_t
 			if (e != hipSuccess) {
 				return e;
 			}
-			return launch_kernel(KIND_GEMM, gemm_tiled_kernel<TM, false, 4, STREAM, true>, dim3(grid.x, grid.y, static_cast<unsigned>(cut.kz)), dim3(1024), 0, s, w, a, C, R, sums, m, n, groups, partials,
+			return launch_kernel(KIND_GEMM, gemm_tiled_kernel<TM, false, 4, STREAM, true>, dim3(grid.x, grid.y, static_cast<unsigned>(cut.kz)), dim3(1024), 0, s, w, a, m, n, groups, C, R, sums, partials,
 				counters);
 		}
 	}
 	if (ks == 4) {
-		return launch_kernel(KIND_GEMM, gemm_tiled_kernel<TM, false, 4, STREAM>, grid, dim3(1024), 0, s, w, a, C, R, sums, m, n, groups, static_cast<float*>(nullptr), static_cast<unsigned*>(nullptr));
+		return launch_kernel(KIND_GEMM, gemm_tiled_kernel<TM, false, 4, STREAM>, grid, dim3(1024), 0, s, w, a, m, n, groups, C, R, sums, static_cast<float*>(nullptr), static_cast<unsigned*>(nullptr));
 	}
 	if (ks == 2) {
-		return launch_kernel(KIND_GEMM, gemm_tiled_kernel<TM, false, 2, STREAM>, grid, dim3(512), 0, s, w, a, C, R, sums, m, n, groups, static_cast<float*>(nullptr), static_cast<unsigned*>(nullptr));
+		return launch_kernel(KIND_GEMM, gemm_tiled_kernel<TM, false, 2, STREAM>, grid, dim3(512), 0, s, w, a, m, n, groups, C, R, sums, static_cast<float*>(nullptr), static_cast<unsigned*>(nullptr));
 	}
-	return launch_kernel(KIND_GEMM, gemm_tiled_kernel<TM, false, 1, STREAM>, grid, dim3(256), 0, s, w, a, C, R, sums, m, n, groups, static_cast<float*>(nullptr), static_cast<unsigned*>(nullptr));
+	return launch_kernel(KIND_GEMM, gemm_tiled_kernel<TM, false, 1, STREAM>, grid, dim3(256), 0, s, w, a, m, n, groups, C, R, sums, static_cast<float*>(nullptr), static_cast<unsigned*>(nullptr));
 }
 
 // stream: the weights are read once and not again (a batch of decode rows against a large matrix), so their loads bypass the caches.
@@ -773,7 +773,7 @@ hipError_t launch_gemm_gate_up_silu(const void* w_gate, const void* w_up, const 
 		const dim3 grid(t.grid_x, t.grid_y);
 		auto launch = [&](auto kernel) {
 			return launch_kernel(KIND_GEMM, kernel, grid, dim3(static_cast<unsigned>(256 * t.ks)), 0, s, static_cast<const uint8_t*>(w_gate), static_cast<const uint8_t*>(w_up), static_cast<const uint8_t*>(aq),
-				static_cast<uint8_t*>(act_out), gate_dbg, up_dbg, static_cast<int>(M), static_cast<int>(n_ff), static_cast<int>(K / GROUP_K), cut.passes, cut.tree);
+				static_cast<int>(M), static_cast<int>(n_ff), static_cast<int>(K / GROUP_K), cut.passes, cut.tree, static_cast<uint8_t*>(act_out), gate_dbg, up_dbg);
 		};
 		if (t.tm == 1) { // 17 to 32 rows on matrices of 192 column blocks and more (the rows kernel has the others)
 			return t.ks == 1 ? launch(gemm_gate_up_kernel<1, 1, true, false>) : cut.passes > 1 ? launch(gemm_gate_up_kernel<1, 2, true, true>) : launch(gemm_gate_up_kernel<1, 2, true, false>);

@@ -232,31 +232,55 @@ template<int R, int T, int MATS, int SETS> __device__ __forceinline__ float rows
 } // namespace
 
 template<int R, int T, int SETS>
-__global__ __launch_bounds__(SK_WAVES * 64, 4) void gemm_rows_kernel(const uint8_t* __restrict__ W, const uint8_t* __restrict__ A, float* C, const float* residual, uint64_t* __restrict__ tagged,
-	unsigned epoch, int M, int N, int groups, int split_shift) {
+__global__ __launch_bounds__(SK_WAVES * 64, 4) void gemm_rows_kernel(const uint8_t* __restrict__ W, const uint8_t* __restrict__ A, int groups, int split_shift, int M, int N, const float* residual, float* C,
+	uint64_t* __restrict__ tagged, unsigned epoch) {
 	__shared__ __align__(16) uint8_t lds[rows_lds<R, T, 1, SETS>::BYTES];
 	const int tid	= threadIdx.x;
 	const int lane	= tid & 63;
 	const int wave	= __builtin_amdgcn_readfirstlane(tid >> 6);
 	const int strip = static_cast<int>(blockIdx.x >> split_shift);
 	const int split = static_cast<int>(blockIdx.x) & ((1 << split_shift) - 1);
-	rows_strip<R, T, 1, SETS>(W + macro_offset(strip, 0, groups), nullptr, A, lds, groups, split_shift, split, lane, wave);
+	// thread t finishes outputs (row t / 32 + 16 i, strip column t % 32); their residuals (which may be those outputs) are requested here, a memory
+	// latency ahead of their use
+	constexpr int OWN = (R + 15) / 16;
+	const int m0 = tid >> 5, l = tid & 31, n = strip * STRIP_ROWS + l;
+	const int rows = min(M, R);
+	float res[OWN];
 #pragma unroll
-	for (int o = 0; o < R * STRIP_ROWS; o += SK_WAVES * 64) {
-		const int m = (o + tid) >> 5, l = tid & 31;
-		if (m >= M || m >= R) {
-			continue;
+	for (int i = 0; i < OWN; ++i) {
+		res[i] = 0.0f;
+		if (residual && m0 + 16 * i < rows && n < N) {
+			res[i] = residual[static_cast<int64_t>(m0 + 16 * i) * N + n];
 		}
-		const float total = rows_total<R, T, 1, SETS>(lds, 0, m, l);
-		const int n		  = strip * STRIP_ROWS + l;
-		float* cm		  = C + static_cast<int64_t>(m) * N;
-		const float* rm	  = residual ? residual + static_cast<int64_t>(m) * N : nullptr; // may be cm: read before the write, by the same thread
-		if (split_shift == 0) {
-			if (n < N) {
-				cm[n] = rm ? total + rm[n] : total;
+	}
+	rows_strip<R, T, 1, SETS>(W + macro_offset(strip, 0, groups), nullptr, A, lds, groups, split_shift, split, lane, wave);
+	float total[OWN];
+#pragma unroll
+	for (int i = 0; i < OWN; ++i) {
+		if (m0 + 16 * i < rows) {
+			total[i] = rows_total<R, T, 1, SETS>(lds, 0, m0 + 16 * i, l);
+		}
+	}
+	if (split_shift == 0) {
+#pragma unroll
+		for (int i = 0; i < OWN; ++i) {
+			if (m0 + 16 * i < rows && n < N) {
+				C[static_cast<int64_t>(m0 + 16 * i) * N + n] = residual ? total[i] + res[i] : total[i];
 			}
-		} else {
-			split_k_finish(tagged, epoch, strip * R + m, 1 << split_shift, split, l, total, cm, n, N, rm);
+		}
+		return;
+	}
+#pragma unroll
+	for (int i = 0; i < OWN; ++i) {
+		if (m0 + 16 * i < rows) {
+			split_k_publish(tagged, epoch, strip * R + m0 + 16 * i, 1 << split_shift, split, l, total[i], res[i]);
+		}
+	}
+	wait_stores_acknowledged();
+#pragma unroll
+	for (int i = 0; i < OWN; ++i) {
+		if (m0 + 16 * i < rows) {
+			split_k_collect(tagged, epoch, strip * R + m0 + 16 * i, 1 << split_shift, l, C + static_cast<int64_t>(m0 + 16 * i) * N, n, N, residual != nullptr, res[i]);
 		}
 	}
 }
@@ -265,7 +289,7 @@ __global__ __launch_bounds__(SK_WAVES * 64, 4) void gemm_rows_kernel(const uint8
 // activation row are one block of the down projection's operand and sit in one half-wave.
 template<int R, int T, int SETS>
 __global__ __launch_bounds__(SK_WAVES * 64, 4) void gemm_rows_gate_up_kernel(const uint8_t* __restrict__ W_gate, const uint8_t* __restrict__ W_up, const uint8_t* __restrict__ A,
-	uint8_t* __restrict__ act_out, float* __restrict__ gate_out, float* __restrict__ up_out, int M, int N, int groups) {
+	int groups, int M, int N, uint8_t* __restrict__ act_out, float* __restrict__ gate_out, float* __restrict__ up_out) {
 	__shared__ __align__(16) uint8_t lds[rows_lds<R, T, 2, SETS>::BYTES];
 	const int tid	= threadIdx.x;
 	const int lane	= tid & 63;
@@ -369,7 +393,7 @@ template<int SETS> static hipError_t launch_rows_t(const uint8_t* w, const uint8
 		++shift;
 	}
 	const dim3 grid(static_cast<unsigned>((n + STRIP_ROWS - 1) / STRIP_ROWS * splits)), block(SK_WAVES * 64);
-	auto launch = [&](auto kernel) { return launch_kernel(KIND_GEMM, kernel, grid, block, 0, s, w, a, C, residual, sc.tagged, sc.epoch, m, n, groups, shift); };
+	auto launch = [&](auto kernel) { return launch_kernel(KIND_GEMM, kernel, grid, block, 0, s, w, a, groups, shift, m, n, residual, C, sc.tagged, sc.epoch); };
 	return m <= 8 ? launch(gemm_rows_kernel<8, 2, SETS>) : m <= 16 ? launch(gemm_rows_kernel<16, 2, SETS>) : m <= 24 ? launch(gemm_rows_kernel<24, 2, SETS>) : launch(gemm_rows_kernel<32, 2, SETS>);
 }
 
@@ -389,7 +413,7 @@ hipError_t launch_gemm_rows(const void* W, const void* Aq, float* C, const float
 }
 
 template<int SETS> static hipError_t launch_rows_gate_up_t(const uint8_t* wg, const uint8_t* wu, const uint8_t* a, uint8_t* out, float* gate_dbg, float* up_dbg, int m, int n, int groups, hipStream_t s) {
-	auto launch = [&](auto kernel) { return launch_kernel(KIND_GEMM, kernel, dim3(static_cast<unsigned>(n / STRIP_ROWS)), dim3(SK_WAVES * 64), 0, s, wg, wu, a, out, gate_dbg, up_dbg, m, n, groups); };
+	auto launch = [&](auto kernel) { return launch_kernel(KIND_GEMM, kernel, dim3(static_cast<unsigned>(n / STRIP_ROWS)), dim3(SK_WAVES * 64), 0, s, wg, wu, a, groups, m, n, out, gate_dbg, up_dbg); };
 	return m <= 8 ? launch(gemm_rows_gate_up_kernel<8, 1, SETS>) : m <= 16 ? launch(gemm_rows_gate_up_kernel<16, 1, SETS>) : m <= 24 ? launch(gemm_rows_gate_up_kernel<24, 1, SETS>) : launch(gemm_rows_gate_up_kernel<32, 1, SETS>);
 }
 

@@ -29,8 +29,8 @@ template<bool NT, typename T> __device__ __forceinline__ T load_weights(const T*
 }
 
 template<int MS, int GC, int WAVES, bool NT>
-__global__ __launch_bounds__(WAVES * 64, 4) void gemm_skinny_kernel(const uint8_t* __restrict__ W, const uint8_t* __restrict__ A, float* C, const float* R,
-	float* __restrict__ partials, unsigned* __restrict__ counters, int M, int N, int groups, int split_shift) {
+__global__ __launch_bounds__(WAVES * 64, 4) void gemm_skinny_kernel(const uint8_t* __restrict__ W, const uint8_t* __restrict__ A, int groups, int split_shift, int M, int N,
+	float* C, const float* R, float* __restrict__ partials, unsigned* __restrict__ counters) {
 	__shared__ float red[MS * 16][WAVES][64];
 	__shared__ int last_flag;
 
@@ -349,7 +349,7 @@ template<int MS> static hipError_t launch_skinny_t(int splits, int waves, const 
 	// group ([8192 x 4096] at 40 rows 12.3 as it is, 13.2 through the caches), nor with two whose workgroups are on one XCD (workgroups go to the eight in turn) at
 	// the same time: the second finds the first's lines on their way ([4096 x 4096] at 64 rows 8.1 / 8.25, at 117 rows the same).
 	const bool nt = m_groups == 1 || (m_groups == 2 && (strips * splits) % 8 == 0);
-	const auto launch = [&](auto kernel) { return launch_kernel(KIND_GEMM, kernel, grid, block, 0, s, w, a, C, R, sc.partials, sc.counters, m, n, groups, shift); };
+	const auto launch = [&](auto kernel) { return launch_kernel(KIND_GEMM, kernel, grid, block, 0, s, w, a, groups, shift, m, n, C, R, sc.partials, sc.counters); };
 	if (waves == SK_WIDE_WAVES) {
 		return nt ? launch(gemm_skinny_kernel<MS, 2, SK_WIDE_WAVES, true>) : launch(gemm_skinny_kernel<MS, 2, SK_WIDE_WAVES, false>);
 	}

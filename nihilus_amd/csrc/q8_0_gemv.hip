@@ -139,6 +139,20 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_tiled_kernel(gemv_segmen
 	wave_k_range(groups, RS > 1 ? 0 : split_shift, split, GEMV_WAVES, wave, g0, g1);
 
 	const uint8_t* w_strip = DUMP == DUMP_X ? nullptr : seg.W[sidx] + macro_offset(strip, 0, groups);
+	// thread t stores row t of the workgroup's; its residual (which may be that output) is requested here, a memory latency ahead of its use (with the norm, whose
+	// launches have none and whose long walks no register for it, in front of the reduction)
+	constexpr int PART_ROWS = STRIP_ROWS / RS; // rows this workgroup owns: 64 / PART_ROWS lanes of every wave hold a share of each
+	const int row			= strip * STRIP_ROWS + rowpart * PART_ROWS + tid;
+	const float* residual	= DUMP == DUMP_NONE ? seg.residual[sidx] : nullptr;
+	float res				= 0.0f;
+	const auto request_residual = [&] {
+		if (residual && tid < PART_ROWS && row < N) {
+			res = residual[row];
+		}
+	};
+	if constexpr (!NORM) {
+		request_residual();
+	}
 	const int row_l		   = strip * STRIP_ROWS + (lane & 31);
 	float acc			   = 0.0f;
 	// the wave's K range, in one piece when the host picked splits so that g1 - g0 <= TILES (straight-line code, every load of the
@@ -184,11 +198,13 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_tiled_kernel(gemv_segmen
 		return;
 	}
 
+	if constexpr (NORM) {
+		request_residual();
+	}
 	// ---- one reduction per workgroup, fixed order ----
 	red[wave][lane] = acc;
 	__syncthreads();
-	constexpr int PART_ROWS = STRIP_ROWS / RS; // rows this workgroup owns: 64 / PART_ROWS lanes of every wave hold a share of each
-	float total				= 0.0f;
+	float total = 0.0f;
 	if (tid < PART_ROWS) {
 #pragma unroll
 		for (int w = 0; w < GEMV_WAVES; ++w) {
@@ -200,19 +216,17 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_tiled_kernel(gemv_segmen
 			total += part;
 		}
 	}
-	const int row = strip * STRIP_ROWS + rowpart * PART_ROWS + tid;
-	float* y		  = seg.y[sidx];
-	const float* res  = seg.residual[sidx];
+	float* y = seg.y[sidx];
 	if (splits == 1) {
 		if (tid < PART_ROWS && row < N) {
-			y[row] = res ? total + res[row] : total;
+			y[row] = residual ? total + res : total;
 		}
 		return;
 	}
 
 	// ---- K split over several workgroups ----
 	if (tid < STRIP_ROWS) {
-		split_k_finish(tagged, epoch, gstrip, splits, split, tid, total, y, row, N, res);
+		split_k_finish(tagged, epoch, gstrip, splits, split, tid, total, y, row, N, residual != nullptr, res);
 	}
 }
 

@@ -49,6 +49,13 @@ template<int TILES> __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_grou
 	int g0, g1;
 	wave_k_range(groups, shift, split, GEMV_WAVES, wave, g0, g1);
 
+	// thread t stores row t of the strip; its residual (which may be that output) is requested here, a memory latency ahead of its use
+	const int row		  = strip * STRIP_ROWS + tid;
+	const float* residual = g.residual[m];
+	float res			  = 0.0f;
+	if (residual && tid < STRIP_ROWS && row < N) {
+		res = residual[row];
+	}
 	const uint8_t* w_strip = g.W[m] + macro_offset(strip, 0, groups);
 	const int row_l		   = strip * STRIP_ROWS + (lane & 31);
 	// the host only groups matrices whose waves own at most TILES groups: every load of the wave in flight at once
@@ -63,17 +70,15 @@ template<int TILES> __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_grou
 			total += red[w][tid] + red[w][32 + tid];
 		}
 	}
-	const int row	 = strip * STRIP_ROWS + tid;
-	float* y		 = g.y[m];
-	const float* res = g.residual[m];
+	float* y = g.y[m];
 	if (splits == 1) {
 		if (tid < STRIP_ROWS && row < N) {
-			y[row] = res ? total + res[row] : total;
+			y[row] = residual ? total + res : total;
 		}
 		return;
 	}
 	if (tid < STRIP_ROWS) {
-		split_k_finish(tagged + static_cast<int64_t>(g.unit0[m]) * STRIP_ROWS, epoch, strip, splits, split, tid, total, y, row, N, res);
+		split_k_finish(tagged + static_cast<int64_t>(g.unit0[m]) * STRIP_ROWS, epoch, strip, splits, split, tid, total, y, row, N, residual != nullptr, res);
 	}
 }
 

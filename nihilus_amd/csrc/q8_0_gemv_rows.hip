@@ -114,8 +114,8 @@ __device__ __forceinline__ void gemv_rows_chunk(const uint8_t* __restrict__ w_st
 // TILES <= 2 groups per wave and chunk: MR slices of fp32 activations sit in registers next to the weight tiles (two rows fit
 // in 64 registers = two workgroups per CU; three take 65 and run as one, which measured faster than spilling to stay at two).
 template<int TILES, int MR, bool LOOP>
-__global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_rows_kernel(const uint8_t* __restrict__ W, const float* __restrict__ x, float* y, const float* residual, uint64_t* __restrict__ tagged, unsigned epoch,
-	int N, int groups, int split_shift) {
+__global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_rows_kernel(const uint8_t* __restrict__ W, const float* __restrict__ x, int groups, int split_shift, int N, const float* residual, float* y,
+	uint64_t* __restrict__ tagged, unsigned epoch) {
 	__shared__ __align__(16) uint8_t xs_q[GEMV_WAVES][MR][TILES * GROUP_K]; // each wave's quantized slices, block jj of row m at 32*jj
 	__shared__ float xs_d[GEMV_WAVES][MR][TILES * GROUP_BLOCKS];
 	__shared__ float red[MR][GEMV_WAVES][64];
@@ -129,6 +129,12 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_rows_kernel(const uint8_
 	wave_k_range(groups, split_shift, split, GEMV_WAVES, wave, g0, g1);
 	const int64_t K	 = static_cast<int64_t>(groups) * GROUP_K;
 
+	// thread 32 * m + l stores output (row m, strip row l); its residual (which may be that output) is requested here, a memory latency ahead of its use
+	const int m = tid >> 5, l = tid & 31, row = strip * STRIP_ROWS + l;
+	float res	= 0.0f;
+	if (residual && m < MR && row < N) {
+		res = residual[static_cast<int64_t>(m) * N + row];
+	}
 	const uint8_t* w_strip = W + macro_offset(strip, 0, groups);
 	float acc[MR];
 #pragma unroll
@@ -153,22 +159,19 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_rows_kernel(const uint8_
 	if (tid >= MR * STRIP_ROWS) {
 		return;
 	}
-	const int m = tid >> 5, l = tid & 31;
 	float total = 0.0f;
 #pragma unroll
 	for (int w = 0; w < GEMV_WAVES; ++w) {
 		total += red[m][w][l] + red[m][w][32 + l];
 	}
-	const int row = strip * STRIP_ROWS + l;
-	float* ym		= y + static_cast<int64_t>(m) * N;
-	const float* rm = residual ? residual + static_cast<int64_t>(m) * N : nullptr; // may be ym: read before the write, by the same thread
+	float* ym = y + static_cast<int64_t>(m) * N;
 	if (splits == 1) {
 		if (row < N) {
-			ym[row] = rm ? total + rm[row] : total;
+			ym[row] = residual ? total + res : total;
 		}
 		return;
 	}
-	split_k_finish(tagged, epoch, strip * MR + m, splits, split, l, total, ym, row, N, rm);
+	split_k_finish(tagged, epoch, strip * MR + m, splits, split, l, total, ym, row, N, residual != nullptr, res);
 }
 
 template<int TILES, int MR, bool LOOP> static hipError_t launch_rows_n(const gemv_plan& p, const uint8_t* W, const float* x, float* y, const float* r, int N, const gemv_scratch& sc, hipStream_t s) {
@@ -177,7 +180,7 @@ template<int TILES, int MR, bool LOOP> static hipError_t launch_rows_n(const gem
 	while ((1 << shift) < p.splits) {
 		++shift;
 	}
-	return launch_kernel(KIND_GEMV, gemv_rows_kernel<TILES, MR, LOOP>, grid, block, 0, s, W, x, y, r, sc.tagged, sc.epoch, N, p.groups, shift);
+	return launch_kernel(KIND_GEMV, gemv_rows_kernel<TILES, MR, LOOP>, grid, block, 0, s, W, x, p.groups, shift, N, r, y, sc.tagged, sc.epoch);
 }
 
 template<int MR> static hipError_t launch_rows_m(const gemv_plan& p, const uint8_t* W, const float* x, float* y, const float* r, int N, const gemv_scratch& sc, hipStream_t s) {

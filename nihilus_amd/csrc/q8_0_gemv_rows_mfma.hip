@@ -123,8 +123,8 @@ __device__ __forceinline__ void rows8_chunk(const uint8_t* __restrict__ w_strip,
 }
 
 template<int R, int TILES, bool LOOP>
-__global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_rows8_kernel(const uint8_t* __restrict__ W, const float* __restrict__ x, float* y, const float* residual, uint64_t* __restrict__ tagged,
-	unsigned epoch, int M, int N, int groups, int split_shift) {
+__global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_rows8_kernel(const uint8_t* __restrict__ W, const float* __restrict__ x, int groups, int split_shift, int M, int N, const float* residual, float* y,
+	uint64_t* __restrict__ tagged, unsigned epoch) {
 	constexpr int ROWS8 = R, ROWS8_A_HALF = rows_a_half<R>, ROWS8_A_TILE = rows_a_tile<R>;
 	__shared__ __align__(16) uint8_t a_tiles[GEMV_WAVES][TILES * GROUP_BLOCKS * ROWS8_A_TILE];
 	__shared__ __align__(16) float a_scales[GEMV_WAVES][TILES * GROUP_BLOCKS * ROWS8];
@@ -145,6 +145,18 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_rows8_kernel(const uint8
 	}
 	__builtin_amdgcn_wave_barrier();
 
+	// thread 32 * m + l stores output (row m, strip row l); its residual (which may be that output) is requested here, a memory latency ahead of its use (behind
+	// a walk of several chunks, which has no register for it)
+	const int m = tid >> 5, l = tid & 31, row = strip * STRIP_ROWS + l;
+	float res	= 0.0f;
+	const auto request_residual = [&] {
+		if (residual && m < M && row < N) {
+			res = residual[static_cast<int64_t>(m) * N + row];
+		}
+	};
+	if constexpr (!LOOP) {
+		request_residual();
+	}
 	const uint8_t* w_strip = W + macro_offset(strip, 0, groups);
 	float acc[R / 2];
 #pragma unroll
@@ -158,6 +170,7 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_rows8_kernel(const uint8
 			rows8_chunk<R, TILES>(w_strip, x, K, M, a_tiles[wave], a_scales[wave], gc, min(TILES, g1 - gc), lane, acc);
 			__builtin_amdgcn_wave_barrier(); // the next chunk overwrites this wave's tiles
 		}
+		request_residual();
 	}
 
 	// ---- one reduction per workgroup, fixed order: thread 32 * m + l owns output (row m, strip row l) ----
@@ -166,7 +179,6 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_rows8_kernel(const uint8
 		red[e][wave][lane] = acc[e];
 	}
 	__syncthreads();
-	const int m = tid >> 5, l = tid & 31;
 	if (m >= M || m >= R) {
 		return;
 	}
@@ -175,16 +187,14 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_rows8_kernel(const uint8
 	for (int w = 0; w < GEMV_WAVES; ++w) {
 		total += red[4 * (m >> 3) + (m & 3)][w][32 * ((m >> 2) & 1) + l]; // row m = 8 e4 + 4 half + i sits in lanes of that half, sum 4 e4 + i
 	}
-	const int row	= strip * STRIP_ROWS + l;
-	float* ym		= y + static_cast<int64_t>(m) * N;
-	const float* rm = residual ? residual + static_cast<int64_t>(m) * N : nullptr; // may be ym: read before the write, by the same thread
+	float* ym = y + static_cast<int64_t>(m) * N;
 	if (splits == 1) {
 		if (row < N) {
-			ym[row] = rm ? total + rm[row] : total;
+			ym[row] = residual ? total + res : total;
 		}
 		return;
 	}
-	split_k_finish(tagged, epoch, strip * R + m, splits, split, l, total, ym, row, N, rm);
+	split_k_finish(tagged, epoch, strip * R + m, splits, split, l, total, ym, row, N, residual != nullptr, res);
 }
 
 template<int R, int TILES, bool LOOP> static hipError_t launch_rows8_n(const gemv_plan& p, const uint8_t* W, const float* x, float* y, const float* r, int M, int N, const gemv_scratch& sc, hipStream_t s) {
@@ -193,7 +203,7 @@ template<int R, int TILES, bool LOOP> static hipError_t launch_rows8_n(const gem
 	while ((1 << shift) < p.splits) {
 		++shift;
 	}
-	return launch_kernel(KIND_GEMV, gemv_rows8_kernel<R, TILES, LOOP>, grid, block, 0, s, W, x, y, r, sc.tagged, sc.epoch, M, N, p.groups, shift);
+	return launch_kernel(KIND_GEMV, gemv_rows8_kernel<R, TILES, LOOP>, grid, block, 0, s, W, x, p.groups, shift, M, N, r, y, sc.tagged, sc.epoch);
 }
 
 // 1 <= M <= 16 fp32 activation rows [M][K] against a tiled weight [N][K]; y is [M][N].  K % 128 == 0 (checked by the caller).

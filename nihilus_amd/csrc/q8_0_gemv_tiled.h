@@ -432,21 +432,19 @@ __device__ __forceinline__ float gemv_chunk(const uint8_t* __restrict__ w_strip,
 // to / read from the memory side).  A device-wide fence would also order them, but it writes back and invalidates the
 // whole L2 under the other workgroups' streaming loads.
 // Call from the first 32 threads of the workgroup (one wave), total = the row's partial sum over this split.
-__device__ __forceinline__ void split_k_finish(uint64_t* __restrict__ tagged, unsigned epoch, int gstrip, int splits, int split, int lane, float total, float* __restrict__ y, int row,
-	int N, const float* __restrict__ residual) {
-	uint64_t* mine = tagged + static_cast<int64_t>(gstrip) * splits * STRIP_ROWS + lane;
-	// The residual may be y itself, and more than one workgroup may store the row: each takes its copy of the residual before
-	// it publishes its own share.  Nobody can have stored the row by then (that takes every share, this one included), so all
-	// of them add the same value, whoever stores first.
-	float res = 0.0f;
-	if (residual && row < N) {
-		res = residual[row];
-	}
+//
+// The residual may be y itself, and more than one workgroup may store the row: each has its copy of the residual (`res`) before it publishes its own
+// share.  Nobody can have stored the row by then (that takes every share, this one included), so all of them add the same value,
+// whoever stores first.
+__device__ __forceinline__ void split_k_publish(uint64_t* __restrict__ tagged, unsigned epoch, int gstrip, int splits, int split, int lane, float total, float& res) {
 	asm volatile("" : "+v"(res)::"memory"); // the value is in a register (the load has returned) before the share goes out
-	__hip_atomic_store(&mine[split * STRIP_ROWS], (static_cast<uint64_t>(epoch) << 32) | __float_as_uint(total), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-	wait_stores_acknowledged();
-	bool all  = true;
-	float sum = 0.0f;
+	__hip_atomic_store(&tagged[(static_cast<int64_t>(gstrip) * splits + split) * STRIP_ROWS + lane], (static_cast<uint64_t>(epoch) << 32) | __float_as_uint(total), __ATOMIC_RELAXED,
+		__HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void split_k_collect(uint64_t* __restrict__ tagged, unsigned epoch, int gstrip, int splits, int lane, float* __restrict__ y, int row, int N, bool add, float res) {
+	uint64_t* mine = tagged + static_cast<int64_t>(gstrip) * splits * STRIP_ROWS + lane;
+	bool all	   = true;
+	float sum	   = 0.0f;
 	for (int sp0 = 0; sp0 < splits; sp0 += 8) { // every share requested before the first is waited for
 		uint64_t v[8];
 #pragma unroll
@@ -462,8 +460,14 @@ __device__ __forceinline__ void split_k_finish(uint64_t* __restrict__ tagged, un
 		}
 	}
 	if (all && row < N) {
-		y[row] = residual ? sum + res : sum;
+		y[row] = add ? sum + res : sum;
 	}
+}
+__device__ __forceinline__ void split_k_finish(uint64_t* __restrict__ tagged, unsigned epoch, int gstrip, int splits, int split, int lane, float total, float* __restrict__ y, int row, int N, bool add,
+	float res) {
+	split_k_publish(tagged, epoch, gstrip, splits, split, lane, total, res);
+	wait_stores_acknowledged();
+	split_k_collect(tagged, epoch, gstrip, splits, lane, y, row, N, add, res);
 }
 
 // Scratch of the K-split path (tagged partial sums) and of the fused FFN launch (the gate and up

@@ -96,7 +96,7 @@ template<int GC> __global__ __launch_bounds__(F32ACT_WAVES * 64, GC <= 2 ? 8 : 4
 		}
 		const int row = strip * STRIP_ROWS + tid;
 		if (splits > 1) {
-			split_k_finish(tagged, epoch, strip, splits, split, tid, total, y, row, N, nullptr);
+			split_k_finish(tagged, epoch, strip, splits, split, tid, total, y, row, N, false, 0.0f);
 		} else if (row < N) {
 			y[m * N + row] = total;
 		}

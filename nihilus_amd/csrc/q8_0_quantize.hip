@@ -92,7 +92,7 @@ __global__ __launch_bounds__(256) void quantize_kernel(const float* __restrict__
 // one 1024-thread workgroup per row; the row's scale first (fixed-order sum of squares, see rms_scale_workgroup), then
 // every thread normalises and quantizes its float4s.  The row is read twice, the second time from cache.
 template<bool TILED>
-__global__ __launch_bounds__(1024) void rms_norm_quantize_kernel(const float* __restrict__ x, const float* __restrict__ norm_w, float eps, uint8_t* __restrict__ out, int64_t M, int K) {
+__global__ __launch_bounds__(1024) void rms_norm_quantize_kernel(const float* __restrict__ x, const float* __restrict__ norm_w, int K, float eps, uint8_t* __restrict__ out, int64_t M) {
 	__shared__ float red[16];
 	const int tid	  = threadIdx.x;
 	const int lane	  = tid & 63;
@@ -148,7 +148,7 @@ __global__ __launch_bounds__(1024) void rms_norm_quantize_kernel(const float* __
 // once (non-temporal loads of the rows measured no different: the launch is bound by its stores).  The quants and scales go to an LDS image of the eight rows' share of the tiles ([group][tile][half][row][16 bytes], then
 // [group][row][4 scales]) and from there to memory as whole lines, 16 bytes per lane.  F4: float4s per lane and run.
 template<int F4>
-__global__ __launch_bounds__(1024, F4 == 1 ? 8 : 4) void rms_norm_quantize_rows8_kernel(const float* __restrict__ x, const float* __restrict__ norm_w, float eps, uint8_t* __restrict__ out, int64_t M, int K) {
+__global__ __launch_bounds__(1024, F4 == 1 ? 8 : 4) void rms_norm_quantize_rows8_kernel(const float* __restrict__ x, const float* __restrict__ norm_w, int K, float eps, uint8_t* __restrict__ out, int64_t M) {
 	__shared__ __align__(16) uint8_t image[F4 * 4096 * 8 + F4 * 32 * 64]; // K * 8 bytes of quants, then K / 128 * 64 bytes of scales (K <= 4096 F4)
 	__shared__ float red[8][16];
 	const int tid	 = threadIdx.x;
@@ -246,15 +246,15 @@ hipError_t launch_rms_norm_quantize(const float* x, const float* norm_w, float e
 		const dim3 g8(static_cast<unsigned>(rows_out / 8)), b8(1024);
 		uint8_t* o		 = static_cast<uint8_t*>(out);
 		if (K <= 4096) {
-			return launch_kernel(KIND_QUANTIZE, rms_norm_quantize_rows8_kernel<1>, g8, b8, 0, s, x, norm_w, eps, o, M, static_cast<int>(K));
+			return launch_kernel(KIND_QUANTIZE, rms_norm_quantize_rows8_kernel<1>, g8, b8, 0, s, x, norm_w, static_cast<int>(K), eps, o, M);
 		}
-		return launch_kernel(KIND_QUANTIZE, rms_norm_quantize_rows8_kernel<2>, g8, b8, 0, s, x, norm_w, eps, o, M, static_cast<int>(K));
+		return launch_kernel(KIND_QUANTIZE, rms_norm_quantize_rows8_kernel<2>, g8, b8, 0, s, x, norm_w, static_cast<int>(K), eps, o, M);
 	}
 	const dim3 g(static_cast<unsigned>(rows_out)), b(1024);
 	if (tiled) {
-		return launch_kernel(KIND_QUANTIZE, rms_norm_quantize_kernel<true>, g, b, 0, s, x, norm_w, eps, static_cast<uint8_t*>(out), M, static_cast<int>(K));
+		return launch_kernel(KIND_QUANTIZE, rms_norm_quantize_kernel<true>, g, b, 0, s, x, norm_w, static_cast<int>(K), eps, static_cast<uint8_t*>(out), M);
 	}
-	return launch_kernel(KIND_QUANTIZE, rms_norm_quantize_kernel<false>, g, b, 0, s, x, norm_w, eps, static_cast<uint8_t*>(out), M, static_cast<int>(K));
+	return launch_kernel(KIND_QUANTIZE, rms_norm_quantize_kernel<false>, g, b, 0, s, x, norm_w, static_cast<int>(K), eps, static_cast<uint8_t*>(out), M);
 }
 
 template<bool SILU_MUL> static hipError_t launch_quantize_t(const float* x, const float* u, void* out, int64_t M, int64_t K, bool tiled, hipStream_t s) {
