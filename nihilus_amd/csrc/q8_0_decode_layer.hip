@@ -31,7 +31,6 @@ namespace nh {
 
 constexpr int CHAIN_TILES = 4; // groups a wave stages at once: LDS slices are sized for it
 constexpr int CHAIN_DOWN_ROWS_TILES = 8; // ... in the down stage when it is cut by rows (half-size groups)
-constexpr int CHAIN_NORM_F4 = CHAIN_MAX_EMBD / GROUP_K / GEMV_WAVES * 32 / 64; // float4 per lane of a norm workgroup's wave: 2
 
 struct layer_args {
 	// attn_out
@@ -85,78 +84,118 @@ __device__ __forceinline__ bool give_up(int& spins, int limit, unsigned* error_w
 // The norm workgroup: the fp32 row `row` (tagged words, written by the workgroups of the stage before) -> (row * scale) * norm_w
 // -> quantize_row_q8_0 -> published blocks.  Sixteen waves; wave w takes run w of the fixed-order sum of squares (q8_0_device.h),
 // lane l the float4s l, l + 64, ... of that run -- for the sum and for the quantizer alike, so the row is read once, into registers.
+// F4: float4s per lane, 1 for rows of up to 4096 values, 2 up to CHAIN_MAX_EMBD.  (A second one that a short row leaves zero cost the quantizer's slow route:
+// 0.5 us of the 1.2 from the row's scale to its publication.)
 // The same sequence of fp32 operations as rms_norm_quantize_kernel and the mat-vec kernels' own norm, hence the same bytes.
-__device__ __forceinline__ void norm_workgroup(const uint64_t* __restrict__ row, const float* __restrict__ norm_w, uint64_t* __restrict__ out, int groups, float eps, unsigned epoch,
-	unsigned* error_word, int spin_limit, float* red, int lane, int wave) {
+template<int F4> __device__ __forceinline__ void norm_workgroup(const uint64_t* __restrict__ row, const float* __restrict__ norm_w, uint64_t* __restrict__ out, int groups, float eps, unsigned epoch,
+	unsigned* error_word, int spin_limit, float* red, uint32_t* words, int lane, int wave) {
 	const int q = groups / GEMV_WAVES, r = groups % GEMV_WAVES;
 	const int g0 = wave * q + min(wave, r);
 	const int n4 = (q + (wave < r ? 1 : 0)) * 32; // float4s in this wave's run
 	const float4* w4 = reinterpret_cast<const float4*>(norm_w) + g0 * 32;
-	float4 wv[CHAIN_NORM_F4], xf[CHAIN_NORM_F4];
+	float4 wv[F4], xf[F4];
 #pragma unroll
-	for (int i = 0; i < CHAIN_NORM_F4; ++i) {
+	for (int i = 0; i < F4; ++i) {
 		const int v = lane + 64 * i;
 		wv[i]		= v < n4 ? w4[v] : make_float4(0.f, 0.f, 0.f, 0.f);
 	}
 	const uint64_t* mine = row + static_cast<int64_t>(g0) * GROUP_K;
 	int spins			 = 0;
-	for (;;) {
-		bool fresh = true;
+	// Everything behind the wait runs once beforehand, on ones, with nothing published: no other workgroup of the launch runs this code, and fetched
+	// from memory when the row was there it was most of the time from the row to its publication.
+	int passes = 2;
+	asm volatile("" : "+s"(passes)); // one copy of the code
 #pragma unroll
-		for (int i = 0; i < CHAIN_NORM_F4; ++i) {
+	for (int i = 0; i < F4; ++i) {
+		xf[i] = lane + 64 * i < n4 ? make_float4(1.f, 1.f, 1.f, 1.f) : make_float4(0.f, 0.f, 0.f, 0.f);
+	}
+#pragma unroll 1
+	for (int pass = 1; pass <= passes; ++pass) {
+		const bool real = pass == passes;
+		if (real) {
+			for (;;) {
+				bool fresh = true;
+#pragma unroll
+				for (int i = 0; i < F4; ++i) {
+					const int v = lane + 64 * i;
+					uint64_t t[4];
+#pragma unroll
+					for (int c = 0; c < 4; ++c) {
+						t[c] = v < n4 ? __hip_atomic_load(mine + 4 * v + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : (static_cast<uint64_t>(epoch) << 32);
+					}
+#pragma unroll
+					for (int c = 0; c < 4; ++c) {
+						fresh = fresh && static_cast<unsigned>(t[c] >> 32) == epoch;
+					}
+					xf[i] = make_float4(__uint_as_float(static_cast<uint32_t>(t[0])), __uint_as_float(static_cast<uint32_t>(t[1])), __uint_as_float(static_cast<uint32_t>(t[2])),
+						__uint_as_float(static_cast<uint32_t>(t[3])));
+				}
+				if (__builtin_amdgcn_ballot_w64(!fresh) == 0) {
+					break;
+				}
+				if (give_up(spins, spin_limit, error_word, lane)) {
+					// the stage before never delivered: what is published below is NaN, and everything downstream inherits it
+#pragma unroll
+					for (int i = 0; i < F4; ++i) {
+						const float nan = __uint_as_float(0x7FC00000u);
+						xf[i]			= make_float4(nan, nan, nan, nan);
+					}
+					break;
+				}
+			}
+		}
+		float p = 0.0f;
+#pragma unroll
+		for (int i = 0; i < F4; ++i) {
+			if (lane + 64 * i < n4) {
+				p = sumsq_fold(p, xf[i]);
+			}
+		}
+		const float scale = rms_scale_workgroup(p, red, wave, lane, groups * GROUP_K, eps); // a workgroup barrier inside
+#pragma unroll
+		for (int i = 0; i < F4; ++i) {
 			const int v = lane + 64 * i;
-			uint64_t t[4];
-#pragma unroll
-			for (int c = 0; c < 4; ++c) {
-				t[c] = v < n4 ? __hip_atomic_load(mine + 4 * v + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : (static_cast<uint64_t>(epoch) << 32);
-			}
-#pragma unroll
-			for (int c = 0; c < 4; ++c) {
-				fresh = fresh && static_cast<unsigned>(t[c] >> 32) == epoch;
-			}
-			xf[i] = make_float4(__uint_as_float(static_cast<uint32_t>(t[0])), __uint_as_float(static_cast<uint32_t>(t[1])), __uint_as_float(static_cast<uint32_t>(t[2])),
-				__uint_as_float(static_cast<uint32_t>(t[3])));
-		}
-		if (__builtin_amdgcn_ballot_w64(!fresh) == 0) {
-			break;
-		}
-		if (give_up(spins, spin_limit, error_word, lane)) {
-			// the stage before never delivered: what is published below is NaN, and everything downstream inherits it
-#pragma unroll
-			for (int i = 0; i < CHAIN_NORM_F4; ++i) {
-				const float nan = __uint_as_float(0x7FC00000u);
-				xf[i]			= make_float4(nan, nan, nan, nan);
-			}
-			break;
-		}
-	}
-	float p = 0.0f;
-#pragma unroll
-	for (int i = 0; i < CHAIN_NORM_F4; ++i) {
-		if (lane + 64 * i < n4) {
-			p = sumsq_fold(p, xf[i]);
-		}
-	}
-	const float scale = rms_scale_workgroup(p, red, wave, lane, groups * GROUP_K, eps); // a workgroup barrier inside
-#pragma unroll
-	for (int i = 0; i < CHAIN_NORM_F4; ++i) {
-		const int v = lane + 64 * i;
-		uint16_t dh;
-		const uint32_t packed = quantize_block_lane(norm_mul4(xf[i], scale, wv[i]), &dh); // every lane takes part; lanes past the run hold zeros
-		if (v < n4) {
-			uint64_t* blk = out + (static_cast<int64_t>(g0) * GROUP_BLOCKS + (v >> 3)) * PUBLISHED_WORDS;
-			__hip_atomic_store(blk + (v & 7), (static_cast<uint64_t>(epoch) << 32) | packed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-			if ((v & 7) == 0) {
-				__hip_atomic_store(blk + 8, (static_cast<uint64_t>(epoch) << 32) | __float_as_uint(half_bits_to_float(dh)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+			uint16_t dh;
+			const uint32_t packed = quantize_block_lane(norm_mul4(xf[i], scale, wv[i]), &dh); // every lane takes part; lanes past the run hold zeros
+			if (v < n4) {
+				words[(v >> 3) * PUBLISHED_WORDS + (v & 7)] = packed;
+				if ((v & 7) == 0) {
+					words[(v >> 3) * PUBLISHED_WORDS + 8] = __float_as_uint(half_bits_to_float(dh));
+				}
 			}
 		}
+		__builtin_amdgcn_wave_barrier(); // the same wave wrote and reads
+		// in the order of the words, through LDS: whole lines go out
+		uint64_t* mine_out = out + static_cast<int64_t>(g0) * (GROUP_BLOCKS * PUBLISHED_WORDS);
+#pragma unroll
+		for (int i = 0; i < (F4 * 8 * PUBLISHED_WORDS + 63) / 64; ++i) {
+			const int v = lane + 64 * i;
+			if (real && v < n4 / 8 * PUBLISHED_WORDS) {
+				__hip_atomic_store(mine_out + v, (static_cast<uint64_t>(epoch) << 32) | words[v], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+			}
+		}
+		__syncthreads(); // the first pass's sums are read before the second's are written
 	}
 }
 
 // A finished row goes out twice: as the plain output tensor (read by later launches) and as a tagged word for this launch's next stage.
 __device__ __forceinline__ void store_row(float* __restrict__ y, uint64_t* __restrict__ y_tagged, unsigned epoch, int row, float v) {
-	y[row] = v;
 	__hip_atomic_store(&y_tagged[row], (static_cast<uint64_t>(epoch) << 32) | __float_as_uint(v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+	y[row] = v;
+}
+
+// A down row's residual is this launch's own attn_out row, which other workgroups have published.  It is requested at a workgroup's start, a memory latency
+// ahead of its use: published by then, as a down workgroup only becomes resident behind gate/up workgroups, which wait for all of attn_out.  Should
+// its word not be there yet, it is read again where it is used, when it is certain to be: the workgroup's activation exists only because the norm workgroup
+// read every row.  (A word that does not carry the epoch even then poisons the row.)
+__device__ __forceinline__ uint64_t request_attn_row(const uint64_t* __restrict__ attn_row, int row, bool real) {
+	return real ? __hip_atomic_load(&attn_row[row], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
+}
+__device__ __forceinline__ float attn_row_value(uint64_t word, const uint64_t* __restrict__ attn_row, int row, unsigned epoch) {
+	if (static_cast<unsigned>(word >> 32) != epoch) {
+		word = __hip_atomic_load(&attn_row[row], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+	}
+	return static_cast<unsigned>(word >> 32) == epoch ? __uint_as_float(static_cast<uint32_t>(word)) : __uint_as_float(0x7FC00000u);
 }
 
 // Every gate/up wave takes a K range of both matrices (one staged slice of the input row for the two), two groups of each at a time:
@@ -178,6 +217,8 @@ template<int CHUNKS> __global__ __launch_bounds__(GEMV_WAVES * 64) void decode_l
 		const int strip = wg;
 		int g0, g1;
 		wave_k_range(a.groups_e, 0, 0, GEMV_WAVES, wave, g0, g1);
+		const int row		   = strip * STRIP_ROWS + tid; // thread t's output; its residual is requested here, a memory latency ahead of its use
+		const float res		   = tid < STRIP_ROWS && row < a.n_embd ? a.layer_in[row] : 0.0f;
 		const uint8_t* w_strip = a.w_o + macro_offset(strip, 0, a.groups_e);
 		const int row_l		   = strip * STRIP_ROWS + (lane & 31);
 		const float acc		   = gemv_chunk<CHAIN_TILES, X_F32, DUMP_NONE, false>(w_strip, a.attn, nullptr, xs_q[wave], xs_d[wave], g0, g1 - g0, a.groups_e, lane, row_l, a.n_embd, false, 0, nullptr);
@@ -189,15 +230,14 @@ template<int CHUNKS> __global__ __launch_bounds__(GEMV_WAVES * 64) void decode_l
 			for (int w = 0; w < GEMV_WAVES; ++w) {
 				total += red[w][tid] + red[w][32 + tid];
 			}
-			const int row = strip * STRIP_ROWS + tid;
 			if (row < a.n_embd) {
-				store_row(a.ffn_inp, a.attn_row, a.epoch, row, total + a.layer_in[row]);
+				store_row(a.ffn_inp, a.attn_row, a.epoch, row, total + res);
 			}
 		}
 		return;
 	}
 	if (wg == a.first_norm) {
-		norm_workgroup(a.attn_row, a.ffn_norm_w, a.x_words, a.groups_e, a.eps, a.epoch, a.error_word, a.spin_limit, norm_red, lane, wave);
+		norm_workgroup<CHUNKS>(a.attn_row, a.ffn_norm_w, a.x_words, a.groups_e, a.eps, a.epoch, a.error_word, a.spin_limit, norm_red, reinterpret_cast<uint32_t*>(xs_q[wave]), lane, wave);
 		return;
 	}
 	if (wg < a.first_consumer) {
@@ -225,13 +265,15 @@ template<int CHUNKS> __global__ __launch_bounds__(GEMV_WAVES * 64) void decode_l
 		red[wave][lane] = acc;
 		__syncthreads();
 		if (wave == 0) {
-			if (lane < STRIP_ROWS) {
-				float g = 0.0f, u = 0.0f;
+			// lanes 0..31 add up gate's rows, lanes 32..63 up's
+			const float(*sums)[64] = lane < STRIP_ROWS ? red : red_up;
+			float total			   = 0.0f;
 #pragma unroll
-				for (int w = 0; w < GEMV_WAVES; ++w) {
-					g += red[w][lane] + red[w][32 + lane];
-					u += red_up[w][lane] + red_up[w][32 + lane];
-				}
+			for (int w = 0; w < GEMV_WAVES; ++w) {
+				total += sums[w][lane & 31] + sums[w][32 + (lane & 31)];
+			}
+			const float g = total, u = __shfl_down(total, STRIP_ROWS);
+			if (lane < STRIP_ROWS) {
 				act_f[lane]									  = silu_mul(g, u);
 				a.gate_up[strip * STRIP_ROWS + lane]				  = g; // inspection copies, not read by this launch
 				a.gate_up[FFN_MAX_HIDDEN + strip * STRIP_ROWS + lane] = u;
@@ -258,6 +300,8 @@ template<int CHUNKS> __global__ __launch_bounds__(GEMV_WAVES * 64) void decode_l
 			wave_k_range(a.groups_f, 0, 0, GEMV_WAVES, wave, g0, g1);
 			const uint8_t* w_strip = a.w_down + macro_offset(gstrip, 0, a.groups_f);
 			const int row_l		   = gstrip * STRIP_ROWS + (lane & 31);
+			const int row		   = gstrip * STRIP_ROWS + rowpart * (STRIP_ROWS / 2) + tid;
+			const uint64_t res	   = request_attn_row(a.attn_row, row, tid < STRIP_ROWS / 2 && row < a.n_embd);
 			const float acc = gemv_chunk<CHAIN_DOWN_ROWS_TILES, X_PUBLISHED_WATCH, DUMP_NONE, false, 2>(w_strip, a.act_words, a.error_word, xs_q[wave], xs_d[wave], g0, g1 - g0, a.groups_f, lane, row_l, a.n_embd, false,
 				a.epoch, nullptr, rowpart, a.spin_limit);
 			red[wave][lane] = acc;
@@ -273,11 +317,8 @@ template<int CHUNKS> __global__ __launch_bounds__(GEMV_WAVES * 64) void decode_l
 					}
 					total += part;
 				}
-				const int row = gstrip * STRIP_ROWS + rowpart * (STRIP_ROWS / 2) + tid;
 				if (row < a.n_embd) {
-					const uint64_t t = __hip_atomic_load(&a.attn_row[row], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-					const float res	 = static_cast<unsigned>(t >> 32) == a.epoch ? __uint_as_float(static_cast<uint32_t>(t)) : __uint_as_float(0x7FC00000u);
-					store_row(a.l_out, a.down_row, a.epoch, row, total + res);
+					store_row(a.l_out, a.down_row, a.epoch, row, total + attn_row_value(res, a.attn_row, row, a.epoch));
 				}
 			}
 			return;
@@ -292,8 +333,10 @@ template<int CHUNKS> __global__ __launch_bounds__(GEMV_WAVES * 64) void decode_l
 		const int gstrip   = c - split * strips_d;
 		int g0, g1;
 		wave_k_range(a.groups_f, a.split_shift, split, GEMV_WAVES, wave, g0, g1);
-		const uint8_t* w_strip = a.w_down + macro_offset(gstrip, 0, a.groups_f);
-		const int row_l		   = gstrip * STRIP_ROWS + (lane & 31);
+		const uint8_t* w_strip	   = a.w_down + macro_offset(gstrip, 0, a.groups_f);
+		const int row_l			   = gstrip * STRIP_ROWS + (lane & 31);
+		const int row			   = gstrip * STRIP_ROWS + tid;
+		const uint64_t res_word	   = request_attn_row(a.attn_row, row, tid < STRIP_ROWS && row < a.n_embd);
 		const float acc = gemv_chunk<CHAIN_TILES, X_PUBLISHED, DUMP_NONE>(w_strip, a.act_words, a.error_word, xs_q[wave], xs_d[wave], g0, g1 - g0, a.groups_f, lane, row_l, a.n_embd, false, a.epoch, nullptr, 0,
 			a.spin_limit);
 		red[wave][lane] = acc;
@@ -306,14 +349,7 @@ template<int CHUNKS> __global__ __launch_bounds__(GEMV_WAVES * 64) void decode_l
 		for (int w = 0; w < GEMV_WAVES; ++w) {
 			total += red[w][tid] + red[w][32 + tid];
 		}
-		const int row = gstrip * STRIP_ROWS + tid;
-		// the residual is this launch's own attn_out row.  Its words are final: this workgroup's activation exists only because the
-		// norm workgroup read all of them.  (A word that does not carry the epoch all the same poisons the row.)
-		float res = 0.0f;
-		if (row < a.n_embd) {
-			const uint64_t t = __hip_atomic_load(&a.attn_row[row], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-			res				 = static_cast<unsigned>(t >> 32) == a.epoch ? __uint_as_float(static_cast<uint32_t>(t)) : __uint_as_float(0x7FC00000u);
-		}
+		float res = row < a.n_embd ? attn_row_value(res_word, a.attn_row, row, a.epoch) : 0.0f;
 		if (splits == 1) {
 			if (row < a.n_embd) {
 				store_row(a.l_out, a.down_row, a.epoch, row, total + res);
@@ -347,7 +383,7 @@ template<int CHUNKS> __global__ __launch_bounds__(GEMV_WAVES * 64) void decode_l
 		return;
 	}
 	if (wg == a.second_norm) {
-		norm_workgroup(a.down_row, a.next_norm_w, a.x_words_next, a.groups_e, a.eps, a.epoch, a.error_word, a.spin_limit, norm_red, lane, wave);
+		norm_workgroup<CHUNKS>(a.down_row, a.next_norm_w, a.x_words_next, a.groups_e, a.eps, a.epoch, a.error_word, a.spin_limit, norm_red, reinterpret_cast<uint32_t*>(xs_q[wave]), lane, wave);
 		return;
 	}
 	// ---- the projections behind the next norm: rows of W_next[i] against Q(n2) ----
