@@ -32,6 +32,9 @@ namespace nh {
 constexpr int CHAIN_TILES = 4; // groups a wave stages at once: LDS slices are sized for it
 constexpr int CHAIN_DOWN_ROWS_TILES = 8; // ... in the down stage when it is cut by rows (half-size groups)
 
+constexpr int CHAIN_CUS			= 256;
+constexpr int CHAIN_HOLD_CLOCKS = 6144; // how long a held down workgroup waits before its first request
+
 struct layer_args {
 	// attn_out
 	const uint8_t* w_o;
@@ -56,6 +59,7 @@ struct layer_args {
 	int p_per_slot, p_rem; // a producer strip's K range over its waves
 	int split_shift; // a down strip's K range goes over (1 << split_shift) workgroups
 	int down_by_rows; // instead: two workgroups per down strip, each 16 rows and all of K (nothing to hand over)
+	int down_held; // down workgroups that hold their weight requests back a while
 	// scratch
 	uint64_t* attn_row; // [n_embd] {epoch, fp32}: ffn_inp as published
 	uint64_t* x_words; // [n_embd / 32][9]: Q(n1)
@@ -292,6 +296,9 @@ template<int CHUNKS> __global__ __launch_bounds__(GEMV_WAVES * 64) void decode_l
 	}
 	if (wg < a.second_norm) {
 		const int c = wg - a.first_consumer;
+		if (c < a.down_held) {
+			__builtin_amdgcn_s_sleep(CHAIN_HOLD_CLOCKS / 64); // at most 127
+		}
 		if (a.down_by_rows) {
 			// ---- 16 rows of a down strip against the whole published activation, + ffn_inp: the row is complete in this workgroup, so
 			// what the next stage waits for leaves without the two trips through memory of a K-split hand-off ----
@@ -513,6 +520,20 @@ hipError_t launch_decode_layer(const void* w_o, const float* attn, const float* 
 	a.first_producer = a.first_norm + 1;
 	a.first_consumer = a.first_producer + static_cast<int>(n_ff / STRIP_ROWS);
 	a.second_norm	 = a.first_consumer + strips_e * splits;
+	// A CU holds one workgroup.  The last round of gate/up strips leaves some CUs to the first down workgroups, which cannot work before that round is through:
+	// requested at once, their weights only take bandwidth from the strips that everybody waits for.  They hold their requests back for CHAIN_HOLD_CLOCKS
+	// (measured at the [4096 / 14336] block: 41.35 us without, 40.8 with 4096 clocks, 40.45 with 6144; without / with 6144 [4096 / 11008] 37.0 / 35.9,
+	// [3200 / 10880] 31.9 / 30.7, [4096 / 20480] 55.3 / 53.1, [7168 / 20480] 98.5 / 97.0, [8192 / 22016] 117.8 / 117.1).  Not where they are much of the chip: then their
+	// bytes are what the round has to move ([2560 / 10240] with 191 of them 24.75 / 25.2, [8192 / 18560] with 187 103.8 / 105.3, [6144 / 11008] with 167 57.0 / 58.1; up
+	// to 4096 values, whose strips are shorter, [4096 / 11008] with 167 still gains).  Nor where they are the stage, all but an eighth ([2048 / 11008] 23.1 / 23.9,
+	// [1024 / 14336] 20.8 / 22.2), or it takes a part of a second round ([6144 / 13824], 384 workgroups: 63.6 / 66.1; [2176 / 19072], 272: 35.5 / 36.9), nor behind a third
+	// round, by when the strips no longer change in step ([8192 / 28672] 143.1 / 143.9), nor for a handful ([2560 / 16256], 3: 32.8 / 33.2).
+	const int down_wgs	  = strips_e * splits;
+	const int rounds_left = a.first_consumer - a.first_producer - (CHAIN_CUS - 1); // strips behind those that start with attn_out's end or before
+	const int beside	  = (CHAIN_CUS - rounds_left % CHAIN_CUS) % CHAIN_CUS;
+	const bool held		  = rounds_left > 0 && rounds_left <= 2 * CHAIN_CUS && beside >= CHAIN_CUS / 16 && beside <= (one_chunk ? CHAIN_CUS * 11 / 16 : CHAIN_CUS / 2) && beside * 8 <= down_wgs * 7
+		&& (down_wgs <= CHAIN_CUS || down_wgs >= 2 * CHAIN_CUS);
+	a.down_held			  = held ? beside : 0;
 	a.first_next	 = a.second_norm + 1;
 	const unsigned grid = static_cast<unsigned>(next_strips > 0 ? a.first_next + next_strips : a.second_norm);
 	a.attn_row		= sc.row_tagged[0];
