@@ -89,6 +89,7 @@ constexpr int64_t GEMM_ROWS_MAX = 32;
 inline int gemm_rows_operand(int64_t M) { // operand rows the rows kernel is instantiated for
 	return M <= 8 ? 8 : M <= 16 ? 16 : M <= 24 ? 24 : 32;
 }
+// This one decides how many shares K goes over (also for the forms that stand in for this kernel); how more than 32 rows carry them out: plan_gemm_streaming.
 inline gemm_skinny_cut plan_gemm_skinny(int64_t M, int64_t N, int64_t K) {
 	gemm_skinny_cut c{};
 	const int groups	 = static_cast<int>(K / GROUP_K);
@@ -142,6 +143,45 @@ inline gemm_skinny_cut plan_gemm_skinny(int64_t M, int64_t N, int64_t K) {
 	// 117 rows) and 9.6 / 12.2 (K = 8192); at 256, 12.8 / 12.5 ([4096 x 4096] at 117 rows) and 8.5 / 8.8 (at 64).
 	c.waves	 = (units > 128 && units < 256 && groups >= 4 * SK_WAVES) ? SK_WIDE_WAVES : SK_WAVES;
 	c.splits = sets_for(c.waves);
+	return c;
+}
+
+// The streaming kernel's own mat-mats of more than 32 rows: never fewer shares of K than above, in another cut where that is faster (random shapes whose
+// cut differs: 1.08 times as fast; measured, us, cut above / this).
+// - One strip per workgroup instead of two, up to 512 workgroups of one (of three strips, whose fourth would be work for nothing, up to 640): half as many leave
+//   a part of the chip's last round idle ([4864 x 2432] at 94 rows 11.4 / 8.2, [5632 x 3968] at 72 17.3 / 13.1, [3016 x 7424] at 148 24.4 / 21.7; with five strips
+//   [3346 x 2176] at 144, 525 of one, 10.3 / 11.0).
+// - Two strips instead of one, with sixteen waves, where those fit a workgroup per CU and ones of a strip do not, from K = 5248 on: the weights cross L2 once for
+//   two strips ([7296 x 8832] at 36 rows 24.5 / 19.9, [5888 x 13568] at 48 37.8 / 31, [2658 x 14464] at 170 33.7 / 28.9; at K = 4608 11.6 / 12.0).  With more than 64
+//   rows from 360 workgroups on ([2560 x 6144] at 103 rows, 320, 12.7 / 14.1), and up to 192 ([1152 x 9856] at 310 18.4 / 19.0).
+// - Sixteen waves instead of eight for 65 to 160 workgroups and eleven to 31 groups, and for more workgroups while a wave of eight has two groups or so: all of a wave's
+//   share is on its way at once ([768 x 2048] at 104 rows 5.1 / 4.2, [1569 x 1664] at 57 5.0 / 4.3; [2048 x 2304] at 127, 256 workgroups, 5.8 / 6.0;
+//   up to 64 workgroups it may lose, [611 x 2688] at 80 rows 5.3 / 5.65).  The same instead of two workgroups of eight for 65 to 128 and up to 40
+//   groups: nothing to hand over ([1024 x 4096] at 117 rows 6.4 / 5.6, the same bits; up to 64 rows [1792 x 5120] at 35 7.35 / 8.0).
+// - Four workgroups along K instead of two for up to 64 and from 34 groups on, as a CU more costs nothing there ([457 x 6272] at 40 rows 7.8 / 6.1, [384 x 8064] at
+//   34 8.5 / 6.7).
+inline gemm_skinny_cut plan_gemm_streaming(int64_t M, int64_t N, int64_t K) {
+	gemm_skinny_cut c = plan_gemm_skinny(M, N, K);
+	if (M <= GEMM_ROWS_MAX) {
+		return c;
+	}
+	const int groups	 = static_cast<int>(K / GROUP_K);
+	const int64_t strips = (N + STRIP_ROWS - 1) / STRIP_ROWS, m_strips = (M + STRIP_ROWS - 1) / STRIP_ROWS;
+	const int64_t ones = strips * m_strips, twos = strips * ((m_strips + 1) / 2); // workgroups of one strip, of two
+	if (c.ms == 2 && c.splits == 1 && twos > 256 && ones <= (m_strips == 3 ? 640 : 512)) {
+		c.ms = 1;
+	} else if (c.ms == 1 && ones > 256 && twos < 256 && (M <= 64 || (M <= 192 && ones >= 360)) && groups >= 41 && c.splits * c.waves <= SK_WIDE_WAVES) {
+		c = gemm_skinny_cut{ 2, 1, SK_WIDE_WAVES };
+	} else if (c.ms == 1 && c.waves == SK_WAVES) {
+		if (c.splits == 1 && ones > 64 && groups >= 11 && (ones <= 160 || (ones <= 256 && groups < 18))) {
+			c.waves = SK_WIDE_WAVES;
+		} else if (c.splits == 2 && M > 64 && ones > 64 && ones <= 128 && groups <= 40) {
+			c.splits = 1;
+			c.waves	 = SK_WIDE_WAVES;
+		} else if (c.splits == 2 && ones <= 64 && groups >= 34) {
+			c.splits = 4;
+		}
+	}
 	return c;
 }
 
@@ -293,7 +333,7 @@ inline gemm_plan plan_gemm(int64_t M, int64_t N, int64_t K) {
 		p.kernel = MM_GEMM_TILE;
 	} else if (M <= GEMM_SKINNY_MAX_M || tile_workgroups <= 256) {
 		p.kernel = MM_GEMM_SKINNY;
-		p.skinny = plan_gemm_skinny(M, N, K);
+		p.skinny = plan_gemm_streaming(M, N, K);
 		if (wide) {
 			p.skinny.waves = SK_WIDE_WAVES;
 		}
@@ -370,7 +410,8 @@ inline bool plan_gate_up_with(bool even, int64_t M, int64_t n_ff, int64_t K, gat
 		return false;
 	} else {
 		const bool tree	 = g.kernel == MM_GEMM_SKINNY || (g.kernel == MM_GEMM_TILE && g.tile.kz > 1);
-		int shares		 = g.kernel == MM_GEMM_SKINNY ? g.skinny.splits * g.skinny.waves : g.tile.ks * g.tile.kz;
+		const gemm_skinny_cut own = plan_gemm_skinny(M, n_ff, K);
+		int shares				  = g.kernel == MM_GEMM_SKINNY ? own.splits * own.waves : g.tile.ks * g.tile.kz;
 		if (g.kernel != MM_GEMM_SKINNY && g.tile.kz == 1) {
 			// K does not divide over the mat-mats' sets: a second pass for the last bits only ([2 x 11008 x 4352] at 100 rows 49.4 -> 55.1 us, [2 x 24832 x 6912] at 40 rows
 			// 79.8 -> 88.2), or no single launch at all where there is one set ([2 x 41856 x 13184] at 21 rows 196 us, three launches 231)
@@ -381,8 +422,7 @@ inline bool plan_gate_up_with(bool even, int64_t M, int64_t n_ff, int64_t K, gat
 		} else if (g.kernel == MM_GEMM_TILE && shares > 2 * c.tile.ks && groups % shares != 0 && groups % c.tile.ks == 0) {
 			// Sixteen shares that differ by a group, from K over workgroups: eight, if the streaming kernel would have no more, so that a pair which is one launch
 			// with a K that sixteen divide is one here too.  ([2 x 768 x 11264] at 484 rows: 56 us, the three launches 49 through a workspace.)
-			const gemm_skinny_cut own = plan_gemm_skinny(M, n_ff, K);
-			shares					  = shares / 2 >= own.splits * own.waves ? shares / 2 : shares;
+			shares = shares / 2 >= own.splits * own.waves ? shares / 2 : shares;
 		}
 		if (K > GATE_UP_SHORT_K) {
 			c.passes = shares / c.tile.ks;
