@@ -150,7 +150,8 @@ inline gemm_skinny_cut plan_gemm_skinny(int64_t M, int64_t N, int64_t K) {
 // cut differs: 1.08 times as fast; measured, us, cut above / this).
 // - One strip per workgroup instead of two, up to 512 workgroups of one (of three strips, whose fourth would be work for nothing, up to 640): half as many leave
 //   a part of the chip's last round idle ([4864 x 2432] at 94 rows 11.4 / 8.2, [5632 x 3968] at 72 17.3 / 13.1, [3016 x 7424] at 148 24.4 / 21.7; with five strips
-//   [3346 x 2176] at 144, 525 of one, 10.3 / 11.0).
+//   [3346 x 2176] at 144, 525 of one, 10.3 / 11.0.  Also where two strips make just a workgroup per CU, if those are of eight row strips and more: two workgroups
+//   on a CU wait for their loads in turn ([1024 x 4096] at 512 rows 9.3 / 8.8, [2048 x 1024] at 256 4.9 / 4.3; [4096 x 4096] at 128 12.3 / 12.4).
 // - Two strips instead of one, with sixteen waves, where those fit a workgroup per CU and ones of a strip do not, from K = 5248 on: the weights cross L2 once for
 //   two strips ([7296 x 8832] at 36 rows 24.5 / 19.9, [5888 x 13568] at 48 37.8 / 31, [2658 x 14464] at 170 33.7 / 28.9; at K = 4608 11.6 / 12.0).  With more than 64
 //   rows from 360 workgroups on ([2560 x 6144] at 103 rows, 320, 12.7 / 14.1), and up to 192 ([1152 x 9856] at 310 18.4 / 19.0).
@@ -168,7 +169,7 @@ inline gemm_skinny_cut plan_gemm_streaming(int64_t M, int64_t N, int64_t K) {
 	const int groups	 = static_cast<int>(K / GROUP_K);
 	const int64_t strips = (N + STRIP_ROWS - 1) / STRIP_ROWS, m_strips = (M + STRIP_ROWS - 1) / STRIP_ROWS;
 	const int64_t ones = strips * m_strips, twos = strips * ((m_strips + 1) / 2); // workgroups of one strip, of two
-	if (c.ms == 2 && c.splits == 1 && twos > 256 && ones <= (m_strips == 3 ? 640 : 512)) {
+	if (c.ms == 2 && c.splits == 1 && (twos > 256 || (twos == 256 && m_strips >= 8)) && ones <= (m_strips == 3 ? 640 : 512)) {
 		c.ms = 1;
 	} else if (c.ms == 1 && ones > 256 && twos < 256 && (M <= 64 || (M <= 192 && ones >= 360)) && groups >= 41 && c.splits * c.waves <= SK_WIDE_WAVES) {
 		c = gemm_skinny_cut{ 2, 1, SK_WIDE_WAVES };
