@@ -273,8 +273,23 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 	const int half	   = lane >> 5;
 	const int m_strips = (M + 31) / 32;
 	const int n_strips = (N + 31) / 32;
-	const int ms0	   = blockIdx.y * TM;
-	const int ns	   = GATE_UP ? blockIdx.x * 2 + (wave & 1) : blockIdx.x * 4 + wave;
+	int bx = blockIdx.x, by = blockIdx.y; // block of weight strips, group of activation strips
+	if constexpr (!GATE_UP && !SPLIT && !STREAM) {
+		// Workgroups go to the eight XCDs in turn.  With a number of column blocks that eight divides, a block's row groups are all on one XCD, whose L2 has its weights
+		// then; otherwise every XCD would read nearly all of them ([24171 x 10240] at 145 rows 162 us, [3117 x 10752] at 912 101).  There each XCD takes the tiles of
+		// some consecutive column blocks instead, row groups fastest: 126 and 92 us, 106 random shapes of that kind 1.09 times as fast (with the one-strip
+		// form for some of them, q8_0_plan.h, which needs this: 182 and 134 us without).  Not with eight dividing: a round of workgroups is a wider piece of the
+		// matrix then as it is ([8192 x 8192] at 330 rows 72 us, 76 this way).
+		const unsigned gx = static_cast<unsigned>(n_strips + 3) / 4, gy = static_cast<unsigned>(m_strips + TM - 1) / TM;
+		if (gx % 8 != 0 && gy > 1) {
+			const unsigned total = gx * gy, id = by * gx + bx, xcd = id % 8;
+			const unsigned t	 = xcd * (total / 8) + min(xcd, total % 8) + id / 8; // XCDs 0 .. total % 8 - 1 have one more
+			bx					 = __builtin_amdgcn_readfirstlane(static_cast<int>(t / gy));
+			by					 = __builtin_amdgcn_readfirstlane(static_cast<int>(t % gy));
+		}
+	}
+	const int ms0	   = by * TM;
+	const int ns	   = GATE_UP ? bx * 2 + (wave & 1) : bx * 4 + wave;
 	const uint8_t* Wm  = (GATE_UP && wave >= 2) ? W2 : W; // wave-uniform
 	// every address below is a wave-uniform part (scalar registers, advanced by scalar adds) plus one of three lane constants
 	uint32_t lane16 = 16u * lane;
@@ -533,7 +548,7 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 				// counts itself in, and the last to arrive adds the tiles in z order -- whoever that is -- and stores
 				__shared__ int last_flag;
 				const int kz_count = static_cast<int>(gridDim.z);
-				const int unit	   = static_cast<int>(blockIdx.y * gridDim.x + blockIdx.x);
+				const int unit	   = static_cast<int>(by * gridDim.x + bx);
 				constexpr int TILE_FLOATS = 4 * KS * TM * PER * 64; // = TM * 4096: a workgroup's tile
 				float* tile = partials + (static_cast<int64_t>(unit) * kz_count) * TILE_FLOATS + wave_all * (TM * PER * 64) + lane;
 				float* dst	= tile + static_cast<int64_t>(blockIdx.z) * TILE_FLOATS;

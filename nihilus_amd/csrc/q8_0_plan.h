@@ -71,12 +71,25 @@ inline gemm_tile_cut plan_gemm_tile(int64_t M, int64_t N, int64_t K, bool stream
 //                                 [4096 x 6912] at 512 43.2 / 40.9, [24832 x 5376] at 64 38.2 / 34.9.  One strip [32000 x 6400] at 24 38.4 / 40.0
 //   one set / two uneven          [60032 x 1152] at 64 rows 21.4 / 25.3, [16640 x 1920] at 117 25.3 / 26.9, [28672 x 2176] at 117 31.2 / 30.3; one strip
 //                                 [40064 x 1152] at 24 12.7 / 14.6, [60032 x 7296] 72.8 / 74.4
-inline gemm_tile_cut gemm_tile_mat_mat(gemm_tile_cut c, int groups) {
+inline gemm_tile_cut gemm_tile_mat_mat(gemm_tile_cut c, int groups, int64_t m_strips, bool stream) {
 	if (c.ks == 4 && c.kz == 1 && groups % 4 == 2 && (c.tm == 1 || groups < 40)) {
 		c.ks = 2;
 	}
 	if (c.ks == 2 && groups % 2 != 0 && static_cast<int64_t>(c.grid_x) * c.grid_y > 256 && (c.tm == 1 || groups < 24)) {
 		c.ks = 1;
+	}
+	// One activation strip per wave, twice the workgroups, where two leave the chip's last round mostly idle: a little more than one round of workgroups, or than two.
+	// Weight tiles are fetched twice as often then, which costs 8 % in a grid that is full anyway.  Measured, us, two strips / one: 272 to 376 workgroups [1024 x 4096]
+	// at 2100 / 3001 rows 39.5 / 35.6 and 42.5 / 38.2, [4096 x 14336] at 600 126 / 118, [4096 x 1024] at 740 13.7 / 12.3, [8192 x 8192] at 330 80 / 74, [14336 x 4096] at 160 41 / 39
+	// (with four strips in all the weights come from memory for most of them: [20480 x 4096] at 100 41 / 43); 544 to 576 [4096 x 4096] at 1050 62.2 / 58.8, [4096 x 14336] at 1100
+	// 205 / 195, [8192 x 8192] at 520 122 / 116; but 640 [16384 x 4096] at 300 67.3 / 67.8, 800 [4096 x 4096] at 1600 82 / 83.
+	const int64_t wgs = static_cast<int64_t>(c.grid_x) * c.grid_y;
+	if (!stream && c.tm == 2 && c.kz == 1 && m_strips > 4 && ((wgs > 256 && wgs <= 384) || (wgs > 512 && wgs <= 608))) {
+		c.tm	 = 1;
+		c.grid_y = static_cast<unsigned>(m_strips);
+		if (c.ks == 1 && groups >= 8 && groups % 2 == 0) {
+			c.ks = 2; // two waves on a SIMD of every CU
+		}
 	}
 	return c;
 }
@@ -150,7 +163,7 @@ inline gemm_skinny_cut plan_gemm_skinny(int64_t M, int64_t N, int64_t K) {
 // cut differs: 1.08 times as fast; measured, us, cut above / this).
 // - One strip per workgroup instead of two, up to 512 workgroups of one (of three strips, whose fourth would be work for nothing, up to 640): half as many leave
 //   a part of the chip's last round idle ([4864 x 2432] at 94 rows 11.4 / 8.2, [5632 x 3968] at 72 17.3 / 13.1, [3016 x 7424] at 148 24.4 / 21.7; with five strips
-//   [3346 x 2176] at 144, 525 of one, 10.3 / 11.0.  Also where two strips make just a workgroup per CU, if those are of eight row strips and more: two workgroups
+//   [3346 x 2176] at 144, 525 of one, 10.3 / 11.0).  Also where two strips make just a workgroup per CU, if those are of eight row strips and more: two workgroups
 //   on a CU wait for their loads in turn ([1024 x 4096] at 512 rows 9.3 / 8.8, [2048 x 1024] at 256 4.9 / 4.3; [4096 x 4096] at 128 12.3 / 12.4).
 // - Two strips instead of one, with sixteen waves, where those fit a workgroup per CU and ones of a strip do not, from K = 5248 on: the weights cross L2 once for
 //   two strips ([7296 x 8832] at 36 rows 24.5 / 19.9, [5888 x 13568] at 48 37.8 / 31, [2658 x 14464] at 170 33.7 / 28.9; at K = 4608 11.6 / 12.0).  With more than 64
@@ -329,7 +342,7 @@ inline gemm_plan plan_gemm(int64_t M, int64_t N, int64_t K) {
 	}
 	if (stream_tile) {
 		p.kernel = MM_GEMM_TILE_STREAM;
-		p.tile	 = gemm_tile_mat_mat(plan_gemm_tile(M, N, K, true), static_cast<int>(K / GROUP_K));
+		p.tile	 = gemm_tile_mat_mat(plan_gemm_tile(M, N, K, true), static_cast<int>(K / GROUP_K), (M + 31) / 32, true);
 	} else if (M > GEMM_SKINNY_MAX_M && tile_workgroups <= 256 && plan_gemm_tile_split(M, N, K, &p.tile, &p.skinny)) {
 		p.kernel = MM_GEMM_TILE;
 	} else if (M <= GEMM_SKINNY_MAX_M || tile_workgroups <= 256) {
@@ -341,7 +354,7 @@ inline gemm_plan plan_gemm(int64_t M, int64_t N, int64_t K) {
 		p.rows = gemm_rows_suits(M, N, K) && gemm_rows_fits(M, N, p.skinny);
 	} else {
 		p.kernel = MM_GEMM_TILE;
-		p.tile	 = gemm_tile_mat_mat(plan_gemm_tile(M, N, K, false), static_cast<int>(K / GROUP_K));
+		p.tile	 = gemm_tile_mat_mat(plan_gemm_tile(M, N, K, false), static_cast<int>(K / GROUP_K), (M + 31) / 32, false);
 	}
 	return p;
 }
