@@ -274,13 +274,12 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 	const int m_strips = (M + 31) / 32;
 	const int n_strips = (N + 31) / 32;
 	int bx = blockIdx.x, by = blockIdx.y; // block of weight strips, group of activation strips
-	if constexpr (!GATE_UP && !SPLIT && !STREAM) {
+	if constexpr (!SPLIT && !STREAM) {
 		// Workgroups go to the eight XCDs in turn.  With a number of column blocks that eight divides, a block's row groups are all on one XCD, whose L2 has its weights
-		// then; otherwise every XCD would read nearly all of them ([24171 x 10240] at 145 rows 162 us, [3117 x 10752] at 912 101).  There each XCD takes the tiles of
-		// some consecutive column blocks instead, row groups fastest: 126 and 92 us, 106 random shapes of that kind 1.09 times as fast (with the one-strip
-		// form for some of them, q8_0_plan.h, which needs this: 182 and 134 us without).  Not with eight dividing: a round of workgroups is a wider piece of the
-		// matrix then as it is ([8192 x 8192] at 330 rows 72 us, 76 this way).
-		const unsigned gx = static_cast<unsigned>(n_strips + 3) / 4, gy = static_cast<unsigned>(m_strips + TM - 1) / TM;
+		// then; otherwise every XCD would read nearly all of them.  There each XCD takes the tiles of some consecutive column blocks instead, row groups fastest
+		// ([24171 x 10240] at 145 rows 182 -> 126 us, [3117 x 10752] at 912 134 -> 92, [2 x 3968 x 6528] at 274 77 -> 59 with one strip per wave; with two, 50 random shapes
+		// 1.02 times as fast).  Not with eight dividing: a round of workgroups is a wider piece of the matrix then as it is ([8192 x 8192] at 330 rows 72 us, 76 this way).
+		const unsigned gx = static_cast<unsigned>(GATE_UP ? (n_strips + 1) / 2 : (n_strips + 3) / 4), gy = static_cast<unsigned>(m_strips + TM - 1) / TM;
 		if (gx % 8 != 0 && gy > 1) {
 			const unsigned total = gx * gy, id = by * gx + bx, xcd = id % 8;
 			const unsigned t	 = xcd * (total / 8) + min(xcd, total % 8) + id / 8; // XCDs 0 .. total % 8 - 1 have one more
@@ -790,6 +789,9 @@ hipError_t launch_gemm_gate_up_silu(const void* w_gate, const void* w_up, const 
 			return launch_kernel(KIND_GEMM, kernel, grid, dim3(static_cast<unsigned>(256 * t.ks)), 0, s, static_cast<const uint8_t*>(w_gate), static_cast<const uint8_t*>(w_up), static_cast<const uint8_t*>(aq),
 				static_cast<int>(M), static_cast<int>(n_ff), static_cast<int>(K / GROUP_K), cut.passes, cut.tree, static_cast<uint8_t*>(act_out), gate_dbg, up_dbg);
 		};
+		if (t.tm == 1 && t.grid_y > 1) {
+			return t.ks == 1 ? launch(gemm_gate_up_kernel<1, 1, false, false>) : cut.passes > 1 ? launch(gemm_gate_up_kernel<1, 2, false, true>) : launch(gemm_gate_up_kernel<1, 2, false, false>);
+		}
 		if (t.tm == 1) { // 17 to 32 rows on matrices of 192 column blocks and more (the rows kernel has the others)
 			return t.ks == 1 ? launch(gemm_gate_up_kernel<1, 1, true, false>) : cut.passes > 1 ? launch(gemm_gate_up_kernel<1, 2, true, true>) : launch(gemm_gate_up_kernel<1, 2, true, false>);
 		}

@@ -64,6 +64,26 @@ inline gemm_tile_cut plan_gemm_tile(int64_t M, int64_t N, int64_t K, bool stream
 	return c;
 }
 
+// One activation strip per wave instead of two where that fills the chip's last round better: twice the workgroups of half the work, and no second strip that is none
+// where their number is odd.  `percent`: what a round of them takes of a half round of the others, as weight tiles are fetched twice as often.  Measured, us, two strips / one:
+//   mat-mats  [1024 x 4096] at 3001 rows (three half rounds for two rounds) 42.5 / 38.2, [4096 x 14336] at 600 126 / 118, [4096 x 1024] at 740 13.7 / 12.3, [8192 x 8192] at 330
+//             80 / 72, [19712 x 3456] at 81 37.0 / 26.4; [4096 x 4096] at 1050 (five for three) 62.2 / 58.8, [8192 x 8192] at 520 122 / 116; [26752 x 6784] at 201 (six for four)
+//             140 / 121; but seven for four [10496 x 3072] at 640 63.4 / 65.0, [25472 x 1024] at 234 27.0 / 29.4
+//   gate/up   [2 x 1280 x 1280] at 788 rows (three for two) 32 / 20, [2 x 8960 x 5760] at 233 (five for three) 96 / 94, [2 x 2560 x 4608] at 787 79 / 58, [2 x 5248 x 3200] at 578
+//             (seven for four) 72.6 / 68.5, [2 x 17792 x 4096] at 266 (ten for six) 142 / 128, [2 x 10368 x 7936] at 543 (eleven for six) 257 / 252; but with the same number
+//             [2 x 5376 x 2048] at 326 30.8 / 33.4, and thirteen for seven [2 x 25600 x 5248] at 243 210 / 302
+// Not with four strips, whose weights come from memory for most of them ([20480 x 4096] at 100 rows 41 / 43, [2 x 9344 x 7808] at 119 78 / 80).
+constexpr int ONE_STRIP_MAT_MAT = 115, ONE_STRIP_GATE_UP = 108;
+inline bool gemm_tile_take_one_strip(gemm_tile_cut* c, int64_t m_strips, int percent) {
+	const int64_t twos = int64_t{ c->grid_x } * c->grid_y, ones = int64_t{ c->grid_x } * m_strips;
+	if (c->tm != 2 || c->kz != 1 || m_strips <= 2 || m_strips == 4 || twos <= 256 || (ones + 255) / 256 * percent > (twos + 255) / 256 * 200) {
+		return false;
+	}
+	c->tm	  = 1;
+	c->grid_y = static_cast<unsigned>(m_strips);
+	return true;
+}
+
 // The tile kernel's cut for a mat-mat of its own (K not over workgroups).  Uneven sets walk as many trips as the longest, so short ones multiply up to a tenth
 // more for nothing, and behind two sets, or more workgroups than CUs, there are two waves on a SIMD already.  Measured, us:
 //   two even sets / four uneven   [4096 x 2304] at 512 rows 16.1 / 17.1, [8064 x 2816] at 200 22.9 / 25.5, [2048 x 3328] at 1000 22.8 / 23.1; of streamed weights
@@ -78,18 +98,8 @@ inline gemm_tile_cut gemm_tile_mat_mat(gemm_tile_cut c, int groups, int64_t m_st
 	if (c.ks == 2 && groups % 2 != 0 && static_cast<int64_t>(c.grid_x) * c.grid_y > 256 && (c.tm == 1 || groups < 24)) {
 		c.ks = 1;
 	}
-	// One activation strip per wave, twice the workgroups, where two leave the chip's last round mostly idle: a little more than one round of workgroups, or than two.
-	// Weight tiles are fetched twice as often then, which costs 8 % in a grid that is full anyway.  Measured, us, two strips / one: 272 to 376 workgroups [1024 x 4096]
-	// at 2100 / 3001 rows 39.5 / 35.6 and 42.5 / 38.2, [4096 x 14336] at 600 126 / 118, [4096 x 1024] at 740 13.7 / 12.3, [8192 x 8192] at 330 80 / 74, [14336 x 4096] at 160 41 / 39
-	// (with four strips in all the weights come from memory for most of them: [20480 x 4096] at 100 41 / 43); 544 to 576 [4096 x 4096] at 1050 62.2 / 58.8, [4096 x 14336] at 1100
-	// 205 / 195, [8192 x 8192] at 520 122 / 116; but 640 [16384 x 4096] at 300 67.3 / 67.8, 800 [4096 x 4096] at 1600 82 / 83.
-	const int64_t wgs = static_cast<int64_t>(c.grid_x) * c.grid_y;
-	if (!stream && c.tm == 2 && c.kz == 1 && m_strips > 4 && ((wgs > 256 && wgs <= 384) || (wgs > 512 && wgs <= 608))) {
-		c.tm	 = 1;
-		c.grid_y = static_cast<unsigned>(m_strips);
-		if (c.ks == 1 && groups >= 8 && groups % 2 == 0) {
-			c.ks = 2; // two waves on a SIMD of every CU
-		}
+	if (!stream && gemm_tile_take_one_strip(&c, m_strips, ONE_STRIP_MAT_MAT) && c.ks == 1 && groups >= 8 && groups % 2 == 0 && c.grid_x * m_strips <= 1280) {
+		c.ks = 2; // so few of them are less than four waves on a SIMD ([4096 x 4096] at 1100 rows 59.7 / 58.8; at 1600, seven rounds, 80.8 / 83.4)
 	}
 	return c;
 }
@@ -455,6 +465,9 @@ inline bool plan_gate_up_with(bool even, int64_t M, int64_t n_ff, int64_t K, gat
 				return false;
 			}
 		}
+	}
+	if (c.tile.ks <= 2) {
+		gemm_tile_take_one_strip(&c.tile, (M + STRIP_ROWS - 1) / STRIP_ROWS, ONE_STRIP_GATE_UP);
 	}
 	if (cut) {
 		*cut = c;
