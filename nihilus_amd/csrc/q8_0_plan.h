@@ -70,10 +70,10 @@ inline gemm_tile_cut plan_gemm_tile(int64_t M, int64_t N, int64_t K, bool stream
 //             80 / 72, [19712 x 3456] at 81 37.0 / 26.4; [4096 x 4096] at 1050 (five for three) 62.2 / 58.8, [8192 x 8192] at 520 122 / 116; [26752 x 6784] at 201 (six for four)
 //             140 / 121; but seven for four [10496 x 3072] at 640 63.4 / 65.0, [25472 x 1024] at 234 27.0 / 29.4
 //   gate/up   [2 x 1280 x 1280] at 788 rows (three for two) 32 / 20, [2 x 8960 x 5760] at 233 (five for three) 96 / 94, [2 x 2560 x 4608] at 787 79 / 58, [2 x 5248 x 3200] at 578
-//             (seven for four) 72.6 / 68.5, [2 x 17792 x 4096] at 266 (ten for six) 142 / 128, [2 x 10368 x 7936] at 543 (eleven for six) 257 / 252; but with the same number
-//             [2 x 5376 x 2048] at 326 30.8 / 33.4, and thirteen for seven [2 x 25600 x 5248] at 243 210 / 302
+//             (seven for four) 72.6 / 68.5, [2 x 17792 x 4096] at 266 (ten for six) 142 / 128; but with eleven for six [2 x 28672 x 8192] at 178 261 / 274,
+//             [2 x 22016 x 5632] at 236 181 / 189, [2 x 5376 x 2048] at 326 30.8 / 33.4 ([2 x 10368 x 7936] at 543 257 / 252), thirteen for seven [2 x 25600 x 5248] at 243 210 / 302
 // Not with four strips, whose weights come from memory for most of them ([20480 x 4096] at 100 rows 41 / 43, [2 x 9344 x 7808] at 119 78 / 80).
-constexpr int ONE_STRIP_MAT_MAT = 115, ONE_STRIP_GATE_UP = 108;
+constexpr int ONE_STRIP_MAT_MAT = 115, ONE_STRIP_GATE_UP = 110;
 inline bool gemm_tile_take_one_strip(gemm_tile_cut* c, int64_t m_strips, int percent) {
 	const int64_t twos = int64_t{ c->grid_x } * c->grid_y, ones = int64_t{ c->grid_x } * m_strips;
 	if (c->tm != 2 || c->kz != 1 || m_strips <= 2 || m_strips == 4 || twos <= 256 || (ones + 255) / 256 * percent > (twos + 255) / 256 * 200) {
@@ -82,6 +82,19 @@ inline bool gemm_tile_take_one_strip(gemm_tile_cut* c, int64_t m_strips, int per
 	c->tm	  = 1;
 	c->grid_y = static_cast<unsigned>(m_strips);
 	return true;
+}
+
+// The order of the tile kernel's tiles where eight divides the number of column blocks (the kernel has one of its own for others): column blocks per band, whose row groups
+// are all done before the next band is begun, 0 for one band.  With one, every group of rows walks the whole matrix, from memory again where it is no longer cached, and the
+// workgroups that run together share only their activations; a band's weights are still in its XCDs' L2 when the next row group comes.  Measured, us, one band / this:
+//   gate/up   [2 x 28672 x 8192] at 512 rows 745 / 598, at 178 two strips 293 / 261; [2 x 14336 x 4096] at 512 / 3001 170 / 162, 938 / 881; [2 x 26624 x 9344] at 858 1394 / 1062;
+//             with one strip per wave [2 x 21504 x 7808] at 200 318 / 226, [2 x 24576 x 1920] at 273 122 / 89
+//   mat-mats  [27648 x 4736] at 1058 363 / 344, [20475 x 9984] at 1965 980 / 941, [25530 x 6784] at 738 343 / 326
+// Bands of 16 to 64 column blocks are within 1 % of each other.  Below 128 nothing changes ([2 x 5632 x 7680] at 660 rows 159 / 161, [9146 x 9216] at 326 88.5 / 88.5), and two
+// row groups of a mat-mat find each other's weights on their way as it is ([22528 x 2944] at 118 rows 32.8 / 34.2; gate / up [2 x 24064 x 8320] at 125 159 / 153).
+constexpr int GEMM_TILE_BAND = 32;
+inline int gemm_tile_band(const gemm_tile_cut& c, bool gate_up) {
+	return c.grid_x % 8 == 0 && c.grid_x >= 128 && c.grid_y > (gate_up ? 1u : 2u) && c.kz == 1 ? GEMM_TILE_BAND : 0;
 }
 
 // The tile kernel's cut for a mat-mat of its own (K not over workgroups).  Uneven sets walk as many trips as the longest, so short ones multiply up to a tenth
