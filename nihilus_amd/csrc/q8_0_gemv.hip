@@ -139,20 +139,6 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_tiled_kernel(gemv_segmen
 	wave_k_range(groups, RS > 1 ? 0 : split_shift, split, GEMV_WAVES, wave, g0, g1);
 
 	const uint8_t* w_strip = DUMP == DUMP_X ? nullptr : seg.W[sidx] + macro_offset(strip, 0, groups);
-	// thread t stores row t of the workgroup's; its residual (which may be that output) is requested here, a memory latency ahead of its use (with the norm, whose
-	// launches have none and whose long walks no register for it, in front of the reduction)
-	constexpr int PART_ROWS = STRIP_ROWS / RS; // rows this workgroup owns: 64 / PART_ROWS lanes of every wave hold a share of each
-	const int row			= strip * STRIP_ROWS + rowpart * PART_ROWS + tid;
-	const float* residual	= DUMP == DUMP_NONE ? seg.residual[sidx] : nullptr;
-	float res				= 0.0f;
-	const auto request_residual = [&] {
-		if (residual && tid < PART_ROWS && row < N) {
-			res = residual[row];
-		}
-	};
-	if constexpr (!NORM) {
-		request_residual();
-	}
 	const int row_l		   = strip * STRIP_ROWS + (lane & 31);
 	float acc			   = 0.0f;
 	// the wave's K range, in one piece when the host picked splits so that g1 - g0 <= TILES (straight-line code, every load of the
@@ -198,8 +184,15 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_tiled_kernel(gemv_segmen
 		return;
 	}
 
-	if constexpr (NORM) {
-		request_residual();
+	// Thread t stores row t of the workgroup's; its residual (which may be that output) is requested here, in front of the reduction.  Not at the launch's start:
+	// there the look at its pointer holds the weight loads up ([1024 x 8192] without one 4.77 us with the read behind the reduction, 4.90 at the start, 4.80 here;
+	// with one 4.87 / 4.90 / 4.78; [4096 x 14336] with one 11.55 / 11.47 / 11.51).
+	constexpr int PART_ROWS = STRIP_ROWS / RS; // rows this workgroup owns: 64 / PART_ROWS lanes of every wave hold a share of each
+	const int row			= strip * STRIP_ROWS + rowpart * PART_ROWS + tid;
+	const float* residual	= seg.residual[sidx];
+	float res				= 0.0f;
+	if (residual && tid < PART_ROWS && row < N) {
+		res = residual[row];
 	}
 	// ---- one reduction per workgroup, fixed order ----
 	red[wave][lane] = acc;
