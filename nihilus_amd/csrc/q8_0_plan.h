@@ -197,8 +197,13 @@ inline gemm_skinny_cut plan_gemm_skinny(int64_t M, int64_t N, int64_t K) {
 //   groups: nothing to hand over ([1024 x 4096] at 117 rows 6.4 / 5.6, the same bits; up to 64 rows [1792 x 5120] at 35 7.35 / 8.0).
 // - Four workgroups along K instead of two for up to 64 and from 34 groups on, as a CU more costs nothing there ([457 x 6272] at 40 rows 7.8 / 6.1, [384 x 8064] at
 //   34 8.5 / 6.7).
+// Not in more shares where gate / up of such a pair are one launch, which has no room for sixteen (plan_gate_up_with): one launch and three give the same bytes
+// there (one in a hundred of the pairs whose mat-mats run here: [2 x 2688 x 2048] at 69 rows, [2 x 3840 x 6144] at 98), and
+// the mat-mats cost no more: 40 random ones of those with sixteen shares / these 0.91 to 1.09, mean 1.01.
+inline bool gate_up_one_launch_beside(const gemm_skinny_cut& mat_mat, int64_t M, int64_t n_ff, int64_t K); // below
 inline gemm_skinny_cut plan_gemm_streaming(int64_t M, int64_t N, int64_t K) {
-	gemm_skinny_cut c = plan_gemm_skinny(M, N, K);
+	const gemm_skinny_cut own = plan_gemm_skinny(M, N, K);
+	gemm_skinny_cut c		  = own;
 	if (M <= GEMM_ROWS_MAX) {
 		return c;
 	}
@@ -218,6 +223,9 @@ inline gemm_skinny_cut plan_gemm_streaming(int64_t M, int64_t N, int64_t K) {
 		} else if (c.splits == 2 && ones <= 64 && groups >= 34) {
 			c.splits = 4;
 		}
+	}
+	if (c.splits * c.waves != own.splits * own.waves && gate_up_one_launch_beside(own, M, N, K)) {
+		return own;
 	}
 	return c;
 }
@@ -423,14 +431,14 @@ struct gate_up_cut {
 	bool tree; // eight shares in two passes, added as the streaming kernel adds them
 };
 constexpr int64_t GATE_UP_MIN_WAVES = 2048, GATE_UP_MIN_WAVES_SMALL = 1100, GATE_UP_SMALL_WEIGHTS = 48ll << 20, GATE_UP_SHORT_K = 1024, GATE_UP_UNEVEN_MIN_GROUPS = 12;
-inline bool plan_gate_up_with(bool even, int64_t M, int64_t n_ff, int64_t K, gate_up_cut* cut) { // even: no more sets than K divides over
+// even: no more sets than K divides over; g: the mat-mats it stands for
+inline bool plan_gate_up_with(bool even, const gemm_plan& g, int64_t M, int64_t n_ff, int64_t K, gate_up_cut* cut) {
 	if (M <= 0 || n_ff <= 0 || K <= 0 || n_ff % GROUP_K != 0 || K % GROUP_K != 0) {
 		return false;
 	}
 	gate_up_cut c{ {}, 1, false };
 	c.tile			  = plan_gemm_tile(M, 2 * n_ff, K, false); // grid_x = n_ff / 64 workgroups of two gate and two up strips
 	const int groups  = static_cast<int>(K / GROUP_K);
-	const gemm_plan g = plan_gemm(M, n_ff, K);
 	while (even && groups % c.tile.ks != 0) {
 		c.tile.ks /= 2;
 	}
@@ -447,8 +455,7 @@ inline bool plan_gate_up_with(bool even, int64_t M, int64_t n_ff, int64_t K, gat
 		return false;
 	} else {
 		const bool tree	 = g.kernel == MM_GEMM_SKINNY || (g.kernel == MM_GEMM_TILE && g.tile.kz > 1);
-		const gemm_skinny_cut own = plan_gemm_skinny(M, n_ff, K);
-		int shares				  = g.kernel == MM_GEMM_SKINNY ? own.splits * own.waves : g.tile.ks * g.tile.kz;
+		int shares		 = g.kernel == MM_GEMM_SKINNY ? g.skinny.splits * g.skinny.waves : g.tile.ks * g.tile.kz;
 		if (g.kernel != MM_GEMM_SKINNY && g.tile.kz == 1) {
 			// K does not divide over the mat-mats' sets: a second pass for the last bits only ([2 x 11008 x 4352] at 100 rows 49.4 -> 55.1 us, [2 x 24832 x 6912] at 40 rows
 			// 79.8 -> 88.2), or no single launch at all where there is one set ([2 x 41856 x 13184] at 21 rows 196 us, three launches 231)
@@ -459,7 +466,8 @@ inline bool plan_gate_up_with(bool even, int64_t M, int64_t n_ff, int64_t K, gat
 		} else if (g.kernel == MM_GEMM_TILE && shares > 2 * c.tile.ks && groups % shares != 0 && groups % c.tile.ks == 0) {
 			// Sixteen shares that differ by a group, from K over workgroups: eight, if the streaming kernel would have no more, so that a pair which is one launch
 			// with a K that sixteen divide is one here too.  ([2 x 768 x 11264] at 484 rows: 56 us, the three launches 49 through a workspace.)
-			shares = shares / 2 >= own.splits * own.waves ? shares / 2 : shares;
+			const gemm_skinny_cut own = plan_gemm_skinny(M, n_ff, K);
+			shares					  = shares / 2 >= own.splits * own.waves ? shares / 2 : shares;
 		}
 		if (K > GATE_UP_SHORT_K) {
 			c.passes = shares / c.tile.ks;
@@ -488,7 +496,12 @@ inline bool plan_gate_up_with(bool even, int64_t M, int64_t n_ff, int64_t K, gat
 	return true;
 }
 inline bool plan_gate_up_fused(int64_t M, int64_t n_ff, int64_t K, gate_up_cut* cut = nullptr) {
-	return plan_gate_up_with(false, M, n_ff, K, cut) || plan_gate_up_with(true, M, n_ff, K, cut);
+	const gemm_plan g = plan_gemm(M, n_ff, K);
+	return plan_gate_up_with(false, g, M, n_ff, K, cut) || plan_gate_up_with(true, g, M, n_ff, K, cut);
+}
+inline bool gate_up_one_launch_beside(const gemm_skinny_cut& mat_mat, int64_t M, int64_t n_ff, int64_t K) {
+	const gemm_plan g{ MM_GEMM_SKINNY, {}, mat_mat, false };
+	return plan_gate_up_with(false, g, M, n_ff, K, nullptr) || plan_gate_up_with(true, g, M, n_ff, K, nullptr);
 }
 
 // The MFMA mat-vec's cut (q8_0_gemv_rows_mfma.hip): K over workgroups until a wave owns at most two groups (one with the

@@ -110,9 +110,11 @@ def test_gate_up_silu_k_sets(q8, oracle, m, n_ff, k):
 
 # One launch, the bytes of the three it stands for: four K sets in two passes as two workgroups' sums (40 rows: K over two workgroups per
 # tile in the mat-mats) and as the streaming kernel's tree, with even shares, with shares that differ by a group, and for mat-mats with K
-# over workgroups; two K sets in two passes, of two row strips and of one; one pass.  Infinite scales at the ends of the shares: what
+# over workgroups; two K sets in two passes, of two row strips and of one; one pass; shapes on which the streaming kernel would have sixteen shares
+# of K if there were no such launch.  Infinite scales at the ends of the shares: what
 # stands for the group that a smaller share does not have must add nothing to them.
-@pytest.mark.parametrize("m,n_ff,k", [(40, 12800, 4096), (64, 4608, 2048), (64, 4608, 2560), (97, 2304, 4608), (66, 4224, 5120), (64, 24576, 2048), (33, 24576, 2048), (24, 24576, 2048), (100, 12288, 512)])
+@pytest.mark.parametrize("m,n_ff,k", [(40, 12800, 4096), (64, 4608, 2048), (64, 4608, 2560), (97, 2304, 4608), (66, 4224, 5120), (64, 24576, 2048), (33, 24576, 2048), (24, 24576, 2048), (100, 12288, 512),
+                                        (69, 2688, 2048), (75, 2560, 2048), (57, 4736, 5248), (98, 3840, 6144), (115, 3712, 6144), (148, 2432, 9728)])
 def test_gate_up_silu_has_the_bytes_of_three_launches(q8, oracle, m, n_ff, k):
     assert q8._lib.lib().nh_q8_0_gate_up_silu_workspace_bytes(m, n_ff, k) == 0
     tg, tu = (q8.tile(q8.fill_weight_blocks(s + m, n_ff, k), n_ff, k) for s in (31, 32))

@@ -127,6 +127,19 @@ def test_k_that_no_number_of_sets_divides():
     assert size(65, 3712, 11648) > 0 and size(58, 6400, 2304) > 0
 
 
+def test_gate_up_in_one_launch_has_the_shares_of_the_streaming_mat_mats():
+    # where the mat-mats run on the streaming kernel, one launch adds as many shares of K as they do (K above 1024: below, one pass is enough)
+    seen = 0
+    for m in (33, 48, 57, 64, 69, 75, 92, 98, 115, 128, 135, 148, 160, 186, 270):
+        for n_ff in range(896, 4993, 128):
+            for k in (1152, 1408, 2048, 2176, 3072, 4096, 5248, 5632, 6144, 6656, 7680, 8192, 9728):
+                gate_up, mat_mat = q8_0.plan_gate_up_silu(m, n_ff, k), q8_0.plan_mul_mat(m, n_ff, k)
+                if gate_up["form"] == "tile" and mat_mat["kernel"] == "gemm_skinny":
+                    assert mat_mat["k_splits"] * mat_mat["waves"] == gate_up["k_sets"] * gate_up["passes"], (m, n_ff, k)
+                    seen += 1
+    assert seen > 500
+
+
 def test_what_leaves_a_callers_workspace_untouched():
     # nh_q8_0_mul_mat's promise: 4 to 16 rows on matrices of up to 40 MB, 4 rows up to 80 MB.  Without a workspace of the caller's the faster way
     moved = 0
