@@ -367,10 +367,11 @@ int nh_q8_0_debug_ffn_gate_up(float* gate_out, float* up_out, int64_t N_ff, void
  *   [1] 1 when the activations are quantized by a launch of their own into the workspace (kernels 3, 4, 5);
  *   kernel 1, 6: [2] workgroups per 32-row strip along K, [3] 128-quant groups per wave, [4] row parts per strip;
  *   kernel 3:    [2] 32-row activation strips per workgroup, [3] workgroups per weight strip along K, [4] shares of K that a workgroup
- *                adds, one per wave (with few rows eight waves may take sixteen);
+ *                adds, one per wave (with few rows eight waves may take sixteen), [5] 1 when its weights go past the caches;
  *   kernel 4, 5: [2] activation strips per wave, [3] K sets of four waves per workgroup, [4] workgroups per tile along K,
- *                [5], [6] the grid (column blocks of 128 weight rows, groups of activation strips);
- *   [7] 1 when nh_q8_0_gemm_tiled runs this shape, up to 32 rows, on the kernel for few rows (as kernel 3 here does then);
+ *                [5], [6] the grid (column blocks of 128 weight rows, groups of activation strips), [7] the order of the tiles: 0 as the
+ *                grid has them, 1 by XCD, n > 1 in bands of n column blocks;
+ *   other kernels: [7] 1 when nh_q8_0_gemm_tiled runs this shape, up to 32 rows, on the kernel for few rows (as kernel 3 here does then);
  *   the rest 0.  The same shape under HIP graph capture may take a form without state between launches (no K split). */
 int nh_q8_0_debug_plan_mul_mat(int64_t M, int64_t N, int64_t K, int32_t* host_plan);
 /* ... and nh_q8_0_mul_mat_scratch */
@@ -379,7 +380,7 @@ int nh_q8_0_debug_plan_mul_mat_scratch(int64_t M, int64_t N, int64_t K, int32_t*
  * for few rows, 2 one launch of the MFMA tile kernel;
  *   1: [1] shares of K that a workgroup adds;
  *   2: [1] activation strips per wave, [2] K sets of four waves per workgroup, [3] passes over K, [4] 1 when the shares are added in the
- *      streaming kernel's order, [5], [6] the grid (blocks of 64 rows of both matrices, groups of activation strips). */
+ *      streaming kernel's order, [5], [6] the grid (blocks of 64 rows of both matrices, groups of activation strips), [7] the order of the tiles, as above. */
 int nh_q8_0_debug_plan_gate_up_silu(int64_t M, int64_t N_ff, int64_t K, int32_t* host_plan);
 
 /* nh_q8_0_gemm_tiled_gate_up_silu with the fp32 outputs of the two mat-mats copied out as well (gate_out, up_out: [M][N_ff]), so that

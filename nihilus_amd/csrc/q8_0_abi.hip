@@ -709,6 +709,7 @@ static int debug_plan_common(int64_t M, int64_t N, int64_t K, int32_t* host_plan
 			host_plan[2] = p.gemm.skinny.ms;
 			host_plan[3] = p.gemm.skinny.splits;
 			host_plan[4] = p.gemm.skinny.waves;
+			host_plan[5] = !p.gemm.rows && nh::gemm_skinny_past_caches(M, N, p.gemm.skinny);
 			break;
 		case nh::MM_GEMM_TILE_STREAM:
 		case nh::MM_GEMM_TILE:
@@ -717,6 +718,7 @@ static int debug_plan_common(int64_t M, int64_t N, int64_t K, int32_t* host_plan
 			host_plan[4] = p.gemm.tile.kz;
 			host_plan[5] = static_cast<int32_t>(p.gemm.tile.grid_x);
 			host_plan[6] = static_cast<int32_t>(p.gemm.tile.grid_y);
+			host_plan[7] = p.gemm.tile.order;
 			break;
 		default:
 			break;
@@ -751,6 +753,7 @@ int nh_q8_0_debug_plan_gate_up_silu(int64_t M, int64_t N_ff, int64_t K, int32_t*
 		host_plan[4] = cut.tree;
 		host_plan[5] = static_cast<int32_t>(cut.tile.grid_x);
 		host_plan[6] = static_cast<int32_t>(cut.tile.grid_y);
+		host_plan[7] = cut.tile.order;
 	}
 	return NH_OK;
 }

@@ -211,7 +211,7 @@ template<typename T, bool NT> __device__ __forceinline__ T load_sv(gptr_u8 p, ui
 // C / C2 (optional, inspection): the fp32 gate / up tiles as the launch computed them.
 template<int TM, bool DUMP, int KS, bool STREAM, bool SPLIT, bool GATE_UP, bool PASSES = false>
 __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, const uint8_t* __restrict__ A, float* C, const float* R, int32_t* __restrict__ sums, int M, int N, int groups,
-	float* __restrict__ partials, unsigned* __restrict__ counters, const uint8_t* __restrict__ W2, uint8_t* __restrict__ act_out, float* __restrict__ C2, int band, int passes = 1, bool tree = false) {
+	float* __restrict__ partials, unsigned* __restrict__ counters, const uint8_t* __restrict__ W2, uint8_t* __restrict__ act_out, float* __restrict__ C2, int order, int passes = 1, bool tree = false) {
 	static_assert(!SPLIT || (KS > 1 && !DUMP), "K over several workgroups continues the K sets' sum");
 	static_assert(!GATE_UP || (!DUMP && !SPLIT), "the fused gate/up form leaves a workgroup's tile quantized");
 	constexpr int STAGE_BYTES = TM * MACRO_BYTES; // the activation strips' macro-tiles of a group, as in memory
@@ -275,18 +275,14 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 	const int n_strips = (N + 31) / 32;
 	int bx = blockIdx.x, by = blockIdx.y; // block of weight strips, group of activation strips
 	if constexpr (!SPLIT && !STREAM) {
-		// Workgroups go to the eight XCDs in turn.  With a number of column blocks that eight divides, a block's row groups are all on one XCD, whose L2 has its weights
-		// then; otherwise every XCD would read nearly all of them.  There each XCD takes the tiles of some consecutive column blocks instead, row groups fastest
-		// ([24171 x 10240] at 145 rows 182 -> 126 us, [3117 x 10752] at 912 134 -> 92, [2 x 3968 x 6528] at 274 77 -> 59 with one strip per wave; with two, 50 random shapes
-		// 1.02 times as fast).  Not with eight dividing: a round of workgroups is a wider piece of the matrix then as it is ([8192 x 8192] at 330 rows 72 us, 76 this way).
-		// Wide matrices of that kind are walked in bands of column blocks (gemm_tile_band in q8_0_plan.h), all row groups of a band before the next band.
+		// three permutations of the grid; which one, and why: gemm_tile_order in q8_0_plan.h
 		const unsigned gx = static_cast<unsigned>(GATE_UP ? (n_strips + 1) / 2 : (n_strips + 3) / 4), gy = static_cast<unsigned>(m_strips + TM - 1) / TM;
-		if (band > 0) {
-			const unsigned b = static_cast<unsigned>(band), id = by * gx + bx, first = id / (b * gy) * b;
+		if (order > TILE_ORDER_XCD) { // bands of that many column blocks
+			const unsigned b = static_cast<unsigned>(order), id = by * gx + bx, first = id / (b * gy) * b;
 			const unsigned r = id - first * gy, width = min(b, gx - first); // the last band may be narrower
 			by				 = __builtin_amdgcn_readfirstlane(static_cast<int>(r / width));
 			bx				 = __builtin_amdgcn_readfirstlane(static_cast<int>(first + r % width));
-		} else if (gx % 8 != 0 && gy > 1) {
+		} else if (order == TILE_ORDER_XCD) {
 			const unsigned total = gx * gy, id = by * gx + bx, xcd = id % 8;
 			const unsigned t	 = xcd * (total / 8) + min(xcd, total % 8) + id / 8; // XCDs 0 .. total % 8 - 1 have one more
 			bx					 = __builtin_amdgcn_readfirstlane(static_cast<int>(t / gy));
@@ -725,26 +721,25 @@ __device__ __forceinline__ void gemm_tiled_body(const uint8_t* __restrict__ W, c
 }
 
 template<int TM, bool DUMP, int KS = 1, bool STREAM = false, bool SPLIT = false>
-__global__ __launch_bounds__(256 * KS, 4) void gemm_tiled_kernel(const uint8_t* __restrict__ W, const uint8_t* __restrict__ A, int M, int N, int groups, int band, float* C, const float* R,
+__global__ __launch_bounds__(256 * KS, 4) void gemm_tiled_kernel(const uint8_t* __restrict__ W, const uint8_t* __restrict__ A, int M, int N, int groups, int order, float* C, const float* R,
 	int32_t* __restrict__ sums, float* __restrict__ partials, unsigned* __restrict__ counters) {
-	gemm_tiled_body<TM, DUMP, KS, STREAM, SPLIT, false>(W, A, C, R, sums, M, N, groups, partials, counters, nullptr, nullptr, nullptr, band);
+	gemm_tiled_body<TM, DUMP, KS, STREAM, SPLIT, false>(W, A, C, R, sums, M, N, groups, partials, counters, nullptr, nullptr, nullptr, order);
 }
 
 // the fused gate / up form (GATE_UP above): N = rows of each of the two matrices; gate_out / up_out optional
 template<int TM, int KS, bool STREAM, bool PASSES>
 __global__ __launch_bounds__(256 * KS, 4) void gemm_gate_up_kernel(const uint8_t* __restrict__ W_gate, const uint8_t* __restrict__ W_up, const uint8_t* __restrict__ A, int M, int N, int groups,
-	int band, int passes, bool tree, uint8_t* __restrict__ act_out, float* __restrict__ gate_out, float* __restrict__ up_out) {
-	gemm_tiled_body<TM, false, KS, STREAM, false, true, PASSES>(W_gate, A, gate_out, nullptr, nullptr, M, N, groups, nullptr, nullptr, W_up, act_out, up_out, band, passes, tree);
+	int order, int passes, bool tree, uint8_t* __restrict__ act_out, float* __restrict__ gate_out, float* __restrict__ up_out) {
+	gemm_tiled_body<TM, false, KS, STREAM, false, true, PASSES>(W_gate, A, gate_out, nullptr, nullptr, M, N, groups, nullptr, nullptr, W_up, act_out, up_out, order, passes, tree);
 }
 
 // Executes a cut made by plan_gemm_tile (q8_0_plan.h): TM activation strips per wave, KS sets of four waves per workgroup,
 // and K over kz workgroups per tile whose tiles are added through the scratch.
 template<int TM, bool STREAM> static hipError_t launch_gemm_tiled_t(const gemm_tile_cut& cut, const uint8_t* w, const uint8_t* a, float* C, const float* R, int32_t* sums, int m, int n, int k, hipStream_t s) {
 	const int groups = k / GROUP_K;
-	const int band	 = gemm_tile_band(cut, false);
 	const dim3 grid(cut.grid_x, cut.grid_y);
 	if (sums) {
-		gemm_tiled_kernel<TM, true><<<grid, dim3(256), 0, s>>>(w, a, m, n, groups, band, C, R, sums, nullptr, nullptr);
+		gemm_tiled_kernel<TM, true><<<grid, dim3(256), 0, s>>>(w, a, m, n, groups, cut.order, C, R, sums, nullptr, nullptr);
 		return hipGetLastError();
 	}
 	const int ks = cut.ks;
@@ -757,17 +752,17 @@ template<int TM, bool STREAM> static hipError_t launch_gemm_tiled_t(const gemm_t
 			if (e != hipSuccess) {
 				return e;
 			}
-			return launch_kernel(KIND_GEMM, gemm_tiled_kernel<TM, false, 4, STREAM, true>, dim3(grid.x, grid.y, static_cast<unsigned>(cut.kz)), dim3(1024), 0, s, w, a, m, n, groups, band, C, R, sums, partials,
+			return launch_kernel(KIND_GEMM, gemm_tiled_kernel<TM, false, 4, STREAM, true>, dim3(grid.x, grid.y, static_cast<unsigned>(cut.kz)), dim3(1024), 0, s, w, a, m, n, groups, cut.order, C, R, sums, partials,
 				counters);
 		}
 	}
 	if (ks == 4) {
-		return launch_kernel(KIND_GEMM, gemm_tiled_kernel<TM, false, 4, STREAM>, grid, dim3(1024), 0, s, w, a, m, n, groups, band, C, R, sums, static_cast<float*>(nullptr), static_cast<unsigned*>(nullptr));
+		return launch_kernel(KIND_GEMM, gemm_tiled_kernel<TM, false, 4, STREAM>, grid, dim3(1024), 0, s, w, a, m, n, groups, cut.order, C, R, sums, static_cast<float*>(nullptr), static_cast<unsigned*>(nullptr));
 	}
 	if (ks == 2) {
-		return launch_kernel(KIND_GEMM, gemm_tiled_kernel<TM, false, 2, STREAM>, grid, dim3(512), 0, s, w, a, m, n, groups, band, C, R, sums, static_cast<float*>(nullptr), static_cast<unsigned*>(nullptr));
+		return launch_kernel(KIND_GEMM, gemm_tiled_kernel<TM, false, 2, STREAM>, grid, dim3(512), 0, s, w, a, m, n, groups, cut.order, C, R, sums, static_cast<float*>(nullptr), static_cast<unsigned*>(nullptr));
 	}
-	return launch_kernel(KIND_GEMM, gemm_tiled_kernel<TM, false, 1, STREAM>, grid, dim3(256), 0, s, w, a, m, n, groups, band, C, R, sums, static_cast<float*>(nullptr), static_cast<unsigned*>(nullptr));
+	return launch_kernel(KIND_GEMM, gemm_tiled_kernel<TM, false, 1, STREAM>, grid, dim3(256), 0, s, w, a, m, n, groups, cut.order, C, R, sums, static_cast<float*>(nullptr), static_cast<unsigned*>(nullptr));
 }
 
 // stream: the weights are read once and not again (a batch of decode rows against a large matrix), so their loads bypass the caches.
@@ -791,11 +786,10 @@ hipError_t launch_gemm_gate_up_silu(const void* w_gate, const void* w_up, const 
 	gate_up_cut cut{};
 	if (plan_gate_up_fused(M, n_ff, K, &cut)) {
 		const gemm_tile_cut& t = cut.tile;
-		const int band		   = gemm_tile_band(t, true);
 		const dim3 grid(t.grid_x, t.grid_y);
 		auto launch = [&](auto kernel) {
 			return launch_kernel(KIND_GEMM, kernel, grid, dim3(static_cast<unsigned>(256 * t.ks)), 0, s, static_cast<const uint8_t*>(w_gate), static_cast<const uint8_t*>(w_up), static_cast<const uint8_t*>(aq),
-				static_cast<int>(M), static_cast<int>(n_ff), static_cast<int>(K / GROUP_K), band, cut.passes, cut.tree, static_cast<uint8_t*>(act_out), gate_dbg, up_dbg);
+				static_cast<int>(M), static_cast<int>(n_ff), static_cast<int>(K / GROUP_K), t.order, cut.passes, cut.tree, static_cast<uint8_t*>(act_out), gate_dbg, up_dbg);
 		};
 		if (t.tm == 1 && t.grid_y > 1) {
 			return t.ks == 1 ? launch(gemm_gate_up_kernel<1, 1, false, false>) : cut.passes > 1 ? launch(gemm_gate_up_kernel<1, 2, false, true>) : launch(gemm_gate_up_kernel<1, 2, false, false>);

@@ -344,11 +344,7 @@ template<int MS> static hipError_t launch_skinny_t(int splits, int waves, const 
 		++shift;
 	}
 	const dim3 grid(static_cast<unsigned>(strips * splits), static_cast<unsigned>(m_groups)), block(static_cast<unsigned>(64 * waves));
-	// The groups of rows read the same weights: past the caches each would take them from memory again ([896 x 6400] at 316 rows 17.1 -> 11.4 us, [4319 x 4224]
-	// at 35 rows 13.9 -> 11.5, [4096 x 4096] at 200 rows 18.4 -> 16.8, [1024 x 4096] at 512 / 250 / 117 rows 10.6 -> 9.6, 7.3 -> 6.6, 7.1 -> 6.7).  Not with one
-	// group ([8192 x 4096] at 40 rows 12.3 as it is, 13.2 through the caches), nor with two whose workgroups are on one XCD (workgroups go to the eight in turn) at
-	// the same time: the second finds the first's lines on their way ([4096 x 4096] at 64 rows 8.1 / 8.25, at 117 rows the same).
-	const bool nt = m_groups == 1 || (m_groups == 2 && (strips * splits) % 8 == 0);
+	const bool nt	  = gemm_skinny_past_caches(m, n, gemm_skinny_cut{ MS, splits, waves });
 	const auto launch = [&](auto kernel) { return launch_kernel(KIND_GEMM, kernel, grid, block, 0, s, w, a, groups, shift, m, n, C, R, sc.partials, sc.counters); };
 	if (waves == SK_WIDE_WAVES) {
 		return nt ? launch(gemm_skinny_kernel<MS, 2, SK_WIDE_WAVES, true>) : launch(gemm_skinny_kernel<MS, 2, SK_WIDE_WAVES, false>);

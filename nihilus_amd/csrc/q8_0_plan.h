@@ -35,6 +35,7 @@ constexpr int GEMM_STREAM_TILE_MIN_COLUMN_BLOCKS = 192; // 128-row column blocks
 struct gemm_tile_cut {
 	int tm, ks, kz;
 	unsigned grid_x, grid_y;
+	int order; // in which the workgroups take the tiles (gemm_tile_order)
 };
 inline gemm_tile_cut plan_gemm_tile(int64_t M, int64_t N, int64_t K, bool stream) {
 	gemm_tile_cut c{};
@@ -84,17 +85,26 @@ inline bool gemm_tile_take_one_strip(gemm_tile_cut* c, int64_t m_strips, int per
 	return true;
 }
 
-// The order of the tile kernel's tiles where eight divides the number of column blocks (the kernel has one of its own for others): column blocks per band, whose row groups
-// are all done before the next band is begun, 0 for one band.  With one, every group of rows walks the whole matrix, from memory again where it is no longer cached, and the
-// workgroups that run together share only their activations; a band's weights are still in its XCDs' L2 when the next row group comes.  Measured, us, one band / this:
+// The order in which the tile kernel's workgroups take its tiles (not those with K over workgroups or with streamed weights, which have one row of workgroups or few).
+//
+// By XCD: workgroups go to the eight XCDs in turn.  With a number of column blocks that eight divides, a block's row groups are all on one XCD, whose L2 has its weights then;
+// otherwise every XCD would read nearly all of them.  There each XCD takes the tiles of some consecutive column blocks instead, row groups fastest ([24171 x 10240] at 145 rows
+// 182 -> 126 us, [3117 x 10752] at 912 134 -> 92, [2 x 3968 x 6528] at 274 77 -> 59 with one strip per wave; with two, 50 random shapes 1.02 times as fast).  Not with eight
+// dividing: a round of workgroups is a wider piece of the matrix then as it is ([8192 x 8192] at 330 rows 72 us, 76 this way).
+//
+// In bands of that many column blocks, all row groups of a band before the next band is begun, where eight divides their number.  With one band, every group of rows walks the
+// whole matrix, from memory again where it is no longer cached, and the workgroups that run together share only their activations.  Measured, us, one band / this:
 //   gate/up   [2 x 28672 x 8192] at 512 rows 745 / 598, at 178 two strips 293 / 261; [2 x 14336 x 4096] at 512 / 3001 170 / 162, 938 / 881; [2 x 26624 x 9344] at 858 1394 / 1062;
 //             with one strip per wave [2 x 21504 x 7808] at 200 318 / 226, [2 x 24576 x 1920] at 273 122 / 89
 //   mat-mats  [27648 x 4736] at 1058 363 / 344, [20475 x 9984] at 1965 980 / 941, [25530 x 6784] at 738 343 / 326
 // Bands of 16 to 64 column blocks are within 1 % of each other.  Below 128 nothing changes ([2 x 5632 x 7680] at 660 rows 159 / 161, [9146 x 9216] at 326 88.5 / 88.5), and two
 // row groups of a mat-mat find each other's weights on their way as it is ([22528 x 2944] at 118 rows 32.8 / 34.2; gate / up [2 x 24064 x 8320] at 125 159 / 153).
-constexpr int GEMM_TILE_BAND = 32;
-inline int gemm_tile_band(const gemm_tile_cut& c, bool gate_up) {
-	return c.grid_x % 8 == 0 && c.grid_x >= 128 && c.grid_y > (gate_up ? 1u : 2u) && c.kz == 1 ? GEMM_TILE_BAND : 0;
+constexpr int TILE_ORDER_GRID = 0, TILE_ORDER_XCD = 1, TILE_ORDER_BANDS = 32;
+inline int gemm_tile_order(const gemm_tile_cut& c, bool gate_up) {
+	if (c.grid_x % 8 != 0) {
+		return c.grid_y > 1 ? TILE_ORDER_XCD : TILE_ORDER_GRID;
+	}
+	return c.grid_x >= 128 && c.grid_y > (gate_up ? 1u : 2u) ? TILE_ORDER_BANDS : TILE_ORDER_GRID;
 }
 
 // The tile kernel's cut for a mat-mat of its own (K not over workgroups).  Uneven sets walk as many trips as the longest, so short ones multiply up to a tenth
@@ -180,6 +190,16 @@ inline gemm_skinny_cut plan_gemm_skinny(int64_t M, int64_t N, int64_t K) {
 	c.waves	 = (units > 128 && units < 256 && groups >= 4 * SK_WAVES) ? SK_WIDE_WAVES : SK_WAVES;
 	c.splits = sets_for(c.waves);
 	return c;
+}
+
+// Its weights go past the caches where no other workgroup reads them.  The groups of rows read the same ones: past the caches each would take them from memory again
+// ([896 x 6400] at 316 rows 17.1 -> 11.4 us, [4319 x 4224] at 35 rows 13.9 -> 11.5, [4096 x 4096] at 200 rows 18.4 -> 16.8, [1024 x 4096] at 512 / 250 / 117 rows
+// 10.6 -> 9.6, 7.3 -> 6.6, 7.1 -> 6.7).  Not with one group ([8192 x 4096] at 40 rows 12.3 as it is, 13.2 through the caches), nor with two whose workgroups are on
+// one XCD (workgroups go to the eight in turn) at the same time: the second finds the first's lines on their way ([4096 x 4096] at 64 rows 8.1 / 8.25, at 117 rows
+// the same).
+inline bool gemm_skinny_past_caches(int64_t M, int64_t N, const gemm_skinny_cut& cut) {
+	const int64_t strips = (N + STRIP_ROWS - 1) / STRIP_ROWS, m_strips = (M + STRIP_ROWS - 1) / STRIP_ROWS, m_groups = (m_strips + cut.ms - 1) / cut.ms;
+	return m_groups == 1 || (m_groups == 2 && (strips * cut.splits) % 8 == 0);
 }
 
 // The streaming kernel's own mat-mats of more than 32 rows: never fewer shares of K than above, in another cut where that is faster (random shapes whose
@@ -386,6 +406,7 @@ inline gemm_plan plan_gemm(int64_t M, int64_t N, int64_t K) {
 	} else {
 		p.kernel = MM_GEMM_TILE;
 		p.tile	 = gemm_tile_mat_mat(plan_gemm_tile(M, N, K, false), static_cast<int>(K / GROUP_K), (M + 31) / 32, false);
+		p.tile.order = gemm_tile_order(p.tile, false);
 	}
 	return p;
 }
@@ -490,6 +511,7 @@ inline bool plan_gate_up_with(bool even, const gemm_plan& g, int64_t M, int64_t 
 	if (c.tile.ks <= 2) {
 		gemm_tile_take_one_strip(&c.tile, (M + STRIP_ROWS - 1) / STRIP_ROWS, ONE_STRIP_GATE_UP);
 	}
+	c.tile.order = gemm_tile_order(c.tile, true);
 	if (cut) {
 		*cut = c;
 	}

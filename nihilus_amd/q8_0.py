@@ -80,6 +80,10 @@ def tiled_bytes(rows: int, k: int) -> int:
 KERNEL_NAMES = {0: "nothing", 1: "gemv", 2: "gemv_rows", 3: "gemm_skinny", 4: "gemm_tile_stream", 5: "gemm_tile", 6: "gemv_rows_mfma"}
 
 
+def _tile_order(raw: int):
+    return {0: "grid", 1: "by_xcd"}.get(raw, f"bands_of_{raw}")
+
+
 def plan_mul_mat(m: int, n: int, k: int, own_workspace: bool = False) -> dict:
     """Which kernel mul_mat runs for fp32 activations [m, k] against a tiled weight [n, k], and its cut (no GPU needed);
     own_workspace: with a workspace of the caller's."""
@@ -88,13 +92,13 @@ def plan_mul_mat(m: int, n: int, k: int, own_workspace: bool = False) -> dict:
     raw = (ctypes.c_int32 * 8)()
     fn = "nh_q8_0_debug_plan_mul_mat" if own_workspace else "nh_q8_0_debug_plan_mul_mat_scratch"
     _lib.check("nh_q8_0_debug_plan_mul_mat", getattr(_lib.lib(), fn)(m, n, k, raw))
-    plan = {"kernel": KERNEL_NAMES[raw[0]], "quantize_launch": bool(raw[1]), "gemm_rows": bool(raw[7])}
+    plan = {"kernel": KERNEL_NAMES[raw[0]], "quantize_launch": bool(raw[1]), "gemm_rows": raw[0] not in (4, 5) and bool(raw[7])}
     if raw[0] in (1, 6):
         plan.update(k_splits=raw[2], groups_per_wave=raw[3], row_parts=raw[4])
     elif raw[0] == 3:
-        plan.update(activation_strips=raw[2], k_splits=raw[3], waves=raw[4])
+        plan.update(activation_strips=raw[2], k_splits=raw[3], waves=raw[4], past_caches=bool(raw[5]))
     elif raw[0] in (4, 5):
-        plan.update(activation_strips=raw[2], k_sets=raw[3], k_splits=raw[4], grid=(raw[5], raw[6]))
+        plan.update(activation_strips=raw[2], k_sets=raw[3], k_splits=raw[4], grid=(raw[5], raw[6]), order=_tile_order(raw[7]))
     return plan
 
 
@@ -107,7 +111,7 @@ def plan_gate_up_silu(m: int, n_ff: int, k: int) -> dict:
     if raw[0] == 1:
         return {"form": "rows", "waves": raw[1]}
     if raw[0] == 2:
-        return {"form": "tile", "activation_strips": raw[1], "k_sets": raw[2], "passes": raw[3], "tree": bool(raw[4]), "grid": (raw[5], raw[6])}
+        return {"form": "tile", "activation_strips": raw[1], "k_sets": raw[2], "passes": raw[3], "tree": bool(raw[4]), "grid": (raw[5], raw[6]), "order": _tile_order(raw[7])}
     return {"form": "three_launches"}
 
 

@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 )
 def test_bands(q8, oracle, m, n, k, grid):
     p = q8.plan_mul_mat(m, n, k)
-    assert p["kernel"] == "gemm_tile" and p["grid"] == grid and p["k_splits"] == 1, p
+    assert p["kernel"] == "gemm_tile" and p["grid"] == grid and p["k_splits"] == 1 and p["order"] == ("bands_of_32" if grid[0] >= 128 and grid[1] > 2 else "grid"), p
     w = oracle.fill_weights(m + n, n, k)
     x = oracle.fill_activations(m + k, m * k).reshape(m, k)
     aq = oracle.quantize_rows(x)
@@ -31,7 +31,7 @@ def test_bands(q8, oracle, m, n, k, grid):
 @pytest.mark.parametrize("m,n_ff,k,grid", [(100, 8192, 1024, (128, 2)), (100, 8704, 2048, (136, 2)), (193, 8192, 1024, (128, 4)), (290, 9216, 256, (144, 5)), (161, 9728, 128, (152, 3)), (385, 8704, 256, (136, 13))])
 def test_gate_up_bands(q8, oracle, m, n_ff, k, grid):
     p = q8.plan_gate_up_silu(m, n_ff, k)
-    assert p["form"] == "tile" and p["grid"] == grid, p
+    assert p["form"] == "tile" and p["grid"] == grid and p["order"] == "bands_of_32", p
     wg, wu = oracle.fill_weights(21 + m, n_ff, k), oracle.fill_weights(22 + m, n_ff, k)
     x = oracle.fill_activations(m + k, m * k).reshape(m, k)
     aq_cpu = oracle.quantize_rows(x)

@@ -140,6 +140,23 @@ def test_gate_up_in_one_launch_has_the_shares_of_the_streaming_mat_mats():
     assert seen > 500
 
 
+@pytest.mark.parametrize(
+    "m,n,k,order",
+    [(129, 128 * 127, 256, "by_xcd"), (129, 128 * 120, 256, "grid"), (129, 128 * 128, 256, "bands_of_32"), (1000, 128 * 129, 4096, "by_xcd"), (100, 128 * 136, 256, "grid"), (117, 128 * 137, 256, "by_xcd")],
+)
+def test_order_of_the_tiles(m, n, k, order):
+    # the number of column blocks: eight does not divide it, divides fewer than 128, and more; two row groups and more
+    p = q8_0.plan_mul_mat(m, n, k)
+    assert p["kernel"] == "gemm_tile" and p["order"] == order, p
+
+
+@pytest.mark.parametrize("m,n,k,past", [(64, 8192, 1024, True), (33, 4096, 1024, True), (33, 4128, 1024, False), (97, 1024, 256, False), (40, 128, 128 * 33, True), (64, 480, 128 * 33, False)])
+def test_weights_past_the_caches(m, n, k, past):
+    # streaming kernel: one group of rows; two whose workgroups are on one XCD, and not; more
+    p = q8_0.plan_mul_mat(m, n, k)
+    assert p["kernel"] == "gemm_skinny" and p["past_caches"] == past, p
+
+
 def test_what_leaves_a_callers_workspace_untouched():
     # nh_q8_0_mul_mat's promise: 4 to 16 rows on matrices of up to 40 MB, 4 rows up to 80 MB.  Without a workspace of the caller's the faster way
     moved = 0
