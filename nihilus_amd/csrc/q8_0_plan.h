@@ -94,17 +94,25 @@ inline bool gemm_tile_take_one_strip(gemm_tile_cut* c, int64_t m_strips, int per
 //
 // In bands of that many column blocks, all row groups of a band before the next band is begun, where eight divides their number.  With one band, every group of rows walks the
 // whole matrix, from memory again where it is no longer cached, and the workgroups that run together share only their activations.  Measured, us, one band / this:
-//   gate/up   [2 x 28672 x 8192] at 512 rows 745 / 598, at 178 two strips 293 / 261; [2 x 14336 x 4096] at 512 / 3001 170 / 162, 938 / 881; [2 x 26624 x 9344] at 858 1394 / 1062;
-//             with one strip per wave [2 x 21504 x 7808] at 200 318 / 226, [2 x 24576 x 1920] at 273 122 / 89
-//   mat-mats  [27648 x 4736] at 1058 363 / 344, [20475 x 9984] at 1965 980 / 941, [25530 x 6784] at 738 343 / 326
-// Bands of 16 to 64 column blocks are within 1 % of each other.  Below 128 nothing changes ([2 x 5632 x 7680] at 660 rows 159 / 161, [9146 x 9216] at 326 88.5 / 88.5), and two
-// row groups of a mat-mat find each other's weights on their way as it is ([22528 x 2944] at 118 rows 32.8 / 34.2; gate / up [2 x 24064 x 8320] at 125 159 / 153).
+//   gate/up   [2 x 28672 x 8192] at 512 rows 740 / 628, at 178 two strips 285 / 274; [2 x 14336 x 4096] at 3001 933 / 897; [2 x 26624 x 9344] at 858 1377 / 1122;
+//             with one strip per wave [2 x 21504 x 7808] at 200 318 / 231, [2 x 24576 x 1920] at 273 123 / 91
+//   mat-mats  [27648 x 4736] at 1058 365 / 357, [20475 x 9984] at 1965 988 / 956
+// Bands of 16 to 64 column blocks are within 1 % of each other.  Not where the matrix is found in a cache again as it is, or the launch is over before its workgroups have
+// drifted apart (random shapes, one band / this):
+//   two strips per wave, less than 8e10 products     83 mat-mats 0.90 to 1.01, mean 0.98 ([18432 x 2048] at 500 rows 56 / 60), 302 gate/up 0.96 to 1.05, mean 0.99;
+//                        more                        67 mat-mats 0.98 to 1.14, mean 1.02, 93 gate/up 0.98 to 1.22, mean 1.03
+//   one strip per wave   less than 80 MiB of weights 60 mat-mats 0.81 to 1.03, mean 0.95; more 40, 0.94 to 1.39, mean 1.09
+//                        gate/up, less than 48 MiB   9, 0.95 to 1.01, mean 0.99; more 66, 0.98 to 1.55, mean 1.11
+// Below 128 column blocks nothing changes ([2 x 5632 x 7680] at 660 rows 164 / 163, [9146 x 9216] at 326 90.4 / 91.0), and two row groups of a mat-mat find each other's weights
+// on their way as it is ([22528 x 2944] at 118 rows 33.2 / 33.3).
 constexpr int TILE_ORDER_GRID = 0, TILE_ORDER_XCD = 1, TILE_ORDER_BANDS = 32;
-inline int gemm_tile_order(const gemm_tile_cut& c, bool gate_up) {
+constexpr int64_t TILE_BANDS_MIN_PRODUCTS = 80'000'000'000, TILE_BANDS_ONE_STRIP_BYTES = 80ll << 20, TILE_BANDS_ONE_STRIP_BYTES_GATE_UP = 48ll << 20;
+inline int gemm_tile_order(const gemm_tile_cut& c, bool gate_up, int64_t M, int64_t N, int64_t K) { // N: rows of weights, of both matrices for gate/up
 	if (c.grid_x % 8 != 0) {
 		return c.grid_y > 1 ? TILE_ORDER_XCD : TILE_ORDER_GRID;
 	}
-	return c.grid_x >= 128 && c.grid_y > (gate_up ? 1u : 2u) ? TILE_ORDER_BANDS : TILE_ORDER_GRID;
+	const bool enough = c.tm == 1 ? N * (K / QK) * BLOCK_BYTES >= (gate_up ? TILE_BANDS_ONE_STRIP_BYTES_GATE_UP : TILE_BANDS_ONE_STRIP_BYTES) : M * N * K >= TILE_BANDS_MIN_PRODUCTS;
+	return c.grid_x >= 128 && c.grid_y > (gate_up ? 1u : 2u) && enough ? TILE_ORDER_BANDS : TILE_ORDER_GRID;
 }
 
 // The tile kernel's cut for a mat-mat of its own (K not over workgroups).  Uneven sets walk as many trips as the longest, so short ones multiply up to a tenth
@@ -406,7 +414,7 @@ inline gemm_plan plan_gemm(int64_t M, int64_t N, int64_t K) {
 	} else {
 		p.kernel = MM_GEMM_TILE;
 		p.tile	 = gemm_tile_mat_mat(plan_gemm_tile(M, N, K, false), static_cast<int>(K / GROUP_K), (M + 31) / 32, false);
-		p.tile.order = gemm_tile_order(p.tile, false);
+		p.tile.order = gemm_tile_order(p.tile, false, M, N, K);
 	}
 	return p;
 }
@@ -511,7 +519,7 @@ inline bool plan_gate_up_with(bool even, const gemm_plan& g, int64_t M, int64_t 
 	if (c.tile.ks <= 2) {
 		gemm_tile_take_one_strip(&c.tile, (M + STRIP_ROWS - 1) / STRIP_ROWS, ONE_STRIP_GATE_UP);
 	}
-	c.tile.order = gemm_tile_order(c.tile, true);
+	c.tile.order = gemm_tile_order(c.tile, true, M, 2 * n_ff, K);
 	if (cut) {
 		*cut = c;
 	}

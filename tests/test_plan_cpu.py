@@ -141,13 +141,24 @@ def test_gate_up_in_one_launch_has_the_shares_of_the_streaming_mat_mats():
 
 
 @pytest.mark.parametrize(
-    "m,n,k,order",
-    [(129, 128 * 127, 256, "by_xcd"), (129, 128 * 120, 256, "grid"), (129, 128 * 128, 256, "bands_of_32"), (1000, 128 * 129, 4096, "by_xcd"), (100, 128 * 136, 256, "grid"), (117, 128 * 137, 256, "by_xcd")],
+    "m,n,k,strips,order",
+    [(129, 128 * 127, 256, 1, "by_xcd"), (1000, 128 * 129, 4096, 2, "by_xcd"), (117, 128 * 137, 256, 2, "by_xcd"),  # a number of column blocks that eight does not divide
+     (129, 128 * 128, 4864, 1, "bands_of_32"), (129, 128 * 128, 4736, 1, "grid"), (140, 128 * 120, 8192, 1, "grid"),  # one strip per wave: 80 MiB of weights, 128 column blocks
+     (512, 128 * 144, 8576, 2, "bands_of_32"), (512, 128 * 144, 8448, 2, "grid"), (3001, 14336, 4096, 2, "grid"), (128, 128 * 136, 40960, 2, "grid")],  # two: 8e10 products, three row groups
 )
-def test_order_of_the_tiles(m, n, k, order):
-    # the number of column blocks: eight does not divide it, divides fewer than 128, and more; two row groups and more
+def test_order_of_the_tiles(m, n, k, strips, order):
     p = q8_0.plan_mul_mat(m, n, k)
-    assert p["kernel"] == "gemm_tile" and p["order"] == order, p
+    assert (p["kernel"], p["activation_strips"], p["order"]) == ("gemm_tile", strips, order), p
+
+
+@pytest.mark.parametrize(
+    "m,n_ff,k,strips,order",
+    [(385, 8704, 2816, 1, "bands_of_32"), (385, 8704, 2688, 1, "grid"), (300, 9728, 13824, 2, "bands_of_32"), (300, 9728, 13568, 2, "grid"), (128, 24576, 12800, 2, "bands_of_32"), (128, 24576, 12672, 2, "grid"),
+     (512, 14336, 4096, 2, "grid"), (3001, 14336, 4096, 2, "bands_of_32"), (512, 11008, 4096, 2, "by_xcd")],
+)
+def test_order_of_the_gate_up_tiles(m, n_ff, k, strips, order):
+    p = q8_0.plan_gate_up_silu(m, n_ff, k)
+    assert (p["form"], p["activation_strips"], p["order"]) == ("tile", strips, order), p
 
 
 @pytest.mark.parametrize("m,n,k,past", [(64, 8192, 1024, True), (33, 4096, 1024, True), (33, 4128, 1024, False), (97, 1024, 256, False), (40, 128, 128 * 33, True), (64, 480, 128 * 33, False)])
