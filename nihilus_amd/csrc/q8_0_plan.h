@@ -210,21 +210,22 @@ inline bool gemm_skinny_past_caches(int64_t M, int64_t N, const gemm_skinny_cut&
 	return m_groups == 1 || (m_groups == 2 && (strips * cut.splits) % 8 == 0);
 }
 
-// The streaming kernel's own mat-mats of more than 32 rows: never fewer shares of K than above, in another cut where that is faster (random shapes whose
-// cut differs: 1.08 times as fast; measured, us, cut above / this).
+// The streaming kernel's own mat-mats of more than 32 rows: never fewer shares of K than above, in another cut where that is faster (measured, us, cut above / this; in
+// brackets 70 random shapes of each kind).
 // - One strip per workgroup instead of two, up to 512 workgroups of one (of three strips, whose fourth would be work for nothing, up to 640): half as many leave
-//   a part of the chip's last round idle ([4864 x 2432] at 94 rows 11.4 / 8.2, [5632 x 3968] at 72 17.3 / 13.1, [3016 x 7424] at 148 24.4 / 21.7; with five strips
-//   [3346 x 2176] at 144, 525 of one, 10.3 / 11.0).  Also where two strips make just a workgroup per CU, if those are of eight row strips and more: two workgroups
-//   on a CU wait for their loads in turn ([1024 x 4096] at 512 rows 9.3 / 8.8, [2048 x 1024] at 256 4.9 / 4.3; [4096 x 4096] at 128 12.3 / 12.4).
+//   a part of the chip's last round idle ([4864 x 2432] at 94 rows 11.4 / 7.9, [5632 x 3968] at 72 16.8 / 13.0, [3016 x 7424] at 148 24.1 / 21.5; with five strips
+//   [3346 x 2176] at 144, 525 of one, 10.3 / 11.0; 0.98 to 1.45, mean 1.24).  Also where two strips make just a workgroup per CU, if those are of eight row strips and
+//   more: two workgroups on a CU wait for their loads in turn ([2048 x 1024] at 256 5.3 / 4.7, [1024 x 4096] at 512 10.4 / 10.4; [4096 x 4096] at 128 12.3 / 12.4).
 // - Two strips instead of one, with sixteen waves, where those fit a workgroup per CU and ones of a strip do not, from K = 5248 on: the weights cross L2 once for
-//   two strips ([7296 x 8832] at 36 rows 24.5 / 19.9, [5888 x 13568] at 48 37.8 / 31, [2658 x 14464] at 170 33.7 / 28.9; at K = 4608 11.6 / 12.0).  With more than 64
-//   rows from 360 workgroups on ([2560 x 6144] at 103 rows, 320, 12.7 / 14.1), and up to 192 ([1152 x 9856] at 310 18.4 / 19.0).
+//   two strips ([7296 x 8832] at 36 rows 24.6 / 19.5, [5888 x 13568] at 48 37.7 / 28.8; at K = 4608 11.6 / 12.0).  With more than 64
+//   rows from 360 workgroups on ([2560 x 6144] at 103 rows, 320, 12.7 / 14.1), and up to 192 ([1152 x 9856] at 310 18.4 / 19.0): 0.92 ([3200 x 5504] at 120) to 1.14 times
+//   as fast below K = 7680, [2658 x 14464] at 170 33.1 / 28.2.  (Of all 70 0.92 to 1.33, mean 1.15.)
 // - Sixteen waves instead of eight for 65 to 160 workgroups and eleven to 31 groups, and for more workgroups while a wave of eight has two groups or so: all of a wave's
-//   share is on its way at once ([768 x 2048] at 104 rows 5.1 / 4.2, [1569 x 1664] at 57 5.0 / 4.3; [2048 x 2304] at 127, 256 workgroups, 5.8 / 6.0;
-//   up to 64 workgroups it may lose, [611 x 2688] at 80 rows 5.3 / 5.65).  The same instead of two workgroups of eight for 65 to 128 and up to 40
-//   groups: nothing to hand over ([1024 x 4096] at 117 rows 6.4 / 5.6, the same bits; up to 64 rows [1792 x 5120] at 35 7.35 / 8.0).
-// - Four workgroups along K instead of two for up to 64 and from 34 groups on, as a CU more costs nothing there ([457 x 6272] at 40 rows 7.8 / 6.1, [384 x 8064] at
-//   34 8.5 / 6.7).
+//   share is on its way at once ([768 x 2048] at 104 rows 4.8 / 4.5, [1569 x 1664] at 57 4.8 / 4.7; [2048 x 2304] at 127, 256 workgroups, 5.8 / 6.0; up to 64
+//   workgroups it may lose, [611 x 2688] at 80 rows 5.3 / 5.65; 0.94 to 1.29, mean 1.02).  Not instead of two workgroups of eight: 65 to 128 of them, with more than 64 rows
+//   and up to 40 groups, 0.91 to 1.01, mean 0.96 ([1024 x 4096] at 117 rows 6.7 / 7.1, the same bits).
+// - Four workgroups along K instead of two for up to 64 and from 34 groups on, as a CU more costs nothing there ([457 x 6272] at 40 rows 7.5 / 6.1, [384 x 8064] at
+//   34 8.2 / 6.4; 1.09 to 1.29, mean 1.18).
 // Not in more shares where gate / up of such a pair are one launch, which has no room for sixteen (plan_gate_up_with): one launch and three give the same bytes
 // there (one in a hundred of the pairs whose mat-mats run here: [2 x 2688 x 2048] at 69 rows, [2 x 3840 x 6144] at 98), and
 // the mat-mats cost no more: 40 random ones of those with sixteen shares / these 0.91 to 1.09, mean 1.01.
@@ -245,9 +246,6 @@ inline gemm_skinny_cut plan_gemm_streaming(int64_t M, int64_t N, int64_t K) {
 	} else if (c.ms == 1 && c.waves == SK_WAVES) {
 		if (c.splits == 1 && ones > 64 && groups >= 11 && (ones <= 160 || (ones <= 256 && groups < 18))) {
 			c.waves = SK_WIDE_WAVES;
-		} else if (c.splits == 2 && M > 64 && ones > 64 && ones <= 128 && groups <= 40) {
-			c.splits = 1;
-			c.waves	 = SK_WIDE_WAVES;
 		} else if (c.splits == 2 && ones <= 64 && groups >= 34) {
 			c.splits = 4;
 		}

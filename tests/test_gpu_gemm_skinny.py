@@ -40,7 +40,7 @@ def test_gemm_skinny(q8, oracle, m, n, k):
     [(65, 2752, 256, (1, 8, 1)), (96, 6816, 256, (1, 8, 1)), (65, 6880, 256, (2, 8, 1)), (100, 4096, 256, (2, 8, 1)), (129, 3264, 256, (1, 8, 1)), (160, 3300, 256, (2, 8, 1)), (250, 2048, 256, (1, 8, 1)),
      (34, 4128, 128 * 41, (2, 16, 1)), (34, 4128, 128 * 40, (1, 8, 1)), (34, 4096, 128 * 41, (1, 8, 1)), (190, 1910, 128 * 41, (2, 16, 1)), (193, 1910, 128 * 41, (1, 8, 1)),
      (64, 1056, 128 * 11, (1, 16, 1)), (64, 1024, 128 * 11, (1, 8, 1)), (64, 1056, 128 * 10, (1, 8, 1)), (33, 2570, 128 * 31, (1, 8, 1)), (256, 1000, 128 * 17, (1, 16, 1)), (256, 1000, 128 * 18, (1, 8, 1)),
-     (97, 1000, 128 * 40, (1, 16, 1)), (97, 1000, 128 * 41, (1, 8, 2)), (33, 1056, 128 * 33, (1, 8, 2)), (64, 1000, 128 * 34, (1, 8, 4)), (64, 1000, 128 * 33, (1, 8, 2))],
+     (97, 1000, 128 * 31, (1, 16, 1)), (97, 1000, 128 * 32, (1, 8, 2)), (97, 1000, 128 * 41, (1, 8, 2)), (33, 1056, 128 * 33, (1, 8, 2)), (64, 1000, 128 * 34, (1, 8, 4)), (64, 1000, 128 * 33, (1, 8, 2))],
 )
 def test_cuts(q8, oracle, m, n, k, cut):
     p = q8.plan_mul_mat(m, n, k)
