@@ -382,6 +382,9 @@ int nh_q8_0_debug_plan_mul_mat_scratch(int64_t M, int64_t N, int64_t K, int32_t*
  *   2: [1] activation strips per wave, [2] K sets of four waves per workgroup, [3] passes over K, [4] 1 when the shares are added in the
  *      streaming kernel's order, [5], [6] the grid (blocks of 64 rows of both matrices, groups of activation strips), [7] the order of the tiles, as above. */
 int nh_q8_0_debug_plan_gate_up_silu(int64_t M, int64_t N_ff, int64_t K, int32_t* host_plan);
+/* ... and of nh_q8_0_decode_layer_f32, four int32: [0] 1 when it is one launch, and then [1] workgroups per strip of the down projection, [2] 1 when they share it by
+ * rows and not along K, [3] how many of them hold their weight requests back a while. */
+int nh_q8_0_debug_plan_decode_layer(int64_t N_embd, int64_t N_ff, int32_t* host_plan);
 
 /* nh_q8_0_gemm_tiled_gate_up_silu with the fp32 outputs of the two mat-mats copied out as well (gate_out, up_out: [M][N_ff]), so that
  * the quantized activation can be compared with the CPU quantizer applied to exactly the sums the launch computed. */

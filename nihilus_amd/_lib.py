@@ -57,6 +57,7 @@ SIGNATURES = {
     "nh_q8_0_debug_plan_mul_mat": (_int, [_i64, _i64, _i64, _vp]),
     "nh_q8_0_debug_plan_mul_mat_scratch": (_int, [_i64, _i64, _i64, _vp]),
     "nh_q8_0_debug_plan_gate_up_silu": (_int, [_i64, _i64, _i64, _vp]),
+    "nh_q8_0_debug_plan_decode_layer": (_int, [_i64, _i64, _vp]),
     "nh_q8_0_gemv_tiled_residual_f32": (_int, [_vp, _vp, _vp, _vp, _i64, _i64, _vp]),
     "nh_q8_0_gemv_tiled_multi_f32": (_int, [C.POINTER(_vp), C.POINTER(_vp), C.POINTER(_i64), _i64, _vp, _i64, _vp]),
     "nh_q8_0_debug_fused_quantize": (_int, [_vp, _vp, _i64, _vp]),

@@ -758,6 +758,18 @@ int nh_q8_0_debug_plan_gate_up_silu(int64_t M, int64_t N_ff, int64_t K, int32_t*
 	return NH_OK;
 }
 
+int nh_q8_0_debug_plan_decode_layer(int64_t N_embd, int64_t N_ff, int32_t* host_plan) {
+	NH_TRY(check_shape(1, N_ff, N_embd, true));
+	NH_REQUIRE(N_ff % nh::GROUP_K == 0, NH_ERR_SHAPE);
+	NH_REQUIRE(host_plan, NH_ERR_NULL_POINTER);
+	const nh::decode_layer_plan p = nh::plan_decode_layer(N_embd, N_ff, 0);
+	host_plan[0]				  = p.one_launch;
+	host_plan[1]				  = p.one_launch ? p.splits : 0;
+	host_plan[2]				  = p.down_by_rows;
+	host_plan[3]				  = p.held;
+	return NH_OK;
+}
+
 int nh_q8_0_mul_mat(const void* W_tiled, const float* x, float* y, int64_t M, int64_t N, int64_t K, void* workspace, int64_t workspace_bytes, void* stream) {
 	return mul_mat_common(W_tiled, x, nullptr, y, M, N, K, workspace, workspace_bytes, stream);
 }

@@ -25,15 +25,11 @@
 // Progress: every workgroup waits only for workgroups with lower indices, and workgroups are dispatched in index order within each
 // XCD's share of the grid, so the lowest unfinished workgroup can always run; every wait is bounded all the same (the wave gives
 // up, leaves NaN and a code in the device-visible error word).
-#include "q8_0_gemv_tiled.h"
+#include "q8_0_plan.h"
 
 namespace nh {
 
-constexpr int CHAIN_TILES = 4; // groups a wave stages at once: LDS slices are sized for it
-constexpr int CHAIN_DOWN_ROWS_TILES = 8; // ... in the down stage when it is cut by rows (half-size groups)
-
-constexpr int CHAIN_CUS			= 256;
-constexpr int CHAIN_HOLD_CLOCKS = 6144; // how long a held down workgroup waits before its first request
+constexpr int CHAIN_HOLD_CLOCKS = 6144; // how long a held down workgroup waits before its first request (plan_decode_layer in q8_0_plan.h)
 
 struct layer_args {
 	// attn_out
@@ -421,31 +417,14 @@ template<int CHUNKS> __global__ __launch_bounds__(GEMV_WAVES * 64) void decode_l
 	}
 }
 
-// Whether the shape takes the one-launch form; otherwise (and under HIP graph capture, where a replay could not renew the epoch) the
-// layer runs as its three launches.
-bool decode_layer_chains(int64_t n_embd, int64_t n_ff, int64_t next_strips) {
-	if (n_embd <= 0 || n_ff <= 0 || n_embd % GROUP_K != 0 || n_ff % GROUP_K != 0 || n_embd > CHAIN_MAX_EMBD || n_ff > FFN_MAX_HIDDEN) {
-		return false;
-	}
-	const int64_t strips_e = n_embd / STRIP_ROWS, groups_f = n_ff / GROUP_K;
-	// the down projection's K split must bring a wave's share to four groups within the scratch
-	int splits = 1;
-	while ((groups_f + GEMV_WAVES * splits - 1) / (GEMV_WAVES * splits) > CHAIN_TILES && strips_e <= GEMV_MAX_SPLIT_STRIPS && strips_e * splits * 2 <= GEMV_MAX_SPLIT_UNITS) {
-		splits *= 2;
-	}
-	if ((groups_f + GEMV_WAVES * splits - 1) / (GEMV_WAVES * splits) > CHAIN_TILES) {
-		return false;
-	}
-	return next_strips >= 0 && next_strips < (1 << 20);
-}
-
 hipError_t launch_decode_layer(const void* w_o, const float* attn, const float* layer_in, float* ffn_inp, const void* w_gate, const void* w_up, const void* w_down, const float* ffn_norm_w,
 	float* l_out, const void* const* w_next, float* const* y_next, const int64_t* n_next, int count_next, const float* next_norm_w, float eps, int64_t n_embd, int64_t n_ff, hipStream_t s) {
 	int64_t next_strips = 0;
 	for (int i = 0; i < count_next; ++i) {
 		next_strips += (n_next[i] + STRIP_ROWS - 1) / STRIP_ROWS;
 	}
-	if (!decode_layer_chains(n_embd, n_ff, next_strips) || stream_is_capturing(s) || !in_kernel_waits_enabled()) {
+	const decode_layer_plan p = plan_decode_layer(n_embd, n_ff, next_strips); // otherwise (and under HIP graph capture, where a replay could not renew the epoch)
+	if (!p.one_launch || stream_is_capturing(s) || !in_kernel_waits_enabled()) {
 		// the same three steps as launches of their own
 		const void* w1[1]  = { w_o };
 		float* y1[1]	   = { ffn_inp };
@@ -500,40 +479,17 @@ hipError_t launch_decode_layer(const void* w_o, const float* attn, const float* 
 	// gate/up: sixteen K ranges per workgroup, both matrices per wave, two groups of each at a time: one such chunk covers a wave's
 	// share up to 4096 values of hidden state, two up to 8192 (CHAIN_MAX_EMBD).  (Up to 8192 the stage used to give eight waves to each
 	// matrix, four groups at a time: 128 registers and spills, the LLaMA-3-70B block 160.8 us against 150.3 us in this form.)
-	const bool one_chunk = (a.groups_e + GEMV_WAVES - 1) / GEMV_WAVES <= 2;
 	a.p_per_slot		 = a.groups_e / GEMV_WAVES;
 	a.p_rem				 = a.groups_e % GEMV_WAVES;
-	int splits = 1;
-	while ((a.groups_f + GEMV_WAVES * splits - 1) / (GEMV_WAVES * splits) > CHAIN_TILES) {
-		splits *= 2;
-	}
-	while ((1 << a.split_shift) < splits) {
+	while ((1 << a.split_shift) < p.splits) {
 		++a.split_shift;
 	}
-	// Down cut by rows instead of K where two workgroups per strip are what the K split would make anyway, they put a workgroup on
-	// every CU and a wave can hold its whole share of K (the LLaMA-3-8B block: 256 workgroups of 16 rows, seven half-size groups per
-	// wave): a finished row then leaves its workgroup directly, without the K-split hand-off's two trips through memory, on the path
-	// that ends the launch.  Measured at that block: 42.6 against 43.1 us (the stage behind the down projection 6.2 against 6.8 us).
-	// As a launch of its own, or in the one-launch FFN, the same cut measured no different from the K split.
-	a.down_by_rows = splits == 2 && strips_e * 2 <= 256 && (a.groups_f + GEMV_WAVES - 1) / GEMV_WAVES <= CHAIN_DOWN_ROWS_TILES;
+	a.down_by_rows	 = p.down_by_rows;
+	a.down_held		 = p.held;
 	a.first_norm	 = strips_e;
 	a.first_producer = a.first_norm + 1;
 	a.first_consumer = a.first_producer + static_cast<int>(n_ff / STRIP_ROWS);
-	a.second_norm	 = a.first_consumer + strips_e * splits;
-	// A CU holds one workgroup.  The last round of gate/up strips leaves some CUs to the first down workgroups, which cannot work before that round is through:
-	// requested at once, their weights only take bandwidth from the strips that everybody waits for.  They hold their requests back for CHAIN_HOLD_CLOCKS
-	// (measured at the [4096 / 14336] block: 41.35 us without, 40.8 with 4096 clocks, 40.45 with 6144; without / with 6144 [4096 / 11008] 37.0 / 35.9,
-	// [3200 / 10880] 31.9 / 30.7, [4096 / 20480] 55.3 / 53.1, [7168 / 20480] 98.5 / 97.0, [8192 / 22016] 117.8 / 117.1).  Not where they are much of the chip: then their
-	// bytes are what the round has to move ([2560 / 10240] with 191 of them 24.75 / 25.2, [8192 / 18560] with 187 103.8 / 105.3, [6144 / 11008] with 167 57.0 / 58.1; up
-	// to 4096 values, whose strips are shorter, [4096 / 11008] with 167 still gains).  Nor where they are the stage, all but an eighth ([2048 / 11008] 23.1 / 23.9,
-	// [1024 / 14336] 20.8 / 22.2), or it takes a part of a second round ([6144 / 13824], 384 workgroups: 63.6 / 66.1; [2176 / 19072], 272: 35.5 / 36.9), nor behind a third
-	// round, by when the strips no longer change in step ([8192 / 28672] 143.1 / 143.9), nor for a handful ([2560 / 16256], 3: 32.8 / 33.2).
-	const int down_wgs	  = strips_e * splits;
-	const int rounds_left = a.first_consumer - a.first_producer - (CHAIN_CUS - 1); // strips behind those that start with attn_out's end or before
-	const int beside	  = (CHAIN_CUS - rounds_left % CHAIN_CUS) % CHAIN_CUS;
-	const bool held		  = rounds_left > 0 && rounds_left <= 2 * CHAIN_CUS && beside >= CHAIN_CUS / 16 && beside <= (one_chunk ? CHAIN_CUS * 11 / 16 : CHAIN_CUS / 2) && beside * 8 <= down_wgs * 7
-		&& (down_wgs <= CHAIN_CUS || down_wgs >= 2 * CHAIN_CUS);
-	a.down_held			  = held ? beside : 0;
+	a.second_norm	 = a.first_consumer + strips_e * p.splits;
 	a.first_next	 = a.second_norm + 1;
 	const unsigned grid = static_cast<unsigned>(next_strips > 0 ? a.first_next + next_strips : a.second_norm);
 	a.attn_row		= sc.row_tagged[0];
@@ -547,7 +503,7 @@ hipError_t launch_decode_layer(const void* w_o, const float* attn, const float* 
 	a.error_word	= sc.error_word;
 	a.spin_limit	= sc.spin_limit;
 	const dim3 block(GEMV_WAVES * 64);
-	return one_chunk ? launch_kernel(KIND_GEMV, decode_layer_kernel<1>, dim3(grid), block, 0, s, a) : launch_kernel(KIND_GEMV, decode_layer_kernel<2>, dim3(grid), block, 0, s, a);
+	return p.one_chunk ? launch_kernel(KIND_GEMV, decode_layer_kernel<1>, dim3(grid), block, 0, s, a) : launch_kernel(KIND_GEMV, decode_layer_kernel<2>, dim3(grid), block, 0, s, a);
 }
 
 } // namespace nh

@@ -368,8 +368,7 @@ hipError_t launch_ffn_decode(const void* w_gate, const void* w_up, const void* w
 	int64_t K, int64_t n_out, hipStream_t s);
 hipError_t copy_ffn_gate_up(float* gate_out, float* up_out, int64_t n_ff, hipStream_t s);
 // attn_out + residual -> norm -> gate/up -> SiLU * up -> down + residual -> norm -> up to GEMV_MAX_SEGMENTS projections, one launch where
-// the shape allows it (decode_layer_chains), else the three launches it stands for (q8_0_decode_layer.hip).  ffn_inp != l_out.
-bool decode_layer_chains(int64_t n_embd, int64_t n_ff, int64_t next_strips);
+// the shape allows it (plan_decode_layer in q8_0_plan.h), else the three launches it stands for (q8_0_decode_layer.hip).  ffn_inp != l_out.
 hipError_t launch_decode_layer(const void* w_o, const float* attn, const float* layer_in, float* ffn_inp, const void* w_gate, const void* w_up, const void* w_down, const float* ffn_norm_w,
 	float* l_out, const void* const* w_next, float* const* y_next, const int64_t* n_next, int count_next, const float* next_norm_w, float eps, int64_t n_embd, int64_t n_ff, hipStream_t s);
 // Runs only the activation staging of the fused kernel and writes what it staged as packed blocks (parity check).

@@ -636,4 +636,54 @@ inline mul_mat_plan plan_mul_mat(int64_t M, int64_t N, int64_t K, bool scratch =
 	return p;
 }
 
+// A decode block as one launch (q8_0_decode_layer.hip): whether the shape takes that form, and how its stages are cut.
+//
+// gate/up: a wave holds two groups of each matrix at a time: one such chunk covers its share up to 4096 values of hidden state, two up to 8192.
+//
+// Down: K over workgroups until a wave's share is four groups, within the scratch.  Cut by rows instead where two workgroups per strip are what that makes anyway, they put a
+// workgroup on every CU and a wave can hold its whole share of K (the LLaMA-3-8B block: 256 workgroups of 16 rows, seven half-size groups per wave): a finished row then leaves its
+// workgroup directly, without the K-split hand-off's two trips through memory, on the path that ends the launch.  Measured at that block: 42.6 against 43.1 us (the stage behind the
+// down projection 6.2 against 6.8 us).  As a launch of its own, or in the one-launch FFN, the same cut measured no different from the K split.
+constexpr int CHAIN_TILES = 4; // groups a wave stages at once: LDS slices are sized for it
+constexpr int CHAIN_DOWN_ROWS_TILES = 8; // ... in the down stage when it is cut by rows (half-size groups)
+constexpr int CHAIN_CUS = 256;
+struct decode_layer_plan {
+	bool one_launch, one_chunk, down_by_rows;
+	int splits; // workgroups per down strip
+	int held; // down workgroups that hold their weight requests back a while
+};
+inline decode_layer_plan plan_decode_layer(int64_t n_embd, int64_t n_ff, int64_t next_strips) {
+	decode_layer_plan p{};
+	if (n_embd <= 0 || n_ff <= 0 || n_embd % GROUP_K != 0 || n_ff % GROUP_K != 0 || n_embd > CHAIN_MAX_EMBD || n_ff > FFN_MAX_HIDDEN) {
+		return p;
+	}
+	const int strips_e = static_cast<int>(n_embd / STRIP_ROWS), groups_e = static_cast<int>(n_embd / GROUP_K), groups_f = static_cast<int>(n_ff / GROUP_K);
+	const auto share   = [&] { return (groups_f + GEMV_WAVES * p.splits - 1) / (GEMV_WAVES * p.splits); };
+	p.splits		   = 1;
+	while (share() > CHAIN_TILES && strips_e <= GEMV_MAX_SPLIT_STRIPS && strips_e * p.splits * 2 <= GEMV_MAX_SPLIT_UNITS) {
+		p.splits *= 2;
+	}
+	if (share() > CHAIN_TILES || next_strips < 0 || next_strips >= (1 << 20)) {
+		return p;
+	}
+	p.one_launch   = true;
+	p.one_chunk	   = (groups_e + GEMV_WAVES - 1) / GEMV_WAVES <= 2;
+	p.down_by_rows = p.splits == 2 && strips_e * 2 <= 256 && (groups_f + GEMV_WAVES - 1) / GEMV_WAVES <= CHAIN_DOWN_ROWS_TILES;
+	// A CU holds one workgroup.  The last round of gate/up strips leaves some CUs to the first down workgroups, whose weights, requested at once, take bandwidth from the strips that
+	// everybody waits for: also where K goes over workgroups and the first of them have their activation early.  They hold their requests back, up to 4096 values of hidden state
+	// (a fixed time, chosen at the [4096 / 14336] block: 41.35 us without, 40.8 with 4096 clocks, 40.45 with 6144).  117 random shapes within the lines below gain 1 to 5 %, mean 3.
+	// Above 4096 values, whose strips take two chunks, nothing is gained: 60 random shapes 0.98 to 1.03, mean 1.00 ([5760 / 21248] 79.9 / 81.5 us).
+	// Not where they are the stage, all but an eighth (40 random shapes 0.95 to 1.04, mean 0.98; with more than 176 of them as well 0.89 to 1.03, mean 0.97), where there are more than
+	// 176 and the stage takes a part of a second round (0.94 to 1.02, mean 0.96), nor for a handful (no different).  Either of the last two alone would gain as well (0.96 to 1.05,
+	// mean 1.03) and is left out.  Nor behind a third round, by when the strips no longer change in step ([8192 / 28672] 143.1 / 143.9).
+	const int down_wgs	  = strips_e * p.splits;
+	const int rounds_left = static_cast<int>(n_ff / STRIP_ROWS) - (CHAIN_CUS - 1); // strips behind those that start with attn_out's end or before
+	const int beside	  = (CHAIN_CUS - rounds_left % CHAIN_CUS) % CHAIN_CUS;
+	if (p.one_chunk && rounds_left > 0 && rounds_left <= 2 * CHAIN_CUS && beside >= CHAIN_CUS / 16 && beside <= CHAIN_CUS * 11 / 16 && beside * 8 <= down_wgs * 7 &&
+		(down_wgs <= CHAIN_CUS || down_wgs >= 2 * CHAIN_CUS)) {
+		p.held = beside;
+	}
+	return p;
+}
+
 } // namespace nh

@@ -115,6 +115,15 @@ def plan_gate_up_silu(m: int, n_ff: int, k: int) -> dict:
     return {"form": "three_launches"}
 
 
+def plan_decode_layer(n_embd: int, n_ff: int) -> dict:
+    """How decode_layer runs, and the cut of its down projection (no GPU needed)."""
+    import ctypes
+
+    raw = (ctypes.c_int32 * 4)()
+    _lib.check("nh_q8_0_debug_plan_decode_layer", _lib.lib().nh_q8_0_debug_plan_decode_layer(n_embd, n_ff, raw))
+    return {"one_launch": bool(raw[0]), "down_splits": raw[1], "down_by_rows": bool(raw[2]), "down_held": raw[3]}
+
+
 def quantize_row_q8_0(x: torch.Tensor, tiled: bool = False) -> torch.Tensor:
     """x fp32 [M, K] (or [K]) -> uint8 blocks [M, K/32*34] (or the tiled byte stream)."""
     x = _dev(x, torch.float32, "x")

@@ -51,20 +51,14 @@ SHAPES = [
 ]
 
 
-@pytest.mark.parametrize("n_embd,n_ff,next_rows,same_cut", SHAPES, ids=[f"{s[0]}x{s[1]}" for s in SHAPES])
-def test_decode_layer_one_launch(q8, oracle, n_embd, n_ff, next_rows, same_cut):
-    rng = np.random.default_rng(n_embd + n_ff)
-    host, dev, norms = _weights(q8, rng, n_embd, n_ff, next_rows)
-    attn = rng.standard_normal(n_embd).astype(np.float32)
-    layer_in = rng.standard_normal(n_embd).astype(np.float32)
-    d_attn, d_in = to_dev(attn), to_dev(layer_in)
+def _one_launch_stage_by_stage(q8, oracle, host, dev, norms, d_attn, d_in, n_embd, n_ff, next_rows):
+    # the checker on the launch's own previous stage
+    attn, layer_in = to_host(d_attn), to_host(d_in)
     h, y, nxt = q8.decode_layer(dev["o"], d_attn, d_in, dev["g"], dev["u"], dev["d"], to_dev(norms[0]), [dev[f"n{i}"] for i in range(len(next_rows))], list(next_rows),
                                 to_dev(norms[1]) if next_rows else None, EPS, n_embd, n_ff)
     g_gpu, u_gpu = (to_host(a) for a in q8.debug_ffn_gate_up(n_ff))
     h_gpu, y_gpu = to_host(h), to_host(y)
     assert np.isfinite(h_gpu).all() and np.isfinite(y_gpu).all()
-
-    # (1) stage by stage: the checker on the launch's own previous stage
     assert rel_l2(h_gpu, oracle.gemv(host["o"][0], oracle.quantize_rows(attn[None, :])[0], n_embd, n_embd) + layer_in) <= REL_L2_TOL
     hq = oracle.rms_norm_quantize_rows(h_gpu[None, :], norms[0], EPS)[0]
     assert rel_l2(g_gpu, oracle.gemv(host["g"][0], hq, n_ff, n_embd)) <= REL_L2_TOL
@@ -75,6 +69,17 @@ def test_decode_layer_one_launch(q8, oracle, n_embd, n_ff, next_rows, same_cut):
         yq = oracle.rms_norm_quantize_rows(y_gpu[None, :], norms[1], EPS)[0]
         for i, n in enumerate(next_rows):
             assert rel_l2(to_host(nxt[i]), oracle.gemv(host[f"n{i}"][0], yq, n, n_embd)) <= REL_L2_TOL, i
+    return h_gpu, y_gpu, nxt
+
+
+@pytest.mark.parametrize("n_embd,n_ff,next_rows,same_cut", SHAPES, ids=[f"{s[0]}x{s[1]}" for s in SHAPES])
+def test_decode_layer_one_launch(q8, oracle, n_embd, n_ff, next_rows, same_cut):
+    rng = np.random.default_rng(n_embd + n_ff)
+    host, dev, norms = _weights(q8, rng, n_embd, n_ff, next_rows)
+    attn = rng.standard_normal(n_embd).astype(np.float32)
+    layer_in = rng.standard_normal(n_embd).astype(np.float32)
+    d_attn, d_in = to_dev(attn), to_dev(layer_in)
+    h_gpu, y_gpu, nxt = _one_launch_stage_by_stage(q8, oracle, host, dev, norms, d_attn, d_in, n_embd, n_ff, next_rows)  # (1)
 
     # (2) the three launches it stands for
     h3, y3, nxt3 = _three_launches(q8, dev, norms, d_attn, d_in, n_embd, n_ff, next_rows)
@@ -90,10 +95,25 @@ def test_decode_layer_one_launch(q8, oracle, n_embd, n_ff, next_rows, same_cut):
             assert rel_l2(to_host(a), to_host(b)) <= 2e-3
 
 
-def test_decode_layer_launches_back_to_back_do_not_mix(q8, oracle):
+# Norm workgroups whose waves have runs of unequal length, of two groups and one and of three and two (the second float4 of a lane partly live); held workgroups in front of a down
+# stage cut by rows and in front of one with K over four workgroups.
+@pytest.mark.parametrize(
+    "n_embd,n_ff,next_rows,held",
+    [(3200, 10880, (3200, 640, 640), True), (2176, 12672, (2176, 256), True), (5120, 13824, (5120, 1024, 1024), False), (7168, 20480, (7168, 1024, 1024), False), (4096, 20480, (4096, 1024), True)],
+)
+def test_decode_layer_uneven_runs_and_holds(q8, oracle, n_embd, n_ff, next_rows, held):
+    p = q8.plan_decode_layer(n_embd, n_ff)
+    assert p["one_launch"] and (p["down_held"] > 0) == held, p
+    rng = np.random.default_rng(n_embd + n_ff)
+    host, dev, norms = _weights(q8, rng, n_embd, n_ff, next_rows)
+    attn, layer_in = (to_dev(rng.standard_normal(n_embd).astype(np.float32)) for _ in range(2))
+    _one_launch_stage_by_stage(q8, oracle, host, dev, norms, attn, layer_in, n_embd, n_ff, next_rows)
+
+
+@pytest.mark.parametrize("n_embd,n_ff,next_rows,blocks", [(1024, 3584, (1024, 256, 256), 6), (2176, 12672, (2176, 256, 256), 3), (4096, 20480, (4096, 128, 128), 2), (5120, 10240, (5120, 128, 128), 2)])
+def test_decode_layer_launches_back_to_back_do_not_mix(q8, oracle, n_embd, n_ff, next_rows, blocks):
     # a token's worth of launches on one stream without a wait in between, each block fed by the one before, then the same again
     # with one launch at a time: every word handed over inside a launch must be that launch's own
-    n_embd, n_ff, next_rows, blocks = 1024, 3584, (1024, 256, 256), 6
     rng = np.random.default_rng(5)
     layers = [_weights(q8, rng, n_embd, n_ff, next_rows) for _ in range(blocks)]
     x0 = to_dev(rng.standard_normal(n_embd).astype(np.float32))

@@ -168,6 +168,22 @@ def test_weights_past_the_caches(m, n, k, past):
     assert p["kernel"] == "gemm_skinny" and p["past_caches"] == past, p
 
 
+@pytest.mark.parametrize(
+    "n_embd,n_ff,splits,by_rows,held",
+    [(4096, 14336, 2, True, 63), (3200, 10880, 2, True, 171), (4096, 20480, 4, False, 127), (4096, 15872, 2, True, 0), (4096, 15744, 2, True, 19),  # cut by rows, along K; a handful
+     (4096, 10752, 2, True, 175), (4096, 10624, 2, True, 0), (2048, 11008, 2, True, 0), (3200, 17408, 4, False, 0), (4096, 8192, 1, False, 0),  # more than 176; most of the stage; a part of a second round; no round left
+     (4224, 20480, 4, False, 0), (5760, 21248, 4, False, 0), (8192, 22016, 4, False, 0), (8192, 28672, 4, False, 0)],  # above 4096 values
+)
+def test_decode_layer_holds(n_embd, n_ff, splits, by_rows, held):
+    assert q8_0.plan_decode_layer(n_embd, n_ff) == {"one_launch": True, "down_splits": splits, "down_by_rows": by_rows, "down_held": held}
+
+
+def test_decode_layer_beyond_the_one_launch():
+    assert not q8_0.plan_decode_layer(8320, 16384)["one_launch"]
+    with pytest.raises(q8_0._lib.Q8Error):
+        q8_0.plan_decode_layer(4096, 14400)
+
+
 def test_what_leaves_a_callers_workspace_untouched():
     # nh_q8_0_mul_mat's promise: 4 to 16 rows on matrices of up to 40 MB, 4 rows up to 80 MB.  Without a workspace of the caller's the faster way
     moved = 0
