@@ -145,17 +145,16 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_rows8_kernel(const uint8
 	}
 	__builtin_amdgcn_wave_barrier();
 
-	// thread 32 * m + l stores output (row m, strip row l); its residual (which may be that output) is requested here, a memory latency ahead of its use (behind
-	// a walk of several chunks, which has no register for it)
-	const int m = tid >> 5, l = tid & 31, row = strip * STRIP_ROWS + l;
-	float res	= 0.0f;
-	const auto request_residual = [&] {
+	// thread 32 * m + l stores output (row m, strip row l).  With the sixteen-row operand its residual (which may be that output) is requested here, a memory latency ahead of its
+	// use, but for a walk of several chunks, which has no register for it.  With the eight-row one behind the reduction: requested here it takes longer (100 random shapes of four
+	// rows 1.029 times as long, [2800 x 3072] 5.03 us for 4.81; of 5 to 8 rows 1.004; of 9 to 16 with the other one 0.994)
+	constexpr bool RESIDUAL_AHEAD = R > 8 && !LOOP;
+	float res					  = 0.0f;
+	if constexpr (RESIDUAL_AHEAD) {
+		const int m = tid >> 5, row = strip * STRIP_ROWS + (tid & 31);
 		if (residual && m < M && row < N) {
 			res = residual[static_cast<int64_t>(m) * N + row];
 		}
-	};
-	if constexpr (!LOOP) {
-		request_residual();
 	}
 	const uint8_t* w_strip = W + macro_offset(strip, 0, groups);
 	float acc[R / 2];
@@ -170,7 +169,6 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_rows8_kernel(const uint8
 			rows8_chunk<R, TILES>(w_strip, x, K, M, a_tiles[wave], a_scales[wave], gc, min(TILES, g1 - gc), lane, acc);
 			__builtin_amdgcn_wave_barrier(); // the next chunk overwrites this wave's tiles
 		}
-		request_residual();
 	}
 
 	// ---- one reduction per workgroup, fixed order: thread 32 * m + l owns output (row m, strip row l) ----
@@ -179,6 +177,7 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_rows8_kernel(const uint8
 		red[e][wave][lane] = acc[e];
 	}
 	__syncthreads();
+	const int m = tid >> 5, l = tid & 31, row = strip * STRIP_ROWS + l;
 	if (m >= M || m >= R) {
 		return;
 	}
@@ -186,6 +185,11 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_rows8_kernel(const uint8
 #pragma unroll
 	for (int w = 0; w < GEMV_WAVES; ++w) {
 		total += red[4 * (m >> 3) + (m & 3)][w][32 * ((m >> 2) & 1) + l]; // row m = 8 e4 + 4 half + i sits in lanes of that half, sum 4 e4 + i
+	}
+	if constexpr (!RESIDUAL_AHEAD) {
+		if (residual && row < N) {
+			res = residual[static_cast<int64_t>(m) * N + row];
+		}
 	}
 	float* ym = y + static_cast<int64_t>(m) * N;
 	if (splits == 1) {
