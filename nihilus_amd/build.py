@@ -33,8 +33,8 @@ HIPCC_FLAGS = [
     "-mllvm", "-amdgpu-mfma-vgpr-form",
 ]
 # A kernel's first arguments (up to sixteen dwords) arrive in scalar registers with the wave instead of being read from memory by it, a miss of the scalar
-# cache in front of the first address; kernels name what that address takes first.  norm + quantize of 4 rows 3.02 -> 2.77 us, [1024 x 4096] at 4 rows
-# 4.17 -> 3.99, mul_mat of 4 / 16 rows [4096 x 4096] 6.3 -> 5.9 and 10.2 -> 9.5, [1024 x 4096] at 512 rows 10.3 -> 10.1.
+# cache in front of the first address; kernels name what that address takes first.  norm + quantize of 4 rows 3.14 -> 2.95 us, of 16 3.48 -> 3.33, of [64 x 8192]
+# 4.38 -> 4.14; mul_mat of 2 to 16 rows, 60 random shapes of each number, 1.03 to 1.05 times as fast.
 PRELOAD_FLAGS = ["-mllvm", "-amdgpu-kernarg-preload-count=16"]
 # not where a launch is many short waves, each of which then starts later: embedding rows of 4 tokens 1.83 us without, 1.99 with; [14336 x 4096] into the
 # device layout 25.0 / 25.8

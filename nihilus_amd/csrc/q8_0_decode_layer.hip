@@ -84,8 +84,8 @@ __device__ __forceinline__ bool give_up(int& spins, int limit, unsigned* error_w
 // The norm workgroup: the fp32 row `row` (tagged words, written by the workgroups of the stage before) -> (row * scale) * norm_w
 // -> quantize_row_q8_0 -> published blocks.  Sixteen waves; wave w takes run w of the fixed-order sum of squares (q8_0_device.h),
 // lane l the float4s l, l + 64, ... of that run -- for the sum and for the quantizer alike, so the row is read once, into registers.
-// F4: float4s per lane, 1 for rows of up to 4096 values, 2 up to CHAIN_MAX_EMBD.  (A second one that a short row leaves zero cost the quantizer's slow route:
-// 0.5 us of the 1.2 from the row's scale to its publication.)
+// F4: float4s per lane, 1 for rows of up to 4096 values, 2 up to CHAIN_MAX_EMBD.  (With a second one that a short row leaves zero the way from the row's scale to its publication,
+// a second pass of the quantizer among it, took 1.2 us instead of 0.7.)
 // The same sequence of fp32 operations as rms_norm_quantize_kernel and the mat-vec kernels' own norm, hence the same bytes.
 template<int F4> __device__ __forceinline__ void norm_workgroup(const uint64_t* __restrict__ row, const float* __restrict__ norm_w, uint64_t* __restrict__ out, int groups, float eps, unsigned epoch,
 	unsigned* error_word, int spin_limit, float* red, uint32_t* words, int lane, int wave) {
@@ -184,9 +184,9 @@ __device__ __forceinline__ void store_row(float* __restrict__ y, uint64_t* __res
 	y[row] = v;
 }
 
-// A down row's residual is this launch's own attn_out row, which other workgroups have published.  It is requested at a workgroup's start, a memory latency
-// ahead of its use: published by then, as a down workgroup only becomes resident behind gate/up workgroups, which wait for all of attn_out.  Should
-// its word not be there yet, it is read again where it is used, when it is certain to be: the workgroup's activation exists only because the norm workgroup
+// A down row's residual is this launch's own attn_out row, which other workgroups publish.  It is requested at a workgroup's start, a memory latency ahead of its use.  Where the down
+// workgroup became resident behind gate/up workgroups, which wait for all of attn_out, its word is there; where all of the stages in front fit the CUs ([2048 / 5632]: 241 workgroups)
+// it may not be, and is read again where it is used, when it is certain to be: the workgroup's activation exists only because the norm workgroup
 // read every row.  (A word that does not carry the epoch even then poisons the row.)
 __device__ __forceinline__ uint64_t request_attn_row(const uint64_t* __restrict__ attn_row, int row, bool real) {
 	return real ? __hip_atomic_load(&attn_row[row], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;

@@ -171,7 +171,8 @@ template<int TILES, bool LOOP, bool NORM, bool PAIR = false> __global__ __launch
 	int g0, g1;
 	wave_k_range(a.groups_c, a.split_shift, split, GEMV_WAVES, wave, g0, g1);
 
-	// thread t stores row t of the strip; its residual (which may be that output) is requested here, a memory latency ahead of its use
+	// thread t stores row t of the strip; its residual (which may be that output) is requested here, a memory latency ahead of its use (100 random FFNs with one: 1.005 times
+	// as fast as with the read behind the reduction, 1.002 with it in front of the reduction)
 	const int row = gstrip * STRIP_ROWS + tid;
 	float res	  = 0.0f;
 	if (a.residual && tid < STRIP_ROWS && row < a.n_out) {

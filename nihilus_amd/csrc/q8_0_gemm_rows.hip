@@ -241,7 +241,7 @@ __global__ __launch_bounds__(SK_WAVES * 64, 4) void gemm_rows_kernel(const uint8
 	const int strip = static_cast<int>(blockIdx.x >> split_shift);
 	const int split = static_cast<int>(blockIdx.x) & ((1 << split_shift) - 1);
 	// thread t finishes outputs (row t / 32 + 16 i, strip column t % 32); their residuals (which may be those outputs) are requested here, a memory
-	// latency ahead of their use
+	// latency ahead of their use (100 random shapes, half of them with one: as fast as with the read behind the reduction, 0.98 to 1.04)
 	constexpr int OWN = (R + 15) / 16;
 	const int m0 = tid >> 5, l = tid & 31, n = strip * STRIP_ROWS + l;
 	const int rows = min(M, R);

@@ -352,7 +352,7 @@ template<int MS> static hipError_t launch_skinny_t(int splits, int waves, const 
 	return nt ? launch(gemm_skinny_kernel<MS, 2, SK_WAVES, true>) : launch(gemm_skinny_kernel<MS, 2, SK_WAVES, false>);
 }
 
-// cut: plan_gemm_skinny, or the stand-in for a tile kernel's (q8_0_plan.h)
+// cut: plan_gemm_streaming, or the stand-in for the rows kernel's or the tile kernel's (q8_0_plan.h)
 hipError_t launch_gemm_skinny(const void* W, const void* Aq, float* C, int64_t M, int64_t N, int64_t K, const gemm_skinny_cut& cut, hipStream_t s, const float* residual) {
 	const uint8_t* w = static_cast<const uint8_t*>(W);
 	const uint8_t* a = static_cast<const uint8_t*>(Aq);

@@ -23,7 +23,7 @@ enum mul_mat_kernel : int {
 };
 
 constexpr int SK_WAVES			  = 8; // waves per workgroup of the weight-streaming MFMA kernel
-constexpr int SK_WIDE_WAVES		  = 16; // the same in grids of 129 to 255 workgroups (plan_gemm_skinny)
+constexpr int SK_WIDE_WAVES		  = 16; // the same where K over eight more is better than over another workgroup (plan_gemm_skinny, plan_gemm_streaming)
 constexpr int SK_MAX_SPLIT_UNITS  = 2048; // strips * splits when splits > 1
 constexpr int SK_MAX_SPLIT_STRIPS = 512;
 constexpr int GEMM_SPLIT_MIN_TRIPS = 2; // K goes over more workgroups only while each K set keeps this many 128-quant groups
@@ -73,7 +73,8 @@ inline gemm_tile_cut plan_gemm_tile(int64_t M, int64_t N, int64_t K, bool stream
 //   gate/up   [2 x 1280 x 1280] at 788 rows (three for two) 32 / 20, [2 x 8960 x 5760] at 233 (five for three) 96 / 94, [2 x 2560 x 4608] at 787 79 / 58, [2 x 5248 x 3200] at 578
 //             (seven for four) 72.6 / 68.5, [2 x 17792 x 4096] at 266 (ten for six) 142 / 128; but with eleven for six [2 x 28672 x 8192] at 178 261 / 274,
 //             [2 x 22016 x 5632] at 236 181 / 189, [2 x 5376 x 2048] at 326 30.8 / 33.4 ([2 x 10368 x 7936] at 543 257 / 252), thirteen for seven [2 x 25600 x 5248] at 243 210 / 302
-// Not with four strips, whose weights come from memory for most of them ([20480 x 4096] at 100 rows 41 / 43, [2 x 9344 x 7808] at 119 78 / 80).
+// Over 70 random shapes each whose cut differs: mat-mats 0.94 to 1.44 times as fast, mean 1.07; gate/up 0.98 to 1.60, mean 1.10.  Not with four strips ([20480 x 4096] at 100 rows 41 / 43,
+// [2 x 9344 x 7808] at 119 78 / 80): of 50 random shapes each mat-mats 0.91 to 1.27, mean 0.98, gate/up 0.91 to 1.29, mean 1.01.
 constexpr int ONE_STRIP_MAT_MAT = 115, ONE_STRIP_GATE_UP = 110;
 inline bool gemm_tile_take_one_strip(gemm_tile_cut* c, int64_t m_strips, int percent) {
 	const int64_t twos = int64_t{ c->grid_x } * c->grid_y, ones = int64_t{ c->grid_x } * m_strips;
@@ -89,30 +90,31 @@ inline bool gemm_tile_take_one_strip(gemm_tile_cut* c, int64_t m_strips, int per
 //
 // By XCD: workgroups go to the eight XCDs in turn.  With a number of column blocks that eight divides, a block's row groups are all on one XCD, whose L2 has its weights then;
 // otherwise every XCD would read nearly all of them.  There each XCD takes the tiles of some consecutive column blocks instead, row groups fastest ([24171 x 10240] at 145 rows
-// 182 -> 126 us, [3117 x 10752] at 912 134 -> 92, [2 x 3968 x 6528] at 274 77 -> 59 with one strip per wave; with two, 50 random shapes 1.02 times as fast).  Not with eight
-// dividing: a round of workgroups is a wider piece of the matrix then as it is ([8192 x 8192] at 330 rows 72 us, 76 this way).
+// 182 -> 126 us, [3117 x 10752] at 912 134 -> 92, [2 x 3968 x 6528] at 274 77 -> 59 with one strip per wave; 60 random shapes with one 0.99 to 1.62 times as fast, mean 1.20, 120 with two
+// 0.98 to 1.17, mean 1.04).  Not with eight dividing: a round of workgroups is a wider piece of the matrix then as it is ([8192 x 8192] at 330 rows 72 us, 76 this way).
 //
 // In bands of that many column blocks, all row groups of a band before the next band is begun, where eight divides their number.  With one band, every group of rows walks the
 // whole matrix, from memory again where it is no longer cached, and the workgroups that run together share only their activations.  Measured, us, one band / this:
-//   gate/up   [2 x 28672 x 8192] at 512 rows 740 / 628, at 178 two strips 285 / 274; [2 x 14336 x 4096] at 3001 933 / 897; [2 x 26624 x 9344] at 858 1377 / 1122;
-//             with one strip per wave [2 x 21504 x 7808] at 200 318 / 231, [2 x 24576 x 1920] at 273 123 / 91
-//   mat-mats  [27648 x 4736] at 1058 365 / 357, [20475 x 9984] at 1965 988 / 956
-// Bands of 16 to 64 column blocks are within 1 % of each other.  Not where the matrix is found in a cache again as it is, or the launch is over before its workgroups have
-// drifted apart (random shapes, one band / this):
-//   two strips per wave, less than 8e10 products     83 mat-mats 0.90 to 1.01, mean 0.98 ([18432 x 2048] at 500 rows 56 / 60), 302 gate/up 0.96 to 1.05, mean 0.99;
-//                        more                        67 mat-mats 0.98 to 1.14, mean 1.02, 93 gate/up 0.98 to 1.22, mean 1.03
-//   one strip per wave   less than 80 MiB of weights 60 mat-mats 0.81 to 1.03, mean 0.95; more 40, 0.94 to 1.39, mean 1.09
-//                        gate/up, less than 48 MiB   9, 0.95 to 1.01, mean 0.99; more 66, 0.98 to 1.55, mean 1.11
-// Below 128 column blocks nothing changes ([2 x 5632 x 7680] at 660 rows 164 / 163, [9146 x 9216] at 326 90.4 / 91.0), and two row groups of a mat-mat find each other's weights
-// on their way as it is ([22528 x 2944] at 118 rows 33.2 / 33.3).
+//   gate/up   [2 x 28672 x 8192] at 512 rows 740 / 578, at 178 two strips 289 / 252; [2 x 14336 x 4096] at 512 / 3001 166 / 157, 917 / 855; [2 x 26624 x 9344] at 858 1365 / 1064;
+//             with one strip per wave [2 x 21504 x 7808] at 200 316 / 223, [2 x 24576 x 1920] at 273 121 / 88; 61 random shapes 0.97 to 1.73 times as fast, mean 1.15, 149 with two strips
+//             0.98 to 1.22, mean 1.04
+//   mat-mats  [27648 x 4736] at 1058 360 / 341, [20475 x 9984] at 1965 973 / 930, [25530 x 6784] at 738 340 / 325; 39 random shapes 0.99 to 1.16, mean 1.05, 59 with one strip 0.94 to 1.47,
+//             mean 1.07; but below 2e10 products 8 of 0.95 to 1.01, mean 0.98 ([17408 x 2432] at 162 0.95), and with one strip below 40 MiB of weights 34 of 0.85 to 1.01, mean 0.95
+//             ([22528 x 384] at 216 0.85): there it stays as it is
+// (In runs of some milliseconds with waits between them the bands look worse than this, by up to 5 %: launches one after the other for tens of milliseconds run at a lower clock, as a
+// prompt's do, and there the bytes saved count.  The figures are of such.)
+// Bands of 16 to 64 column blocks are within 1 % of each other.  Below 128 nothing changes ([2 x 5632 x 7680] at 660 rows 161 / 161, [9146 x 9216] at 326 88.0 / 88.1), and two
+// row groups of a mat-mat find each other's weights on their way as it is ([22528 x 2944] at 118 rows 32.9 / 32.9; gate / up [2 x 24064 x 8320] at 125 159 / 152).
 constexpr int TILE_ORDER_GRID = 0, TILE_ORDER_XCD = 1, TILE_ORDER_BANDS = 32;
-constexpr int64_t TILE_BANDS_MIN_PRODUCTS = 80'000'000'000, TILE_BANDS_ONE_STRIP_BYTES = 80ll << 20, TILE_BANDS_ONE_STRIP_BYTES_GATE_UP = 48ll << 20;
-inline int gemm_tile_order(const gemm_tile_cut& c, bool gate_up, int64_t M, int64_t N, int64_t K) { // N: rows of weights, of both matrices for gate/up
+constexpr int64_t TILE_BANDS_MIN_PRODUCTS = 20'000'000'000, TILE_BANDS_ONE_STRIP_BYTES = 40ll << 20;
+inline int gemm_tile_order(const gemm_tile_cut& c, bool gate_up, int64_t M, int64_t N, int64_t K) {
 	if (c.grid_x % 8 != 0) {
 		return c.grid_y > 1 ? TILE_ORDER_XCD : TILE_ORDER_GRID;
 	}
-	const bool enough = c.tm == 1 ? N * (K / QK) * BLOCK_BYTES >= (gate_up ? TILE_BANDS_ONE_STRIP_BYTES_GATE_UP : TILE_BANDS_ONE_STRIP_BYTES) : M * N * K >= TILE_BANDS_MIN_PRODUCTS;
-	return c.grid_x >= 128 && c.grid_y > (gate_up ? 1u : 2u) && enough ? TILE_ORDER_BANDS : TILE_ORDER_GRID;
+	if (c.grid_x < 128 || c.grid_y < (gate_up ? 2u : 3u)) {
+		return TILE_ORDER_GRID;
+	}
+	return gate_up || (c.tm == 1 ? N * (K / QK) * BLOCK_BYTES >= TILE_BANDS_ONE_STRIP_BYTES : M * N * K >= TILE_BANDS_MIN_PRODUCTS) ? TILE_ORDER_BANDS : TILE_ORDER_GRID;
 }
 
 // The tile kernel's cut for a mat-mat of its own (K not over workgroups).  Uneven sets walk as many trips as the longest, so short ones multiply up to a tenth
@@ -211,21 +213,21 @@ inline bool gemm_skinny_past_caches(int64_t M, int64_t N, const gemm_skinny_cut&
 }
 
 // The streaming kernel's own mat-mats of more than 32 rows: never fewer shares of K than above, in another cut where that is faster (measured, us, cut above / this; in
-// brackets 70 random shapes of each kind).
+// brackets 50 random shapes of each kind).
 // - One strip per workgroup instead of two, up to 512 workgroups of one (of three strips, whose fourth would be work for nothing, up to 640): half as many leave
 //   a part of the chip's last round idle ([4864 x 2432] at 94 rows 11.4 / 7.9, [5632 x 3968] at 72 16.8 / 13.0, [3016 x 7424] at 148 24.1 / 21.5; with five strips
-//   [3346 x 2176] at 144, 525 of one, 10.3 / 11.0; 0.98 to 1.45, mean 1.24).  Also where two strips make just a workgroup per CU, if those are of eight row strips and
+//   [3346 x 2176] at 144, 525 of one, 10.3 / 11.0; 0.98 to 1.47, mean 1.23).  Also where two strips make just a workgroup per CU, if those are of eight row strips and
 //   more: two workgroups on a CU wait for their loads in turn ([2048 x 1024] at 256 5.3 / 4.7, [1024 x 4096] at 512 10.4 / 10.4; [4096 x 4096] at 128 12.3 / 12.4).
 // - Two strips instead of one, with sixteen waves, where those fit a workgroup per CU and ones of a strip do not, from K = 5248 on: the weights cross L2 once for
 //   two strips ([7296 x 8832] at 36 rows 24.6 / 19.5, [5888 x 13568] at 48 37.7 / 28.8; at K = 4608 11.6 / 12.0).  With more than 64
 //   rows from 360 workgroups on ([2560 x 6144] at 103 rows, 320, 12.7 / 14.1), and up to 192 ([1152 x 9856] at 310 18.4 / 19.0): 0.92 ([3200 x 5504] at 120) to 1.14 times
-//   as fast below K = 7680, [2658 x 14464] at 170 33.1 / 28.2.  (Of all 70 0.92 to 1.33, mean 1.15.)
+//   as fast below K = 7680, [2658 x 14464] at 170 33.1 / 28.2.  (Of all 0.92 to 1.40, mean 1.13.)
 // - Sixteen waves instead of eight for 65 to 160 workgroups and eleven to 31 groups, and for more workgroups while a wave of eight has two groups or so: all of a wave's
 //   share is on its way at once ([768 x 2048] at 104 rows 4.8 / 4.5, [1569 x 1664] at 57 4.8 / 4.7; [2048 x 2304] at 127, 256 workgroups, 5.8 / 6.0; up to 64
-//   workgroups it may lose, [611 x 2688] at 80 rows 5.3 / 5.65; 0.94 to 1.29, mean 1.02).  Not instead of two workgroups of eight: 65 to 128 of them, with more than 64 rows
-//   and up to 40 groups, 0.91 to 1.01, mean 0.96 ([1024 x 4096] at 117 rows 6.7 / 7.1, the same bits).
+//   workgroups it may lose, [611 x 2688] at 80 rows 5.3 / 5.65; 0.95 to 1.08, mean 1.02).  Not instead of two workgroups of eight: 65 to 128 of them, with more than 64 rows
+//   and up to 40 groups, 0.92 to 1.00, mean 0.96 ([1024 x 4096] at 117 rows 6.7 / 7.1, the same bits).
 // - Four workgroups along K instead of two for up to 64 and from 34 groups on, as a CU more costs nothing there ([457 x 6272] at 40 rows 7.5 / 6.1, [384 x 8064] at
-//   34 8.2 / 6.4; 1.09 to 1.29, mean 1.18).
+//   34 8.2 / 6.4; 1.08 to 1.30, mean 1.20).
 // Not in more shares where gate / up of such a pair are one launch, which has no room for sixteen (plan_gate_up_with): one launch and three give the same bytes
 // there (one in a hundred of the pairs whose mat-mats run here: [2 x 2688 x 2048] at 69 rows, [2 x 3840 x 6144] at 98), and
 // the mat-mats cost no more: 40 random ones of those with sixteen shares / these 0.91 to 1.09, mean 1.01.
@@ -517,7 +519,7 @@ inline bool plan_gate_up_with(bool even, const gemm_plan& g, int64_t M, int64_t 
 	if (c.tile.ks <= 2) {
 		gemm_tile_take_one_strip(&c.tile, (M + STRIP_ROWS - 1) / STRIP_ROWS, ONE_STRIP_GATE_UP);
 	}
-	c.tile.order = gemm_tile_order(c.tile, true, M, 2 * n_ff, K);
+	c.tile.order = gemm_tile_order(c.tile, true, M, n_ff, K);
 	if (cut) {
 		*cut = c;
 	}
@@ -672,7 +674,7 @@ inline decode_layer_plan plan_decode_layer(int64_t n_embd, int64_t n_ff, int64_t
 	// A CU holds one workgroup.  The last round of gate/up strips leaves some CUs to the first down workgroups, whose weights, requested at once, take bandwidth from the strips that
 	// everybody waits for: also where K goes over workgroups and the first of them have their activation early.  They hold their requests back, up to 4096 values of hidden state
 	// (a fixed time, chosen at the [4096 / 14336] block: 41.35 us without, 40.8 with 4096 clocks, 40.45 with 6144).  117 random shapes within the lines below gain 1 to 5 %, mean 3.
-	// Above 4096 values, whose strips take two chunks, nothing is gained: 60 random shapes 0.98 to 1.03, mean 1.00 ([5760 / 21248] 79.9 / 81.5 us).
+	// Above 4096 values, whose strips take two chunks, it goes either way: 100 random shapes 0.98 to 1.03, mean 1.00 ([5760 / 21248] 79.9 / 81.5 us, [7296 / 22528] 109.2 / 107.0).
 	// Not where they are the stage, all but an eighth (40 random shapes 0.95 to 1.04, mean 0.98; with more than 176 of them as well 0.89 to 1.03, mean 0.97), where there are more than
 	// 176 and the stage takes a part of a second round (0.94 to 1.02, mean 0.96), nor for a handful (no different).  Either of the last two alone would gain as well (0.96 to 1.05,
 	// mean 1.03) and is left out.  Nor behind a third round, by when the strips no longer change in step ([8192 / 28672] 143.1 / 143.9).

@@ -1,4 +1,4 @@
-"""GPU parity: the MFMA tile kernel on wide matrices, whose column blocks it goes through in bands where the launch is large enough, and as its grid has them otherwise."""
+"""GPU parity: the MFMA tile kernel on matrices wide enough that it goes through their column blocks in bands, where the launch is large enough."""
 import numpy as np
 import pytest
 
@@ -32,7 +32,7 @@ def edge_rows(m):
 
 # In bands: whole ones (the narrowest matrix that has them, 128 column blocks) and a last one of 8, 16 and 24; one strip per wave and two, one K set and two; ragged rows and columns.
 # The rows on both sides of the strips' and row groups' edges, all columns.
-@pytest.mark.parametrize("m,n,k,cut", [(129, 128 * 128, 4864, (1, 2)), (140, 128 * 152 - 127, 4352, (1, 2)), (70, 128 * 168, 4096, (1, 2)), (500, 128 * 144 - 70, 9216, (2, 1)), (1030, 128 * 136, 4608, (2, 1))])
+@pytest.mark.parametrize("m,n,k,cut", [(129, 128 * 128, 2432, (1, 1)), (140, 128 * 152 - 127, 2176, (1, 1)), (70, 128 * 168, 2048, (1, 2)), (500, 128 * 144 - 70, 2304, (2, 1)), (1030, 128 * 136, 1152, (2, 1))])
 def test_bands(q8, oracle, m, n, k, cut):
     p = q8.plan_mul_mat(m, n, k)
     assert p["kernel"] == "gemm_tile" and p["order"] == "bands_of_32" and (p["activation_strips"], p["k_sets"]) == cut, p
@@ -46,28 +46,11 @@ def test_bands(q8, oracle, m, n, k, cut):
         assert rel_l2(to_host(got[row]), want[i]) <= REL_L2_TOL, row
 
 
-# The fused gate/up launch in bands against the two mat-mats, which take their tiles in another order or have none: one strip per wave, in one pass and in four, two strips, two row
-# groups; a last band of 8, 24 and none.
-@pytest.mark.parametrize("m,n_ff,k,grid", [(385, 8704, 2816, (136, 13)), (72, 8704, 2816, (136, 3)), (300, 9728, 13824, (152, 5)), (128, 24576, 12800, (384, 2))])
+# The fused gate/up launch: two row groups too; one K set, two, and two in passes.
+@pytest.mark.parametrize("m,n_ff,k,grid", [(100, 8192, 1024, (128, 2)), (100, 8704, 2048, (136, 2)), (193, 8192, 1024, (128, 4)), (290, 9216, 256, (144, 5)), (161, 9728, 128, (152, 3)), (385, 8704, 256, (136, 13))])
 def test_gate_up_bands(q8, oracle, m, n_ff, k, grid):
     p = q8.plan_gate_up_silu(m, n_ff, k)
-    assert p["form"] == "tile" and p["grid"] == grid and p["order"] == "bands_of_32" and q8.plan_mul_mat(m, n_ff, k).get("order") != "bands_of_32", p
-    tg, tu = (q8.tile(q8.fill_weight_blocks(s + m, n_ff, k), n_ff, k) for s in (21, 22))
-    aq = q8.quantize_row_q8_0(q8.fill_activations(m + k, m * k).reshape(m, k), tiled=True)
-    act, gate, up = q8.gate_up_silu(tg, tu, aq, m, n_ff, k, debug=True)
-    for got, w in ((to_host(gate), tg), (to_host(up), tu)):
-        want = to_host(q8.gemm(w, aq, m, n_ff, k, tiled=True))
-        for i in range(m):
-            assert rel_l2(got[i], want[i]) <= REL_L2_TOL, i
-    assert np.array_equal(to_host(act), to_host(q8.silu_mul_quantize(gate, up, tiled=True)))
-    assert np.array_equal(to_host(act), to_host(q8.gate_up_silu(tg, tu, aq, m, n_ff, k)))
-
-
-# The fused gate/up launch as its grid has the tiles: two row groups too; one K set, two, and two in passes.
-@pytest.mark.parametrize("m,n_ff,k,grid", [(100, 8192, 1024, (128, 2)), (100, 8704, 2048, (136, 2)), (193, 8192, 1024, (128, 4)), (290, 9216, 256, (144, 5)), (161, 9728, 128, (152, 3)), (385, 8704, 256, (136, 13))])
-def test_gate_up_wide_as_the_grid_has_it(q8, oracle, m, n_ff, k, grid):
-    p = q8.plan_gate_up_silu(m, n_ff, k)
-    assert p["form"] == "tile" and p["grid"] == grid and p["order"] == "grid", p
+    assert p["form"] == "tile" and p["grid"] == grid and p["order"] == "bands_of_32", p
     wg, wu = oracle.fill_weights(21 + m, n_ff, k), oracle.fill_weights(22 + m, n_ff, k)
     x = oracle.fill_activations(m + k, m * k).reshape(m, k)
     aq_cpu = oracle.quantize_rows(x)

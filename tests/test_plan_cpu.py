@@ -143,8 +143,8 @@ def test_gate_up_in_one_launch_has_the_shares_of_the_streaming_mat_mats():
 @pytest.mark.parametrize(
     "m,n,k,strips,order",
     [(129, 128 * 127, 256, 1, "by_xcd"), (1000, 128 * 129, 4096, 2, "by_xcd"), (117, 128 * 137, 256, 2, "by_xcd"),  # a number of column blocks that eight does not divide
-     (129, 128 * 128, 4864, 1, "bands_of_32"), (129, 128 * 128, 4736, 1, "grid"), (140, 128 * 120, 8192, 1, "grid"),  # one strip per wave: 80 MiB of weights, 128 column blocks
-     (512, 128 * 144, 8576, 2, "bands_of_32"), (512, 128 * 144, 8448, 2, "grid"), (3001, 14336, 4096, 2, "grid"), (128, 128 * 136, 40960, 2, "grid")],  # two: 8e10 products, three row groups
+     (129, 128 * 128, 2432, 1, "bands_of_32"), (129, 128 * 128, 2304, 1, "grid"), (140, 128 * 120, 8192, 1, "grid"),  # one strip per wave: 40 MiB of weights, 128 column blocks
+     (512, 128 * 144, 2176, 2, "bands_of_32"), (512, 128 * 144, 2048, 2, "grid"), (3001, 14336, 4096, 2, "grid"), (128, 128 * 136, 40960, 2, "grid")],  # two: 2e10 products, three row groups
 )
 def test_order_of_the_tiles(m, n, k, strips, order):
     p = q8_0.plan_mul_mat(m, n, k)
@@ -153,8 +153,8 @@ def test_order_of_the_tiles(m, n, k, strips, order):
 
 @pytest.mark.parametrize(
     "m,n_ff,k,strips,order",
-    [(385, 8704, 2816, 1, "bands_of_32"), (385, 8704, 2688, 1, "grid"), (300, 9728, 13824, 2, "bands_of_32"), (300, 9728, 13568, 2, "grid"), (128, 24576, 12800, 2, "bands_of_32"), (128, 24576, 12672, 2, "grid"),
-     (512, 14336, 4096, 2, "grid"), (3001, 14336, 4096, 2, "bands_of_32"), (512, 11008, 4096, 2, "by_xcd")],
+    [(385, 8704, 256, 1, "bands_of_32"), (193, 8192, 1024, 2, "bands_of_32"), (100, 8192, 1024, 2, "bands_of_32"), (512, 14336, 4096, 2, "bands_of_32"), (512, 7680, 4096, 2, "grid"), (60, 9216, 4096, 2, "grid"),
+     (512, 11008, 4096, 2, "by_xcd")],
 )
 def test_order_of_the_gate_up_tiles(m, n_ff, k, strips, order):
     p = q8_0.plan_gate_up_silu(m, n_ff, k)
