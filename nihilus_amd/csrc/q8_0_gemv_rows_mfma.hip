@@ -122,7 +122,7 @@ __device__ __forceinline__ void rows8_chunk(const uint8_t* __restrict__ w_strip,
 	}
 }
 
-template<int R, int TILES, bool LOOP>
+template<int R, int TILES, bool LOOP, bool RESIDUAL_AHEAD>
 __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_rows8_kernel(const uint8_t* __restrict__ W, const float* __restrict__ x, int groups, int split_shift, int M, int N, const float* residual, float* y,
 	uint64_t* __restrict__ tagged, unsigned epoch) {
 	constexpr int ROWS8 = R, ROWS8_A_HALF = rows_a_half<R>, ROWS8_A_TILE = rows_a_tile<R>;
@@ -145,11 +145,8 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_rows8_kernel(const uint8
 	}
 	__builtin_amdgcn_wave_barrier();
 
-	// thread 32 * m + l stores output (row m, strip row l).  With the sixteen-row operand its residual (which may be that output) is requested here, a memory latency ahead of its
-	// use, but for a walk of several chunks, which has no register for it.  With the eight-row one behind the reduction: requested here it takes longer (100 random shapes of four
-	// rows 1.029 times as long, [2800 x 3072] 5.03 us for 4.81; of 5 to 8 rows 1.004; of 9 to 16 with the other one 0.994)
-	constexpr bool RESIDUAL_AHEAD = R > 8 && !LOOP;
-	float res					  = 0.0f;
+	// thread 32 * m + l stores output (row m, strip row l); RESIDUAL_AHEAD: its residual (which may be that output) is requested here, a memory latency ahead of its use
+	float res = 0.0f;
 	if constexpr (RESIDUAL_AHEAD) {
 		const int m = tid >> 5, row = strip * STRIP_ROWS + (tid & 31);
 		if (residual && m < M && row < N) {
@@ -201,13 +198,22 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_rows8_kernel(const uint8
 	split_k_finish(tagged, epoch, strip * R + m, splits, split, l, total, ym, row, N, residual != nullptr, res);
 }
 
+// The residual's request goes ahead of the weights where every wave has the same share of K, or sixteen operand rows.  With eight of them and shares that differ it takes longer than
+// behind the reduction, also where there is none: 100 random shapes of four rows 1.028 times as long, [2800 x 3072] 5.02 us for 4.76, [3139 x 2304] with one 4.97 / 4.48, of 5 to 8 rows
+// 1.004; but [4096 x 4096] at 5 rows with one 6.51 / 6.59 and of 9 to 16 rows 0.994.  (A walk of several chunks has no register for it.)
 template<int R, int TILES, bool LOOP> static hipError_t launch_rows8_n(const gemv_plan& p, const uint8_t* W, const float* x, float* y, const float* r, int M, int N, const gemv_scratch& sc, hipStream_t s) {
 	const dim3 grid(static_cast<unsigned>(p.strips * p.splits)), block(GEMV_WAVES * 64);
 	int shift = 0;
 	while ((1 << shift) < p.splits) {
 		++shift;
 	}
-	return launch_kernel(KIND_GEMV, gemv_rows8_kernel<R, TILES, LOOP>, grid, block, 0, s, W, x, p.groups, shift, M, N, r, y, sc.tagged, sc.epoch);
+	const auto launch = [&](auto kernel) { return launch_kernel(KIND_GEMV, kernel, grid, block, 0, s, W, x, p.groups, shift, M, N, r, y, sc.tagged, sc.epoch); };
+	if constexpr (R == 8 && !LOOP) {
+		if (p.groups % (GEMV_WAVES * p.splits) != 0) {
+			return launch(gemv_rows8_kernel<R, TILES, LOOP, false>);
+		}
+	}
+	return launch(gemv_rows8_kernel<R, TILES, LOOP, !LOOP>);
 }
 
 // 1 <= M <= 16 fp32 activation rows [M][K] against a tiled weight [N][K]; y is [M][N].  K % 128 == 0 (checked by the caller).
