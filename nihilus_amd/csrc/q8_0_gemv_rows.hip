@@ -129,6 +129,17 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_rows_kernel(const uint8_
 	wave_k_range(groups, split_shift, split, GEMV_WAVES, wave, g0, g1);
 	const int64_t K	 = static_cast<int64_t>(groups) * GROUP_K;
 
+	// thread 32 * m + l stores output (row m, strip row l); RESIDUAL_AHEAD: its residual (which may be that output) is requested here, a memory latency ahead of its use.  Three rows at
+	// two groups a wave then take 64 registers, two workgroups per CU, where behind the reduction they take 65 ([13415 x 2176] 12 % faster).  Elsewhere it costs the first loads more
+	// than it saves: 80 random shapes 1.005 times as long with two rows, 1.019 with three
+	constexpr bool RESIDUAL_AHEAD = MR == 3 && TILES == 2 && !LOOP;
+	float res					  = 0.0f;
+	if constexpr (RESIDUAL_AHEAD) {
+		const int m = tid >> 5, row = strip * STRIP_ROWS + (tid & 31);
+		if (residual && m < MR && row < N) {
+			res = residual[static_cast<int64_t>(m) * N + row];
+		}
+	}
 	const uint8_t* w_strip = W + macro_offset(strip, 0, groups);
 	float acc[MR];
 #pragma unroll
@@ -159,11 +170,10 @@ __global__ __launch_bounds__(GEMV_WAVES * 64) void gemv_rows_kernel(const uint8_
 	for (int w = 0; w < GEMV_WAVES; ++w) {
 		total += red[m][w][l] + red[m][w][32 + l];
 	}
-	// the residual (which may be the output) is read here.  Requested at the launch's start, a memory latency ahead, it costs the first loads more than it saves: 100
-	// random shapes with one / without take 1.010 / 1.001 times as long with two rows, 1.020 / 1.016 with three
-	float res = 0.0f;
-	if (residual && row < N) {
-		res = residual[static_cast<int64_t>(m) * N + row];
+	if constexpr (!RESIDUAL_AHEAD) {
+		if (residual && row < N) {
+			res = residual[static_cast<int64_t>(m) * N + row];
+		}
 	}
 	float* ym = y + static_cast<int64_t>(m) * N;
 	if (splits == 1) {

@@ -104,3 +104,18 @@ def test_the_line_to_the_quantize_launch(q8, oracle, m, n, k, fused):
     y, want = to_host(q8.mul_mat(wt, to_dev(x), n, k)), _want(oracle, w, x, n, k)
     assert max(rel_l2(y[i], want[i]) for i in range(m)) <= REL_L2_TOL
     assert np.array_equal(to_host(q8.mul_mat(wt, to_dev(x), n, k, residual=to_dev(res))), y + res)
+
+
+# The residual requested ahead of the weights and behind the reduction: shares of K that are the same for every wave and not, K over workgroups and not, a ragged last strip, one and two
+# groups per wave; into a buffer of its own and into the residual's.
+@pytest.mark.parametrize("m", [2, 3, 4, 8, 9])
+@pytest.mark.parametrize("n,k", [(2800, 3072), (1000, 2304), (1024, 4096), (4096, 2048), (8200, 2048), (8200, 2176), (96, 128)])
+def test_residual_in_place(q8, m, n, k):
+    wt = q8.tile(q8.fill_weight_blocks(m + n, n, k), n, k)
+    x, res = q8.fill_activations(k, m * k).reshape(m, k), q8.fill_activations(n, m * n).reshape(m, n)
+    plain = to_host(q8.mul_mat(wt, x, n, k))
+    assert np.array_equal(to_host(q8.mul_mat(wt, x, n, k, residual=res)), plain + to_host(res))
+    want, lib = plain + to_host(res), q8._lib.lib()
+    ws = torch.empty(max(1, lib.nh_q8_0_mul_mat_workspace_bytes(m, k)), dtype=torch.uint8, device="cuda")
+    status = lib.nh_q8_0_mul_mat_scratch(wt.data_ptr(), x.data_ptr(), res.data_ptr(), res.data_ptr(), m, n, k, ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream)
+    assert status == 0 and np.array_equal(to_host(res), want)
