@@ -1,5 +1,5 @@
 // Which kernel a mul_mat call runs, and how that kernel cuts the work: decided here, on the host, in one place, from the
-// shape alone.  The launchers execute the plan they get from these functions and decide nothing themselves -- but for a call that is being
+// shape alone.  The launchers execute the plan they get from these functions and decide no cut, order or route themselves -- but for a call that is being
 // captured, or finds the hand-off scratch of its form in use on another stream, which runs as the form without it that the plan has
 // for it: in the mat-mats the same additions in the same order -- so a test can
 // ask (nh_q8_0_debug_plan_mul_mat, no GPU needed) what a shape will run and pin it.
