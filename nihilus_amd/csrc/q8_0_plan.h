@@ -131,8 +131,10 @@ inline gemm_tile_cut gemm_tile_mat_mat(gemm_tile_cut c, int groups, int64_t m_st
 	if (c.ks == 2 && groups % 2 != 0 && static_cast<int64_t>(c.grid_x) * c.grid_y > 256 && (c.tm == 1 || groups < 24)) {
 		c.ks = 1;
 	}
-	if (!stream && gemm_tile_take_one_strip(&c, m_strips, ONE_STRIP_MAT_MAT) && c.ks == 1 && groups >= 8 && groups % 2 == 0 && c.grid_x * m_strips <= 1280) {
-		c.ks = 2; // so few of them are less than four waves on a SIMD ([4096 x 4096] at 1100 rows 59.7 / 58.8; at 1600, seven rounds, 80.8 / 83.4)
+	// One set of K into two behind that: up to five rounds of them are less than four waves on a SIMD.  From K = 3072 on and with more than four rounds: 183 random shapes 0.97 to 1.07 times
+	// as fast, mean 1.02 ([4096 x 4096] at 1100 rows 59.7 / 58.8; at 1600, seven rounds, 80.8 / 83.4); shorter 145 of 0.90 to 1.05, mean 0.98 ([13568 x 1024] at 294 0.94), with up to four rounds 32, 0.98.
+	if (!stream && gemm_tile_take_one_strip(&c, m_strips, ONE_STRIP_MAT_MAT) && c.ks == 1 && groups >= 24 && groups % 2 == 0 && c.grid_x * m_strips > 1024 && c.grid_x * m_strips <= 1280) {
+		c.ks = 2;
 	}
 	return c;
 }

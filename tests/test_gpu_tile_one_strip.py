@@ -7,12 +7,12 @@ from helpers import REL_L2_TOL, rel_l2, to_dev, to_host
 pytestmark = pytest.mark.gpu
 
 
-# Both sides of the lines: workgroups of two strips just over one round and two, of one strip up to three and five; three strips, four and five; a last strip of one row, ragged
+# Both sides of the lines: workgroups of two strips just over one round and two, of one strip up to three and five (with two sets of K there, from 24 groups and above four rounds on); three strips, four and five; a last strip of one row, ragged
 # columns, a number of column blocks that eight divides and others; one K set and two, even and uneven.
 @pytest.mark.parametrize(
     "m,n,k,cut",
     [(161, 11008, 1024, (1, 2)), (161, 10960, 128 * 9, (1, 1)), (192, 16384, 512, (1, 1)), (192, 16385, 512, (2, 1)), (129, 12000, 1024, (1, 2)), (128, 24576, 512, (2, 1)), (1000, 2900, 1024, (1, 2)),
-     (161, 21860, 1024, (1, 2)), (161, 21888, 128 * 9, (1, 1)), (180, 21760, 512, (2, 1)), (256, 20480, 1024, (1, 2)), (256, 20481, 1024, (2, 1)), (96, 21760, 512, (1, 1)), (65, 16500, 1024, (1, 2)), (160, 12000, 128 * 25, (1, 2))],
+     (161, 21860, 1024, (1, 1)), (161, 21888, 128 * 9, (1, 1)), (161, 21860, 3072, (1, 2)), (161, 21860, 128 * 22, (1, 1)), (200, 18688, 3072, (1, 1)), (200, 18689, 3072, (1, 2)), (180, 21760, 512, (2, 1)), (256, 20480, 1024, (1, 1)), (256, 20480, 3072, (1, 2)), (256, 20481, 1024, (2, 1)), (96, 21760, 512, (1, 1)), (65, 16500, 1024, (1, 2)), (160, 12000, 128 * 25, (1, 2))],
 )
 def test_one_strip_per_wave(q8, oracle, m, n, k, cut):
     p = q8.plan_mul_mat(m, n, k)
